@@ -25,7 +25,7 @@ import torch
 
 from . import codegen, library, verify
 from .configs import supported_configs
-from .gfx950_space import NoValidConfigError
+from .gfx950_space import MIN_LENGTH, NoValidConfigError
 
 _PKG = os.path.normpath(os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))
 DEFAULT_CACHE_DIR = os.environ.get("AAT_CACHE_DIR", os.path.join(_PKG, "cache"))
@@ -89,7 +89,8 @@ class BaseTunner:
             return self.validate_shared_fuse(config)
         return self.validate_kernel(config)
 
-    def _fits_problem(self, config):
+    def _fits_problem(self, config, whole_tiles=False):
+        """Whether ``config``'s library takes this problem.  ``whole_tiles``: only if its tiles divide the lengths."""
         s = self.problem_shape
         ns = getattr(config, "kv_splits", 1)
         if ns > 1 and (s["Sk"] // config.Bc) % ns:
@@ -97,7 +98,12 @@ class BaseTunner:
         if config.operation in ("ret_bwd", "attn_bwd"):   # both lengths are resident in one pass, streamed in another
             return all(s[n] % config.Br == 0 and s[n] % config.Bc == 0 for n in ("Sq", "Sk")) and \
                 s["Sk"] % getattr(config, "row_Bc", config.Bc) == 0
-        return s["Sq"] % config.Br == 0 and s["Sk"] % config.Bc == 0
+        if s["Sq"] % config.Br == 0 and s["Sk"] % config.Bc == 0:
+            return True
+        # the register-fused attention forward has a kernel for partial tiles at the end of either length
+        ragged = config.operation == "attn" and config.fuse_type == "register" and getattr(self.arch, "platform", "") == "ROCm"
+        return ragged and not whole_tiles and config.Br <= s["Sq"] and config.Bc <= s["Sk"] and \
+            s["Sq"] % MIN_LENGTH == 0 and s["Sk"] % MIN_LENGTH == 0
 
     def get_tuned_configs(self):
         dq, dv = self.problem_key["dim_qk"], self.problem_key["dim_v"]
@@ -201,7 +207,7 @@ class BaseTunner:
 
     nearest_limit = 12.0       # e.g. one length and the row count a factor 16 apart
 
-    def nearest_cached(self):
+    def nearest_cached(self, limit=None):
         """The tuned configuration of the closest problem this cache holds for the same operator, head sizes and mask
         walk whose tiles also divide this problem's lengths, or None.  For callers that do not want a tuning run on a
         miss: the reference keys its cache by the two head sizes alone (python/autotuner/base_tunner.py:190-208), i.e. it always launches
@@ -224,7 +230,7 @@ class BaseTunner:
             b, h, sq, sk = (int(x) for x in m.groups())
             far = 2 * abs(math.log2(sq / s["Sq"])) + 2 * abs(math.log2(sk / s["Sk"])) + \
                 abs(math.log2((b * h * sq) / (s["B"] * s["H"] * s["Sq"])))
-            if far <= self.nearest_limit:
+            if far <= (self.nearest_limit if limit is None else limit):
                 found.append((far, name))
         for _, name in sorted(found):
             try:
@@ -233,7 +239,7 @@ class BaseTunner:
                 cfg = supported_configs[dd["operation"]].from_dict(dd)
             except (OSError, ValueError, KeyError):
                 continue
-            if self._fits_problem(cfg):
+            if self._fits_problem(cfg, whole_tiles=True):
                 _memo[self._memo_key()] = cfg             # this process keeps launching it for this problem
                 return cfg
         return None

@@ -6,6 +6,8 @@ whole-tile buffers; and the register file is split between the resident waves of
 occupancy target (``waves_per_eu``) is itself a knob.  Validity is LDS bytes (160 KB per CU, shared by
 all resident blocks) and a per-lane register estimate (512 / waves_per_eu).
 """
+import math
+
 from .configs import AttnConfig, RetConfig, RetBwdConfig, AttnBwdConfig
 
 
@@ -222,6 +224,69 @@ def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None):
         if forward_valid(cfg, arch):
             return cfg
     raise NoValidConfigError(f"no default {op} configuration fits dim_qk={dim_qk} dim_v={dim_v} seq=({seq_q},{seq_k})")
+
+
+# ---- attention forward without a tuned entry -----------------------------------------------------------
+# Tile shapes the rule below chooses from, per pair of head sizes: (Br, Bc, unit rows, K buffers, V buffers, threads,
+# waves per SIMD).  Of 38 shapes timed on 26 problems (64 ... 16384 rows, ragged lengths, 1 ... 32 kv parts) these are the ones
+# without which some problem loses: with one of them at hand a problem is on the mean 4 % (d 64, 128, 192) to 6 % (d 256)
+# slower than with the best of the 38.
+RULE_SHAPES = {
+    (64, 64): ((128, 64, 64, 2, 2, 256, 3), (256, 64, 64, 2, 1, 256, 2)),
+    (128, 128): ((128, 64, 64, 2, 2, 256, 2), (256, 64, 64, 2, 2, 512, 2), (256, 64, 32, 2, 2, 256, 2), (512, 128, 32, 2, 2, 512, 2)),
+    (192, 192): ((128, 32, 32, 2, 2, 256, 2), (256, 64, 64, 2, 2, 512, 2)),
+    (256, 256): ((64, 64, 64, 1, 1, 128, 1), (128, 32, 32, 2, 1, 256, 2), (256, 32, 32, 2, 2, 512, 2)),
+}
+MIN_LENGTH = 32               # the register-fused attention forward takes any lengths that are multiples of this
+
+
+def rule_configs(dim_qk, dim_v):
+    return [AttnConfig(br, bc, dim_qk, dim_v, dim_qk, unit, nk, nv, nt, True, waves_per_eu=wpe).set_fuse_type("register")
+            for br, bc, unit, nk, nv, nt, wpe in RULE_SHAPES.get((dim_qk, dim_v), ())]
+
+
+def forward_estimate_us(cfg, arch, b, h, seq_q, seq_k, causal, parts):
+    """Time of one attention forward launch; the same estimate the library takes to cut the kv range into parts
+    (csrc/kernels/attention/regfuse/kv_parts.h says where it comes from)."""
+    waves = _waves(cfg)
+    lds = cfg.Bc * (cfg.num_stages_qk * cfg.Kd + cfg.num_stages_v * cfg.D) * 2
+    per_block = max(1, min(cfg.waves_per_eu * 4 // waves, 160 * 1024 // lds))
+    single = (cfg.num_stages_qk == 1) + (cfg.num_stages_v == 1)
+    tile = cfg.Br * cfg.Bc * 2.0 * (cfg.Kd + cfg.D) / 4.5e6 * (1.0 + 17.0 / cfg.D)
+    alone = 4.55 / waves * tile
+    shared = (0.72 if cfg.Br >= 512 else 0.77 if cfg.Br >= 256 else 0.87 if cfg.Br >= 128 else 1.25) * (1.0 + 0.034 * single) * tile
+    start = 0.7 + 2.6e-5 * cfg.Br * (cfg.Kd + cfg.D)
+    row_blocks = -(-seq_q // cfg.Br)
+    tiles = -(-(-(-seq_k // cfg.Bc)) // parts)
+    per_cu = b * h * row_blocks * parts / arch.compute_max_core
+    us = start + tiles * alone
+    if per_cu > 1.0:
+        triangle = causal and seq_q == seq_k
+        walked = (row_blocks + 1) / (2.0 * row_blocks) if triangle else 1.0
+        queue = math.ceil(per_cu) if per_cu < 3.0 else per_cu + (0.3 if triangle else 0.6)
+        rounds = math.ceil(queue / per_block) if per_cu < 3.0 * per_block else queue / per_block
+        us = max(us if triangle else rounds * us, start + queue * walked * tiles * shared)
+    if parts > 1:
+        us += 4.0 + 1.6e-6 * parts * b * h * seq_q * cfg.D
+    return us
+
+
+def kv_parts(cfg, arch, b, h, seq_q, seq_k, causal):
+    """Into how many parts the library of ``cfg`` cuts the kv range of a problem."""
+    if cfg.kv_splits > 1:
+        return 1 if causal else cfg.kv_splits
+    if seq_k < 1024 or b * h * -(-seq_q // cfg.Br) >= 2 * arch.compute_max_core:
+        return 1
+    return min(range(1, min(64, seq_k // 256) + 1), key=lambda p: forward_estimate_us(cfg, arch, b, h, seq_q, seq_k, causal, p))
+
+
+def rule_forward_config(dim_qk, dim_v, arch, b, h, seq_q, seq_k, causal):
+    """The tile shape for an attention forward problem nobody tuned, or None (head sizes or lengths the rule does not
+    cover): the one of RULE_SHAPES with the smallest estimate at the kv parts its library will take."""
+    if seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
+        return None
+    return min(rule_configs(dim_qk, dim_v), default=None,
+               key=lambda c: forward_estimate_us(c, arch, b, h, seq_q, seq_k, causal, kv_parts(c, arch, b, h, seq_q, seq_k, causal)))
 
 
 # ---- backward (RetNet) ---------------------------------------------------------------------------------

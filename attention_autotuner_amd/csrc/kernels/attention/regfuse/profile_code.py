@@ -9,6 +9,7 @@ global_vars = r"""
 #define AAT_OP_ATTN 1
 #include <atomic>
 #include "aat_kernel_abi.h"
+#include "kernels/attention/regfuse/kv_parts.h"
 #include "kernels/attention/regfuse/regfuse.h"
 #include "kernels/utils/host_launch.h"
 
@@ -21,17 +22,19 @@ constexpr int Nthreads = {Nthreads};
 constexpr int num_stages_qk = {num_stages_qk};   // LDS buffers for the K tile
 constexpr int num_stages_v = {num_stages_v};     // LDS buffers for the V tile
 constexpr int waves_per_eu = {waves_per_eu};
-constexpr int kv_splits = {kv_splits};           // > 1: the kv range is cut into that many parts (non-causal only)
+constexpr int kv_splits = {kv_splits};           // > 1: a non-causal problem's kv range is cut into that many parts, a causal one's not; 1: as many as pay (kv_parts.h)
 constexpr bool sw_pipeline = {sw_pipeline};      // next tile's QK^T MFMAs interleaved with this tile's exponentials
 constexpr int unit_rows = sw_pipeline ? Bc : {BlockKSmem2};   // plain schedule: kv rows per scores -> softmax -> PV unit inside a tile of Bc rows
 constexpr float kReferenceScale = 0.125f;        // what the reference kernels hard-code
 
 using Traits = aat::AttnFwdRegfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v>;
 constexpr int shared_mem = Traits::kSmemBytes;
-const auto kernel = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, sw_pipeline, false>;
-const auto kernel_causal = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, sw_pipeline, true>;
-const auto kernel_causal_paired = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, sw_pipeline, true, false, false, true>;
-const auto kernel_split = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, sw_pipeline, false, true>;
+const auto kernel = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, sw_pipeline, false>;
+const auto kernel_causal = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, sw_pipeline, true>;
+const auto kernel_causal_paired = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, sw_pipeline, true, false, false, true>;
+// any lengths that are multiples of 32, causal or not; and the same with the kv range cut into parts
+const auto kernel_gen = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, false, true>;
+const auto kernel_split = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, false, true, true>;
 constexpr int shared_mem_split = Traits::kSmemBytesSplit;
 
 // Persistent variant (a block walks several row blocks, prefetching across them): exists for two K and two V
@@ -46,7 +49,7 @@ using PersistTraits = Traits::Persist<waves_per_eu>;
 constexpr int shared_mem_persist = PersistTraits::kSmemBytes;
 template <bool OK> auto persistent_kernel() {{
   if constexpr (OK)
-    return &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, false, false, false, true>;
+    return &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, false, false, false, true>;
   else
     return static_cast<decltype(kernel)>(nullptr);
 }}
@@ -100,25 +103,47 @@ bool pairs_fill_the_chip(int n) {{
   return n % resident == 0 || n >= 8 * resident;
 }}
 
-size_t split_workspace_bytes(int B, int H, int Seq_q) {{
-  return kv_splits > 1 ? (size_t)kv_splits * B * H * Seq_q * (D + 1) * sizeof(float) : 0;
+bool lengths_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, 32); }}
+bool whole_tiles(int Seq_q, int Seq_k) {{ return Seq_q % Br == 0 && Seq_k % Bc == 0; }}
+int row_blocks(int Seq_q) {{ return (Seq_q + Br - 1) / Br; }}
+
+constexpr aat::ForwardShape kShape = {{Br, Bc, Kd, D, Nthreads / 64, aat::forward_blocks_per_cu(Nthreads / 64, waves_per_eu, shared_mem_split),
+                                      (num_stages_qk == 1) + (num_stages_v == 1)}};
+int kv_parts(int B, int H, int Seq_q, int Seq_k, int causal) {{
+  if (kv_splits > 1) return causal ? 1 : kv_splits;
+  return aat::choose_kv_parts(kShape, B, H, Seq_q, Seq_k, causal);
 }}
-bool split_applies(int Seq_k, int causal) {{ return kv_splits > 1 && !causal && (Seq_k / Bc) % kv_splits == 0; }}
+size_t split_workspace_bytes(int parts, int B, int H, int Seq_q) {{
+  return parts > 1 ? (size_t)parts * B * H * Seq_q * (D + 1) * sizeof(float) : 0;
+}}
+size_t needed_workspace(int B, int H, int Seq_q, int Seq_k, int causal) {{
+  return split_workspace_bytes(kv_parts(B, H, Seq_q, Seq_k, causal), B, H, Seq_q);
+}}
 
 hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
-                  float softmax_scale, int causal, void* workspace, hipStream_t stream, float* lse = nullptr) {{
-  if (split_applies(Seq_k, causal) && workspace != nullptr) {{
+                  float softmax_scale, int causal, void* workspace, size_t workspace_bytes, hipStream_t stream, float* lse = nullptr) {{
+  const int parts = kv_parts(B, H, Seq_q, Seq_k, causal);
+  if (parts > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(parts, B, H, Seq_q)) {{
     static const hipError_t lds_ok_split = aat::allow_lds(kernel_split, shared_mem_split);
     if (lds_ok_split != hipSuccess) return lds_ok_split;
     const size_t rows = (size_t)B * H * Seq_q;
     float* part_o = static_cast<float*>(workspace);
-    float* part_lse = part_o + (size_t)kv_splits * rows * D;
-    kernel_split<<<dim3(B * H * (Seq_q / Br), kv_splits), dim3(Nthreads), shared_mem_split, stream>>>(
+    float* part_lse = part_o + (size_t)parts * rows * D;
+    kernel_split<<<dim3(B * H * row_blocks(Seq_q), parts), dim3(Nthreads), shared_mem_split, stream>>>(
         reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
-        reinterpret_cast<const aat::half_t*>(v), nullptr, nullptr, H, Seq_k, Seq_q, softmax_scale, part_o, part_lse, 0);
+        reinterpret_cast<const aat::half_t*>(v), nullptr, nullptr, H, Seq_k, Seq_q, softmax_scale, part_o, part_lse, (int)rows, causal);
     const size_t threads = rows * (D / 8);
     aat::attn_split_merge<D><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream>>>(
-        part_o, part_lse, reinterpret_cast<aat::half_t*>(o), lse, (int)rows, kv_splits);
+        part_o, part_lse, reinterpret_cast<aat::half_t*>(o), lse, (int)rows, parts);
+    return hipGetLastError();
+  }}
+  if (!whole_tiles(Seq_q, Seq_k)) {{
+    static const hipError_t lds_ok_gen = aat::allow_lds(kernel_gen, shared_mem);
+    if (lds_ok_gen != hipSuccess) return lds_ok_gen;
+    kernel_gen<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
+        reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
+        reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<aat::half_t*>(o), lse, H, Seq_k, Seq_q, softmax_scale, nullptr,
+        nullptr, 0, causal);
     return hipGetLastError();
   }}
   const int items = B * H * (Seq_q / Br);
@@ -128,7 +153,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int
       kernel_persist<<<dim3(resident), dim3(Nthreads), shared_mem_persist, stream>>>(
           reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
           reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<aat::half_t*>(o), lse, H, Seq_k, Seq_q,
-          softmax_scale, nullptr, nullptr, items);
+          softmax_scale, nullptr, nullptr, items, 0);
       return hipGetLastError();
     }}
   }}
@@ -145,50 +170,51 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int
   (paired ? kernel_causal_paired : causal ? kernel_causal : kernel)<<<dim3(paired ? items / 2 : items), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<aat::half_t*>(o), lse, H, Seq_k, Seq_q,
-      softmax_scale, nullptr, nullptr, 0);
+      softmax_scale, nullptr, nullptr, 0, causal);
   return hipGetLastError();
 }}
 }}  // namespace
 
 extern "C" int abi_version(void) {{ return AAT_ABI_VERSION; }}
 extern "C" const char* config_string(void) {{ return "{config_name}"; }}
-extern "C" size_t workspace_size(int B, int H, int Seq_q, int) {{ return split_workspace_bytes(B, H, Seq_q); }}
+extern "C" size_t workspace_size(int B, int H, int Seq_q, int Seq_k) {{   // room for either kind of call
+  const size_t full = needed_workspace(B, H, Seq_q, Seq_k, 0), causal = needed_workspace(B, H, Seq_q, Seq_k, 1);
+  return full > causal ? full : causal;
+}}
 """
 
 profile_func = r"""
 extern "C" float profile_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
                             float softmax_scale, int causal, void* workspace, size_t workspace_bytes, void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return -1.f;
-  if (split_applies(Seq_k, causal) && (workspace == nullptr || workspace_bytes < split_workspace_bytes(B, H, Seq_q))) return -1.f;
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;
+  if (kv_splits > 1 && (workspace == nullptr ? 0 : workspace_bytes) < needed_workspace(B, H, Seq_q, Seq_k, causal)) return -1.f;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return aat::timed_mean_ms(s, [&] {{ return launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, s); }});
+  return aat::timed_mean_ms(s, [&] {{ return launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, workspace_bytes, s); }});
 }}
 // The reference signature has no workspace argument: a kv-splitting configuration runs unsplit here.
 extern "C" float profile(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return -1.f;
-  return aat::timed_mean_ms(nullptr, [&] {{ return launch(q, k, v, o, B, H, Seq_q, Seq_k, kReferenceScale, 0, nullptr, nullptr); }});
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;
+  return aat::timed_mean_ms(nullptr, [&] {{ return launch(q, k, v, o, B, H, Seq_q, Seq_k, kReferenceScale, 0, nullptr, 0, nullptr); }});
 }}
 """
 
 kernel_entry = r"""
 extern "C" int kernel_entry_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
                                float softmax_scale, int causal, void* workspace, size_t workspace_bytes, void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return AAT_ERR_SHAPE;
-  if (split_applies(Seq_k, causal) && (workspace == nullptr || workspace_bytes < split_workspace_bytes(B, H, Seq_q)))
-    return AAT_ERR_WORKSPACE;
-  return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, static_cast<hipStream_t>(stream));
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
+  if (kv_splits > 1 && (workspace == nullptr ? 0 : workspace_bytes) < needed_workspace(B, H, Seq_q, Seq_k, causal)) return AAT_ERR_WORKSPACE;
+  return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }}
 extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_k, int Seq_q) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return AAT_ERR_SHAPE;
-  return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, kReferenceScale, 0, nullptr, nullptr);
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
+  return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, kReferenceScale, 0, nullptr, 0, nullptr);
 }}
 extern "C" int kernel_entry_lse(aat_half* q, aat_half* k, aat_half* v, aat_half* o, float* lse, int B, int H, int Seq_q,
                                 int Seq_k, float softmax_scale, int causal, void* workspace, size_t workspace_bytes,
                                 void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return AAT_ERR_SHAPE;
-  if (split_applies(Seq_k, causal) && (workspace == nullptr || workspace_bytes < split_workspace_bytes(B, H, Seq_q)))
-    return AAT_ERR_WORKSPACE;
-  return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, static_cast<hipStream_t>(stream), lse);
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
+  if (kv_splits > 1 && (workspace == nullptr ? 0 : workspace_bytes) < needed_workspace(B, H, Seq_q, Seq_k, causal)) return AAT_ERR_WORKSPACE;
+  return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, workspace_bytes, static_cast<hipStream_t>(stream), lse);
 }}
 """
 

@@ -113,10 +113,21 @@ template <bool CAUSAL, class F> AAT_DEV void run_tiles(F& tile, int n_full, int 
 // compile-time switch so that the non-causal kernel carries no masking code at all; in the causal
 // kernel the tiles the diagonal cannot touch still run the unmasked tile body.
 //
-// SPLIT: the kv range is cut into gridDim.y equal parts (few query rows, long kv: not enough row
+// SPLIT: the kv range of every row block is cut into gridDim.y parts (few query rows, long kv: not enough row
 // blocks to fill the chip).  Part s handles kv tiles [s, s+1) * n_tiles / parts and writes its own
 // normalised output (fp32) and log-sum-exp to part_o / part_lse, laid out [part][B*H*S_q][D] and
-// [part][B*H*S_q]; attn_split_merge combines them.  o and lse are not touched.
+// [part][B*H*S_q]; attn_split_merge combines them.  o and lse are not touched.  n_items = B*H*S_q.
+//
+// GEN: any lengths that are multiples of 32, causal or not as `causal` says, one kernel.  The last row block of a head may
+// be partial: its missing 32-row groups load rows of the block that exist, compute nothing (a wave that owns none that
+// exist) or something nobody reads, and are not stored.  The last kv tile may be partial: the missing rows are copies of
+// rows that exist (TileDma::issue_rows) and their scores are masked like those above the diagonal -- the causal walk
+// does that by itself, because the last row that exists sees up to kv row seq_k - 1, and a non-causal walk is a causal one
+// in which every row sees that far.
+// What it replaces at such lengths is the one tile shape that divides them, 64 x 32 on two waves with one buffer: batch 3,
+// 12 heads, 1088 rows, d 128, causal 44 -> 29 us with 128 x 64 tiles; 8 x 12 x 1984 rows 195 -> 118 us; d 64, 4 x 8 x 3392 rows
+// 271 -> 117 us.  The waste is the missing groups of one row block per head and the missing rows of one kv tile; matrix work
+// bounds it as it does the other forms.  With SPLIT, 3 x 12 x 192 queries on 4160 keys: 110 -> 32 us (2.5 TB/s of K and V).
 //
 // PERSIST: the grid is as many blocks as the chip holds at once and block b works through row blocks
 // b, b + gridDim.x, ... of the n_items = B*H*S_q/Br there are.  A block that is alone on its CU otherwise
@@ -128,13 +139,13 @@ template <bool CAUSAL, class F> AAT_DEV void run_tiles(F& tile, int n_full, int 
 // the copies only: memory operations complete in order, so "at most as many outstanding as stores were issued
 // after them" leaves the stores in flight.  Needs two K and two V buffers and an even number of kv tiles (the
 // buffer parity must wrap); plain schedule, non-causal, unsplit.
-template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int WPE = 1, int BU = Bc, bool PIPE = false,
-          bool CAUSAL = false, bool SPLIT = false, bool PERSIST = false, bool PAIR = false>
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int WPE = 1, int BU = Bc, int GEN = 0,
+          bool PIPE = false, bool CAUSAL = false, bool SPLIT = false, bool PERSIST = false, bool PAIR = false>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k,
                       const half_t* __restrict__ v, half_t* __restrict__ o, float* __restrict__ lse,
                       int H, int seq_k, int seq_q, float softmax_scale, float* __restrict__ part_o = nullptr,
-                      float* __restrict__ part_lse = nullptr, int n_items = 0) {
+                      float* __restrict__ part_lse = nullptr, int n_items = 0, int causal = 1) {
   using T = AttnFwdRegfuse<Kd, D, Br, Bc, Nthreads, NSK, NSV>;
   constexpr int RT = T::RT, NT = T::NT, KS = T::KS, DT = T::DT, NCK = T::NCK, NCV = T::NCV, WM = T::WM, NW = T::NW;
   constexpr int PF = AAT_PF;                     // operand prefetch distance, in MFMA steps
@@ -154,7 +165,8 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
   // does not runs the contractions for the late group alone.
   constexpr bool ILV = CAUSAL && RT == 2 && !PIPE && NSK == 2 && NSV == 2;
   static_assert(!PIPE || T::kPipeOk, "the pipelined schedule needs 2+2 buffers and unit-aligned K copies");
-  static_assert(!(SPLIT && CAUSAL), "kv splitting is for non-causal problems");
+  static_assert(!GEN || (CAUSAL && !PIPE && !PERSIST && !PAIR), "the general kernel is a form of the causal plain schedule");
+  static_assert(!SPLIT || GEN, "kv splitting is part of the general kernel");
   using TP = typename T::template Persist<WPE>;
   static_assert(!PERSIST || (!PIPE && !CAUSAL && !SPLIT && TP::kOk), "persistent blocks: plain schedule, 2+2 buffers, room to stage the output");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -166,7 +178,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
-  const int Tr = seq_q / Br;
+  const int Tr = GEN ? (seq_q + Br - 1) / Br : seq_q / Br;
   TileDma<Bc, NCK, Nthreads, Swz::Rows16, 0, XA> kdma;
   TileDma<Bc, NCV, Nthreads, Swz::Rows4, 0, XA> vdma;
   kdma.init(tid);
@@ -186,7 +198,9 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
   }
 
   const float c2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, softmax_scale * kLog2e)));   // wave-uniform: a scalar register
-  const int diag = seq_k - seq_q;               // kv index allowed for query i is <= i + diag
+  // kv index allowed for query i is <= i * slope + diag
+  const int slope = GEN ? causal : 1;
+  const int diag = !GEN || causal ? seq_k - seq_q : seq_k - 1;
 
   // One pass per row block: a single one unless PERSIST -- or PAIR (a variant of the causal kernel): then the grid is half
   // the row blocks and block p of a head walks row block Tr-1-p and then row block p.  The two lengths add up to the same
@@ -211,31 +225,43 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
       }
     }
     const int q0 = rb * Br;
-    int n_tiles = seq_k / Bc;
+    int n_tiles = GEN ? (seq_k + Bc - 1) / Bc : seq_k / Bc;
     int n_full = n_tiles;                         // tiles [0, n_full) are visible to every row of the block
     if constexpr (CAUSAL) {
-      const int last = q0 + Br - 1 + diag;        // last visible kv index for this block
+      const int last = (GEN && q0 + Br > seq_q ? seq_q - 1 : q0 + Br - 1) * slope + diag;   // last visible kv index for this block
       const int lim = last < 0 ? 0 : last / Bc + 1;
       n_tiles = lim < n_tiles ? lim : n_tiles;
-      const int full = (q0 + diag + 1) / Bc;
+      const int full = (q0 * slope + diag + 1) / Bc;
       n_full = full < 0 ? 0 : (full < n_tiles ? full : n_tiles);
-      n_full &= ~1;                               // keep the masked loop on an even tile: buffer parity 0
     }
-
     int tile0 = 0;                                // first kv tile of this block's range
     if constexpr (SPLIT) {
-      const int per = n_tiles / (int)gridDim.y;   // the launcher guarantees divisibility
-      tile0 = (int)blockIdx.y * per;
-      n_tiles = per;
-      n_full = per;
+      tile0 = (int)((int64_t)n_tiles * blockIdx.y / gridDim.y);
+      n_tiles = (int)((int64_t)n_tiles * (blockIdx.y + 1) / gridDim.y) - tile0;
+      n_full = n_full > tile0 ? n_full - tile0 : 0;
+      n_full = n_full < n_tiles ? n_full : n_tiles;
     }
+    if constexpr (CAUSAL) n_full &= ~1;           // keep the masked loop on an even tile: buffer parity 0
+    const int kv_first = SPLIT ? tile0 * Bc : 0;  // first kv row of the range
     const char* kg = reinterpret_cast<const char*>(k + ((size_t)bh * seq_k + (size_t)tile0 * Bc) * Kd);
     const char* vg = reinterpret_cast<const char*>(v + ((size_t)bh * seq_k + (size_t)tile0 * Bc) * D);
 
     // first row of the wave's first 32-row group inside the block, and the distance to its second group
     const int wrow0 = ILV ? 32 * wave : wave * WM;
     const int group_rows = ILV ? 32 * (2 * NW - 1 - 2 * wave) : 32;
-    if (!prefetched) load_q_frags<RT, KS, Kd>(qf, q + ((size_t)bh * seq_q + q0 + wrow0 + n) * Kd + 8 * h, group_rows);
+    int groups = RT;                              // 32-row groups of this wave that exist (its first ones)
+    if constexpr (GEN) {
+      groups = 0;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) groups += q0 + wrow0 + rt * group_rows < seq_q ? 1 : 0;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {           // one that does not exist loads rows that do
+        const int row = rt < groups ? wrow0 + rt * group_rows : groups > 0 ? wrow0 : 0;
+        load_q_frags<1, KS, Kd>(reinterpret_cast<h8(&)[1][KS]>(qf[rt]), q + ((size_t)bh * seq_q + q0 + row + n) * Kd + 8 * h);
+      }
+    } else if (!prefetched) {
+      load_q_frags<RT, KS, Kd>(qf, q + ((size_t)bh * seq_q + q0 + wrow0 + n) * Kd + 8 * h, group_rows);
+    }
     // PERSIST: where the next row block of this block starts (tile numbers map to (head, row block) as above)
     const int vb_next = vb + (int)gridDim.x;
     const bool has_next = PERSIST && vb_next < n_items;
@@ -253,13 +279,22 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) oacc[rt][dt] = zero16();
     }
-    const int q_lim0 = q0 + wrow0 + n + diag;       // last kv index row n of row group 0 may see
+    const int q_lim0 = (q0 + wrow0 + n) * slope + diag;       // last kv index row n of row group 0 may see
+    const int group_lim = group_rows * slope;                 // ... and how much further the next row group sees
+    auto issue_k = [&](int j, char* dst) {
+      if constexpr (GEN) kdma.issue_rows(kg + (size_t)j * T::kKBytes, dst, wave_base, seq_k - kv_first - j * Bc);
+      else kdma.issue(kg + (size_t)j * T::kKBytes, dst, wave_base);
+    };
+    auto issue_v = [&](int j, char* dst) {
+      if constexpr (GEN) vdma.issue_rows(vg + (size_t)j * T::kVBytes, dst, wave_base, seq_k - kv_first - j * Bc);
+      else vdma.issue(vg + (size_t)j * T::kVBytes, dst, wave_base);
+    };
 
     if constexpr (!PIPE) {
       // ============================ plain schedule =================================================
       if (n_tiles > 0 && !prefetched) {
-        kdma.issue(kg, kbuf, wave_base);
-        if constexpr (NSV == 2) vdma.issue(vg, vbuf, wave_base);
+        issue_k(0, kbuf);
+        if constexpr (NSV == 2) issue_v(0, vbuf);
       }
       if (!prefetched) wait_vmcnt0_visible();        // the Q fragments are in (cdna4.h); tile 0 is waited for next anyway
       // `parity_tag` carries j & 1 as a compile-time value so that every LDS address of the tile is a
@@ -290,10 +325,10 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
           wait_vmcnt<0>();
         }
         block_sync();
-        if constexpr (NSV == 1) vdma.issue(vg + (size_t)j * T::kVBytes, vcur, wave_base);
+        if constexpr (NSV == 1) issue_v(j, vcur);
         if (more) {
-          if constexpr (NSK == 2) kdma.issue(kg + (size_t)(j + 1) * T::kKBytes, kbuf + (PAR ^ 1) * T::kKBytes, wave_base);
-          if constexpr (NSV == 2) vdma.issue(vg + (size_t)(j + 1) * T::kVBytes, vbuf + (PAR ^ 1) * T::kVBytes, wave_base);
+          if constexpr (NSK == 2) issue_k(j + 1, kbuf + (PAR ^ 1) * T::kKBytes);
+          if constexpr (NSV == 2) issue_v(j + 1, vbuf + (PAR ^ 1) * T::kVBytes);
         }
         if constexpr (PERSIST) {
           if (!more && has_next) {                 // tile 0 of the next row block, into the buffers it will look in
@@ -309,16 +344,17 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
         // (causal forward at three waves per SIMD: -1.4 %; nothing at two).
         static_for<NU>([&](auto unit_tag) {
           constexpr int U = decltype(unit_tag)::value;
-          const int kv0 = j * Bc + U * BU;           // first kv row of the unit
+          const int kv0 = kv_first + j * Bc + U * BU;   // first kv row of the unit
           if constexpr (ILV) {
             // One body for both row groups; in a unit the early group no longer sees (and the late one does) its
             // MFMAs, its softmax step and its packing are branched around one by one.
             bool on0 = true, on1 = true;
             if constexpr (MASKED) {
-              const int last_early = q0 + wrow0 + 31 + diag;            // last kv row the early group sees
+              const int last_early = (q0 + wrow0 + 31) * slope + diag;            // last kv row the early group sees
               on0 = kv0 <= last_early;
-              on1 = kv0 <= last_early + group_rows;
+              on1 = kv0 <= last_early + group_lim;
             }
+            if constexpr (GEN) on1 = on1 && groups > 0;
             if (on1) {
               f16v sacc[RT][NTU];
               AAT_SETPRIO(2);
@@ -327,9 +363,9 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
 #pragma unroll
               for (int rt = 0; rt < RT; ++rt) {
                 if (rt != 0 || on0 || !(MASKED && XA)) {
-                  const int q_lim = q_lim0 + rt * group_rows;
+                  const int q_lim = q_lim0 + rt * group_lim;
                   // only the unit the group's own diagonal runs through has anything to mask (wave-uniform)
-                  const bool crosses = MASKED && kv0 + BU - 1 > q0 + wrow0 + rt * group_rows + diag;
+                  const bool crosses = MASKED && kv0 + BU - 1 > (q0 + wrow0) * slope + rt * group_lim + diag;
                   if (crosses) causal_mask<NTU>(sacc[rt], kv0, q_lim, h);
                   const float mc = lazy_max_step<NTU, DT>(sacc[rt], m_run[rt], l_run[rt], oacc[rt], c2);
                   exp_tile<NTU, XA>(sacc[rt], c2, mc);
@@ -349,7 +385,8 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
             return;
           }
           bool wave_sees = true;
-          if constexpr (MASKED) wave_sees = kv0 <= q0 + wave * WM + WM - 1 + diag;
+          if constexpr (MASKED) wave_sees = kv0 <= (q0 + wave * WM + WM - 1) * slope + diag;
+          if constexpr (GEN) wave_sees = wave_sees && groups > 0;
 
           f16v sacc[RT][NTU];
           if (wave_sees) {
@@ -363,10 +400,10 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
           if (wave_sees) {
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
-              if constexpr (MASKED) causal_mask<NTU>(sacc[rt], kv0, q_lim0 + rt * 32, h);
+              if constexpr (MASKED) causal_mask<NTU>(sacc[rt], kv0, q_lim0 + rt * group_lim, h);
               const float mc = lazy_max_step<NTU, DT>(sacc[rt], m_run[rt], l_run[rt], oacc[rt], c2);
               exp_tile<NTU, XA>(sacc[rt], c2, mc);
-              if constexpr (MASKED) zero_masked<NTU>(sacc[rt], kv0, q_lim0 + rt * 32, h);
+              if constexpr (MASKED) zero_masked<NTU>(sacc[rt], kv0, q_lim0 + rt * group_lim, h);
             }
           }
 
@@ -375,7 +412,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
             if constexpr (NSV == 1) wait_vmcnt<0>();
             block_sync();
             if constexpr (NSK == 1) {
-              if (more) kdma.issue(kg + (size_t)(j + 1) * T::kKBytes, kbuf, wave_base);
+              if (more) issue_k(j + 1, kbuf);
             }
           }
           if (wave_sees) {
@@ -491,21 +528,21 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
       const size_t row = (size_t)bh * seq_q + q0 + wrow0 + rt * group_rows + n;
       const float row_lse = l_tot > 0.f ? m_run[rt] * softmax_scale + __logf(l_tot) : -INFINITY;
       if constexpr (SPLIT) {
-        if (h == 0) part_lse[(size_t)blockIdx.y * gridDim.x * Br + row] = row_lse;   // gridDim.x * Br = B*H*S_q
+        if (h == 0 && rt < groups) part_lse[(size_t)blockIdx.y * n_items + row] = row_lse;
       } else {
-        if (lse != nullptr && h == 0) lse[row] = row_lse;
+        if (lse != nullptr && h == 0 && rt < groups) lse[row] = row_lse;
       }
     }
     if constexpr (SPLIT) {
-      const size_t rows_total = (size_t)gridDim.x * Br;
-      store_o_rows_f32<RT, DT, D>(oacc, inv, part_o + ((size_t)blockIdx.y * rows_total + (size_t)bh * seq_q + q0 + wave * WM) * D, lane);
+      store_o_rows_f32<RT, DT, D>(oacc, inv, part_o + ((size_t)blockIdx.y * n_items + (size_t)bh * seq_q + q0 + wrow0) * D, lane,
+                                  group_rows, groups);
     } else if constexpr (PERSIST) {
       store_o_tile<RT, DT, D, T::kOStride>(oacc, inv, smem + TP::stage_offset(wave),
                                            o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane);
     } else {
       // transposed through LDS for 16-byte coalesced stores
       store_o_tile<RT, DT, D, T::kOStride>(oacc, inv, smem + wave * WM * T::kOStride,
-                                           o + ((size_t)bh * seq_q + q0 + wrow0) * D, lane, group_rows);
+                                           o + ((size_t)bh * seq_q + q0 + wrow0) * D, lane, group_rows, groups);
     }
     if constexpr (PAIR) {
       if (pass == 0) {

@@ -226,6 +226,17 @@ struct TileDma {
 #pragma unroll
     for (int i = I0; i < I1; ++i) issue_one(i, g, lds, wave_base);
   }
+  // The copy of a tile of which only the first `rows` rows exist (a positive multiple of 32; >= ROWS: all of them).  The 64
+  // chunks a wave copies per instruction lie inside one 32-row group, so whether they exist is wave-uniform: the groups
+  // behind the last one that does are filled with copies of group 0 -- finite data no access of which leaves the matrix,
+  // for scores that the caller masks.  32 rows are a multiple of every swizzle's period, so the layout is the same.
+  AAT_DEV void issue_rows(const char* g, char* lds, int wave_base, int rows) const {
+#pragma unroll
+    for (int i = 0; i < kIters; ++i) {
+      const int group = (i * NT + wave_base) / (32 * NC);
+      issue_one(i, 32 * group < rows ? g : g - (size_t)group * 32 * pitch, lds, wave_base);
+    }
+  }
   // Instruction i alone (i must fold to a constant where this is inlined): lets a caller thread the
   // copy of a tile between other instructions one LDS-DMA instruction at a time.
   AAT_DEV void issue_one(int i, const char* g, char* lds, int wave_base) const {

@@ -355,9 +355,10 @@ AAT_DEV void pv_gemm_steps(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const uint
 // transpose through a wave-private LDS staging area and store rows with 16-byte coalesced writes.
 // ostage: wave-private LDS, WM rows of O_STRIDE bytes.  og: global pointer to the wave's first output row.
 // group_rows: rows in global memory from one 32-row group of the wave to the next (32: contiguous).
+// groups: how many of the wave's row groups exist (the others are behind the end of a ragged sequence).
 template <int RT, int DT, int D, int O_STRIDE, class OutT = half_t>
 AAT_DEV void store_o_tile(const f16v (&oacc)[RT][DT], const float (&row_scale)[RT], char* ostage, OutT* og,
-                          int lane, int group_rows = 32) {
+                          int lane, int group_rows = 32, int groups = RT) {
   constexpr int kElem = (int)sizeof(OutT);
   constexpr int kChunksPerRow = D * kElem / 16, WM = RT * 32;
   const int n = lane & 31, h = lane >> 5;
@@ -395,6 +396,7 @@ AAT_DEV void store_o_tile(const f16v (&oacc)[RT][DT], const float (&row_scale)[R
   constexpr int kChunks = WM * kChunksPerRow;
 #pragma unroll
   for (int t = 0; t < kChunks / 64; ++t) {
+    if (t * 64 / (32 * kChunksPerRow) >= groups) break;
     const int idx = t * 64 + lane;
     const int row = idx / kChunksPerRow, c = idx % kChunksPerRow;
     const u4v val = *reinterpret_cast<const u4v*>(ostage + row * O_STRIDE + c * 16);
@@ -407,13 +409,16 @@ AAT_DEV void store_o_tile(const f16v (&oacc)[RT][DT], const float (&row_scale)[R
 // accumulator group, so it stores 16-byte pieces (the two lanes of a row write neighbouring pieces).  Slower per tile
 // than the staged, row-contiguous stores (about twice), which does not matter for the once-per-block partial output of a
 // kv split, and it needs no LDS: a split block then occupies what its K/V buffers take and nothing more.
+// group_rows, groups: as in store_o_tile.
 template <int RT, int DT, int D>
-AAT_DEV void store_o_rows_f32(const f16v (&oacc)[RT][DT], const float (&row_scale)[RT], float* og, int lane) {
+AAT_DEV void store_o_rows_f32(const f16v (&oacc)[RT][DT], const float (&row_scale)[RT], float* og, int lane,
+                              int group_rows = 32, int groups = RT) {
   const int n = lane & 31, h = lane >> 5;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
+    if (rt >= groups) break;
     const float sc = row_scale[rt];
-    float* row = og + (size_t)(rt * 32 + n) * D + 4 * h;
+    float* row = og + (size_t)(rt * group_rows + n) * D + 4 * h;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       f16v blk = oacc[rt][dt];

@@ -43,7 +43,8 @@ class MultiHeadAttnFunc(torch.autograd.Function):
         causal = bool(causal)
         _, rt = planned(("attn", device_type.name, batch_size, nheads, seqlen_q, seqlen_k, key_dim, head_dim, causal),
                         lambda: AttnTunner(arch=device_type, torch_array=[q, k, v, o], causal=causal, softmax_scale=softmax_scale),
-                        lambda: gfx950_space.default_forward_config("attn", key_dim, head_dim, device_type, seqlen_q, seqlen_k))
+                        lambda: gfx950_space.default_forward_config("attn", key_dim, head_dim, device_type, seqlen_q, seqlen_k),
+                        lambda: gfx950_space.rule_forward_config(key_dim, head_dim, device_type, batch_size, nheads, seqlen_q, seqlen_k, causal))
         needs_grad = any(ctx.needs_input_grad[:3])
         lse = torch.empty(batch_size, nheads, seqlen_q, device=q.device, dtype=torch.float32) if needs_grad else None
         rt.apply([q, k, v, o], softmax_scale=softmax_scale, causal=causal, lse=lse)

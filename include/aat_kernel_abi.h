@@ -13,7 +13,8 @@
  *   - q [B,H,Seq_q,Kd], k [B,H,Seq_k,Kd], v [B,H,Seq_k,D], o/dO [B,H,Seq_q,D] are IEEE fp16;
  *     mask [H,Seq_q,Seq_k] fp16; r [B,H,Seq_q] fp32; dqaccum [B,H,Seq_q,Kd] fp32, zero on entry;
  *   - Kd, D and the tile shape are baked into the library (see config_string());
- *   - Seq_q must be a multiple of the library's Br and Seq_k of its Bc;
+ *   - Seq_q must be a multiple of the library's Br and Seq_k of its Bc; the register-fused attention forward takes any
+ *     lengths that are multiples of 32;
  *   - `profile*` launches the kernel repeatedly (one probe launch, then ceil(100 ms / t) launches) and
  *     returns the mean time of one launch in milliseconds, or -1 on any error;
  *   - `kernel_entry*` enqueues one launch and returns without synchronising.
@@ -25,8 +26,9 @@
  *     a positive hipError_t on a launch failure, AAT_ERR_SHAPE for an indivisible shape;
  *   - the *_ex entry points take (Seq_q, Seq_k) in that order plus a runtime softmax scale, a causal
  *     flag, an optional workspace and the stream to launch on (a hipStream_t passed as void*);
- *   - workspace_size() says how many bytes of workspace a problem needs (attention forward: 0 unless the
- *     configuration splits the kv range; RetNet: the mask scan of AAT_MASK_SCAN, not needed by the other
+ *   - workspace_size() says how many bytes of workspace a problem needs (attention forward: 0 unless the kv
+ *     range is worth cutting into parts, and then optional: without it the call runs in one part, except in a
+ *     configuration with a fixed number of parts; RetNet: the mask scan of AAT_MASK_SCAN, not needed by the other
  *     mask modes, and for a backward built with a stored dS the optional room for it); abi_version() and
  *     config_string() identify the library.
  */

@@ -1,0 +1,72 @@
+"""Attention forward at lengths its tiles do not divide and over kv ranges cut into parts: the edges of tiles, against the
+oracle (the forward's own bound, 2e-3 where |ref| < 4)."""
+import math
+
+import pytest
+import torch
+
+import attention_autotuner_amd as aat
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from oracle import ref_op, tolerance
+
+pytestmark = pytest.mark.gpu
+ARCH = aat.MI355X()
+
+# (B, H, Sq, Sk): one 32-row group, a partial first tile, one row group over a tile, one short of it, more queries than keys,
+# kv ranges that are cut (1024 rows and more on few row blocks), parts that see nothing under the causal mask
+SHAPES = [(1, 2, 32, 32), (2, 3, 96, 160), (1, 2, 288, 288), (1, 3, 480, 544), (1, 2, 544, 96), (1, 1, 64, 1056), (1, 2, 192, 4160), (1, 1, 1088, 1088)]
+PAIRS = sorted(gfx950_space.RULE_SHAPES)
+
+
+def _inputs(b, h, sq, sk, d, seed):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(b, h, s, d, generator=g).half() for s in (sq, sk, sk)]
+
+
+@pytest.mark.parametrize("d", [p[0] for p in PAIRS])
+@pytest.mark.parametrize("causal", [False, True])
+def test_every_rule_shape_at_the_edges_of_its_tiles(d, causal):
+    for i, (b, h, sq, sk) in enumerate(SHAPES):
+        q, k, v = _inputs(b, h, sq, sk, d, 100 + i)
+        want, want_lse = ref_op.attention_ref(q, k, v, None, causal, return_lse=True)
+        qc, kc, vc = (t.cuda() for t in (q, k, v))
+        for cfg in gfx950_space.rule_configs(d, d):
+            print(d, causal, (b, h, sq, sk), cfg, flush=True)
+            o = torch.full((b, h, sq, d), 7.0, dtype=torch.float16, device="cuda")
+            lse = torch.full((b, h, sq), 7.0, device="cuda")
+            Runtime(ARCH, cfg).apply([qc, kc, vc, o], softmax_scale=1 / math.sqrt(d), causal=causal, lse=lse)
+            torch.cuda.synchronize()
+            assert (o.float().cpu() - want).abs().max().item() <= 2e-3
+            seen = torch.isfinite(want_lse)                      # rows that see no key: -inf here, output zero
+            assert torch.equal(torch.isfinite(lse.cpu()), seen)
+            assert (lse.cpu() - want_lse)[seen].abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("b,h,sq,sk,causal", [(3, 5, 1088, 1088, True), (2, 3, 192, 4160, True), (1, 4, 64, 8192, False), (2, 3, 96, 96, False)])
+def test_the_operator_takes_them_and_its_calls_agree(b, h, sq, sk, causal):
+    q, k, v = (t.cuda() for t in _inputs(b, h, sq, sk, 128, 7))
+    o = aat.flash_attn_func(q, k, v, ARCH, causal)
+    assert torch.equal(o, aat.flash_attn_func(q, k, v, ARCH, causal))
+    assert (o.float().cpu() - ref_op.attention_ref(q.cpu(), k.cpu(), v.cpu(), None, causal)).abs().max().item() <= 2e-3
+
+
+def test_a_split_call_replays_from_a_captured_graph():
+    q, k, v = (t.cuda() for t in _inputs(1, 2, 192, 4160, 128, 3))
+    cfg = gfx950_space.rule_forward_config(128, 128, ARCH, 1, 2, 192, 4160, True)
+    assert gfx950_space.kv_parts(cfg, ARCH, 1, 2, 192, 4160, True) > 1
+    rt, o = Runtime(ARCH, cfg), torch.empty_like(q)
+    ws = torch.empty(rt.workspace_size(1, 2, 192, 4160), dtype=torch.uint8, device="cuda")
+    rt.apply([q, k, v, o], causal=True, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rt.apply([q, k, v, o], causal=True, workspace=ws)
+    for seed in (4, 5, 6):
+        for t, new in zip((q, k, v), _inputs(1, 2, 192, 4160, 128, seed)):
+            t.copy_(new)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = torch.empty_like(o)
+        rt.apply([q, k, v, eager], causal=True)
+        torch.cuda.synchronize()
+        assert torch.equal(o, eager)

@@ -420,3 +420,16 @@ def test_an_operator_resolves_a_problem_once_and_again_after_a_tuning_result_is_
     built[0]._write_cache(tuned)
     assert _resolve.planned(key, make, lambda: default)[0] == tuned and len(built) == 2
     base_tunner._memo.clear()
+
+
+def test_the_library_cuts_the_kv_range_as_the_tile_shape_rule_assumes():
+    """gfx950_space.kv_parts and the library's own choice (kv_parts.h) are one estimate, written twice."""
+    for d in (64, 128, 256):
+        for cfg in gfx950_space.rule_configs(d, d):
+            lib = library.load(codegen.compile_config(cfg, ARCH, timeout=600), "attn")
+            for b, h, sq, sk in ((1, 1, 64, 32768), (3, 12, 192, 4160), (1, 32, 256, 16384), (2, 8, 64, 1024), (4, 32, 320, 2560), (1, 4, 1536, 1536), (4, 32, 2048, 2048)):
+                parts = [gfx950_space.kv_parts(cfg, ARCH, b, h, sq, sk, causal) for causal in (False, True)]
+                want = max((p * b * h * sq * (d + 1) * 4 for p in parts if p > 1), default=0)
+                assert lib.workspace_size(b, h, sq, sk) == want, (cfg, b, h, sq, sk, parts)
+    assert gfx950_space.rule_forward_config(128, 128, ARCH, 3, 12, 1088, 1088, True) is not None
+    assert gfx950_space.rule_forward_config(128, 128, ARCH, 1, 1, 128, 80, False) is None       # not whole 32-row groups
