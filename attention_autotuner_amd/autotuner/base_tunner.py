@@ -96,14 +96,16 @@ class BaseTunner:
         if ns > 1 and (s["Sk"] // config.Bc) % ns:
             return False
         if config.operation in ("ret_bwd", "attn_bwd"):   # both lengths are resident in one pass, streamed in another
-            return all(s[n] % config.Br == 0 and s[n] % config.Bc == 0 for n in ("Sq", "Sk")) and \
+            divides = all(s[n] % config.Br == 0 and s[n] % config.Bc == 0 for n in ("Sq", "Sk")) and \
                 s["Sk"] % getattr(config, "row_Bc", config.Bc) == 0
-        if s["Sq"] % config.Br == 0 and s["Sk"] % config.Bc == 0:
-            return True
-        # the register-fused attention forward has a kernel for partial tiles at the end of either length
-        ragged = config.operation == "attn" and config.fuse_type == "register" and getattr(self.arch, "platform", "") == "ROCm"
-        return ragged and not whole_tiles and config.Br <= s["Sq"] and config.Bc <= s["Sk"] and \
-            s["Sq"] % MIN_LENGTH == 0 and s["Sk"] % MIN_LENGTH == 0
+            reaches = config.Br <= min(s["Sq"], s["Sk"])
+        else:
+            divides = s["Sq"] % config.Br == 0 and s["Sk"] % config.Bc == 0
+            reaches = config.Br <= s["Sq"] and config.Bc <= s["Sk"]
+        # kernels for partial tiles at the end of either length
+        ragged = (config.operation == "attn" and config.fuse_type == "register") or config.operation == "attn_bwd"
+        return divides or (ragged and reaches and not whole_tiles and getattr(self.arch, "platform", "") == "ROCm" and
+                           s["Sq"] % MIN_LENGTH == 0 and s["Sk"] % MIN_LENGTH == 0)
 
     def get_tuned_configs(self):
         dq, dv = self.problem_key["dim_qk"], self.problem_key["dim_v"]

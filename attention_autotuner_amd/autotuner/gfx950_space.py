@@ -191,8 +191,13 @@ def _shared_candidates(op, br, bc, dim_qk, dim_v, st_qk, st_v, nthreads, wpe):
     return out
 
 
-def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None):
-    """A configuration that is valid for every supported head size; used before/without tuning."""
+def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None, problem=None):
+    """A configuration that is valid for every supported head size; used before/without tuning.  ``problem``: batch, heads
+    and causal, for a choice that looks at the whole problem where there is a rule for one."""
+    if problem is not None and covered_by_rule(op, dim_qk, dim_v):
+        cfg = rule_forward_config(dim_qk, dim_v, arch, *problem[:2], seq_q, seq_k, problem[2])
+        if cfg is not None:
+            return cfg
     prefs = [(256, 64, 512, 2, 2, 2), (128, 64, 256, 2, 2, 2), (128, 64, 256, 1, 1, 2), (128, 64, 256, 1, 1, 1), (128, 32, 256, 1, 1, 1),
              (64, 32, 128, 1, 1, 1)]
     if op == "ret" and dim_v == 512 and not ((seq_q and seq_q % 128) or (seq_k and seq_k % 64)):
@@ -238,6 +243,10 @@ RULE_SHAPES = {
     (256, 256): ((64, 64, 64, 1, 1, 128, 1), (128, 32, 32, 2, 1, 256, 2), (256, 32, 32, 2, 2, 512, 2)),
 }
 MIN_LENGTH = 32               # the register-fused attention forward takes any lengths that are multiples of this
+
+
+def covered_by_rule(op, dim_qk, dim_v):
+    return (dim_qk, dim_v) in {"attn": RULE_SHAPES, "attn_bwd": ATTN_BWD_RULE}.get(op, ())
 
 
 def rule_configs(dim_qk, dim_v):
@@ -534,7 +543,11 @@ def attn_backward_candidates(br, bc, dim_qk, dim_v):
     return out
 
 
-def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None):
+def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, problem=None):
+    if problem is not None:
+        cfg = rule_attn_backward_config(dim_qk, dim_v, *problem[:2], seq_q, seq_k, problem[2])
+        if cfg is not None:
+            return cfg
     for br, bc, nt, st, wpe in ((128, 32, 256, 3, 1), (128, 32, 256, 2, 1), (64, 32, 128, 3, 1), (64, 32, 128, 2, 1), (64, 32, 128, 2, 2)):
         if any(s and (s % br or s % bc) for s in (seq_q, seq_k)):
             continue
@@ -550,3 +563,34 @@ def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None):
         if attn_backward_valid(cfg, arch):
             return cfg
     raise NoValidConfigError(f"no default attn_bwd configuration fits dim_qk={dim_qk} dim_v={dim_v} seq=({seq_q},{seq_k})")
+
+
+# ---- attention backward without a tuned entry -----------------------------------------------------------
+# (few blocks, many blocks) per pair of head sizes, as arguments of AttnBwdConfig behind the head sizes.  Blocks of 64 resident
+# rows are two waves, two of them to a CU; blocks of 128 are four waves that share one stream.  Up to 512 blocks of 64 rows the
+# smaller ones spread over more CUs (B3 H8 S1344 d 128: 112 us against 114 with two more blocks of 128 rows than there are CUs,
+# d 192 156 against 235), beyond that the larger ones stream less (B4 H32 S1984 d 128 non-causal: 1026 against 1027 ... 1148).
+# A causal walk's blocks are of all lengths, and finer ones end together: the line lies at 1600 there (B6 H20 S832 d 128 123
+# against 131 us).  At d 64 the smaller tile leaves room for four blocks to a CU, which lead beyond the line.  On 34 problems
+# the rule is 1 to 2 % slower on the mean than the best of five to eight shapes.
+ATTN_BWD_RULE = {
+    (64, 64): (dict(Br=64, Bc=64, Nthreads=128, num_stages_qk=2, row_waves_per_eu=2, row_Bc=64),
+               dict(Br=64, Bc=32, Nthreads=128, num_stages_qk=2, waves_per_eu=2, row_waves_per_eu=2)),
+    (128, 128): (dict(Br=64, Bc=64, Nthreads=128, num_stages_qk=2, row_waves_per_eu=2, row_Bc=32),
+                 dict(Br=128, Bc=64, Nthreads=256, num_stages_qk=2, row_waves_per_eu=2, row_Bc=32)),
+    (192, 192): (dict(Br=64, Bc=32, Nthreads=128, num_stages_qk=3), dict(Br=128, Bc=32, Nthreads=256, num_stages_qk=2)),
+    (256, 256): (dict(Br=128, Bc=32, Nthreads=256, num_stages_qk=2),) * 2,
+}
+
+
+def rule_attn_backward_configs(dim_qk, dim_v):
+    return [AttnBwdConfig(Kd=dim_qk, D=dim_v, **kw) for kw in ATTN_BWD_RULE.get((dim_qk, dim_v), ())]
+
+
+def rule_attn_backward_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
+    """The configuration for an attention backward problem nobody tuned, or None."""
+    pair = rule_attn_backward_configs(dim_qk, dim_v)
+    if not pair or seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
+        return None
+    blocks = b * h * -(-seq_k // 64)
+    return pair[blocks > (1600 if causal and dim_qk > 64 else 512)]

@@ -38,6 +38,8 @@ def default_configs(arch=None):
                 cfgs.append(gfx950_space.default_attn_backward_config(dqk, dv, arch, seq, seq))
         if op == "attn":
             cfgs += gfx950_space.rule_configs(dqk, dv)
+        if op == "attn_bwd":
+            cfgs += gfx950_space.rule_attn_backward_configs(dqk, dv)
         if op == "ret":
             for seq in (None, 128, 64):
                 cfgs.append(gfx950_space.default_backward_config(dqk, dv, arch, seq, seq))

@@ -107,7 +107,13 @@ __global__ void __launch_bounds__(256) attn_bwd_prepare(const half_t* __restrict
 // ROW: k, v); all [B*H, S, width] fp16.  lse2, delta: [B*H, seq_q] fp32.  COL writes out1 = dV and
 // out2 = dK; ROW writes out2 = dQ.  c2 = softmax_scale * log2(e); out_scale = softmax_scale.
 // OUTS (COL only): 3 = both outputs, 1 = dV only (x2, delta and out2 are not touched), 2 = dK only.
-template <int Kd, int D, int BX, int BY, int Nthreads, int NS, AttnBwdPass PASS, int WPE = 1, int OUTS = 3>
+// GEN: lengths that are multiples of 32 and not of the tiles.  Missing 32-row groups of the last resident block load rows
+// that exist, and are not stored; a wave that owns none that exist keeps the block's copies and barriers going and computes
+// nothing.  Missing rows of the last streamed tile are copies of rows that exist (TileDma::issue_rows) with P = 0, hence dS = 0.
+// The extra comparisons and the per-row-group bounds cost 1 to 5 % at whole tiles (B4 H32 S2048 d 128: 970 -> 975 us, causal
+// 585 -> 592; B2 H8 S1024: 65 -> 67), so those keep the form without them.  At ragged lengths the column and the row kernel
+// on good tiles replace the one shape that divides them: B6 H20 S832 d 128 causal 145 -> 123 us, B4 H32 S1984 d 64 659 -> 545.
+template <int Kd, int D, int BX, int BY, int Nthreads, int NS, AttnBwdPass PASS, int WPE = 1, int OUTS = 3, int GEN = 0>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, const half_t* __restrict__ y1,
                const half_t* __restrict__ y2, const float* __restrict__ lse2, const float* __restrict__ delta,
@@ -129,7 +135,7 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
   const int n = lane & 31, h = lane >> 5;
   const int seq_x = COL ? seq_k : seq_q, seq_y = COL ? seq_q : seq_k;
 
-  const int Tx = seq_x / BX;
+  const int Tx = GEN ? (seq_x + BX - 1) / BX : seq_x / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
   if (causal) {                                   // longest blocks first: the last query blocks, the first kv blocks
@@ -139,13 +145,13 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
   }
   const int x0 = xb * BX;
   const int diag = seq_k - seq_q;                 // causal: score (q, kv) is kept when kv <= q + diag
-  int j_begin = 0, j_end = seq_y / BY;
+  int j_begin = 0, j_end = GEN ? (seq_y + BY - 1) / BY : seq_y / BY;
   if (causal) {
     if constexpr (COL) {                          // q tiles that reach kv >= x0:  q >= x0 - diag
       const int first = x0 - diag;
       j_begin = first <= 0 ? 0 : first / BY;
     } else {                                      // kv tiles with kv <= x0 + BX - 1 + diag
-      const int last = x0 + BX - 1 + diag;
+      const int last = (GEN && x0 + BX > seq_x ? seq_x - 1 : x0 + BX - 1) + diag;
       const int lim = last < 0 ? 0 : last / BY + 1;
       j_end = lim < j_end ? lim : j_end;
     }
@@ -164,8 +170,18 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
 
   // resident operands: this lane's row of X1 (width Kd) and of X2 (width D) as MFMA B fragments
   h8 x1f[RT][KS], x2f[RT][kOut2 ? DS : 1];
-  load_q_frags<RT, KS, Kd>(x1f, x1 + ((size_t)bh * seq_x + x0 + wave * WM + n) * Kd + 8 * h);
-  if constexpr (kOut2) load_q_frags<RT, DS, D>(x2f, x2 + ((size_t)bh * seq_x + x0 + wave * WM + n) * D + 8 * h);
+  int groups = RT, first_row = x0 + wave * WM;    // the wave's 32-row groups that exist, and where its rows start
+  if constexpr (GEN) {
+    groups = first_row >= seq_x ? 0 : (seq_x - first_row) / 32 < RT ? (seq_x - first_row) / 32 : RT;
+    first_row = groups > 0 ? first_row : x0;
+  }
+  const auto row_of = [&](int rt) { return first_row + (!GEN || rt < groups ? 32 * rt : 0); };   // a missing group: rows that exist
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const size_t row = (size_t)bh * seq_x + row_of(rt) + n;
+    load_q_frags<1, KS, Kd>(reinterpret_cast<h8(&)[1][KS]>(x1f[rt]), x1 + row * Kd + 8 * h);
+    if constexpr (kOut2) load_q_frags<1, DS, D>(reinterpret_cast<h8(&)[1][DS]>(x2f[rt]), x2 + row * D + 8 * h);
+  }
 
   // LDS addresses inside stage 0: first-contraction fragments (rows n, chunk 2ks+h) and transposing reads
   uint32_t y1addr[KS], y2addr[DS], z1lo[KT], z1hi[KT], z2lo[DT], z2hi[DT];
@@ -200,8 +216,8 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
   if constexpr (!COL) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      lse_row[rt] = lse_g[x0 + wave * WM + rt * 32 + n];
-      delta_row[rt] = delta_g[x0 + wave * WM + rt * 32 + n];
+      lse_row[rt] = lse_g[row_of(rt) + n];
+      delta_row[rt] = delta_g[row_of(rt) + n];
     }
   }
 
@@ -223,15 +239,22 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
   auto issue = [&](int step, int st) {
     const int j = tile_of(step);
     char* base = smem + st * T::kStageBytes;
-    y1dma.issue(y1g + (size_t)j * T::kY1Bytes, base, wave_base);
-    y2dma.issue(y2g + (size_t)j * T::kY2Bytes, base + T::kY1Bytes, wave_base);
+    if constexpr (GEN) {
+      y1dma.issue_rows(y1g + (size_t)j * T::kY1Bytes, base, wave_base, seq_y - j * BY);
+      y2dma.issue_rows(y2g + (size_t)j * T::kY2Bytes, base + T::kY1Bytes, wave_base, seq_y - j * BY);
+    } else {
+      y1dma.issue(y1g + (size_t)j * T::kY1Bytes, base, wave_base);
+      y2dma.issue(y2g + (size_t)j * T::kY2Bytes, base + T::kY1Bytes, wave_base);
+    }
     if constexpr (COL) {
       // every wave copies the tile's 2*BY statistics (same bytes, same place): uniform instruction counts
 #pragma unroll
       for (int i = 0; i < T::kStatInstr; ++i) {
         const int idx = i * 64 + lane;              // [0, BY): lse2, [BY, 2BY): delta
         const int c = idx < 2 * BY ? idx : 2 * BY - 1;
-        const float* src = c < BY ? lse_g + j * BY + c : delta_g + j * BY + (c - BY);
+        int row = j * BY + (c < BY ? c : c - BY);
+        if constexpr (GEN) row = row < seq_y ? row : seq_y - 1;
+        const float* src = (c < BY ? lse_g : delta_g) + row;
         __builtin_amdgcn_global_load_lds((const AAT_AS1 void*)(uintptr_t)src,
                                          (AAT_AS3 void*)(base + T::kY1Bytes + T::kY2Bytes + i * 256), 4, 0, 0);
       }
@@ -279,6 +302,16 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
     } else {
       if (more) issue(j + 1, st ^ 1);
     }
+    if (GEN && groups == 0) return;
+    if constexpr (!GEN && WPE == 1 && RT * ((kOut1 ? DT : 0) + (kOut2 ? KT : 0)) * 16 >= 192) {
+      // A branch that is never taken, on a value the compiler cannot see through: it ends the basic block here.  With 192 or
+      // more output accumulators the scheduler otherwise lifts operand reads over the copies above and spills for it --
+      // d_qk = d_v = 256, 32-row tiles, two buffers: 292 -> 64 bytes of scratch per lane (20 in GEN, where the branch above
+      // does the same); B4 H32 S2048 non-causal backward 3277 -> 1960 us.
+      int never = 0;
+      asm volatile("" : "+s"(never));
+      if (never) return;
+    }
 
     // first contractions: s = Y1 X1^T (scores), p = Y2 X2^T (dP), both transposed (lane owns resident row)
     // the score tiles accumulate in vector registers when the outputs alone fill the accumulation registers
@@ -296,7 +329,8 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
     // from LDS four rows at a time, read by hand one group ahead (a tracked read here is answered with a
     // full lgkmcnt(0) per group: eight exposed LDS round trips per tile for the only wave of the SIMD).
     const int jt = tile_of(j);                      // the tile of this step
-    const bool diag_tile = causal && (COL ? (x0 + BX - 1 > jt * BY + diag) : ((jt + 1) * BY - 1 > x0 + diag));
+    const bool diag_tile = (causal && (COL ? (x0 + BX - 1 > jt * BY + diag) : ((jt + 1) * BY - 1 > x0 + diag))) ||
+                           (GEN && (jt + 1) * BY > seq_y);
     auto softmax_part = [&](auto masked_tag) {
       constexpr bool MASKED = decltype(masked_tag)::value;
       constexpr int G = RT * NT * 4;                                 // groups of four streamed rows
@@ -324,7 +358,10 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
         // The score of resident row x and streamed row y = jt*BY + c + 4h (c = 32t + 8g + e, a constant) is masked
         // when kv > q + diag: COL (x is kv) x - diag - jt*BY - 4h > c, ROW (x is q) c > x + diag - jt*BY - 4h.
         const int xrow = x0 + wave * WM + rt * 32 + n;               // resident row of this lane
-        const int lim = (COL ? xrow - diag : xrow + diag) - jt * BY - 4 * h;
+        int lim = (COL ? xrow - diag : xrow + diag) - jt * BY - 4 * h;
+        const int have = seq_y - jt * BY - 4 * h;                    // GEN: c < have for streamed rows that exist
+        if (GEN && !causal) lim = COL ? -BY : have - 1;
+        if (GEN && !COL && lim >= have) lim = have - 1;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           constexpr int vbase = 4 * g, cbase = 32 * t + 8 * g;
@@ -332,7 +369,7 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
           const float lrow = COL ? l2[e] : lse_row[rt];
           float p = fast_exp2(s[rt][t][v] * c2 - lrow);
           if constexpr (MASKED) {
-            if (COL ? lim > cbase + e : cbase + e > lim) p = 0.f;
+            if (COL ? lim > cbase + e || (GEN && cbase + e >= have) : cbase + e > lim) p = 0.f;
           }
           s[rt][t][v] = p;
           if constexpr (kOut2) {
@@ -391,6 +428,7 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
     constexpr int kChunks = WM * kChunksPerRow;
 #pragma unroll
     for (int t = 0; t < kChunks / 64; ++t) {
+      if (GEN && t * 64 / (32 * kChunksPerRow) >= groups) break;
       const int idx = t * 64 + lane;
       const int row = idx / kChunksPerRow, c = idx % kChunksPerRow;
       const u4v val = *reinterpret_cast<const u4v*>(ostage + row * T::kOStride + c * 16);

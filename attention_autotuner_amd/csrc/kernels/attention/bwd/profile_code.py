@@ -30,31 +30,34 @@ constexpr int dk_waves_per_eu = {dk_waves_per_eu};
 using aat::AttnBwdPass;
 using TC = aat::AttnBwdChain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col>;
 using TR = aat::AttnBwdChain<Kd, D, Br, BcRow, Nthreads, num_stages, AttnBwdPass::Row>;
+// GEN = 1: lengths the tiles do not divide
 #if AAT_COL_SPLIT
-const auto kernel_dv = &aat::attn_bwd_chain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col, dv_waves_per_eu, 1>;
-const auto kernel_dk = &aat::attn_bwd_chain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col, dk_waves_per_eu, 2>;
+template <int GEN> constexpr auto kernel_dv = &aat::attn_bwd_chain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col, dv_waves_per_eu, 1, GEN>;
+template <int GEN> constexpr auto kernel_dk = &aat::attn_bwd_chain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col, dk_waves_per_eu, 2, GEN>;
 #else
-const auto kernel_col = &aat::attn_bwd_chain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col, waves_per_eu>;
+template <int GEN> constexpr auto kernel_col = &aat::attn_bwd_chain<Kd, D, Br, Bc, Nthreads, num_stages, AttnBwdPass::Col, waves_per_eu, 3, GEN>;
 #endif
-const auto kernel_row = &aat::attn_bwd_chain<Kd, D, Br, BcRow, Nthreads, num_stages, AttnBwdPass::Row, row_waves_per_eu>;
+template <int GEN> constexpr auto kernel_row = &aat::attn_bwd_chain<Kd, D, Br, BcRow, Nthreads, num_stages, AttnBwdPass::Row, row_waves_per_eu, 3, GEN>;
 
-bool bwd_shape_ok(int B, int H, int Seq_q, int Seq_k) {{
-  // every sequence length plays both roles (resident rows in one kernel, streamed rows in the other)
-  return aat::shape_ok(B, H, Seq_q, Seq_k, Br, Br) && aat::shape_ok(B, H, Seq_q, Seq_k, Bc, BcRow);   // q rows stream through the column kernel, kv rows through the row kernel
+bool bwd_shape_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, 32); }}
+bool whole_tiles(int Seq_q, int Seq_k) {{
+  // every sequence length plays both roles: resident rows in one kernel, streamed rows in the other
+  return Seq_q % Br == 0 && Seq_k % Br == 0 && Seq_q % Bc == 0 && Seq_k % BcRow == 0;
 }}
+int blocks_of(int rows) {{ return (rows + Br - 1) / Br; }}
 size_t stats_bytes(int B, int H, int Seq_q) {{ return (size_t)2 * B * H * Seq_q * sizeof(float); }}
 
-hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* dO, float* lse, aat_half* dq,
+template <int GEN> hipError_t launch_kernels(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* dO, float* lse, aat_half* dq,
                   aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, float softmax_scale, int causal,
                   void* workspace, hipStream_t stream) {{
 #if AAT_COL_SPLIT
-  static const hipError_t ok0 = aat::allow_lds(kernel_dv, TC::kSmemBytes);
-  static const hipError_t ok1 = aat::allow_lds(kernel_dk, TC::kSmemBytes);
+  static const hipError_t ok0 = aat::allow_lds(kernel_dv<GEN>, TC::kSmemBytes);
+  static const hipError_t ok1 = aat::allow_lds(kernel_dk<GEN>, TC::kSmemBytes);
   if (ok0 != hipSuccess) return ok0;
 #else
-  static const hipError_t ok1 = aat::allow_lds(kernel_col, TC::kSmemBytes);
+  static const hipError_t ok1 = aat::allow_lds(kernel_col<GEN>, TC::kSmemBytes);
 #endif
-  static const hipError_t ok2 = aat::allow_lds(kernel_row, TR::kSmemBytes);
+  static const hipError_t ok2 = aat::allow_lds(kernel_row<GEN>, TR::kSmemBytes);
   if (ok1 != hipSuccess) return ok1;
   if (ok2 != hipSuccess) return ok2;
   using H16 = aat::half_t;
@@ -67,17 +70,23 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* 
   aat::attn_bwd_prepare<D><<<dim3((rows + rows_per_block - 1) / rows_per_block), dim3(256), 0, stream>>>(O, G, lse, lse2, delta, rows);
   const float c2 = softmax_scale * 1.4426950408889634f;
 #if AAT_COL_SPLIT
-  kernel_dv<<<dim3(B * H * (Seq_k / Br)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
+  kernel_dv<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
       K, V, Q, G, lse2, delta, reinterpret_cast<H16*>(dv), nullptr, H, Seq_k, Seq_q, c2, softmax_scale, causal);
-  kernel_dk<<<dim3(B * H * (Seq_k / Br)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
+  kernel_dk<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
       K, V, Q, G, lse2, delta, nullptr, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #else
-  kernel_col<<<dim3(B * H * (Seq_k / Br)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
+  kernel_col<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
       K, V, Q, G, lse2, delta, reinterpret_cast<H16*>(dv), reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #endif
-  kernel_row<<<dim3(B * H * (Seq_q / Br)), dim3(Nthreads), TR::kSmemBytes, stream>>>(
+  kernel_row<GEN><<<dim3(B * H * blocks_of(Seq_q)), dim3(Nthreads), TR::kSmemBytes, stream>>>(
       Q, G, K, V, lse2, delta, nullptr, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, c2, softmax_scale, causal);
   return hipGetLastError();
+}}
+hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* dO, float* lse, aat_half* dq,
+                  aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, float softmax_scale, int causal,
+                  void* workspace, hipStream_t stream) {{
+  return (whole_tiles(Seq_q, Seq_k) ? launch_kernels<0> : launch_kernels<1>)(q, k, v, o, dO, lse, dq, dk, dv, B, H, Seq_q, Seq_k,
+                                                                             softmax_scale, causal, workspace, stream);
 }}
 }}  // namespace
 

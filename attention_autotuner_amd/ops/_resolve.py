@@ -10,7 +10,8 @@ _PKG = os.path.normpath(os.path.join(os.path.dirname(os.path.abspath(__file__)),
 DEFAULT_LOG_DIR = os.environ.get("AAT_LOG_DIR", os.path.join(_PKG, "logs"))
 
 
-# Octaves (BaseTunner.nearest_cached) within which a tuned problem's entry is taken before an operator's own rule.
+# Octaves (BaseTunner.nearest_cached) within which a tuned problem's entry is taken before a built-in default that looks at the
+# whole problem (gfx950_space.covered_by_rule).
 # Attention forward, random problems: entries up to 3 octaves away run within 1 % of what the rule picks, entries 4 ... 12
 # octaves away are 9 % slower on the mean and up to 32 % (256-row blocks on 256 rows of 60 heads: 10.5 against 8.1 us).
 NEAR_ENOUGH = 1.5
@@ -23,19 +24,17 @@ def tune_on_miss():
     return os.environ.get("AAT_TUNE_ON_MISS", "1") != "0"
 
 
-def resolve(tuner, default_factory, rule=None):
-    """``rule``: a function that gives the operator's configuration for a problem far from every tuned one, or None."""
+def resolve(tuner, default_factory, near=None):
+    """``near``: how far away (octaves) a tuned problem may be for its entry to be taken before the built-in default."""
     cfg = tuner.check_cache()
     if cfg is not None:
         return cfg
     if tune_on_miss():
         return tuner.tune(log_path=DEFAULT_LOG_DIR)
-    if rule is not None:
-        cfg = tuner.nearest_cached(NEAR_ENOUGH) or rule()
-    return cfg or tuner.nearest_cached() or default_factory()
+    return tuner.nearest_cached(near) or default_factory()
 
 
-def planned(key, make_tuner, default_factory, rule=None):
+def planned(key, make_tuner, default_factory, near=None):
     """``(configuration, Runtime)`` for the problem ``key`` (operator, shapes, mask walk): resolved through a tuner the
     first time this process meets the problem and kept in the tuners' own memo, so that every later call costs one
     dictionary lookup instead of a tuner, a cache-file name and a library path (the reference reads its JSON cache,
@@ -45,7 +44,7 @@ def planned(key, make_tuner, default_factory, rule=None):
     plan = base_tunner._memo.get(k)
     if plan is None:
         tuner = make_tuner()
-        cc = resolve(tuner, default_factory, rule)
+        cc = resolve(tuner, default_factory, near)
         plan = base_tunner._memo[k] = (cc, Runtime(tuner.arch, cc))
     return plan
 

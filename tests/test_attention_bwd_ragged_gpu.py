@@ -1,0 +1,35 @@
+"""Attention backward at lengths its tiles do not divide: the edges of tiles, against the oracle's exact form under the
+rounded-operand rule of oracle/tolerance.py."""
+import math
+
+import pytest
+import torch
+
+import attention_autotuner_amd as aat
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from oracle import ref_op, tolerance
+
+pytestmark = pytest.mark.gpu
+ARCH = aat.MI355X()
+# one 32-row group, one group over a tile, one short of it, either side the longer one, several blocks
+SHAPES = [(1, 2, 32, 32), (2, 2, 96, 160), (1, 2, 288, 288), (1, 2, 160, 96), (1, 1, 64, 544), (1, 1, 416, 416)]
+
+
+@pytest.mark.parametrize("d", sorted(p[0] for p in gfx950_space.ATTN_BWD_RULE))
+@pytest.mark.parametrize("causal", [False, True])
+def test_every_rule_shape_at_the_edges_of_its_tiles(d, causal):
+    for i, (b, h, sq, sk) in enumerate(SHAPES):
+        g = torch.Generator().manual_seed(300 + i)
+        q, k, v, do = (torch.randn(b, h, s, d, generator=g).half() for s in (sq, sk, sk, sq))
+        o, lse = ref_op.attention_ref(q, k, v, None, causal, return_lse=True)
+        o = o.half()
+        want = ref_op.attention_bwd_ref(q, k, v, do, None, causal)
+        terms = ref_op.attention_bwd_rounding_bound(q, k, v, do, None, causal, o_stored=o)
+        for cfg in gfx950_space.rule_attn_backward_configs(d, d):
+            print(d, causal, (b, h, sq, sk), cfg, flush=True)
+            out = [torch.full_like(t, 7.0, device="cuda") for t in (q, k, v)]
+            Runtime(ARCH, cfg).apply([q.cuda(), k.cuda(), v.cuda(), o.cuda(), do.cuda(), lse.cuda(), *out], softmax_scale=1 / math.sqrt(d), causal=causal)
+            torch.cuda.synchronize()
+            for name, got, ref, t in zip(("dq", "dk", "dv"), out, want, terms):
+                ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
+                assert ok, (name, worst, ratio)
