@@ -98,12 +98,12 @@ class BaseTunner:
         if config.operation in ("ret_bwd", "attn_bwd"):   # both lengths are resident in one pass, streamed in another
             divides = all(s[n] % config.Br == 0 and s[n] % config.Bc == 0 for n in ("Sq", "Sk")) and \
                 s["Sk"] % getattr(config, "row_Bc", config.Bc) == 0
-            reaches = config.Br <= min(s["Sq"], s["Sk"])
+            reaches = config.Br <= min(s["Sq"], s["Sk"]) and (config.operation == "attn_bwd" or (s["Sq"] % config.Bc == 0 and s["Sk"] % config.Bc == 0))
         else:
             divides = s["Sq"] % config.Br == 0 and s["Sk"] % config.Bc == 0
-            reaches = config.Br <= s["Sq"] and config.Bc <= s["Sk"]
-        # kernels for partial tiles at the end of either length
-        ragged = (config.operation == "attn" and config.fuse_type == "register") or config.operation == "attn_bwd"
+            reaches = config.Br <= s["Sq"] and config.Bc <= s["Sk"] and (config.operation == "attn" or s["Sk"] % config.Bc == 0)
+        # partial tiles at the end of a length: of either one for attention, of resident rows for RetNet
+        ragged = config.fuse_type != "shared"
         return divides or (ragged and reaches and not whole_tiles and getattr(self.arch, "platform", "") == "ROCm" and
                            s["Sq"] % MIN_LENGTH == 0 and s["Sk"] % MIN_LENGTH == 0)
 

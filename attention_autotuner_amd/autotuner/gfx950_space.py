@@ -191,16 +191,26 @@ def _shared_candidates(op, br, bc, dim_qk, dim_v, st_qk, st_v, nthreads, wpe):
     return out
 
 
+MIN_LENGTH = 32               # the register-fused forwards and both backwards take resident lengths that are multiples of this
+
+
+def _takes(seq, tile, step=MIN_LENGTH):
+    """Whether a kernel with tiles of ``tile`` rows runs a length of ``seq`` rows (None: any) without mostly idle tiles;
+    ``step``: what its lengths have to be multiples of."""
+    return not seq or seq % tile == 0 or (seq > tile and seq % step == 0)
+
+
 def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None, problem=None):
     """A configuration that is valid for every supported head size; used before/without tuning.  ``problem``: batch, heads
     and causal, for a choice that looks at the whole problem where there is a rule for one."""
     if problem is not None and covered_by_rule(op, dim_qk, dim_v):
-        cfg = rule_forward_config(dim_qk, dim_v, arch, *problem[:2], seq_q, seq_k, problem[2])
+        cfg = rule_forward_config(dim_qk, dim_v, arch, *problem[:2], seq_q, seq_k, problem[2]) if op == "attn" else \
+            rule_ret_config("ret", dim_qk, dim_v, *problem[:2], seq_q, seq_k, problem[2])
         if cfg is not None:
             return cfg
     prefs = [(256, 64, 512, 2, 2, 2), (128, 64, 256, 2, 2, 2), (128, 64, 256, 1, 1, 2), (128, 64, 256, 1, 1, 1), (128, 32, 256, 1, 1, 1),
              (64, 32, 128, 1, 1, 1)]
-    if op == "ret" and dim_v == 512 and not ((seq_q and seq_q % 128) or (seq_k and seq_k % 64)):
+    if op == "ret" and dim_v == 512 and _takes(seq_q, 128) and _takes(seq_k, 64, 64):
         # 32 rows x 512 columns per wave fill the 256 accumulation registers of a wave that has its SIMD to itself;
         # the RetNet kernel is written so that this builds without scratch, and at d_qk 256 it leads every mask mode
         cfg = RetConfig(128, 64, dim_qk, dim_v, dim_qk, 64, 1, 1, 1, 256, True, waves_per_eu=1)
@@ -208,7 +218,7 @@ def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None, prob
         if forward_valid(cfg, arch):
             return cfg
     for br, bc, nt, sq, sv, wpe in prefs:
-        if (seq_q and seq_q % br) or (seq_k and seq_k % bc):
+        if not _takes(seq_q, br) or not _takes(seq_k, bc, MIN_LENGTH if op == "attn" else bc):
             continue
         if op == "attn":
             cfg = AttnConfig(br, bc, dim_qk, dim_v, dim_qk, bc, sq, sv, nt, True, waves_per_eu=wpe)
@@ -242,11 +252,9 @@ RULE_SHAPES = {
     (192, 192): ((128, 32, 32, 2, 2, 256, 2), (256, 64, 64, 2, 2, 512, 2)),
     (256, 256): ((64, 64, 64, 1, 1, 128, 1), (128, 32, 32, 2, 1, 256, 2), (256, 32, 32, 2, 2, 512, 2)),
 }
-MIN_LENGTH = 32               # the register-fused attention forward takes any lengths that are multiples of this
-
 
 def covered_by_rule(op, dim_qk, dim_v):
-    return (dim_qk, dim_v) in {"attn": RULE_SHAPES, "attn_bwd": ATTN_BWD_RULE}.get(op, ())
+    return (dim_qk, dim_v) in {"attn": RULE_SHAPES, "attn_bwd": ATTN_BWD_RULE, "ret": RET_RULE, "ret_bwd": RET_BWD_RULE}.get(op, ())
 
 
 def rule_configs(dim_qk, dim_v):
@@ -402,13 +410,17 @@ def backward_candidates(br, bc, dim_qk, dim_v):
     return out
 
 
-def default_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None):
+def default_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, problem=None):
+    if problem is not None:
+        cfg = rule_ret_config("ret_bwd", dim_qk, dim_v, *problem[:2], seq_q, seq_k, problem[2])
+        if cfg is not None:
+            return cfg
     prefs = ((128, 32, 256, 3, 2, 1), (128, 32, 256, 2, 2, 1), (64, 32, 128, 2, 2, 1), (64, 32, 128, 1, 1, 1), (64, 32, 128, 1, 1, 2),
              (64, 64, 128, 1, 1, 1))
     if dim_v == 512:            # measured at d_qk 256: 64-row streamed tiles with single buffers lead the three-buffer ring of 32-row tiles
         prefs = ((128, 64, 256, 1, 1, 1),) + prefs
     for br, bc, nt, sy, sz, wpe in prefs:
-        if any(s and (s % br or s % bc) for s in (seq_q, seq_k)):
+        if any(not _takes(s, br) or not _takes(s, bc, bc) for s in (seq_q, seq_k)):
             continue
         n = nt // WAVE
         cfg = RetBwdConfig(br, bc, dim_qk, dim_v, n, n, n, n, nt, True, BlockKSmem=dim_qk, num_stages_qk=sy,
@@ -549,7 +561,7 @@ def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, pr
         if cfg is not None:
             return cfg
     for br, bc, nt, st, wpe in ((128, 32, 256, 3, 1), (128, 32, 256, 2, 1), (64, 32, 128, 3, 1), (64, 32, 128, 2, 1), (64, 32, 128, 2, 2)):
-        if any(s and (s % br or s % bc) for s in (seq_q, seq_k)):
+        if any(not _takes(s, br) or not _takes(s, bc) for s in (seq_q, seq_k)):
             continue
         for row_wpe in ((2, wpe) if wpe == 1 else (wpe,)):            # the row kernel at two waves per SIMD where it fits
             cfg = AttnBwdConfig(br, bc, dim_qk, dim_v, nt, st, waves_per_eu=wpe, row_waves_per_eu=row_wpe)
@@ -557,7 +569,7 @@ def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, pr
                 return cfg
     # head sizes whose dV and dK accumulators cannot share a wave: one column kernel per output
     for br, bc, nt, st in ((128, 32, 256, 3), (128, 32, 256, 2), (64, 32, 128, 2)):
-        if any(s and (s % br or s % bc) for s in (seq_q, seq_k)):
+        if any(not _takes(s, br) or not _takes(s, bc) for s in (seq_q, seq_k)):
             continue
         cfg = AttnBwdConfig(br, bc, dim_qk, dim_v, nt, st, waves_per_eu=1, col_split=1)
         if attn_backward_valid(cfg, arch):
@@ -594,3 +606,58 @@ def rule_attn_backward_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
         return None
     blocks = b * h * -(-seq_k // 64)
     return pair[blocks > (1600 if causal and dim_qk > 64 else 512)]
+
+
+# ---- RetNet without a tuned entry ------------------------------------------------------------------------
+# Per pair of head sizes and walk: (up to `line` blocks of 64 rows, line, beyond).  "dense" is every tile of a mask tensor;
+# "skip" is a walk that leaves zero tiles out (scanned, promised, or decay rates).  Timed on 14 problems of 64 ... 3136 rows;
+# a pair is 1 to 4 % slower on the mean than the best of five to seven shapes, the shape that used to stand in at lengths
+# like 1344 (64 x 32 tiles, single buffers) 10 % at best and up to a half at d_v 512.  Where the line lies: two blocks of 64
+# rows share a CU as one block of 128 does, so up to 512 of them the dense walk keeps more CUs busy with the smaller ones
+# (B3 H8 S1344 256/256, 504 blocks: 43 us against 67 for 264 blocks of 128 rows); the blocks of a skipping walk differ in length
+# and balance at half as many.  Backward: blocks of 64 kv rows lead everywhere up to d 192 for the same reason, with dS stored.
+#   forward  (Br, Bc, K buffers, V buffers, threads, waves per SIMD)
+#   backward (Br, Bc, threads, buffers of the dV pass' two streams, of the others', waves per SIMD, ds_rows)
+RET_RULE = {
+    (64, 64): {"dense": ((128, 64, 2, 2, 256, 2), 0, (128, 64, 2, 2, 256, 2)), "skip": ((128, 64, 2, 2, 256, 2), 0, (128, 64, 2, 2, 256, 2))},
+    (128, 128): {"dense": ((64, 64, 1, 1, 128, 2), 256, (128, 64, 1, 1, 256, 2)), "skip": ((64, 64, 1, 1, 128, 2), 256, (128, 64, 1, 1, 256, 2))},
+    (192, 192): {"dense": ((64, 64, 1, 1, 128, 1), 512, (128, 64, 1, 1, 256, 2)), "skip": ((64, 64, 1, 1, 128, 1), 256, (128, 64, 2, 1, 256, 1))},
+    (256, 256): {"dense": ((64, 64, 1, 1, 128, 1), 512, (128, 32, 1, 1, 256, 2)), "skip": ((64, 64, 1, 1, 128, 1), 1024, (128, 64, 1, 1, 256, 1))},
+    (256, 512): {"dense": ((64, 32, 1, 1, 128, 1), 512, (128, 64, 1, 1, 256, 1)), "skip": ((64, 32, 1, 1, 128, 1), 256, (128, 64, 1, 1, 256, 1))},
+}
+RET_BWD_RULE = {
+    (64, 64): {"dense": ((64, 64, 128, 3, 2, 3, 2, 1, 128), 512, (128, 64, 256, 2, 2, 2, 2, 2, 0)),
+               "skip": ((64, 64, 128, 3, 2, 3, 2, 1, 128), 256, (128, 64, 256, 2, 2, 2, 2, 2, 0))},
+    (128, 128): {"dense": ((64, 64, 128, 1, 1, 1, 1, 1, 128), 512, (256, 64, 256, 1, 1, 1, 1, 1, 256)),
+                 "skip": ((64, 64, 128, 1, 1, 1, 1, 1, 128), 0, (64, 64, 128, 1, 1, 1, 1, 1, 128))},
+    (192, 192): {"dense": ((64, 64, 128, 1, 1, 1, 1, 1, 128), 512, (256, 32, 256, 3, 2, 3, 2, 1, 128)),
+                 "skip": ((64, 64, 128, 1, 1, 1, 1, 1, 128), 0, (64, 64, 128, 1, 1, 1, 1, 1, 128))},
+    (256, 256): {"dense": ((64, 64, 128, 1, 1, 1, 1, 1, 128), 512, (256, 32, 256, 3, 2, 3, 2, 1, 128)),
+                 "skip": ((64, 64, 128, 1, 1, 1, 1, 1, 128), 512, (128, 64, 256, 1, 1, 1, 1, 1, 128))},
+    (256, 512): {"dense": ((64, 32, 128, 1, 1, 1, 1, 1, 0), 128, (128, 64, 256, 1, 1, 1, 1, 1, 128)),
+                 "skip": ((64, 32, 128, 1, 1, 1, 1, 1, 0), 128, (128, 64, 256, 1, 1, 1, 1, 1, 128))},
+}
+
+
+def _ret_config(op, dim_qk, dim_v, args):
+    if op == "ret":
+        br, bc, nk, nv, nt, wpe = args
+        return RetConfig(br, bc, dim_qk, dim_v, dim_qk, bc, nk, nk, nv, nt, True, waves_per_eu=wpe).set_fuse_type("register")
+    br, bc, nt, sy, sz, ds, dq, wpe, rows = args
+    n = nt // WAVE
+    return RetBwdConfig(br, bc, dim_qk, dim_v, n, n, n, n, nt, True, BlockKSmem=dim_qk, num_stages_qk=sy, num_stages_mask=sy,
+                        num_stages_dv=sz, num_stages_ds=ds, num_stages_dq=dq, waves_per_eu=wpe, ds_rows=rows)
+
+
+def rule_ret_configs(op, dim_qk, dim_v):
+    walks = (RET_RULE if op == "ret" else RET_BWD_RULE).get((dim_qk, dim_v), {}).values()
+    return [_ret_config(op, dim_qk, dim_v, args) for args in dict.fromkeys(a for few, _, many in walks for a in (few, many))]
+
+
+def rule_ret_config(op, dim_qk, dim_v, b, h, seq_q, seq_k, skips):
+    """The configuration for a RetNet problem nobody tuned, or None (head sizes or lengths the rule does not cover)."""
+    walks = (RET_RULE if op == "ret" else RET_BWD_RULE).get((dim_qk, dim_v))
+    if walks is None or seq_q % 64 or seq_k % 64:
+        return None
+    few, line, many = walks["skip" if skips else "dense"]
+    return _ret_config(op, dim_qk, dim_v, few if b * h * (seq_q if op == "ret" else seq_k) // 64 <= line else many)

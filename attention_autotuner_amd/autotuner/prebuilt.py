@@ -41,6 +41,7 @@ def default_configs(arch=None):
         if op == "attn_bwd":
             cfgs += gfx950_space.rule_attn_backward_configs(dqk, dv)
         if op == "ret":
+            cfgs += gfx950_space.rule_ret_configs("ret", dqk, dv) + gfx950_space.rule_ret_configs("ret_bwd", dqk, dv)
             for seq in (None, 128, 64):
                 cfgs.append(gfx950_space.default_backward_config(dqk, dv, arch, seq, seq))
     return cfgs

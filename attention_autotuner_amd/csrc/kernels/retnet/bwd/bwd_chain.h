@@ -22,7 +22,8 @@
 //     dQ  ROW   dO   V    K    dQ    q row       x (q)     row-major
 //
 // No atomics, no scratch, deterministic; dQ is written directly in fp16, so the reference's second
-// kernel has no counterpart.  Cost: dO V^T is evaluated twice (3*(d_qk+d_v) instead of 3*d_qk+2*d_v
+// kernel has no counterpart.  Resident rows come in any multiple of 32 (the 32-row groups a last block does not have repeat
+// its first one, see below), streamed rows in multiples of BY.  Cost: dO V^T is evaluated twice (3*(d_qk+d_v) instead of 3*d_qk+2*d_v
 // multiply-adds per score) and, for an output wider than DZB columns, the first contraction is repeated
 // per column slice (grid.y slices).
 #pragma once
@@ -116,7 +117,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   const int n = lane & 31, h = lane >> 5;
   const int seq_x = COL ? seq_k : seq_q, seq_y = COL ? seq_q : seq_k;
 
-  const int Tx = seq_x / BX;
+  const int Tx = (seq_x + BX - 1) / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
   if (causal || extents != nullptr) {             // longest blocks first: the last query blocks, the first kv blocks
@@ -125,21 +126,22 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
     xb = t.blk;
   }
   const int x0 = xb * BX;
+  const int rows = seq_x - x0 < BX ? seq_x - x0 : BX;       // resident rows of this block that exist
   const int dz0 = blockIdx.y * DZB;               // first output column of this block
   const int diag = seq_k - seq_q;                 // mask[q][kv] may be non-zero only for kv <= q + diag
   int j_begin = 0, j_end = seq_y / BY;
   if (extents != nullptr) {                       // the streamed tiles in which the mask has a non-zero entry for these rows
     const MaskExtents e = mask_extents_at(extents, H, seq_q, seq_k);
     int lo, hi;
-    if constexpr (COL) mask_col_range(e, bh % H, seq_q, seq_k, x0, BX, lo, hi);
-    else mask_row_range(e, bh % H, seq_q, x0, BX, lo, hi);
+    if constexpr (COL) mask_col_range(e, bh % H, seq_q, seq_k, x0, rows, lo, hi);
+    else mask_row_range(e, bh % H, seq_q, x0, rows, lo, hi);
     mask_tile_range(lo, hi, BY, j_end, j_begin, j_end);
   } else if (causal) {
     if constexpr (COL) {                          // q tiles that reach kv >= x0:  q >= x0 - diag
       const int first = x0 - diag;
       j_begin = first <= 0 ? 0 : first / BY;
     } else {                                      // kv tiles with kv <= x0 + BX - 1 + diag
-      const int last = x0 + BX - 1 + diag;
+      const int last = x0 + rows - 1 + diag;
       const int lim = last < 0 ? 0 : last / BY + 1;
       j_end = lim < j_end ? lim : j_end;
     }
@@ -158,11 +160,21 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   typename T::MDma mdma;
   ydma.init(tid);
   zdma.init(tid, DZ * 2);
-  mdma.init(tid, seq_k * 2);
+  mdma.init(tid, seq_k * 2, COL ? rows / 8 : T::NCM);       // COL: the block's columns of the mask
   const int wave_base = wave * 64;
 
+  // A 32-row group that does not exist repeats the block's first one in everything: the same rows of X, of r and of the mask
+  // (the mask copies below), the same decays, hence the same E tiles -- DS_OUT stores them to the same place with the same
+  // bits, and the waits that count those stores stay what they are.  Its output is not stored.
   h8 xf[RT][KS];
-  load_q_frags<RT, KS, KX>(xf, x + ((size_t)bh * seq_x + x0 + wave * WM + n) * KX + 8 * h);
+  int groups = 0, row_of[RT];                     // groups of this wave that exist (its first ones); where a group's rows start
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const bool exists = wave * WM + rt * 32 < rows;
+    groups += exists ? 1 : 0;
+    row_of[rt] = x0 + (exists ? wave * WM + rt * 32 : 0);
+    load_q_frags<1, KS, KX>(reinterpret_cast<h8(&)[1][KS]>(xf[rt]), x + ((size_t)bh * seq_x + row_of[rt] + n) * KX + 8 * h);
+  }
   uint32_t yaddr[KS], zaddr[DT], maddr[RT][NT * 4];
   {
     int yoff[KS], zoff[DT];
@@ -191,7 +203,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   float inv_r_row[RT];                            // ROW pass: 1/r of the lane's own query row
   if constexpr (!COL) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) inv_r_row[rt] = fast_rcp(r[(size_t)bh * seq_q + x0 + wave * WM + rt * 32 + n]);
+    for (int rt = 0; rt < RT; ++rt) inv_r_row[rt] = fast_rcp(r[(size_t)bh * seq_q + row_of[rt] + n]);
   }
   const float* rg = r + (size_t)bh * seq_q;       // COL pass: r of the streamed query rows
 
@@ -219,7 +231,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
     ydma.issue(yg + (size_t)jt * T::kYBytes, ybuf + st * T::kYBytes, wave_base);
     if constexpr (!DECAY) {
       const char* msrc = COL ? mg + (size_t)jt * BY * seq_k * 2 : mg + (size_t)jt * BY * 2;
-      mdma.issue(msrc, mbuf + st * T::kMBytes, wave_base);
+      mdma.issue_rows(msrc, mbuf + st * T::kMBytes, wave_base, COL ? BY : rows);
     }
   };
   auto issue_z = [&](int j, int st) {
@@ -304,7 +316,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
         if (NSY > 1 && ym_now) ydma.issue_one(i - kZi, ysrc, ybuf + yslot * T::kYBytes, wave_base);
       } else if (i < kZi + kYi + kMi) {
         if constexpr (!DECAY) {
-          if (NSY > 1 && ym_now) mdma.issue_one(i - kZi - kYi, msrc, mbuf + yslot * T::kMBytes, wave_base);
+          if (NSY > 1 && ym_now) mdma.issue_one_of_rows(i - kZi - kYi, msrc, mbuf + yslot * T::kMBytes, wave_base, COL ? BY : rows);
         }
       }
     };
@@ -336,7 +348,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
     for (int rt = 0; rt < RT; ++rt) {
       if constexpr (DECAY) {
         // this lane's resident index, shifted so that the exponent is (streamed origin) -/+ own
-        const int xrow0 = x0 + wave * WM + rt * 32;
+        const int xrow0 = row_of[rt];
         if constexpr (COL) {                       // lane owns kv = xrow0 + n; registers run over q rows j*BY + off
           const int base = jt * BY - (xrow0 + n - diag);
           const auto inv_r = [&](int t, int v) { return rv[4 * t + (v >> 2)][v & 3]; };
@@ -422,12 +434,16 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
       for (int i = 0; i < kStores; ++i) staged[i] = lds_read_f4_async(st_r, i * kRowsPerInstr * T::kDsStride);
     };
     const auto ds_store = [&]() {
-      half_t* const dst = ds_out + ds_block_offset(bh, x0 + wave * WM + lane / kChunksPerRow, jt * BY + (lane % kChunksPerRow) * 8, seq_q, seq_k);
+      half_t* const dst = ds_out + ds_block_offset(bh, row_of[0] + lane / kChunksPerRow, jt * BY + (lane % kChunksPerRow) * 8, seq_q, seq_k);
+      // Lengths are multiples of 64 here: a wave's two groups both exist, 32 rows apart in one 64-row block, or both repeat the
+      // block's first one.
+      const int second = RT == 2 ? row_of[RT - 1] - row_of[0] : 32;
       static_for<kStores>([&](auto i_tag) {
         constexpr int i = decltype(i_tag)::value;
         lds_wait_younger<kStores - 1 - i>(staged[i]);
         // rows of one store instruction lie in one 64-row block (kRowsPerInstr divides 64): 64 elements apart
-        __builtin_nontemporal_store(staged[i], reinterpret_cast<f4v*>(dst + (size_t)i * kRowsPerInstr * 64));
+        constexpr int row = i * kRowsPerInstr;
+        __builtin_nontemporal_store(staged[i], reinterpret_cast<f4v*>(dst + (row < 32 ? row : row - 32 + second) * 64));
       });
     };
     // What this tile sends to memory from here -- with one Y buffer the copy of the next Y and mask tile, with DS_OUT
@@ -496,6 +512,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
     constexpr int kChunks = WM * kChunksPerRow;
 #pragma unroll
     for (int t = 0; t < kChunks / 64; ++t) {
+      if (t * 64 / (32 * kChunksPerRow) >= groups) break;
       const int idx = t * 64 + lane;
       const int row = idx / kChunksPerRow, c = idx % kChunksPerRow;
       const u4v val = *reinterpret_cast<const u4v*>(ostage + row * T::kOStride + c * 16);

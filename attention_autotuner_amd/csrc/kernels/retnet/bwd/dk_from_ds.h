@@ -49,6 +49,7 @@ struct RetBwdDk {
 
 // q [B*H, seq_q, Kd], ds in 64 x 64 blocks (above), dk [B*H, seq_k, Kd], all fp16.
 // causal / extents: the mask mode of the walk, as in ret_bwd_chain (extents = the scan's ranges or nullptr).
+// seq_q and seq_k are multiples of 64; kv rows a last block does not have are computed from copies and not stored.
 // wr_rows x wr_cols: resident rows and streamed-tile width of the row pass that wrote ds (wr_rows % BY == 0).
 template <int Kd, int BX, int BY, int Nthreads, int NS, int WPE = 2>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
@@ -63,7 +64,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
-  const int Tx = seq_k / BX;
+  const int Tx = (seq_k + BX - 1) / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
   if (causal || extents != nullptr) {             // longest blocks first: the first kv blocks
@@ -72,6 +73,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     xb = t.blk;
   }
   const int x0 = xb * BX;
+  const int cols = seq_k - x0 < BX ? seq_k - x0 : BX;       // kv rows of this block that exist, a multiple of 64
   const int diag = seq_k - seq_q;
   const int head = bh % H;
   int j_begin = 0, j_end = seq_q / BY;
@@ -79,7 +81,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   if (extents != nullptr) {
     ext = mask_extents_at(extents, H, seq_q, seq_k);
     int lo, hi;
-    mask_col_range(ext, head, seq_q, seq_k, x0, BX, lo, hi);
+    mask_col_range(ext, head, seq_q, seq_k, x0, cols, lo, hi);
     mask_tile_range(lo, hi, BY, j_end, j_begin, j_end);
   } else if (causal) {                            // q tiles that reach kv >= x0:  q >= x0 - diag
     const int first = x0 - diag;
@@ -100,7 +102,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     const int jt = tile_of(j);
     char* base = smem + st * T::kStageBytes;
     zdma.issue(zg + (size_t)jt * T::kZBytes, base, wave_base);
-    sdma.issue(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base);
+    sdma.issue_rows(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base, cols / 64 * BY);   // the dS blocks that exist
   };
 
   // LDS addresses inside stage 0: Q^T fragments (A operand, d-tile dt) and this wave's dS columns (B operand);
@@ -150,19 +152,20 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     // the kv range the writer covered for the row block this query tile lies in
     const int jt = tile_of(j);
     const int wx0 = (jt * BY) / wr_rows * wr_rows;
+    const int wrows = seq_q - wx0 < wr_rows ? seq_q - wx0 : wr_rows;
     int wlo = 0, whi = seq_k;
     if (extents != nullptr) {
       int lo, hi, jb, je;
-      mask_row_range(ext, head, seq_q, wx0, wr_rows, lo, hi);
+      mask_row_range(ext, head, seq_q, wx0, wrows, lo, hi);
       mask_tile_range(lo, hi, wr_cols, seq_k / wr_cols, jb, je);
       wlo = jb * wr_cols;
       whi = je * wr_cols;
     } else if (causal) {
-      const int last = wx0 + wr_rows - 1 + diag;
+      const int last = wx0 + wrows - 1 + diag;
       const int lim = last < 0 ? 0 : last / wr_cols + 1;
       whi = lim * wr_cols < seq_k ? lim * wr_cols : seq_k;
     }
-    const bool all_written = wlo <= x0 && x0 + BX <= whi;          // block-uniform
+    const bool all_written = wlo <= x0 && x0 + cols <= whi;        // block-uniform (rows that do not exist are not stored)
     const bool mine_written = my_kv >= wlo && my_kv < whi;
 
     // The operand reads are issued as instructions with counted waits (tile_ops.h): in front of an LDS read it can see
@@ -214,7 +217,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   block_sync();
   const float one[1] = {1.f};
   store_o_tile<1, DT, Kd, T::kOStride>(acc, one, smem + wave * 32 * T::kOStride,
-                                       dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane);
+                                       dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane, 32, wave * 32 < cols ? 1 : 0);
 }
 
 }  // namespace aat

@@ -57,11 +57,15 @@ const auto kernel_dk_ds = &aat::ret_bwd_dk_from_ds<Kd, kDkRows, kDkTile, kDkRows
 static_assert(!kStoredDs || Br % kDkTile == 0, "a query tile of the dK kernel lies inside one block of the row pass");
 
 bool bwd_shape_ok(int B, int H, int Seq_q, int Seq_k) {{
-  // every sequence length plays both roles (resident rows in one pass, streamed rows in another)
-  return aat::shape_ok(B, H, Seq_q, Seq_k, Br, Br) && aat::shape_ok(B, H, Seq_q, Seq_k, Bc, Bc);
+  // every sequence length plays both roles: resident rows (any multiple of 32) in one pass, streamed rows in another
+  return aat::shape_ok(B, H, Seq_q, Seq_k, 32, 32) && aat::shape_ok(B, H, Seq_q, Seq_k, Bc, Bc);
 }}
-// whether this library stores dS for the problem: it is built for it and the lengths fit the dK kernel's tiles
-bool stores_ds(int B, int H, int Seq_q, int Seq_k) {{ return kStoredDs && aat::shape_ok(B, H, Seq_q, Seq_k, kDkTile, kDkRows); }}
+int blocks_of(int rows) {{ return (rows + Br - 1) / Br; }}
+// Whether this library stores dS for the problem: it is built for it and the lengths are whole dS blocks.  Where the kv
+// length is not a multiple of the dK kernel's rows, short walks do not earn the round trip.
+bool stores_ds(int B, int H, int Seq_q, int Seq_k) {{
+  return kStoredDs && aat::shape_ok(B, H, Seq_q, Seq_k, kDkTile, 64) && (Seq_k % kDkRows == 0 || Seq_k >= 512);
+}}
 
 // Workspace: the mask scan's ranges (as the forward lays them out), then, with a stored dS, B*H*Seq_q*Seq_k fp16.
 size_t ds_offset(int H, int Seq_q, int Seq_k) {{ return aat::mask_extent_bytes(H, Seq_q, Seq_k); }}
@@ -95,18 +99,18 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_hal
   const hipError_t scanned = aat::prepare_mask_walk(mask_mode, M, H, Seq_q, Seq_k, workspace, stream, &walk);
   if (scanned != hipSuccess) return scanned;
   const int causal = walk.causal;
-  kernel_dv<<<dim3(B * H * (Seq_k / Br), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
+  kernel_dv<<<dim3(B * H * blocks_of(Seq_k), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
       K, Q, G, M, r, reinterpret_cast<H16*>(dv), H, Seq_k, Seq_q, causal, nullptr, walk.extents, nullptr);
   if (room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k)) {{
     H16* ds = reinterpret_cast<H16*>(static_cast<char*>(workspace) + ds_offset(H, Seq_q, Seq_k));
-    kernel_dq_ds<<<dim3(B * H * (Seq_q / Br), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
+    kernel_dq_ds<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
         G, V, K, M, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, causal, nullptr, walk.extents, ds);
-    kernel_dk_ds<<<dim3(B * H * (Seq_k / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
+    kernel_dk_ds<<<dim3(B * H * ((Seq_k + kDkRows - 1) / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
         Q, ds, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, causal, walk.extents, Br, Bc);
   }} else {{
-    kernel_dk<<<dim3(B * H * (Seq_k / Br), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
+    kernel_dk<<<dim3(B * H * blocks_of(Seq_k), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
         V, G, Q, M, r, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, causal, nullptr, walk.extents, nullptr);
-    kernel_dq<<<dim3(B * H * (Seq_q / Br), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
+    kernel_dq<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
         G, V, K, M, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, causal, nullptr, walk.extents, nullptr);
   }}
   return hipGetLastError();
@@ -125,18 +129,18 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
   using H16 = aat::half_t;
   const H16 *Q = reinterpret_cast<const H16*>(q), *K = reinterpret_cast<const H16*>(k), *V = reinterpret_cast<const H16*>(v),
             *G = reinterpret_cast<const H16*>(dO);
-  decay_dv<<<dim3(B * H * (Seq_k / Br), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
+  decay_dv<<<dim3(B * H * blocks_of(Seq_k), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
       K, Q, G, nullptr, r, reinterpret_cast<H16*>(dv), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, nullptr);
   if (room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k)) {{
     H16* ds = reinterpret_cast<H16*>(static_cast<char*>(workspace) + ds_offset(H, Seq_q, Seq_k));
-    decay_dq_ds<<<dim3(B * H * (Seq_q / Br), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
+    decay_dq_ds<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
         G, V, K, nullptr, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, ds);
-    kernel_dk_ds<<<dim3(B * H * (Seq_k / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
+    kernel_dk_ds<<<dim3(B * H * ((Seq_k + kDkRows - 1) / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
         Q, ds, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, 1, nullptr, Br, Bc);
   }} else {{
-    decay_dk<<<dim3(B * H * (Seq_k / Br), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
+    decay_dk<<<dim3(B * H * blocks_of(Seq_k), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
         V, G, Q, nullptr, r, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, nullptr);
-    decay_dq<<<dim3(B * H * (Seq_q / Br), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
+    decay_dq<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
         G, V, K, nullptr, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, nullptr);
   }}
   return hipGetLastError();

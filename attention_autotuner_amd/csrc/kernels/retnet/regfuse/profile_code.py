@@ -24,6 +24,9 @@ constexpr int shared_mem = Traits::kSmemBytes;
 const auto kernel = &aat::ret_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu>;
 const auto kernel_decay = &aat::ret_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu, true>;
 
+bool lengths_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, Bc); }}
+int row_blocks(int Seq_q) {{ return (Seq_q + Br - 1) / Br; }}
+
 hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* o, float* r, int B, int H,
                   int Seq_q, int Seq_k, int mask_mode, void* workspace, hipStream_t stream) {{
   static const hipError_t lds_ok = aat::allow_lds(kernel, shared_mem);
@@ -32,7 +35,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_hal
   const hipError_t scanned = aat::prepare_mask_walk(mask_mode, reinterpret_cast<const aat::half_t*>(mask), H, Seq_q, Seq_k,
                                                     workspace, stream, &walk);
   if (scanned != hipSuccess) return scanned;
-  kernel<<<dim3(B * H * (Seq_q / Br)), dim3(Nthreads), shared_mem, stream>>>(
+  kernel<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<const aat::half_t*>(mask),
       reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, walk.causal, nullptr, walk.extents);
@@ -43,7 +46,7 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
                         int H, int Seq_q, int Seq_k, hipStream_t stream) {{
   static const hipError_t lds_ok = aat::allow_lds(kernel_decay, shared_mem);
   if (lds_ok != hipSuccess) return lds_ok;
-  kernel_decay<<<dim3(B * H * (Seq_q / Br)), dim3(Nthreads), shared_mem, stream>>>(
+  kernel_decay<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), nullptr, reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, 1,
       log2_gamma, nullptr);
@@ -64,7 +67,7 @@ static_assert(AAT_MASK_DENSE == aat::kMaskDense && AAT_MASK_CAUSAL == aat::kMask
 profile_func = r"""
 extern "C" float profile_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* o, float* r, int B, int H,
                             int Seq_q, int Seq_k, int causal, void* workspace, size_t workspace_bytes, void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return -1.f;
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;
   if (!aat::mask_mode_ok(causal, workspace, workspace_bytes, H, Seq_q, Seq_k)) return -1.f;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return aat::timed_mean_ms(s, [&] {{ return launch(q, k, v, mask, o, r, B, H, Seq_q, Seq_k, causal, workspace, s); }});
@@ -78,7 +81,7 @@ extern "C" float profile(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, 
 kernel_entry = r"""
 extern "C" int kernel_entry_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* o, float* r, int B, int H,
                                int Seq_q, int Seq_k, int causal, void* workspace, size_t workspace_bytes, void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc) || causal < 0 || causal > AAT_MASK_SCANNED) return AAT_ERR_SHAPE;
+  if (!lengths_ok(B, H, Seq_q, Seq_k) || causal < 0 || causal > AAT_MASK_SCANNED) return AAT_ERR_SHAPE;
   if (!aat::mask_mode_ok(causal, workspace, workspace_bytes, H, Seq_q, Seq_k)) return AAT_ERR_WORKSPACE;
   return (int)launch(q, k, v, mask, o, r, B, H, Seq_q, Seq_k, causal, workspace, static_cast<hipStream_t>(stream));
 }}
@@ -91,13 +94,13 @@ extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* mas
 decay_entry = r"""
 extern "C" float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
                                int B, int H, int Seq_q, int Seq_k, void*, size_t, void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return -1.f;
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return aat::timed_mean_ms(s, [&] {{ return launch_decay(q, k, v, log2_gamma, o, r, B, H, Seq_q, Seq_k, s); }});
 }}
 extern "C" int kernel_entry_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
                                   int B, int H, int Seq_q, int Seq_k, void*, size_t, void* stream) {{
-  if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return AAT_ERR_SHAPE;
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
   return (int)launch_decay(q, k, v, log2_gamma, o, r, B, H, Seq_q, Seq_k, static_cast<hipStream_t>(stream));
 }}
 """

@@ -7,6 +7,10 @@
 // and LDS-DMA staging as the attention kernel (attention/regfuse/regfuse.h); the mask tile travels
 // through LDS as a third DMA stream, and the normalisation is lazy (utils/retention.h).
 // `causal` promises a mask that is zero above the diagonal and only shortens the kv walk.
+//
+// seq_q is any multiple of 32, seq_k a multiple of Bc.  The 32-row groups the last row block of a head does not have repeat
+// its first group -- same loads, same arithmetic -- and are not stored: a select per mask copy and per group, nothing in the
+// loop.  (Where no 128-row tile divided the length the row blocks were 64 rows of two waves, with one buffer per stream.)
 #pragma once
 #include <type_traits>
 
@@ -71,7 +75,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
-  const int Tr = seq_q / Br;
+  const int Tr = (seq_q + Br - 1) / Br;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tr, rb = tile % Tr;
   if (causal || extents != nullptr) {             // a scanned mask is taken to be of the causal kind: later rows see more
@@ -80,13 +84,14 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
     rb = t.blk;
   }
   const int q0 = rb * Br;
+  const int rows = seq_q - q0 < Br ? seq_q - q0 : Br;      // of this block that exist
   int n_tiles = seq_k / Bc;
   if (extents != nullptr) {                       // walk up to the last kv tile in which the mask has a non-zero entry
     int lo, hi, j_begin;
-    mask_row_range(mask_extents_at(extents, H, seq_q, seq_k), bh % H, seq_q, q0, Br, lo, hi);
+    mask_row_range(mask_extents_at(extents, H, seq_q, seq_k), bh % H, seq_q, q0, rows, lo, hi);
     mask_tile_range(lo, hi, Bc, n_tiles, j_begin, n_tiles);
   } else if (causal) {
-    const int last = q0 + Br - 1 + (seq_k - seq_q);
+    const int last = q0 + rows - 1 + (seq_k - seq_q);
     const int lim = last < 0 ? 0 : last / Bc + 1;
     n_tiles = lim < n_tiles ? lim : n_tiles;
   }
@@ -107,7 +112,15 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   const int wave_base = wave * 64;
 
   h8 qf[RT][KS];
-  load_q_frags<RT, KS, Kd>(qf, q + ((size_t)bh * seq_q + q0 + wave * WM + n) * Kd + 8 * h);
+  int groups = 0;                                 // 32-row groups of this wave that exist (its first ones)
+  int row_of[RT];                                 // where a group's rows start inside the block
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const bool exists = wave * WM + rt * 32 < rows;
+    groups += exists ? 1 : 0;
+    row_of[rt] = exists ? wave * WM + rt * 32 : 0;
+    load_q_frags<1, KS, Kd>(reinterpret_cast<h8(&)[1][KS]>(qf[rt]), q + ((size_t)bh * seq_q + q0 + row_of[rt] + n) * Kd + 8 * h);
+  }
   // one mask address per 32-row group where the tile's rows are a power of two of chunks (see apply_mask_folded)
   constexpr bool kFoldMask = (NCM & (NCM - 1)) == 0 && NCM <= 16;
   uint32_t kaddr[KS], vaddr[DT], maddr[RT][kFoldMask ? 1 : NT * 4];
@@ -134,7 +147,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   }
   auto issue_km = [&](int j, int par) {          // K tile j and mask tile j travel together
     kdma.issue(kg + (size_t)j * T::kKBytes, kbuf + (NSK == 2 ? par * T::kKBytes : 0), wave_base);
-    if constexpr (!DECAY) mdma.issue(mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base);
+    if constexpr (!DECAY) mdma.issue_rows(mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base, rows);
   };
   if (n_tiles > 0) {
     issue_km(0, 0);
@@ -150,7 +163,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
     constexpr int KI = T::KDma::kIters, VI = T::VDma::kIters, MI = DECAY ? 0 : T::MDma::kIters;
     auto issue_km_one = [&](int j, int par, int i) {          // instruction i of the K copy followed by the mask copy
       if (i < KI) kdma.issue_one(i, kg + (size_t)j * T::kKBytes, kbuf + (NSK == 2 ? par * T::kKBytes : 0), wave_base);
-      else if constexpr (!DECAY) mdma.issue_one(i - KI, mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base);
+      else if constexpr (!DECAY) mdma.issue_one_of_rows(i - KI, mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base, rows);
     };
     // One loop body for both buffer parities: the parity is a run-time value that moves the operand addresses and the
     // copy destinations.
@@ -175,7 +188,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
       static_for<RT>([&](auto rt_tag) {
         constexpr int rt = decltype(rt_tag)::value;
         if constexpr (DECAY) {
-          const int own0 = q0 + wave * WM + rt * 32 + diag;              // q + diag of the group's first row
+          const int own0 = q0 + row_of[rt] + diag;                      // q + diag of the group's first row
           const auto one = [](int, int) { return 1.0f; };
           if ((j + 1) * Bc - 1 > own0) decay.template apply<true>(sacc[rt], own0 + n - j * Bc, one);
           else decay.template apply<false>(sacc[rt], own0 + n - j * Bc, one);
@@ -237,10 +250,10 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
     for (int rt = 0; rt < RT; ++rt) {
       const float r_fin = fmaxf(row[rt].big_r, 1.0f);
       scale[rt] = row[rt].r_ref * fast_rcp(r_fin);
-      if (h == 0) r[(size_t)bh * seq_q + q0 + wave * WM + rt * 32 + n] = r_fin;
+      if (h == 0 && rt < groups) r[(size_t)bh * seq_q + q0 + wave * WM + rt * 32 + n] = r_fin;
     }
     store_o_tile_numbered<RT, DT, D, T::kOStride, 0>(scale, smem + wave * WM * T::kOStride,
-                                                     o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane);
+                                                     o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane, groups);
     return;
   }
 
@@ -268,7 +281,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       if constexpr (DECAY) {
-        const int own0 = q0 + wave * WM + rt * 32 + diag;              // q + diag of the group's first row
+        const int own0 = q0 + row_of[rt] + diag;                      // q + diag of the group's first row
         const auto one = [](int, int) { return 1.0f; };
         if ((j + 1) * Bc - 1 > own0) decay.template apply<true>(sacc[rt], own0 + n - j * Bc, one);
         else decay.template apply<false>(sacc[rt], own0 + n - j * Bc, one);
@@ -308,10 +321,10 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   for (int rt = 0; rt < RT; ++rt) {
     const float r_fin = fmaxf(row[rt].big_r, 1.0f);
     scale[rt] = row[rt].r_ref * fast_rcp(r_fin);
-    if (h == 0) r[(size_t)bh * seq_q + q0 + wave * WM + rt * 32 + n] = r_fin;
+    if (h == 0 && rt < groups) r[(size_t)bh * seq_q + q0 + wave * WM + rt * 32 + n] = r_fin;
   }
   store_o_tile<RT, DT, D, T::kOStride>(oacc, scale, smem + wave * WM * T::kOStride,
-                                       o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane);
+                                       o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane, 32, groups);
 }
 
 }  // namespace aat

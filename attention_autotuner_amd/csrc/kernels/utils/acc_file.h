@@ -120,9 +120,9 @@ AAT_DEV void pv_gemm_steps_numbered(h8 (&pf)[RT][NT][2], const uint32_t (&vaddr)
 }
 
 // store_o_tile for numbered accumulators (after acc_settle): scale per row, round to fp16, transpose through the
-// wave-private staging area, store rows with 16-byte writes.
+// wave-private staging area, store rows with 16-byte writes.  groups: 32-row groups of the wave that exist (store_o_tile).
 template <int RT, int DT, int D, int O_STRIDE, int BASE>
-AAT_DEV void store_o_tile_numbered(const float (&row_scale)[RT], char* ostage, half_t* og, int lane) {
+AAT_DEV void store_o_tile_numbered(const float (&row_scale)[RT], char* ostage, half_t* og, int lane, int groups = RT) {
   constexpr int kChunksPerRow = D * 2 / 16, WM = RT * 32;
   const int n = lane & 31, h = lane >> 5;
   static_for<RT * DT>([&](auto i_tag) {
@@ -143,6 +143,7 @@ AAT_DEV void store_o_tile_numbered(const float (&row_scale)[RT], char* ostage, h
   constexpr int kChunks = WM * kChunksPerRow;
 #pragma unroll
   for (int t = 0; t < kChunks / 64; ++t) {
+    if (t * 64 / (32 * kChunksPerRow) >= groups) break;
     const int idx = t * 64 + lane;
     const int row = idx / kChunksPerRow, c = idx % kChunksPerRow;
     const u4v val = *reinterpret_cast<const u4v*>(ostage + row * O_STRIDE + c * 16);

@@ -205,14 +205,16 @@ struct TileDma {
   int pitch;                                           // bytes between consecutive tile rows in global memory
 
   // `row_pitch_bytes`: distance between rows of the source matrix (defaults to a dense tile-wide matrix).
-  AAT_DEV void init(int tid, int row_pitch_bytes = kRowBytes) {
+  // `chunks`: chunks of a row that exist (4 or more); those behind them are copies of the row's first four.
+  AAT_DEV void init(int tid, int row_pitch_bytes = kRowBytes, int chunks = NC) {
     pitch = row_pitch_bytes;
 #pragma unroll
     for (int i = 0; i < kDistinct; ++i) {
       const int s = i * NT + tid;
       const int row = s / NC, cs = s % NC;
       const int row0 = kRegular ? tid / NC : row;      // the uniform part carries i * kRowsPerIter rows
-      loff[i] = (uint32_t)(row0 * pitch + swz<NC, MODE>(row, cs) * 16);
+      const int c = swz<NC, MODE>(row, cs);
+      loff[i] = (uint32_t)(row0 * pitch + (c < chunks ? c : c & 3) * 16);
     }
   }
   // Issue the copy of one tile.  `g` points at the tile's first row in global memory (wave-uniform),
@@ -232,10 +234,11 @@ struct TileDma {
   // for scores that the caller masks.  32 rows are a multiple of every swizzle's period, so the layout is the same.
   AAT_DEV void issue_rows(const char* g, char* lds, int wave_base, int rows) const {
 #pragma unroll
-    for (int i = 0; i < kIters; ++i) {
-      const int group = (i * NT + wave_base) / (32 * NC);
-      issue_one(i, 32 * group < rows ? g : g - (size_t)group * 32 * pitch, lds, wave_base);
-    }
+    for (int i = 0; i < kIters; ++i) issue_one_of_rows(i, g, lds, wave_base, rows);
+  }
+  AAT_DEV void issue_one_of_rows(int i, const char* g, char* lds, int wave_base, int rows) const {
+    const int group = (i * NT + wave_base) / (32 * NC);
+    issue_one(i, 32 * group < rows ? g : g - (size_t)group * 32 * pitch, lds, wave_base);
   }
   // Instruction i alone (i must fold to a constant where this is inlined): lets a caller thread the
   // copy of a tile between other instructions one LDS-DMA instruction at a time.
