@@ -53,9 +53,39 @@ hipError_t launch_one(const float* q, const float* k, const float* v, const char
   return hipGetLastError();
 }}
 
+template <int KD, int WK>
+hipError_t launch_split(const float* q, const float* k, const float* v, const char* factors, float* out, int batch,
+                        int heads, int kdim, int vdim, int l, hipStream_t stream) {{
+  using T = aat::RetRecurrentSplit<KD, WK>;
+  const auto kernel = &aat::retnet_recurrent_split_kernel<KD, WK>;
+  static const hipError_t ok = aat::allow_lds(kernel, T::kSmemBytes);
+  if (ok != hipSuccess) return ok;
+  kernel<<<dim3((unsigned)batch * heads * (vdim / 32)), dim3(T::kThreads), T::kSmemBytes, stream>>>(q, k, v, factors, out, heads,
+                                                                                             kdim, vdim, l);
+  return hipGetLastError();
+}}
+
+// Whether blocks of 32 value dims that split the key dims between their waves take less time than passes over 128 and
+// 64 key dims with 128 (wide) or 64 value dims per block: microseconds per chunk of a round of blocks, times the rounds on 256
+// compute units (a block fills one; two of the 64 x 64 ones share one), and the addition of the passes' outputs.  Blocks of 64
+// value dims and 128 key dims never came out ahead and are not built.  Measured at 2048 positions, whole calls, passes against
+// split: B4 H8 128/256 353 -> 154 us, B4 H12 128/256 356 -> 276, B8 H16 128/256 398 -> 562; B4 H16 64/128 216 -> 152,
+// B8 H32 64/128 281 -> 491; B4 H16 192/256 618 -> 469, B8 H32 192/128 (1024 positions) 384 -> 463; B4 H16 256/256 758 -> 456,
+// B8 H32 256/256 (1024 positions) 858 -> 882.
+bool split_pays(long bh, int vdim, int block_kdim, bool wide) {{
+  constexpr long kUnits = 256;
+  const auto rounds = [](long blocks, long at_once) {{ return (double)((blocks + at_once - 1) / at_once); }};
+  if (!wide && block_kdim > 64) return true;
+  const double split = (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : 3.4) * rounds(bh * (vdim / 32), kUnits);
+  if (!wide) return split < 3.05 * rounds(bh * (vdim / 64), 2 * kUnits);
+  const double passes = (block_kdim / 128 * 5.8 + block_kdim / 64 % 2 * 4.1) * rounds(bh * (vdim / 128), kUnits);
+  const double add = block_kdim > 128 ? 3.0 * bh * vdim * 32 * 4 / 8e6 : 0.0;      // two reads and a write, partly from the cache
+  return split < passes + add;
+}}
+
 // Two launches: the decay factors of every (head, chunk), then the scan.  A value slice of 128 dims per
-// block halves the traffic of q and k; 64 is taken when vdim asks for it or when 128 would leave most of
-// the compute units without a block.
+// block halves the traffic of q and k; where it would leave most of the compute units without a block or vdim does not
+// allow it, 64 key dims take slices of 64 and more of them the split kernel, which split_pays() may choose elsewhere too.
 hipError_t launch(const float* q, const float* k, const float* v, const float* decay, float* out, int batch, int heads,
                   int kdim, int vdim, int l, int block_kdim, char* workspace, hipStream_t stream) {{
   char* factors = workspace;
@@ -63,14 +93,21 @@ hipError_t launch(const float* q, const float* k, const float* v, const float* d
   aat::retnet_recurrent_factors<<<dim3(heads), dim3(aat::kRecFactorThreads), (size_t)(l / 32) * 16, stream>>>(decay, factors, l);
   hipError_t e = hipGetLastError();
   const bool wide = vdim % 128 == 0 && (long)batch * heads * (vdim / 128) >= 192;
+  if (e == hipSuccess && split_pays((long)batch * heads, vdim, block_kdim, wide)) {{
+    switch (block_kdim) {{
+      case 64: return launch_split<64, 2>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
+      case 128: return launch_split<128, 4>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
+      case 192: return launch_split<192, 3>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
+      default: return launch_split<256, 4>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
+    }}
+  }}
   for (int kd0 = 0; kd0 < block_kdim && e == hipSuccess; ) {{
     const int kd = block_kdim - kd0 >= 128 ? 128 : 64;                 // key dims of this pass
     const float* qp = q + (size_t)kd0 * l;                             // rows kd0.. of every (batch, head) slice
     const float* kp = k + (size_t)kd0 * l;
     float* dst = kd0 == 0 ? out : part;
     if (kd == 128)
-      e = wide ? launch_one<128, 128>(qp, kp, v, factors, dst, batch, heads, kdim, vdim, l, stream)
-               : launch_one<128, 64>(qp, kp, v, factors, dst, batch, heads, kdim, vdim, l, stream);
+      e = launch_one<128, 128>(qp, kp, v, factors, dst, batch, heads, kdim, vdim, l, stream);
     else
       e = wide ? launch_one<64, 128>(qp, kp, v, factors, dst, batch, heads, kdim, vdim, l, stream)
                : launch_one<64, 64>(qp, kp, v, factors, dst, batch, heads, kdim, vdim, l, stream);

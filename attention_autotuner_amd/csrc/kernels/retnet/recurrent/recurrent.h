@@ -488,4 +488,301 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
   asm volatile("s_barrier" ::: "memory");     // the last chunk's output tiles are staged: the data wave stores them
 }
 
+// ---------------------------------------------------------------------------------------------------
+// The same scan for problems whose 64- or 128-wide value slices leave compute units without a block, and for
+// more key dims than those blocks hold: a block owns 32 value dims, and its waves split the key dims between
+// them instead of the value dims.  Wave w holds State[KD/WK key dims][32]; its key dims contribute partial
+// sums of S^T and of O^T, which are exchanged through LDS: every wave adds up 8 of the 32 rows of either
+// (row group g of the C layout goes to wave g % WK), contracts its 8 positions of P with V, and stores its 8
+// rows of the output.  Q is read once per wave and feeds both contractions.
+//
+// Bound by fp32 MFMA like the kernel above; a slice of 32 repeats S^T in every block, so a chunk costs
+// (3 KD + 32) / (2 KD + 32 + KD / 4) of the work of a 128-wide slice, 1.27 to 1.36 times, against four times the blocks.
+// B2 H8 L1056 256/512, 256 blocks: 374 -> 144 us a call; at 2048 positions a chunk takes 3.4 us instead of 5.5 in each of
+// two passes, 2.9 us of them matrix instructions (100 of 64 cycles at 2.2 GHz).
+// All key dims are contracted in one pass, so nothing is written twice and added.  K, Q, V and the factors are
+// double-buffered; S^T partials reuse the wave's own rows of the consumed Q tile.  The products D of the
+// decays, 4 KB per chunk of which a wave needs the rows of its group, skip LDS, which at KD 256 has no room for them.
+template <int KD, int WK>
+struct RetRecurrentSplit {
+  static constexpr int kChunk = 32;
+  static constexpr int kThreads = WK * 64 + 64;
+  static constexpr int kRows = KD / WK;                    // key dims of one wave
+  static constexpr int kKB = kRows / 32;                   // its State tiles
+  static constexpr int kOwn = (4 + WK - 1) / WK;           // row groups of a C tile it adds up (the last may not exist)
+  static constexpr int kQOff = KD * 128, kVOff = 2 * KD * 128, kFOff = kVOff + 4096;
+  static constexpr int kFBytes = kRecFactorBytes - kRecFactorW;
+  static constexpr int kStage = kFOff + kFBytes;
+  static constexpr int kOutOff = 2 * kStage;               // per wave: its partial O^T tile
+  static constexpr int kSmemBytes = kOutOff + WK * 4096;
+  static_assert(KD % (32 * WK) == 0 && WK >= 2 && WK <= 4, "key dims per wave are whole State tiles");
+  static_assert(kQOff + KD * 128 <= 65536, "row offsets go into the 16-bit offset field of the LDS reads");
+  static_assert(kSmemBytes <= 160 * 1024, "LDS");
+};
+
+// Grid: B * H * vdim / 32 blocks, the slices of one (batch, head) on one XCD (they read the same q and k).
+template <int KD, int WK>
+__global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void retnet_recurrent_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    const char* __restrict__ factors, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
+  using T = RetRecurrentSplit<KD, WK>;
+
+  extern __shared__ __align__(16) char smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = xcd_remap(blockIdx.x, gridDim.x), slices = vdim / 32;
+  const int bh = tile / slices, vd0 = (tile % slices) * 32, h = bh % heads;
+  const int nchunk = L / T::kChunk;
+  const char* fg = factors + (size_t)h * nchunk * kRecFactorBytes;
+
+  if (wave == WK) {
+    // data wave: see the kernel above
+    const char* qg = reinterpret_cast<const char*>(q + (size_t)bh * kdim * L);
+    const char* kg = reinterpret_cast<const char*>(k + (size_t)bh * kdim * L);
+    const char* vg = reinterpret_cast<const char*>(v + ((size_t)bh * vdim + vd0) * L);
+    const int orl = lane >> 3, occ = lane & 7, pitch = L * 4;
+    uint32_t toff[KD / 8];
+#pragma unroll
+    for (int i = 0; i < KD / 8; ++i)
+      toff[i] = (uint32_t)((8 * i + rec_pos(orl)) * pitch + (occ ^ (((i & 1) << 2) | (orl >> 1))) * 16);
+    const uint32_t lane16off = lane * 16;
+    auto dma_one = [&](const char* g_uniform, uint32_t lane_off, char* lds) {
+      const uint64_t base = (uint64_t)(uintptr_t)g_uniform;
+      const uint32_t dst = (uint32_t)(uintptr_t)(AAT_AS3 char*)lds;
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :: "v"(lane_off), "s"(base), "s"(dst) : "memory", "m0");
+    };
+    auto dma = [&](int c, int stage) {
+      char* s = smem + stage * T::kStage;
+      const size_t col = (size_t)c * T::kChunk * 4;
+#pragma unroll
+      for (int i = 0; i < KD / 8; ++i) dma_one(kg + col, toff[i], s + i * 1024);
+#pragma unroll
+      for (int i = 0; i < KD / 8; ++i) dma_one(qg + col, toff[i], s + T::kQOff + i * 1024);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dma_one(vg + col, toff[i], s + T::kVOff + i * 1024);
+      dma_one(fg + (size_t)c * kRecFactorBytes + kRecFactorW, lane16off, s + T::kFOff);
+    };
+    dma(0, 0);
+    wait_vmcnt<0>();
+    for (int c = 0; c < nchunk; ++c) {
+      asm volatile("s_barrier" ::: "memory");          // chunk c is in LDS; the matrix waves are done with chunk c-1
+      if (c + 1 < nchunk) dma(c + 1, (c + 1) & 1);
+      asm volatile("s_barrier" ::: "memory");          // (the matrix waves' barrier in front of the S^T sum)
+      wait_vmcnt<0>();
+    }
+    asm volatile("s_barrier" ::: "memory");
+    return;
+  }
+
+  const uint32_t lds0 = lds_addr(smem);
+  const uint32_t row_lane = hi * 128 + (n >> 2) * 16 + (n & 3) * 4;
+  const int cp = rec_pos(n);
+  int own[T::kOwn];                                     // this wave's row groups; a missing one reads like its first
+#pragma unroll
+  for (int s = 0; s < T::kOwn; ++s) own[s] = wave + s * WK < 4 ? wave + s * WK : wave;
+  const bool has_last = wave + (T::kOwn - 1) * WK < 4;
+
+  constexpr int kNumBases = 8 + 4 + 4 + 2 * T::kOwn + 4;
+  uint32_t bases[kNumBases];                            // LDS addresses that move to the other stage after every chunk
+  uint32_t* const rowk = bases;                         // [8]  this wave's key dims along the sequence
+  uint32_t* const colk = bases + 8;                     // [4]  K columns
+  uint32_t* const colv = bases + 12;                    // [4]  V columns
+  uint32_t* const vown = bases + 16;                    // [kOwn]  V columns of the wave's own positions
+  uint32_t* const sown = vown + T::kOwn;                // [kOwn]  S^T partials of the own row groups
+  uint32_t& wbase = sown[T::kOwn];
+  uint32_t& pbase = sown[T::kOwn + 1];
+  uint32_t& fbase = sown[T::kOwn + 2];
+  uint32_t& smine = sown[T::kOwn + 3];                  // this wave's S^T partial
+#pragma unroll
+  for (int sw = 0; sw < 8; ++sw) rowk[sw] = lds0 + wave * T::kRows * 128 + (row_lane ^ (sw << 4));
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const uint32_t col = cp * 128 + rec_slot(cp, 2 * g + hi) * 16;
+    colk[g] = lds0 + wave * T::kRows * 128 + col;
+    colv[g] = lds0 + T::kVOff + col;
+  }
+#pragma unroll
+  for (int s = 0; s < T::kOwn; ++s) {
+    vown[s] = lds0 + T::kVOff + cp * 128 + rec_slot(cp, 2 * own[s] + hi) * 16;
+    sown[s] = lds0 + own[s] * 1024 + lane * 16;
+  }
+  wbase = lds0 + T::kFOff + hi * 64;
+  pbase = lds0 + T::kFOff + (kRecFactorPnl - kRecFactorW) + n * 4;
+  fbase = lds0 + T::kFOff + (kRecFactorFlag - kRecFactorW);
+  smine = lds0 + T::kQOff + wave * T::kRows * 128 + lane * 16;
+  const uint32_t omine = lds0 + T::kOutOff + wave * 4096 + lane * 16;
+  uint32_t oown[T::kOwn];
+  float* orow[T::kOwn];
+  const char* dptr[T::kOwn];
+#pragma unroll
+  for (int s = 0; s < T::kOwn; ++s) {
+    oown[s] = lds0 + T::kOutOff + own[s] * 1024 + lane * 16;
+    orow[s] = out + ((size_t)bh * vdim + vd0 + 8 * own[s] + 4 * hi) * L + n;
+    dptr[s] = fg + own[s] * 1024 + lane * 16;
+  }
+  auto lds_write_f4 = [&](uint32_t a, int imm_g, f4v x) {
+    *reinterpret_cast<f4v*>(smem + (a - lds0) + imm_g * 1024) = x;
+  };
+
+  f16v st[T::kKB];
+#pragma unroll
+  for (int i = 0; i < T::kKB; ++i) st[i] = zero16();
+
+  // One stream of LDS reads per chunk as in the kernel above: rows of K and Q, the previous chunk's O^T
+  // partials, flag, V, w, the K columns of one half of the State update, the S^T partials, p_n, the other half.
+  constexpr int kPF = 6, kRing = kPF + 1, kOwn = T::kOwn;
+  constexpr int nS1 = T::kRows, nUpd = 4 * T::kKB, nHalf = nUpd / 2;
+  constexpr int jO = nS1, jFlag = jO + kOwn * WK, jV = jFlag + 1, jW = jV + 4, jVo = jW + 4, jK1 = jVo + kOwn;
+  constexpr int jRed = jK1 + nHalf, jPnl = jRed + kOwn * WK, jK2 = jPnl + 1, nElem = jK2 + nUpd - nHalf;
+  static_assert(jRed - jO - kPF > kPF, "reads issued after the S^T stores have returned before the barrier that publishes them");
+
+  auto chunk = [&](auto stage_tag, int c) {
+    constexpr int S = decltype(stage_tag)::value;
+    float fr[kRing];
+    f4v vr[kRing];
+    f16v sp = zero16(), oacc = zero16();
+    f4v wv[4], vo[kOwn], pm[kOwn], dd[kOwn], ov[kOwn];
+    float ka = 0.f;
+
+    auto issue = [&](auto jt) {
+      constexpr int j = decltype(jt)::value, slot = j % kRing;
+      if constexpr (j < nS1) {
+        constexpr int i = j / 2, gg = i / 4, e = i % 4, p0 = 8 * gg + 4 * (e & 1) + (e & 2), sw = (p0 >> 1) & 7;
+        fr[slot] = lds_read_f1_async(rowk[sw], (j % 2 ? T::kQOff : 0) + p0 * 128);
+      } else if constexpr (j < jFlag) {
+        vr[slot] = lds_read_f4_async(oown[(j - jO) / WK], (j - jO) % WK * 4096);
+      } else if constexpr (j == jFlag) {
+        vr[slot] = lds_read_f4_async(fbase, 0);
+      } else if constexpr (j < jW) {
+        vr[slot] = lds_read_f4_async(colv[j - jV], 0);
+      } else if constexpr (j < jVo) {
+        vr[slot] = lds_read_f4_async(wbase, (j - jW) * 16);
+      } else if constexpr (j < jK1) {
+        vr[slot] = lds_read_f4_async(vown[j - jVo], 0);
+      } else if constexpr (j < jRed) {
+        vr[slot] = lds_read_f4_async(colk[(j - jK1) % 4], (j - jK1) / 4 * 4096);
+      } else if constexpr (j < jPnl) {
+        vr[slot] = lds_read_f4_async(sown[(j - jRed) / WK], T::kQOff + (j - jRed) % WK * T::kRows * 128);
+      } else if constexpr (j == jPnl) {
+        fr[slot] = lds_read_f1_async(pbase, 0);
+      } else {
+        constexpr int u = nHalf + j - jK2;
+        vr[slot] = lds_read_f4_async(colk[u % 4], u / 4 * 4096);
+      }
+    };
+
+    auto consume = [&](auto jt) {
+      constexpr int j = decltype(jt)::value, slot = j % kRing, younger = (nElem - 1 - j < kPF) ? nElem - 1 - j : kPF;
+      if constexpr (j < nS1) {
+        lds_wait_younger_f<younger>(fr[slot]);
+        if constexpr (j % 2 == 0) ka = fr[slot];
+        else {
+          constexpr int i = j / 2;
+          sp = mfma_32x32x2_f32(ka, fr[slot], sp);
+          oacc = mfma_32x32x2_f32(st[i / 16][i % 16], fr[slot], oacc);
+        }
+        if constexpr (j == nS1 - 1) {          // every row of Q has been read: its place takes the partial tile
+#pragma unroll
+          for (int g = 0; g < 4; ++g) lds_write_f4(smine, g, f4v{sp[4 * g], sp[4 * g + 1], sp[4 * g + 2], sp[4 * g + 3]});
+          asm volatile("" ::: "memory");
+        }
+      } else if constexpr (j < jFlag) {
+        constexpr int s = (j - jO) / WK, t = (j - jO) % WK;
+        lds_wait_younger_f<younger>(vr[slot]);
+        ov[s] = t == 0 ? vr[slot] : ov[s] + vr[slot];
+        if constexpr (t == WK - 1) {
+          if (c > 0 && (s + 1 < kOwn || has_last)) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) orow[s][(size_t)e * L + (size_t)(c - 1) * T::kChunk] = ov[s][e];
+          }
+        }
+      } else if constexpr (j == jFlag) {
+        lds_wait_younger_f<younger>(vr[slot]);
+        if (__builtin_amdgcn_readfirstlane(__float_as_uint(vr[slot][0])) != 0u) {   // lambda left its range: fold it into T
+          const float sc = vr[slot][1];
+#pragma unroll
+          for (int kb = 0; kb < T::kKB; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) st[kb][i] *= sc;
+        }
+      } else if constexpr (j < jW) {
+        lds_wait_younger_f<younger>(vr[slot]);
+        wv[j - jV] = vr[slot];
+      } else if constexpr (j < jVo) {
+        lds_wait_younger_f<younger>(vr[slot]);
+        wv[j - jW] *= vr[slot];
+      } else if constexpr (j < jK1) {
+        lds_wait_younger_f<younger>(vr[slot]);
+        vo[j - jVo] = vr[slot];
+      } else if constexpr (j < jRed) {
+        constexpr int u = j - jK1;
+        lds_wait_younger_f<younger>(vr[slot]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[u / 4] = mfma_32x32x2_f32(vr[slot][e], wv[u % 4][e], st[u / 4]);
+      } else if constexpr (j < jPnl) {
+        constexpr int s = (j - jRed) / WK, t = (j - jRed) % WK;
+        lds_wait_younger_f<younger>(vr[slot]);
+        pm[s] = t == 0 ? vr[slot] : pm[s] + vr[slot];
+        if constexpr (t == WK - 1) pm[s] *= dd[s];
+      } else if constexpr (j == jPnl) {
+        lds_wait_younger_f<younger>(fr[slot]);
+        // O^T = (p_n lambda) T^T Q + V P, over this wave's key dims and positions
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[i] *= fr[slot];
+#pragma unroll
+        for (int s = 0; s < kOwn; ++s)
+          if (s + 1 < kOwn || has_last) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oacc = mfma_32x32x2_f32(vo[s][e], pm[s][e], oacc);
+          }
+      } else {
+        constexpr int u = nHalf + j - jK2;
+        lds_wait_younger_f<younger>(vr[slot]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[u / 4] = mfma_32x32x2_f32(vr[slot][e], wv[u % 4][e], st[u / 4]);
+        if constexpr (j == nElem - 1) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            lds_write_f4(omine, g, f4v{oacc[4 * g], oacc[4 * g + 1], oacc[4 * g + 2], oacc[4 * g + 3]});
+        }
+      }
+    };
+
+    block_sync();        // chunk c is in LDS, chunk c-1's O^T partials are; every wave is done with chunk c-1
+#pragma unroll
+    for (int s = 0; s < kOwn; ++s) dd[s] = *reinterpret_cast<const f4v*>(dptr[s] + (size_t)c * kRecFactorBytes);
+    static_for<kPF>([&](auto jt) { issue(jt); });
+    sched_fence();
+    static_for<nElem>([&](auto jt) {
+      constexpr int j = decltype(jt)::value;
+      if constexpr (j + kPF < nElem) {
+        if constexpr (j + kPF == jRed) asm volatile("s_barrier" ::: "memory");
+        issue(std::integral_constant<int, j + kPF>{});
+      }
+      consume(jt);
+      sched_fence();
+    });
+#pragma unroll
+    for (int i = 0; i < kNumBases; ++i) bases[i] += (S == 0) ? T::kStage : -T::kStage;
+  };
+
+  for (int c = 0; c < nchunk; c += 2) {
+    chunk(std::integral_constant<int, 0>{}, c);
+    if (c + 1 < nchunk) chunk(std::integral_constant<int, 1>{}, c + 1);
+  }
+  block_sync();
+#pragma unroll
+  for (int s = 0; s < kOwn; ++s) {
+    if (s + 1 < kOwn || has_last) {
+      f4v x = *reinterpret_cast<const f4v*>(smem + (oown[s] - lds0));
+#pragma unroll
+      for (int t = 1; t < WK; ++t) x += *reinterpret_cast<const f4v*>(smem + (oown[s] - lds0) + t * 4096);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) orow[s][(size_t)e * L + (size_t)(nchunk - 1) * T::kChunk] = x[e];
+    }
+  }
+}
+
 }  // namespace aat

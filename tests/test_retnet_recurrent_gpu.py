@@ -45,6 +45,21 @@ def test_matches_the_closed_form(b, h, kdim, vdim, seqlen):
     _close(out, ref_op.retnet_recurrent_ref(q, k, v, decay))
 
 
+# blocks whose waves split the key dims: each number of key dims (192: three waves, the first with two row groups), one chunk,
+# odd and even chunk counts, grids that do and do not spread over 8 chiplets, every head against the sequential recurrence;
+# at 64 key dims both sides of the line to 64-wide slices (256 and 258 slices of 32)
+@pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(1, 1, 64, 64, 32), (1, 1, 128, 64, 32), (1, 1, 192, 64, 32), (1, 1, 256, 64, 32),
+                                                   (1, 3, 64, 192, 96), (3, 1, 128, 320, 160), (1, 3, 192, 192, 128),
+                                                   (2, 4, 256, 128, 96), (8, 8, 64, 128, 64), (3, 43, 64, 64, 64)])
+def test_split_key_dims(b, h, kdim, vdim, seqlen):
+    q, k, v, decay = _inputs(11, b, h, kdim, vdim, seqlen, -0.3, 1.2)
+    decay[0, seqlen // 2] = 0.0
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(h):
+        _close(out[:, head], ref[:, head])
+
+
 def test_zero_negative_and_vanishing_decays():
     """Zeros cut the history, negative values flip signs, long runs of small decays drive the carried
     product out of range (the state is then rescaled): all as in the recurrence."""
