@@ -12,6 +12,7 @@ global_vars = r"""
 #include "aat_kernel_abi.h"
 #include "kernels/retnet/recurrent/recurrent.h"
 #include "kernels/utils/host_launch.h"
+#include <algorithm>
 #include <mutex>
 
 namespace {{
@@ -90,7 +91,9 @@ hipError_t launch(const float* q, const float* k, const float* v, const float* d
                   int kdim, int vdim, int l, int block_kdim, char* workspace, hipStream_t stream) {{
   char* factors = workspace;
   float* part = reinterpret_cast<float*>(workspace + (factor_bytes(heads, l) + 255) / 256 * 256);
-  aat::retnet_recurrent_factors<<<dim3(heads), dim3(aat::kRecFactorThreads), (size_t)(l / 32) * 16, stream>>>(decay, factors, l);
+  // one chunk per wave up to 256 chunks; more blocks per head would walk the same long chain of decays once more each
+  const int parts = std::min(16, (l / 32 + aat::kRecFactorWaves - 1) / aat::kRecFactorWaves);
+  aat::retnet_recurrent_factors<<<dim3(heads, parts), dim3(aat::kRecFactorThreads), (size_t)(l / 32) * 8, stream>>>(decay, factors, l);
   hipError_t e = hipGetLastError();
   const bool wide = vdim % 128 == 0 && (long)batch * heads * (vdim / 128) >= 192;
   if (e == hipSuccess && split_pays((long)batch * heads, vdim, block_kdim, wide)) {{

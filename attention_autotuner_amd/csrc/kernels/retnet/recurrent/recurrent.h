@@ -89,19 +89,61 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
 constexpr int kRecFactorBytes = 5120;
 constexpr int kRecFactorW = 4096, kRecFactorPnl = 4224, kRecFactorFlag = 4352;
 
-// decay [H][L] -> factors [H][L/32][kRecFactorBytes].  Grid H, kRecFactorThreads threads, 16 bytes of
-// dynamic LDS per chunk.  The waves of a block share out the chunks of their head (products inside a
-// chunk), one thread then walks lambda through the chunks, and the waves fold it into their records.
+// decay [H][L] -> factors [H][L/32][kRecFactorBytes].  Grid (H, parts of the sequence), kRecFactorThreads threads, 8 bytes of
+// dynamic LDS per chunk.  A head's chunks are shared out over the blocks of its row and the waves of a block.  Each block
+// walks lambda from the first chunk to its own last one by itself (a product per thread and chunk, then one wave chains
+// them); lambda is known before a record is written, so a record is written once.
+//
+// Bound by latency: a load, the walk (one dependent multiplication and comparison per chunk), a load and 32 products, a store.
 constexpr int kRecFactorThreads = 1024;
+constexpr int kRecFactorWaves = kRecFactorThreads / 64;
 __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(const float* __restrict__ decay,
                                                                               char* __restrict__ factors, int L) {
-  extern __shared__ __align__(16) float fsm[];     // per chunk: A, lambda before the chunk, 1/lambda' (or 1), rescale flag
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, hi = lane >> 5, nchunk = L / 32;
-  constexpr int kWavesF = kRecFactorThreads / 64;
-  char* const recs = factors + (size_t)blockIdx.x * nchunk * kRecFactorBytes;
-  for (int c = wave; c < nchunk; c += kWavesF) {
-    const float* dg = decay + (size_t)blockIdx.x * L + c * 32;
-    char* rec = recs + (size_t)c * kRecFactorBytes;
+  extern __shared__ __align__(16) float fsm[];     // per chunk: A, then lambda before the chunk; and A lambda
+  const int lane = threadIdx.x & 63, n = lane & 31, hi = lane >> 5, nchunk = L / 32;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int per_block = (nchunk + gridDim.y - 1) / gridDim.y;
+  const int first = blockIdx.y * per_block, last = min(nchunk, first + per_block);
+  if (first >= last) return;
+  const float* const dh = decay + (size_t)blockIdx.x * L;
+  for (int c = threadIdx.x; c < last; c += kRecFactorThreads) {
+    typedef f4v f4v_dword __attribute__((aligned(4)));                    // decay may start at any float
+    const f4v_dword* p = reinterpret_cast<const f4v_dword*>(dh + (size_t)c * 32);
+    f4v x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = p[i];
+    float w = 1.f;
+#pragma unroll
+    for (int m = 31; m >= 0; --m) w *= x[m / 4][m % 4];
+    fsm[2 * c] = w;                                                                    // A
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float lam = 1.f;
+    for (int base = 0; base < last; base += 64) {
+      const float a = base + lane < last ? fsm[2 * (base + lane)] : 1.f;
+      const int count = min(64, last - base);
+      float before = 1.f, after = 1.f;
+      for (int i = 0; i < count; ++i) {
+        const float lam_new = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(a), i)) * lam;
+        const float mag = __builtin_fabsf(lam_new);
+        before = lane == i ? lam : before;
+        after = lane == i ? lam_new : after;
+        lam = mag >= 0x1p-40f && mag <= 0x1p40f ? lam_new : 1.f;
+      }
+      if (lane < count) {
+        fsm[2 * (base + lane)] = before;
+        fsm[2 * (base + lane) + 1] = after;
+      }
+    }
+  }
+  __syncthreads();
+  for (int c = first + wave; c < last; c += kRecFactorWaves) {
+    const float* dg = dh + (size_t)c * 32;
+    char* rec = factors + ((size_t)blockIdx.x * nchunk + c) * kRecFactorBytes;
+    const float lam = fsm[2 * c], lam_new = fsm[2 * c + 1], mag = __builtin_fabsf(lam_new);
+    const bool rescale = !(mag >= 0x1p-40f && mag <= 0x1p40f);
+    const float inv = rescale ? 1.f : 1.f / lam_new;
     float dsel[16], wsel[16];
     float d = 0.f, w = 1.f;
 #pragma unroll
@@ -117,37 +159,14 @@ __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(co
       f4v x = {dsel[4 * g], dsel[4 * g + 1], dsel[4 * g + 2], dsel[4 * g + 3]};
       *reinterpret_cast<f4v*>(rec + g * 1024 + lane * 16) = x;
       if (n == 0) {
-        f4v y = {wsel[4 * g], wsel[4 * g + 1], wsel[4 * g + 2], wsel[4 * g + 3]};
+        f4v y = {wsel[4 * g] * inv, wsel[4 * g + 1] * inv, wsel[4 * g + 2] * inv, wsel[4 * g + 3] * inv};
         *reinterpret_cast<f4v*>(rec + kRecFactorW + hi * 64 + g * 16) = y;
       }
     }
-    if (hi == 0) *reinterpret_cast<float*>(rec + kRecFactorPnl + n * 4) = d * dg[0];    // p_n
-    if (lane == 0) fsm[4 * c] = w * dg[0];                                             // A
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float lam = 1.f;
-    for (int c = 0; c < nchunk; ++c) {
-      const float lam_new = fsm[4 * c] * lam;
-      const float mag = __builtin_fabsf(lam_new);
-      const bool rescale = !(mag >= 0x1p-40f && mag <= 0x1p40f);
-      char* rec = recs + (size_t)c * kRecFactorBytes;
+    if (hi == 0) *reinterpret_cast<float*>(rec + kRecFactorPnl + n * 4) = d * dg[0] * lam;    // p_n lambda
+    if (lane == 0) {
       *reinterpret_cast<uint32_t*>(rec + kRecFactorFlag) = rescale ? 1u : 0u;
       *reinterpret_cast<float*>(rec + kRecFactorFlag + 4) = lam_new;
-      fsm[4 * c + 1] = lam;
-      fsm[4 * c + 2] = rescale ? 1.f : 1.f / lam_new;
-      lam = rescale ? 1.f : lam_new;
-    }
-  }
-  __syncthreads();
-  for (int c = wave; c < nchunk; c += kWavesF) {
-    char* rec = recs + (size_t)c * kRecFactorBytes;
-    if (lane < 32) {
-      float* w = reinterpret_cast<float*>(rec + kRecFactorW + lane * 4);
-      *w *= fsm[4 * c + 2];
-    } else {
-      float* p = reinterpret_cast<float*>(rec + kRecFactorPnl + (lane - 32) * 4);
-      *p *= fsm[4 * c + 1];
     }
   }
 }

@@ -193,6 +193,20 @@ def test_long_sequence_and_side_stream():
     _close(out, ref)
 
 
+# one block of factors per head and a second one with a single chunk; 300 chunks: several per wave, a short last block, two
+# dozen rescales; decays that do not start on 16 bytes
+@pytest.mark.parametrize("seqlen", [16 * 32, 17 * 32, 300 * 32])
+def test_decay_factors_over_blocks(seqlen):
+    q, k, v, decay = _inputs(12, 1, 2, 64, 64, seqlen, 0.8, 1.0)
+    decay[1, ::97] = -1.5
+    decay[1, seqlen - 40] = 0.0
+    shifted = torch.zeros(2 * seqlen + 1, device="cuda")[1:].view(2, seqlen).copy_(decay)
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), shifted)
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(2):
+        _close(out[:, head], ref[:, head])
+
+
 def test_graph_capture_replays():
     """The extended entry point allocates nothing and launches two kernels: a captured graph of it replays
     correctly with eager work and synchronisations in between, and follows new inputs written in place."""
