@@ -54,15 +54,24 @@ hipError_t launch_one(const float* q, const float* k, const float* v, const char
   return hipGetLastError();
 }}
 
+// Beyond 128 key dims the workspace has an output-sized buffer for the passes (at least 64 value dims: 8 KB per (batch, head,
+// chunk)), which holds P here.
 template <int KD, int WK>
-hipError_t launch_split(const float* q, const float* k, const float* v, const char* factors, float* out, int batch,
+hipError_t launch_split(const float* q, const float* k, const float* v, const char* factors, char* room, float* out, int batch,
                         int heads, int kdim, int vdim, int l, hipStream_t stream) {{
   using T = aat::RetRecurrentSplit<KD, WK>;
-  const auto kernel = &aat::retnet_recurrent_split_kernel<KD, WK>;
+  constexpr bool kPre = KD > 128;
+  const auto kernel = &aat::retnet_recurrent_split_kernel<KD, WK, kPre>;
   static const hipError_t ok = aat::allow_lds(kernel, T::kSmemBytes);
   if (ok != hipSuccess) return ok;
-  kernel<<<dim3((unsigned)batch * heads * (vdim / 32)), dim3(T::kThreads), T::kSmemBytes, stream>>>(q, k, v, factors, out, heads,
-                                                                                             kdim, vdim, l);
+  if constexpr (kPre) {{
+    aat::retnet_recurrent_pmat<KD><<<dim3((unsigned)batch * heads * (l / 32)), dim3(256), 0, stream>>>(q, k, factors, room, heads,
+                                                                                               kdim, l);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }}
+  kernel<<<dim3((unsigned)batch * heads * (vdim / 32)), dim3(T::kThreads), T::kSmemBytes, stream>>>(q, k, v, factors, room, out,
+                                                                                             heads, kdim, vdim, l);
   return hipGetLastError();
 }}
 
@@ -70,14 +79,14 @@ hipError_t launch_split(const float* q, const float* k, const float* v, const ch
 // 64 key dims with 128 (wide) or 64 value dims per block: microseconds per chunk of a round of blocks, times the rounds on 256
 // compute units (a block fills one; two of the 64 x 64 ones share one), and the addition of the passes' outputs.  Blocks of 64
 // value dims and 128 key dims never came out ahead and are not built.  Measured at 2048 positions, whole calls, passes against
-// split: B4 H8 128/256 353 -> 154 us, B4 H12 128/256 356 -> 276, B8 H16 128/256 398 -> 562; B4 H16 64/128 216 -> 152,
-// B8 H32 64/128 281 -> 491; B4 H16 192/256 618 -> 469, B8 H32 192/128 (1024 positions) 384 -> 463; B4 H16 256/256 758 -> 456,
-// B8 H32 256/256 (1024 positions) 858 -> 882.
+// split: B4 H8 128/256 344 -> 147 us, B4 H12 128/256 347 -> 268, B8 H16 128/256 363 -> 552; B4 H16 64/128 207 -> 142,
+// B8 H32 64/128 262 -> 482; B4 H16 192/256 609 -> 371; B4 H16 256/256 748 -> 391.
 bool split_pays(long bh, int vdim, int block_kdim, bool wide) {{
   constexpr long kUnits = 256;
   const auto rounds = [](long blocks, long at_once) {{ return (double)((blocks + at_once - 1) / at_once); }};
   if (!wide && block_kdim > 64) return true;
-  const double split = (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : 3.4) * rounds(bh * (vdim / 32), kUnits);
+  const double pmat = block_kdim > 128 ? 2.0 * bh * block_kdim * 32 * 4 / 5e6 : 0.0;   // P: q and k once more at 5 TB/s
+  const double split = pmat + (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : block_kdim == 192 ? 2.45 : 2.6) * rounds(bh * (vdim / 32), kUnits);
   if (!wide) return split < 3.05 * rounds(bh * (vdim / 64), 2 * kUnits);
   const double passes = (block_kdim / 128 * 5.8 + block_kdim / 64 % 2 * 4.1) * rounds(bh * (vdim / 128), kUnits);
   const double add = block_kdim > 128 ? 3.0 * bh * vdim * 32 * 4 / 8e6 : 0.0;      // two reads and a write, partly from the cache
@@ -95,13 +104,14 @@ hipError_t launch(const float* q, const float* k, const float* v, const float* d
   const int parts = std::min(16, (l / 32 + aat::kRecFactorWaves - 1) / aat::kRecFactorWaves);
   aat::retnet_recurrent_factors<<<dim3(heads, parts), dim3(aat::kRecFactorThreads), (size_t)(l / 32) * 8, stream>>>(decay, factors, l);
   hipError_t e = hipGetLastError();
+  char* const room = reinterpret_cast<char*>(part);
   const bool wide = vdim % 128 == 0 && (long)batch * heads * (vdim / 128) >= 192;
   if (e == hipSuccess && split_pays((long)batch * heads, vdim, block_kdim, wide)) {{
     switch (block_kdim) {{
-      case 64: return launch_split<64, 2>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
-      case 128: return launch_split<128, 4>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
-      case 192: return launch_split<192, 3>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
-      default: return launch_split<256, 4>(q, k, v, factors, out, batch, heads, kdim, vdim, l, stream);
+      case 64: return launch_split<64, 2>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 128: return launch_split<128, 4>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 192: return launch_split<192, 3>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      default: return launch_split<256, 4>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
     }}
   }}
   for (int kd0 = 0; kd0 < block_kdim && e == hipSuccess; ) {{

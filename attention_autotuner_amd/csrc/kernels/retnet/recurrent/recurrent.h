@@ -508,6 +508,41 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // ---------------------------------------------------------------------------------------------------
+// P of every (batch, head, chunk) for the kernel below, as C registers: [B*H][L/32][g][lane][e], 4 KB per chunk.  One block
+// per chunk; its waves split the key dims, read q and k straight from memory (rows of 128 bytes, each used once) and wave w adds
+// up row group w and multiplies it by D.  Bound by the read of q and k.
+template <int KD>
+__global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __restrict__ q, const float* __restrict__ k,
+                                                             const char* __restrict__ factors, char* __restrict__ pmat,
+                                                             int heads, int kdim, int L) {
+  __shared__ __align__(16) f4v part[4][4][64];
+  const int lane = threadIdx.x & 63, n = lane & 31, hi = lane >> 5, nchunk = L / 32;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = xcd_remap(blockIdx.x, gridDim.x), bh = tile / nchunk, c = tile % nchunk;
+  constexpr int kRows = KD / 4;                       // key dims of one wave
+  const size_t at = ((size_t)bh * kdim + wave * kRows + hi) * L + (size_t)c * 32 + n;
+  const float *qp = q + at, *kp = k + at;
+  float kx[kRows / 2], qx[kRows / 2];
+#pragma unroll
+  for (int i = 0; i < kRows / 2; ++i) {
+    kx[i] = kp[(size_t)2 * i * L];
+    qx[i] = qp[(size_t)2 * i * L];
+  }
+  sched_fence();                                      // all loads in flight before the first product
+  f16v sp = zero16();
+#pragma unroll
+  for (int i = 0; i < kRows / 2; ++i) sp = mfma_32x32x2_f32(kx[i], qx[i], sp);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) part[wave][g][lane] = f4v{sp[4 * g], sp[4 * g + 1], sp[4 * g + 2], sp[4 * g + 3]};
+  __syncthreads();
+  f4v x = part[0][wave][lane];
+#pragma unroll
+  for (int t = 1; t < 4; ++t) x += part[t][wave][lane];
+  x *= *reinterpret_cast<const f4v*>(factors + ((size_t)(bh % heads) * nchunk + c) * kRecFactorBytes + wave * 1024 + lane * 16);
+  *reinterpret_cast<f4v*>(pmat + ((size_t)bh * nchunk + c) * 4096 + wave * 1024 + lane * 16) = x;
+}
+
+// ---------------------------------------------------------------------------------------------------
 // The same scan for problems whose 64- or 128-wide value slices leave compute units without a block, and for
 // more key dims than those blocks hold: a block owns 32 value dims, and its waves split the key dims between
 // them instead of the value dims.  Wave w holds State[KD/WK key dims][32]; its key dims contribute partial
@@ -522,6 +557,11 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
 // All key dims are contracted in one pass, so nothing is written twice and added.  K, Q, V and the factors are
 // double-buffered; S^T partials reuse the wave's own rows of the consumed Q tile.  The products D of the
 // decays, 4 KB per chunk of which a wave needs the rows of its group, skip LDS, which at KD 256 has no room for them.
+//
+// PRE: P itself comes from global memory in the same layout, made once per (batch, head) by retnet_recurrent_pmat below, for
+// callers with room for 4 KB per (batch, head, chunk).  That is a third of the matrix instructions of a block (32 of 100 at KD
+// 256) and the exchange of S^T, for one more read of q and k.  B2 H8 L1056 256/512: 136 -> 107 us a call; B4 H16 L2048
+// 192/256: 466 -> 371, 256/256: 447 -> 391.
 template <int KD, int WK>
 struct RetRecurrentSplit {
   static constexpr int kChunk = 32;
@@ -540,10 +580,10 @@ struct RetRecurrentSplit {
 };
 
 // Grid: B * H * vdim / 32 blocks, the slices of one (batch, head) on one XCD (they read the same q and k).
-template <int KD, int WK>
+template <int KD, int WK, bool PRE>
 __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void retnet_recurrent_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const char* __restrict__ factors, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
+    const char* __restrict__ factors, const char* __restrict__ pmat, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
   using T = RetRecurrentSplit<KD, WK>;
 
   extern __shared__ __align__(16) char smem[];
@@ -639,7 +679,7 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
   for (int s = 0; s < T::kOwn; ++s) {
     oown[s] = lds0 + T::kOutOff + own[s] * 1024 + lane * 16;
     orow[s] = out + ((size_t)bh * vdim + vd0 + 8 * own[s] + 4 * hi) * L + n;
-    dptr[s] = fg + own[s] * 1024 + lane * 16;
+    dptr[s] = (PRE ? pmat + (size_t)bh * nchunk * 4096 : fg) + own[s] * 1024 + lane * 16;
   }
   auto lds_write_f4 = [&](uint32_t a, int imm_g, f4v x) {
     *reinterpret_cast<f4v*>(smem + (a - lds0) + imm_g * 1024) = x;
@@ -652,9 +692,9 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
   // One stream of LDS reads per chunk as in the kernel above: rows of K and Q, the previous chunk's O^T
   // partials, flag, V, w, the K columns of one half of the State update, the S^T partials, p_n, the other half.
   constexpr int kPF = 6, kRing = kPF + 1, kOwn = T::kOwn;
-  constexpr int nS1 = T::kRows, nUpd = 4 * T::kKB, nHalf = nUpd / 2;
+  constexpr int nS1 = PRE ? T::kRows / 2 : T::kRows, nUpd = 4 * T::kKB, nHalf = nUpd / 2;
   constexpr int jO = nS1, jFlag = jO + kOwn * WK, jV = jFlag + 1, jW = jV + 4, jVo = jW + 4, jK1 = jVo + kOwn;
-  constexpr int jRed = jK1 + nHalf, jPnl = jRed + kOwn * WK, jK2 = jPnl + 1, nElem = jK2 + nUpd - nHalf;
+  constexpr int jRed = jK1 + nHalf, jPnl = jRed + (PRE ? 0 : kOwn * WK), jK2 = jPnl + 1, nElem = jK2 + nUpd - nHalf;
   static_assert(jRed - jO - kPF > kPF, "reads issued after the S^T stores have returned before the barrier that publishes them");
 
   auto chunk = [&](auto stage_tag, int c) {
@@ -668,8 +708,8 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
     auto issue = [&](auto jt) {
       constexpr int j = decltype(jt)::value, slot = j % kRing;
       if constexpr (j < nS1) {
-        constexpr int i = j / 2, gg = i / 4, e = i % 4, p0 = 8 * gg + 4 * (e & 1) + (e & 2), sw = (p0 >> 1) & 7;
-        fr[slot] = lds_read_f1_async(rowk[sw], (j % 2 ? T::kQOff : 0) + p0 * 128);
+        constexpr int i = PRE ? j : j / 2, gg = i / 4, e = i % 4, p0 = 8 * gg + 4 * (e & 1) + (e & 2), sw = (p0 >> 1) & 7;
+        fr[slot] = lds_read_f1_async(rowk[sw], (PRE || j % 2 ? T::kQOff : 0) + p0 * 128);
       } else if constexpr (j < jFlag) {
         vr[slot] = lds_read_f4_async(oown[(j - jO) / WK], (j - jO) % WK * 4096);
       } else if constexpr (j == jFlag) {
@@ -696,13 +736,14 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
       constexpr int j = decltype(jt)::value, slot = j % kRing, younger = (nElem - 1 - j < kPF) ? nElem - 1 - j : kPF;
       if constexpr (j < nS1) {
         lds_wait_younger_f<younger>(fr[slot]);
-        if constexpr (j % 2 == 0) ka = fr[slot];
+        if constexpr (PRE) oacc = mfma_32x32x2_f32(st[j / 16][j % 16], fr[slot], oacc);
+        else if constexpr (j % 2 == 0) ka = fr[slot];
         else {
           constexpr int i = j / 2;
           sp = mfma_32x32x2_f32(ka, fr[slot], sp);
           oacc = mfma_32x32x2_f32(st[i / 16][i % 16], fr[slot], oacc);
         }
-        if constexpr (j == nS1 - 1) {          // every row of Q has been read: its place takes the partial tile
+        if constexpr (!PRE && j == nS1 - 1) {          // every row of Q has been read: its place takes the partial tile
 #pragma unroll
           for (int g = 0; g < 4; ++g) lds_write_f4(smine, g, f4v{sp[4 * g], sp[4 * g + 1], sp[4 * g + 2], sp[4 * g + 3]});
           asm volatile("" ::: "memory");
@@ -754,7 +795,7 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
         for (int s = 0; s < kOwn; ++s)
           if (s + 1 < kOwn || has_last) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) oacc = mfma_32x32x2_f32(vo[s][e], pm[s][e], oacc);
+            for (int e = 0; e < 4; ++e) oacc = mfma_32x32x2_f32(vo[s][e], PRE ? dd[s][e] : pm[s][e], oacc);
           }
       } else {
         constexpr int u = nHalf + j - jK2;
@@ -771,7 +812,7 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
 
     block_sync();        // chunk c is in LDS, chunk c-1's O^T partials are; every wave is done with chunk c-1
 #pragma unroll
-    for (int s = 0; s < kOwn; ++s) dd[s] = *reinterpret_cast<const f4v*>(dptr[s] + (size_t)c * kRecFactorBytes);
+    for (int s = 0; s < kOwn; ++s) dd[s] = *reinterpret_cast<const f4v*>(dptr[s] + (size_t)c * (PRE ? 4096 : kRecFactorBytes));
     static_for<kPF>([&](auto jt) { issue(jt); });
     sched_fence();
     static_for<nElem>([&](auto jt) {
