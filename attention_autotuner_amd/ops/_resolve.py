@@ -3,7 +3,7 @@ import os
 
 import torch
 
-from ..autotuner import base_tunner
+from ..autotuner import base_tunner, gfx950_space
 from ..autotuner.runtime import Runtime
 
 _PKG = os.path.normpath(os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))
@@ -34,8 +34,9 @@ def resolve(tuner, default_factory, near=None):
     return tuner.nearest_cached(near) or default_factory()
 
 
-def planned(key, make_tuner, default_factory, near=None):
-    """``(configuration, Runtime)`` for the problem ``key`` (operator, shapes, mask walk): resolved through a tuner the
+def planned(key, make_tuner, default_factory):
+    """``(configuration, Runtime)`` for the problem ``key`` (operator, device type, batch, heads, lengths, head sizes, mask
+    walk): resolved through a tuner the
     first time this process meets the problem and kept in the tuners' own memo, so that every later call costs one
     dictionary lookup instead of a tuner, a cache-file name and a library path (the reference reads its JSON cache,
     python/autotuner/base_tunner.py:197-206, and opens the library, python/autotuner/runtime.py:74-82, on every call;
@@ -44,6 +45,8 @@ def planned(key, make_tuner, default_factory, near=None):
     plan = base_tunner._memo.get(k)
     if plan is None:
         tuner = make_tuner()
+        op, key_dim, head_dim = key[0].replace("_decay", ""), key[6], key[7]
+        near = NEAR_ENOUGH if gfx950_space.covered_by_rule(op, key_dim, head_dim) else None
         cc = resolve(tuner, default_factory, near)
         plan = base_tunner._memo[k] = (cc, Runtime(tuner.arch, cc))
     return plan

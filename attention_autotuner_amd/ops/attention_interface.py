@@ -15,7 +15,7 @@ import torch
 from ..arch import Arch
 from ..autotuner import gfx950_space
 from ..autotuner.tunner import AttnBwdTunner, AttnTunner
-from ._resolve import NEAR_ENOUGH, NoGraph, planned, wants_graph
+from ._resolve import NoGraph, planned, wants_graph
 
 REFERENCE_SOFTMAX_SCALE = 0.125
 
@@ -44,8 +44,7 @@ class MultiHeadAttnFunc(torch.autograd.Function):
         _, rt = planned(("attn", device_type.name, batch_size, nheads, seqlen_q, seqlen_k, key_dim, head_dim, causal),
                         lambda: AttnTunner(arch=device_type, torch_array=[q, k, v, o], causal=causal, softmax_scale=softmax_scale),
                         lambda: gfx950_space.default_forward_config("attn", key_dim, head_dim, device_type, seqlen_q, seqlen_k,
-                                                                    (batch_size, nheads, causal)),
-                        NEAR_ENOUGH if gfx950_space.covered_by_rule("attn", key_dim, head_dim) else None)
+                                                                    (batch_size, nheads, causal)))
         needs_grad = any(ctx.needs_input_grad[:3])
         lse = torch.empty(batch_size, nheads, seqlen_q, device=q.device, dtype=torch.float32) if needs_grad else None
         rt.apply([q, k, v, o], softmax_scale=softmax_scale, causal=causal, lse=lse)
@@ -70,8 +69,7 @@ class MultiHeadAttnFunc(torch.autograd.Function):
             _, rt = planned(("attn_bwd", device_type.name, q.shape[0], q.shape[1], seqlen_q, seqlen_k, key_dim, head_dim, ctx.causal),
                             lambda: AttnBwdTunner(arch=device_type, torch_array=arrays, causal=ctx.causal, softmax_scale=ctx.softmax_scale),
                             lambda: gfx950_space.default_attn_backward_config(key_dim, head_dim, device_type, seqlen_q, seqlen_k,
-                                                                              (q.shape[0], q.shape[1], ctx.causal)),
-                            NEAR_ENOUGH if gfx950_space.covered_by_rule("attn_bwd", key_dim, head_dim) else None)
+                                                                              (q.shape[0], q.shape[1], ctx.causal)))
         except gfx950_space.NoValidConfigError as e:      # e.g. d_v = 512: dK and dV do not fit one wave's registers
             raise NotImplementedError(f"attention backward: {e}") from e
         rt.apply(arrays, softmax_scale=ctx.softmax_scale, causal=ctx.causal)

@@ -25,11 +25,7 @@ from ..arch import Arch
 from ..autotuner import gfx950_space
 from ..autotuner.runtime import Runtime
 from ..autotuner.tunner import RetTunner, RetBwdTunner
-from ._resolve import NEAR_ENOUGH, NoGraph, planned, wants_graph
-
-
-def _near(op, key_dim, head_dim):
-    return NEAR_ENOUGH if gfx950_space.covered_by_rule(op, key_dim, head_dim) else None
+from ._resolve import NoGraph, planned, wants_graph
 
 
 def retnet_mask_scan(mask, device_type: Arch):
@@ -77,8 +73,7 @@ class RetNetAttn(torch.autograd.Function):
         walk, mode = causal is None or bool(causal), "scan" if causal is None else None
         _, rt = planned(("ret", device_type.name, batch_size, nheads, seqlen_q, seqlen_k, key_dim, head_dim, walk, mode),
                         lambda: RetTunner(arch=device_type, torch_array=arrays, causal=walk, mask_mode=mode),
-                        lambda: gfx950_space.default_forward_config("ret", key_dim, head_dim, device_type, seqlen_q, seqlen_k, (batch_size, nheads, walk)),
-                        _near("ret", key_dim, head_dim))
+                        lambda: gfx950_space.default_forward_config("ret", key_dim, head_dim, device_type, seqlen_q, seqlen_k, (batch_size, nheads, walk)))
         scan = None
         if reused is not None:
             scan = reused
@@ -115,8 +110,7 @@ class RetNetAttn(torch.autograd.Function):
         walk, mode = ctx.causal is None or bool(ctx.causal), "scan" if ctx.mask_scan is not None else None
         _, rt = planned(("ret_bwd", device_type.name, batch_size, nheads, seqlen_q, seqlen_k, key_dim, head_dim, walk, mode),
                         lambda: RetBwdTunner(arch=device_type, torch_array=arrays, causal=walk, mask_mode=mode),
-                        lambda: gfx950_space.default_backward_config(key_dim, head_dim, device_type, seqlen_q, seqlen_k, (batch_size, nheads, walk)),
-                        _near("ret_bwd", key_dim, head_dim))
+                        lambda: gfx950_space.default_backward_config(key_dim, head_dim, device_type, seqlen_q, seqlen_k, (batch_size, nheads, walk)))
         if ctx.mask_scan is not None:
             rt.apply(arrays, causal="scanned", workspace=ctx.mask_scan)
         else:
@@ -164,8 +158,7 @@ class RetNetDecayAttn(torch.autograd.Function):
         arrays = [q, k, v, lg, o, r]
         _, rt = planned(("ret_decay", device_type.name, batch_size, nheads, seqlen_q, seqlen_k, key_dim, head_dim),
                         lambda: RetTunner(arch=device_type, torch_array=arrays, decay=True),
-                        lambda: gfx950_space.default_forward_config("ret", key_dim, head_dim, device_type, seqlen_q, seqlen_k, (batch_size, nheads, True)),
-                        _near("ret", key_dim, head_dim))
+                        lambda: gfx950_space.default_forward_config("ret", key_dim, head_dim, device_type, seqlen_q, seqlen_k, (batch_size, nheads, True)))
         rt.apply(arrays, decay=True)
         ctx.save_for_backward(q, k, v, lg, r)
         ctx.device_type = device_type
@@ -182,8 +175,7 @@ class RetNetDecayAttn(torch.autograd.Function):
         arrays = [q, k, v, lg, do, r, dq, dk, dv]
         _, rt = planned(("ret_bwd_decay", device_type.name, q.shape[0], q.shape[1], seqlen_q, seqlen_k, key_dim, head_dim),
                         lambda: RetBwdTunner(arch=device_type, torch_array=arrays, decay=True),
-                        lambda: gfx950_space.default_backward_config(key_dim, head_dim, device_type, seqlen_q, seqlen_k, (q.shape[0], q.shape[1], True)),
-                        _near("ret_bwd", key_dim, head_dim))
+                        lambda: gfx950_space.default_backward_config(key_dim, head_dim, device_type, seqlen_q, seqlen_k, (q.shape[0], q.shape[1], True)))
         rt.apply(arrays, decay=True)
         return dq, dk, dv, None, None
 
