@@ -109,7 +109,8 @@ __global__ void __launch_bounds__(256) attn_bwd_prepare(const half_t* __restrict
 // OUTS (COL only): 3 = both outputs, 1 = dV only (x2, delta and out2 are not touched), 2 = dK only.
 // GEN: lengths that are multiples of 32 and not of the tiles.  Missing 32-row groups of the last resident block load rows
 // that exist, and are not stored; a wave that owns none that exist keeps the block's copies and barriers going and computes
-// nothing.  Missing rows of the last streamed tile are copies of rows that exist (TileDma::issue_rows) with P = 0, hence dS = 0.
+// nothing.  Missing rows of the last streamed tile are copies of rows that exist (TileDma::issue_rows) with P = 0; the second
+// contractions leave them out (pv_gemm_steps_hl: TAIL), because such a copy may hold an infinity.
 // The extra comparisons and the per-row-group bounds cost 1 to 5 % at whole tiles (B4 H32 S2048 d 128: 970 -> 975 us, causal
 // 585 -> 592; B2 H8 S1024: 65 -> 67), so those keep the form without them.  At ragged lengths the column and the row kernel
 // on good tiles replace the one shape that divides them: B6 H20 S832 d 128 causal 145 -> 123 us, B4 H32 S1984 d 64 659 -> 545.
@@ -384,17 +385,19 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
 
     // second contractions: COL  dV^T += dO^T P  and  dK^T += Q^T dS;   ROW  dQ^T += K^T dS
     h8 ef[RT][NT][2];
+    constexpr bool TAIL = GEN && NT > 1;
+    const int live = (seq_y - jt * BY) / 16;        // GEN: groups of 16 streamed rows that exist
     if constexpr (kOut1) {
-      pv_gemm_steps_hl<RT, NT, DT, NCD, PF>(acc1, ef, z2lo, z2hi, off, [&](int g) {
+      pv_gemm_steps_hl<RT, NT, DT, NCD, PF, false, TAIL>(acc1, ef, z2lo, z2hi, off, [&](int g) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) ef[rt][g >> 1][g & 1] = pack8_rne(s[rt][g >> 1], 8 * (g & 1));
-      });
+      }, live);
     }
     if constexpr (kOut2) {
-      pv_gemm_steps_hl<RT, NT, KT, NCK, PF>(acc2, ef, z1lo, z1hi, off, [&](int g) {
+      pv_gemm_steps_hl<RT, NT, KT, NCK, PF, false, TAIL>(acc2, ef, z1lo, z1hi, off, [&](int g) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) ef[rt][g >> 1][g & 1] = pack8_rne(dp[rt][g >> 1], 8 * (g & 1));
-      });
+      }, live);
     }
   };
   for (int j = j_begin; j < j_end; j += NS) {

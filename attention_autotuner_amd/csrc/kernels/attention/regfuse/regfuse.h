@@ -123,7 +123,8 @@ template <bool CAUSAL, class F> AAT_DEV void run_tiles(F& tile, int n_full, int 
 // exist) or something nobody reads, and are not stored.  The last kv tile may be partial: the missing rows are copies of
 // rows that exist (TileDma::issue_rows) and their scores are masked like those above the diagonal -- the causal walk
 // does that by itself, because the last row that exists sees up to kv row seq_k - 1, and a non-causal walk is a causal one
-// in which every row sees that far.
+// in which every row sees that far.  The second contraction leaves them out (pv_gemm_steps: TAIL): a copy of a V row with an
+// infinity would make NaN of it.
 // What it replaces at such lengths is the one tile shape that divides them, 64 x 32 on two waves with one buffer: batch 3,
 // 12 heads, 1088 rows, d 128, causal 44 -> 29 us with 128 x 64 tiles; 8 x 12 x 1984 rows 195 -> 118 us; d 64, 4 x 8 x 3392 rows
 // 271 -> 117 us.  The waste is the missing groups of one row block per head and the missing rows of one kv tile; matrix work
@@ -345,6 +346,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
         static_for<NU>([&](auto unit_tag) {
           constexpr int U = decltype(unit_tag)::value;
           const int kv0 = kv_first + j * Bc + U * BU;   // first kv row of the unit
+          constexpr bool TAIL = GEN && MASKED && NTU > 1;   // kv rows of the unit may be missing: they stay out of the second contraction
           if constexpr (ILV) {
             // One body for both row groups; in a unit the early group no longer sees (and the late one does) its
             // MFMAs, its softmax step and its packing are branched around one by one.
@@ -354,7 +356,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
               on0 = kv0 <= last_early;
               on1 = kv0 <= last_early + group_lim;
             }
-            if constexpr (GEN) on1 = on1 && groups > 0;
+            if constexpr (GEN) on1 = on1 && groups > 0 && (!MASKED || kv0 < seq_k);
             if (on1) {
               f16v sacc[RT][NTU];
               AAT_SETPRIO(2);
@@ -374,19 +376,19 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
               }
               h8 pf[RT][NTU][2];
               AAT_SETPRIO(2);
-              pv_gemm_steps<RT, NTU, DT, NCV, PF, false, XA, MASKED && XA>(oacc, pf, vaddr, PAR * T::kVBytes + U * NTU * T::kUnitV, [&](int g) {
+              pv_gemm_steps<RT, NTU, DT, NCV, PF, false, XA, MASKED && XA, TAIL>(oacc, pf, vaddr, PAR * T::kVBytes + U * NTU * T::kUnitV, [&](int g) {
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
                   if (rt != 0 || on0 || !(MASKED && XA)) pack_p_group<NTU, XA>(pf[rt], sacc[rt], g, l_run[rt]);
                 }
-              }, on0);
+              }, on0, (seq_k - kv0) / 16);
               AAT_SETPRIO(0);
             }
             return;
           }
           bool wave_sees = true;
           if constexpr (MASKED) wave_sees = kv0 <= (q0 + wave * WM + WM - 1) * slope + diag;
-          if constexpr (GEN) wave_sees = wave_sees && groups > 0;
+          if constexpr (GEN) wave_sees = wave_sees && groups > 0 && (!MASKED || kv0 < seq_k);
 
           f16v sacc[RT][NTU];
           if (wave_sees) {
@@ -418,10 +420,10 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
           if (wave_sees) {
             h8 pf[RT][NTU][2];
             AAT_SETPRIO(2);
-            pv_gemm_steps<RT, NTU, DT, NCV, PF, false, XA>(oacc, pf, vaddr, (NSV == 2 ? PAR * T::kVBytes : 0) + U * NTU * T::kUnitV, [&](int g) {
+            pv_gemm_steps<RT, NTU, DT, NCV, PF, false, XA, false, TAIL>(oacc, pf, vaddr, (NSV == 2 ? PAR * T::kVBytes : 0) + U * NTU * T::kUnitV, [&](int g) {
 #pragma unroll
               for (int rt = 0; rt < RT; ++rt) pack_p_group<NTU, XA>(pf[rt], sacc[rt], g, l_run[rt]);   // per-lane partial sums
-            });
+            }, true, (seq_k - kv0) / 16);
             AAT_SETPRIO(0);
           }
         });

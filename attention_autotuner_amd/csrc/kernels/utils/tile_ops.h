@@ -250,9 +250,11 @@ AAT_DEV void qk_gemm_steps(f16v (&sacc)[RT][NT], const h8 (&qf)[RT][KS], const u
 // wave on the SIMD nothing covers that wait (RetNet forward at d_qk 256 / d_v 512: -6 % with BLIND); with two or
 // three another wave does, and the counted waits cost a little instead (attention forward, causal: +1.5 %).
 // buf_off must fold to a constant.
-template <int RT, int NT, int DT, int NCV, int PF, bool BLIND = false, class Pack>
+// TAIL: only the first `live` groups of 16 rows exist (wave-uniform, 2 or more).  The others hold copies of rows that do, and
+// a zero P would keep them out of the sums only while they are finite: 0 * inf is NaN.  Their MFMAs are branched around.
+template <int RT, int NT, int DT, int NCV, int PF, bool BLIND = false, bool TAIL = false, class Pack>
 AAT_DEV void pv_gemm_steps_hl(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const uint32_t (&vlo)[DT],
-                              const uint32_t (&vhi)[DT], int buf_off, Pack&& pack) {
+                              const uint32_t (&vhi)[DT], int buf_off, Pack&& pack, int live = 2 * NT) {
   constexpr int G = NT * 2;              // groups of 16 kv rows
   constexpr int S = G * DT;
   constexpr int kRow16 = 16 * NCV * 16;
@@ -277,7 +279,9 @@ AAT_DEV void pv_gemm_steps_hl(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const u
     }
     const h8 vf = cat_h4(clo, chi);
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
+    for (int rt = 0; rt < RT; ++rt) {
+      if (!TAIL || g < 2 || g < live) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
+    }
     if constexpr (dt == 0 && g + 1 < G) pack(g + 1);
     sched_fence();
   });
@@ -289,10 +293,10 @@ AAT_DEV void pv_gemm_steps_hl(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const u
 // BLIND: as in pv_gemm_steps_hl.
 // XA: only vaddr[0] is used; d-tile dt reads at vaddr[0] ^ (dt % 4) << 6 (the Rows4 swizzle XORs the chunk-group
 // bits with row bits); implies hand-issued reads with counted waits.
-// GATE0, group0_on: as in qk_gemm_steps.
-template <int RT, int NT, int DT, int NCV, int PF, bool BLIND = false, bool XA = false, bool GATE0 = false, class Pack>
+// GATE0, group0_on: as in qk_gemm_steps.  TAIL, live: as in pv_gemm_steps_hl.
+template <int RT, int NT, int DT, int NCV, int PF, bool BLIND = false, bool XA = false, bool GATE0 = false, bool TAIL = false, class Pack>
 AAT_DEV void pv_gemm_steps(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const uint32_t (&vaddr)[DT], int buf_off,
-                           Pack&& pack, bool group0_on = true) {
+                           Pack&& pack, bool group0_on = true, int live = 2 * NT) {
   static_assert(!GATE0 || (XA && RT == 2), "the gate is built into the in-place operand ring of two row groups");
   constexpr int G = NT * 2;              // groups of 16 kv rows
   constexpr int S = G * DT;
@@ -335,7 +339,7 @@ AAT_DEV void pv_gemm_steps(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const uint
       const h8 vf = cat_h4(lo[step % PF], hi[step % PF]);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        if (!GATE0 || rt != 0 || group0_on) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
+        if ((!GATE0 || rt != 0 || group0_on) && (!TAIL || g < 2 || g < live)) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
       }
       if constexpr (step + PF < S) read(step + PF, step % PF);
     } else {
@@ -344,7 +348,9 @@ AAT_DEV void pv_gemm_steps(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const uint
       if constexpr (step + PF < S) read(step + PF, step % PF);
       const h8 vf = cat_h4(clo, chi);
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
+      for (int rt = 0; rt < RT; ++rt) {
+        if (!TAIL || g < 2 || g < live) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
+      }
     }
     if constexpr (dt == 0 && g + 1 < G) pack(g + 1);
     sched_fence();

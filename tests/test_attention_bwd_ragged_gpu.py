@@ -33,3 +33,25 @@ def test_every_rule_shape_at_the_edges_of_its_tiles(d, causal):
             for name, got, ref, t in zip(("dq", "dk", "dv"), out, want, terms):
                 ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
                 assert ok, (name, worst, ratio)
+
+
+@pytest.mark.parametrize("d", sorted(p[0] for p in gfx950_space.ATTN_BWD_RULE))
+def test_an_infinite_gradient_in_the_last_partial_tile_stays_an_infinity(d):
+    """dV = P^T dO; the query rows a tile does not have are copies of its first 32 with P = 0, and 0 * inf must not reach dV."""
+    g = torch.Generator().manual_seed(61)
+    q, k, v, do = (torch.randn(1, 2, s, d, generator=g).half() for s in (160, 96, 96, 160))
+    do[..., 5] = 0
+    o, lse = ref_op.attention_ref(q, k, v, None, False, return_lse=True)
+    o = o.half()
+    want = ref_op.attention_bwd_ref(q, k, v, do, None, False)[2]
+    terms = ref_op.attention_bwd_rounding_bound(q, k, v, do, None, False, o_stored=o)[2]
+    do[:, :, 129, 5] = float("inf")
+    for cfg in gfx950_space.rule_attn_backward_configs(d, d):
+        print(d, cfg, flush=True)
+        out = [torch.full_like(t, 7.0, device="cuda") for t in (q, k, v)]
+        Runtime(ARCH, cfg).apply([q.cuda(), k.cuda(), v.cuda(), o.cuda(), do.cuda(), lse.cuda(), *out], softmax_scale=1 / math.sqrt(d))
+        dv = out[2].cpu()
+        assert (dv[..., 5] == float("inf")).all(), cfg
+        dv[..., 5] = 0
+        ok, worst, ratio = tolerance.check_rounded_operand(dv, want, terms)
+        assert ok, (worst, ratio)

@@ -70,3 +70,21 @@ def test_a_split_call_replays_from_a_captured_graph():
         rt.apply([q, k, v, eager], causal=True)
         torch.cuda.synchronize()
         assert torch.equal(o, eager)
+
+
+@pytest.mark.parametrize("d", [p[0] for p in PAIRS])
+@pytest.mark.parametrize("sq,sk", [(96, 160), (64, 1056)])
+def test_an_infinite_value_in_the_last_partial_tile_stays_an_infinity(d, sq, sk):
+    """The kv rows a tile does not have are copies of its first 32: their P is zero, and 0 * inf must not reach the output."""
+    q, k, v = _inputs(1, 2, sq, sk, d, 40)
+    v[..., 5] = 0
+    want = ref_op.attention_ref(q, k, v)
+    v[:, :, sk - 31, 5] = float("inf")
+    for cfg in gfx950_space.rule_configs(d, d):
+        print(d, (sq, sk), cfg, flush=True)
+        o = torch.full((1, 2, sq, d), 7.0, dtype=torch.float16, device="cuda")
+        Runtime(ARCH, cfg).apply([q.cuda(), k.cuda(), v.cuda(), o], softmax_scale=1 / math.sqrt(d))
+        o = o.float().cpu()
+        assert (o[..., 5] == float("inf")).all(), cfg
+        o[..., 5] = 0
+        assert (o - want).abs().max().item() <= 2e-3, cfg
