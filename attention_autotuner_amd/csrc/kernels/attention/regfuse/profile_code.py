@@ -116,6 +116,12 @@ int kv_parts(int B, int H, int Seq_q, int Seq_k, int causal) {{
 size_t split_workspace_bytes(int parts, int B, int H, int Seq_q) {{
   return parts > 1 ? (size_t)parts * B * H * Seq_q * (D + 1) * sizeof(float) : 0;
 }}
+// Whether a call without room for its parts is an error.  A fixed number of parts that divides the kv tiles insists on it, as
+// the caller asked for those parts; everything else runs in one part instead.
+bool room_missing(int B, int H, int Seq_q, int Seq_k, int causal, const void* workspace, size_t workspace_bytes) {{
+  return kv_splits > 1 && !causal && Seq_k % Bc == 0 && (Seq_k / Bc) % kv_splits == 0 &&
+         (workspace == nullptr || workspace_bytes < split_workspace_bytes(kv_splits, B, H, Seq_q));
+}}
 size_t needed_workspace(int B, int H, int Seq_q, int Seq_k, int causal) {{
   return split_workspace_bytes(kv_parts(B, H, Seq_q, Seq_k, causal), B, H, Seq_q);
 }}
@@ -187,7 +193,7 @@ profile_func = r"""
 extern "C" float profile_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
                             float softmax_scale, int causal, void* workspace, size_t workspace_bytes, void* stream) {{
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;
-  if (kv_splits > 1 && (workspace == nullptr ? 0 : workspace_bytes) < needed_workspace(B, H, Seq_q, Seq_k, causal)) return -1.f;
+  if (room_missing(B, H, Seq_q, Seq_k, causal, workspace, workspace_bytes)) return -1.f;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return aat::timed_mean_ms(s, [&] {{ return launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, workspace_bytes, s); }});
 }}
@@ -202,7 +208,7 @@ kernel_entry = r"""
 extern "C" int kernel_entry_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
                                float softmax_scale, int causal, void* workspace, size_t workspace_bytes, void* stream) {{
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
-  if (kv_splits > 1 && (workspace == nullptr ? 0 : workspace_bytes) < needed_workspace(B, H, Seq_q, Seq_k, causal)) return AAT_ERR_WORKSPACE;
+  if (room_missing(B, H, Seq_q, Seq_k, causal, workspace, workspace_bytes)) return AAT_ERR_WORKSPACE;
   return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }}
 extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_k, int Seq_q) {{
@@ -213,7 +219,7 @@ extern "C" int kernel_entry_lse(aat_half* q, aat_half* k, aat_half* v, aat_half*
                                 int Seq_k, float softmax_scale, int causal, void* workspace, size_t workspace_bytes,
                                 void* stream) {{
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
-  if (kv_splits > 1 && (workspace == nullptr ? 0 : workspace_bytes) < needed_workspace(B, H, Seq_q, Seq_k, causal)) return AAT_ERR_WORKSPACE;
+  if (room_missing(B, H, Seq_q, Seq_k, causal, workspace, workspace_bytes)) return AAT_ERR_WORKSPACE;
   return (int)launch(q, k, v, o, B, H, Seq_q, Seq_k, softmax_scale, causal, workspace, workspace_bytes, static_cast<hipStream_t>(stream), lse);
 }}
 """

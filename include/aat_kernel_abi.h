@@ -28,7 +28,7 @@
  *     flag, an optional workspace and the stream to launch on (a hipStream_t passed as void*);
  *   - workspace_size() says how many bytes of workspace a problem needs (attention forward: 0 unless the kv
  *     range is worth cutting into parts, and then optional: without it the call runs in one part, except in a
- *     configuration with a fixed number of parts; RetNet: the mask scan of AAT_MASK_SCAN, not needed by the other
+ *     configuration with a fixed number of parts that divides the kv tiles; RetNet: the mask scan of AAT_MASK_SCAN, not needed by the other
  *     mask modes, and for a backward built with a stored dS the optional room for it); abi_version() and
  *     config_string() identify the library.
  */

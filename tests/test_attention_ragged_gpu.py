@@ -1,12 +1,14 @@
 """Attention forward at lengths its tiles do not divide and over kv ranges cut into parts: the edges of tiles, against the
 oracle (the forward's own bound, 2e-3 where |ref| < 4)."""
+import ctypes
 import math
 
 import pytest
 import torch
 
 import attention_autotuner_amd as aat
-from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space, library
+from attention_autotuner_amd.autotuner.configs import AttnConfig
 from oracle import ref_op, tolerance
 
 pytestmark = pytest.mark.gpu
@@ -88,3 +90,22 @@ def test_an_infinite_value_in_the_last_partial_tile_stays_an_infinity(d, sq, sk)
         assert (o[..., 5] == float("inf")).all(), cfg
         o[..., 5] = 0
         assert (o - want).abs().max().item() <= 2e-3, cfg
+
+
+@pytest.mark.parametrize("sk", [192, 224])
+def test_a_fixed_kv_split_that_does_not_divide_the_tiles_runs_with_and_without_room(sk):
+    q, k, v = _inputs(1, 2, 128, sk, 128, 77)
+    want, want_lse = ref_op.attention_ref(q, k, v, return_lse=True)
+    cfg = AttnConfig(128, 64, 128, 128, 128, 64, 2, 2, 256, True, waves_per_eu=2, kv_splits=4).set_fuse_type("register")
+    rt = Runtime(ARCH, cfg)
+    lib = library.load(rt._path(), "attn")
+    qc, kc, vc = (t.cuda() for t in (q, k, v))
+    room = torch.empty(rt.workspace_size(1, 2, 128, sk), dtype=torch.uint8, device="cuda")
+    for ws, nbytes in ((None, 0), (room.data_ptr(), room.numel() - 1), (room.data_ptr(), room.numel())):
+        o, lse = torch.full((1, 2, 128, 128), 7.0, dtype=torch.float16, device="cuda"), torch.full((1, 2, 128), 7.0, device="cuda")
+        torch.cuda.synchronize()
+        rc = lib.kernel_entry_lse(*[ctypes.c_void_p(t.data_ptr()) for t in (qc, kc, vc, o, lse)], 1, 2, 128, sk, ctypes.c_float(128 ** -0.5), 0,
+                                  ctypes.c_void_p(ws), ctypes.c_size_t(nbytes), None)
+        torch.cuda.synchronize()
+        assert rc == 0
+        assert (o.float().cpu() - want).abs().max().item() <= 2e-3 and (lse.cpu() - want_lse).abs().max().item() <= 1e-3

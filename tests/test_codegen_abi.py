@@ -422,6 +422,18 @@ def test_an_operator_resolves_a_problem_once_and_again_after_a_tuning_result_is_
     base_tunner._memo.clear()
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="hands over null pointers: nothing may be launched")
+def test_a_fixed_kv_split_insists_on_its_room_only_where_its_parts_divide_the_tiles():
+    import ctypes
+    null, scale = ctypes.c_void_p(0), ctypes.c_float(0.1)
+    cfg = AttnConfig(128, 64, 128, 128, 128, 64, 2, 2, 256, True, waves_per_eu=2, kv_splits=8).set_fuse_type("register")
+    lib = library.load(codegen.compile_config(cfg, ARCH, timeout=600), "attn")
+    for sk, causal, refused in ((1024, 0, True), (1024, 1, False), (576, 0, False), (1056, 0, False)):
+        tail = (1, 4, 256, sk, scale, causal, null, ctypes.c_size_t(0), null)
+        for rc in (lib.kernel_entry_ex(*[null] * 4, *tail), lib.kernel_entry_lse(*[null] * 5, *tail)):
+            assert (rc == -3) == refused, (sk, causal, rc)
+
+
 def test_the_library_cuts_the_kv_range_as_the_tile_shape_rule_assumes():
     """gfx950_space.kv_parts and the library's own choice (kv_parts.h) are one estimate, written twice."""
     for d in (64, 128, 256):
