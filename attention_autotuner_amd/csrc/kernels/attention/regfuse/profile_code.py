@@ -128,6 +128,7 @@ size_t needed_workspace(int B, int H, int Seq_q, int Seq_k, int causal) {{
 
 hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
                   float softmax_scale, int causal, void* workspace, size_t workspace_bytes, hipStream_t stream, float* lse = nullptr) {{
+  causal = causal != 0;                          // any value but 0 asks for the causal walk; the general kernel multiplies by it
   const int parts = kv_parts(B, H, Seq_q, Seq_k, causal);
   if (parts > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(parts, B, H, Seq_q)) {{
     static const hipError_t lds_ok_split = aat::allow_lds(kernel_split, shared_mem_split);

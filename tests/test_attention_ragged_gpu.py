@@ -109,3 +109,22 @@ def test_a_fixed_kv_split_that_does_not_divide_the_tiles_runs_with_and_without_r
         torch.cuda.synchronize()
         assert rc == 0
         assert (o.float().cpu() - want).abs().max().item() <= 2e-3 and (lse.cpu() - want_lse).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("sq,sk", [(96, 160), (64, 4160)])
+def test_any_causal_flag_but_zero_asks_for_the_causal_walk(sq, sk):
+    """The C entry takes an int; at lengths the tiles do not divide and over a kv range cut into parts too."""
+    q, k, v = _inputs(1, 2, sq, sk, 128, 91)
+    want = ref_op.attention_ref(q, k, v, None, True)
+    for cfg in gfx950_space.rule_configs(128, 128):
+        rt = Runtime(ARCH, cfg)
+        lib = library.load(rt._path(), "attn")
+        qc, kc, vc = (t.cuda() for t in (q, k, v))
+        room = torch.empty(max(1, rt.workspace_size(1, 2, sq, sk)), dtype=torch.uint8, device="cuda")
+        for causal in (1, 2, -1):
+            o = torch.full((1, 2, sq, 128), 7.0, dtype=torch.float16, device="cuda")
+            torch.cuda.synchronize()
+            rc = lib.kernel_entry_ex(*[ctypes.c_void_p(t.data_ptr()) for t in (qc, kc, vc, o)], 1, 2, sq, sk, ctypes.c_float(128 ** -0.5), causal,
+                                     ctypes.c_void_p(room.data_ptr()), ctypes.c_size_t(room.numel()), None)
+            torch.cuda.synchronize()
+            assert rc == 0 and (o.float().cpu() - want).abs().max().item() <= 2e-3, (cfg, causal)
