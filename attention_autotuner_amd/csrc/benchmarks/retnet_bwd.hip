@@ -122,12 +122,12 @@ static void test_retnet_bwd(const ProblemShape& ps, Tensors& t) {
     std::printf("%-52s skipped: sequence lengths %% %d or %% %d\n", name, Br, Bc);
     return;
   }
-  auto dv_plain = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, false>;
-  auto dk_plain = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, false>;
-  auto dq_plain = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, false>;
-  auto dv_decay = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, true>;
-  auto dk_decay = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, true>;
-  auto dq_decay = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, true>;
+  auto dv_plain = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, 0, false>;
+  auto dk_plain = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, 0, false>;
+  auto dq_plain = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, 0, false>;
+  auto dv_decay = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, 0, true>;
+  auto dk_decay = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, 0, true>;
+  auto dq_decay = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, 0, true>;
   HIP_OK(hipFuncSetAttribute((const void*)dv_plain, hipFuncAttributeMaxDynamicSharedMemorySize, TV::kSmemBytes));
   HIP_OK(hipFuncSetAttribute((const void*)dv_decay, hipFuncAttributeMaxDynamicSharedMemorySize, TV::kSmemBytes));
   HIP_OK(hipFuncSetAttribute((const void*)dk_plain, hipFuncAttributeMaxDynamicSharedMemorySize, TK::kSmemBytes));
@@ -185,10 +185,10 @@ static void test_retnet_bwd_stored_ds(const ProblemShape& ps, Tensors& t) {
     std::printf("%-70s skipped: sequence lengths\n", name);
     return;
   }
-  auto dv_plain = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, false>;
-  auto dq_plain = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, false, true>;
-  auto dv_decay = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, true>;
-  auto dq_decay = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, true, true>;
+  auto dv_plain = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, 0, false>;
+  auto dq_plain = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, 0, false, true>;
+  auto dv_decay = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, NT, NSY, NSZ, BwdPass::Col, WPE, 0, true>;
+  auto dq_decay = &aat::ret_bwd_chain<D, Kd, Kd, Br, Bc, NT, NSY, NSZ, BwdPass::Row, WPE, 0, true, true>;
   auto dk_ds = &aat::ret_bwd_dk_from_ds<Kd, KBX, KBY, KNT, KNS, KWPE>;
   HIP_OK(hipFuncSetAttribute((const void*)dv_plain, hipFuncAttributeMaxDynamicSharedMemorySize, TV::kSmemBytes));
   HIP_OK(hipFuncSetAttribute((const void*)dv_decay, hipFuncAttributeMaxDynamicSharedMemorySize, TV::kSmemBytes));

@@ -22,8 +22,8 @@
 //     dQ  ROW   dO   V    K    dQ    q row       x (q)     row-major
 //
 // No atomics, no scratch, deterministic; dQ is written directly in fp16, so the reference's second
-// kernel has no counterpart.  Resident rows come in any multiple of 32 (the 32-row groups a last block does not have repeat
-// its first one, see below), streamed rows in multiples of BY.  Cost: dO V^T is evaluated twice (3*(d_qk+d_v) instead of 3*d_qk+2*d_v
+// kernel has no counterpart.  Resident rows come in multiples of BX, with GEN in any multiple of 32; streamed rows in
+// multiples of BY.  Cost: dO V^T is evaluated twice (3*(d_qk+d_v) instead of 3*d_qk+2*d_v
 // multiply-adds per score) and, for an output wider than DZB columns, the first contraction is repeated
 // per column slice (grid.y slices).
 #pragma once
@@ -85,8 +85,12 @@ struct RetBwdChain {
 // from lg2gamma[h] = log2(gamma_h); `mask` is not read and tiles above the diagonal are skipped.
 // DS_OUT (row pass only): the fp16 E tiles (= dS) this pass forms are also written to ds_out (64 x 64 blocks, ds_layout.h), for
 // a dK kernel that reads them instead of evaluating them again (dk_from_ds.h).  Only the tiles of the walk are written.
+// GEN: resident lengths that are multiples of 32 and not of BX; the 32-row groups a last block does not have repeat its first
+// one (below).  Whole blocks keep the form without it, because every mask copy of every tile pays a comparison and a 64-bit
+// select for it: 78 scalar registers instead of 70 in the dV pass at 256/512, 86 instead of 74 in dQ + dS, and 538 us instead of
+// 533 for forward + backward at B4 H8 S2048.
 template <int KX, int DZ, int DZB, int BX, int BY, int Nthreads, int NSY, int NSZ, BwdPass PASS, int WPE = 1,
-          bool DECAY = false, bool DS_OUT = false>
+          int GEN = 0, bool DECAY = false, bool DS_OUT = false>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const half_t* __restrict__ z,
               const half_t* __restrict__ mask, const float* __restrict__ r, half_t* __restrict__ out, int H,
@@ -117,7 +121,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   const int n = lane & 31, h = lane >> 5;
   const int seq_x = COL ? seq_k : seq_q, seq_y = COL ? seq_q : seq_k;
 
-  const int Tx = (seq_x + BX - 1) / BX;
+  const int Tx = GEN ? (seq_x + BX - 1) / BX : seq_x / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
   if (causal || extents != nullptr) {             // longest blocks first: the last query blocks, the first kv blocks
@@ -126,7 +130,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
     xb = t.blk;
   }
   const int x0 = xb * BX;
-  const int rows = seq_x - x0 < BX ? seq_x - x0 : BX;       // resident rows of this block that exist
+  const int rows = GEN && seq_x - x0 < BX ? seq_x - x0 : BX;   // resident rows of this block that exist
   const int dz0 = blockIdx.y * DZB;               // first output column of this block
   const int diag = seq_k - seq_q;                 // mask[q][kv] may be non-zero only for kv <= q + diag
   int j_begin = 0, j_end = seq_y / BY;
@@ -160,7 +164,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   typename T::MDma mdma;
   ydma.init(tid);
   zdma.init(tid, DZ * 2);
-  mdma.init(tid, seq_k * 2, COL ? rows / 8 : T::NCM);       // COL: the block's columns of the mask
+  mdma.init(tid, seq_k * 2, GEN && COL ? rows / 8 : T::NCM);   // COL: the block's columns of the mask
   const int wave_base = wave * 64;
 
   // A 32-row group that does not exist repeats the block's first one in everything: the same rows of X, of r and of the mask
@@ -170,7 +174,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   int groups = 0, row_of[RT];                     // groups of this wave that exist (its first ones); where a group's rows start
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    const bool exists = wave * WM + rt * 32 < rows;
+    const bool exists = !GEN || wave * WM + rt * 32 < rows;
     groups += exists ? 1 : 0;
     row_of[rt] = x0 + (exists ? wave * WM + rt * 32 : 0);
     load_q_frags<1, KS, KX>(reinterpret_cast<h8(&)[1][KS]>(xf[rt]), x + ((size_t)bh * seq_x + row_of[rt] + n) * KX + 8 * h);
@@ -231,7 +235,8 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
     ydma.issue(yg + (size_t)jt * T::kYBytes, ybuf + st * T::kYBytes, wave_base);
     if constexpr (!DECAY) {
       const char* msrc = COL ? mg + (size_t)jt * BY * seq_k * 2 : mg + (size_t)jt * BY * 2;
-      mdma.issue_rows(msrc, mbuf + st * T::kMBytes, wave_base, COL ? BY : rows);
+      if constexpr (GEN && !COL) mdma.issue_rows(msrc, mbuf + st * T::kMBytes, wave_base, rows);
+      else mdma.issue(msrc, mbuf + st * T::kMBytes, wave_base);
     }
   };
   auto issue_z = [&](int j, int st) {
@@ -316,7 +321,10 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
         if (NSY > 1 && ym_now) ydma.issue_one(i - kZi, ysrc, ybuf + yslot * T::kYBytes, wave_base);
       } else if (i < kZi + kYi + kMi) {
         if constexpr (!DECAY) {
-          if (NSY > 1 && ym_now) mdma.issue_one_of_rows(i - kZi - kYi, msrc, mbuf + yslot * T::kMBytes, wave_base, COL ? BY : rows);
+          if (NSY > 1 && ym_now) {
+            if constexpr (GEN && !COL) mdma.issue_one_of_rows(i - kZi - kYi, msrc, mbuf + yslot * T::kMBytes, wave_base, rows);
+            else mdma.issue_one(i - kZi - kYi, msrc, mbuf + yslot * T::kMBytes, wave_base);
+          }
         }
       }
     };

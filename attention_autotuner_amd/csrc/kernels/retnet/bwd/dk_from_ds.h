@@ -49,9 +49,10 @@ struct RetBwdDk {
 
 // q [B*H, seq_q, Kd], ds in 64 x 64 blocks (above), dk [B*H, seq_k, Kd], all fp16.
 // causal / extents: the mask mode of the walk, as in ret_bwd_chain (extents = the scan's ranges or nullptr).
-// seq_q and seq_k are multiples of 64; kv rows a last block does not have are computed from copies and not stored.
+// seq_q is a multiple of wr_rows and seq_k of BX; GEN: both of 64, kv rows a last block does not have are computed from copies
+// and not stored.
 // wr_rows x wr_cols: resident rows and streamed-tile width of the row pass that wrote ds (wr_rows % BY == 0).
-template <int Kd, int BX, int BY, int Nthreads, int NS, int WPE = 2>
+template <int Kd, int BX, int BY, int Nthreads, int NS, int WPE = 2, int GEN = 0>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, half_t* __restrict__ dk, int H,
                    int seq_k, int seq_q, int causal, const int* __restrict__ extents, int wr_rows, int wr_cols) {
@@ -64,7 +65,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
-  const int Tx = (seq_k + BX - 1) / BX;
+  const int Tx = GEN ? (seq_k + BX - 1) / BX : seq_k / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
   if (causal || extents != nullptr) {             // longest blocks first: the first kv blocks
@@ -73,7 +74,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     xb = t.blk;
   }
   const int x0 = xb * BX;
-  const int cols = seq_k - x0 < BX ? seq_k - x0 : BX;       // kv rows of this block that exist, a multiple of 64
+  const int cols = GEN && seq_k - x0 < BX ? seq_k - x0 : BX;   // kv rows of this block that exist, a multiple of 64
   const int diag = seq_k - seq_q;
   const int head = bh % H;
   int j_begin = 0, j_end = seq_q / BY;
@@ -102,7 +103,8 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     const int jt = tile_of(j);
     char* base = smem + st * T::kStageBytes;
     zdma.issue(zg + (size_t)jt * T::kZBytes, base, wave_base);
-    sdma.issue_rows(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base, cols / 64 * BY);   // the dS blocks that exist
+    if constexpr (GEN) sdma.issue_rows(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base, cols / 64 * BY);   // the dS blocks that exist
+    else sdma.issue(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base);
   };
 
   // LDS addresses inside stage 0: Q^T fragments (A operand, d-tile dt) and this wave's dS columns (B operand);
@@ -152,7 +154,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     // the kv range the writer covered for the row block this query tile lies in
     const int jt = tile_of(j);
     const int wx0 = (jt * BY) / wr_rows * wr_rows;
-    const int wrows = seq_q - wx0 < wr_rows ? seq_q - wx0 : wr_rows;
+    const int wrows = GEN && seq_q - wx0 < wr_rows ? seq_q - wx0 : wr_rows;
     int wlo = 0, whi = seq_k;
     if (extents != nullptr) {
       int lo, hi, jb, je;
@@ -217,7 +219,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   block_sync();
   const float one[1] = {1.f};
   store_o_tile<1, DT, Kd, T::kOStride>(acc, one, smem + wave * 32 * T::kOStride,
-                                       dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane, 32, wave * 32 < cols ? 1 : 0);
+                                       dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane, 32, !GEN || wave * 32 < cols ? 1 : 0);
 }
 
 }  // namespace aat

@@ -43,17 +43,14 @@ using aat::BwdPass;
 using TV = aat::RetBwdChain<Kd, D, DVB, Br, Bc, Nthreads, num_stages_qk, num_stages_dv, BwdPass::Col>;
 using TK = aat::RetBwdChain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Col>;
 using TQ = aat::RetBwdChain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row>;
-const auto kernel_dv = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, Nthreads, num_stages_qk, num_stages_dv, BwdPass::Col, waves_per_eu>;
-const auto kernel_dk = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Col, waves_per_eu>;
-const auto kernel_dq = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu>;
-const auto decay_dv = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, Nthreads, num_stages_qk, num_stages_dv, BwdPass::Col, waves_per_eu, true>;
-const auto decay_dk = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Col, waves_per_eu, true>;
-const auto decay_dq = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, true>;
+// GEN = 1: resident lengths the blocks do not divide
+template <bool DECAY, int GEN> constexpr auto kernel_dv = &aat::ret_bwd_chain<Kd, D, DVB, Br, Bc, Nthreads, num_stages_qk, num_stages_dv, BwdPass::Col, waves_per_eu, GEN, DECAY, false>;
+template <bool DECAY, int GEN> constexpr auto kernel_dk = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Col, waves_per_eu, GEN, DECAY, false>;
+template <bool DECAY, int GEN> constexpr auto kernel_dq = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, GEN, DECAY, false>;
 // stored dS: the row pass that writes it (the plain one again in a library without it), the dK kernel that reads it
 using TKD = aat::RetBwdDk<Kd, kDkRows, kDkTile, kDkRows * 2, kDkStages>;
-const auto kernel_dq_ds = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, false, kStoredDs>;
-const auto decay_dq_ds = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, true, kStoredDs>;
-const auto kernel_dk_ds = &aat::ret_bwd_dk_from_ds<Kd, kDkRows, kDkTile, kDkRows * 2, kDkStages, kDkWaves>;
+template <bool DECAY, int GEN> constexpr auto kernel_dq_ds = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, GEN, DECAY, kStoredDs>;
+template <int GEN> constexpr auto kernel_dk_ds = &aat::ret_bwd_dk_from_ds<Kd, kDkRows, kDkTile, kDkRows * 2, kDkStages, kDkWaves, GEN>;
 static_assert(!kStoredDs || Br % kDkTile == 0, "a query tile of the dK kernel lies inside one block of the row pass");
 
 bool bwd_shape_ok(int B, int H, int Seq_q, int Seq_k) {{
@@ -82,68 +79,56 @@ bool room_for_ds(const void* workspace, size_t workspace_bytes, int B, int H, in
   return stores_ds(B, H, Seq_q, Seq_k) && workspace != nullptr && workspace_bytes >= ws_bytes_needed(B, H, Seq_q, Seq_k);
 }}
 
-hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* dO, float* r, aat_half* dq,
-                  aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, int mask_mode, void* workspace,
-                  size_t workspace_bytes, hipStream_t stream) {{
-  static const hipError_t ok1 = aat::allow_lds(kernel_dv, TV::kSmemBytes);
-  static const hipError_t ok2 = aat::allow_lds(kernel_dk, TK::kSmemBytes);
-  static const hipError_t ok3 = aat::allow_lds(kernel_dq, TQ::kSmemBytes);
-  static const hipError_t ok4 = kStoredDs ? aat::allow_lds(kernel_dk_ds, TKD::kSmemBytes) : hipSuccess;
-  static const hipError_t ok5 = kStoredDs ? aat::allow_lds(kernel_dq_ds, TQ::kSmemBytesDsOut) : hipSuccess;
-  for (hipError_t e : {{ok1, ok2, ok3, ok4, ok5}})
+// DECAY: the mask is gamma_h^(q + Seq_k - Seq_q - kv) below the diagonal, zero above it, and `mask` and `walk` are not looked at.
+template <bool DECAY> hipError_t launch_passes(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, const float* log2_gamma, aat_half* dO,
+                                               float* r, aat_half* dq, aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k,
+                                               aat::MaskWalk walk, void* workspace, size_t workspace_bytes, hipStream_t stream) {{
+  static const hipError_t allowed[] = {{
+      aat::allow_lds(kernel_dv<DECAY, 0>, TV::kSmemBytes), aat::allow_lds(kernel_dv<DECAY, 1>, TV::kSmemBytes),
+      aat::allow_lds(kernel_dk<DECAY, 0>, TK::kSmemBytes), aat::allow_lds(kernel_dk<DECAY, 1>, TK::kSmemBytes),
+      aat::allow_lds(kernel_dq<DECAY, 0>, TQ::kSmemBytes), aat::allow_lds(kernel_dq<DECAY, 1>, TQ::kSmemBytes),
+      kStoredDs ? aat::allow_lds(kernel_dk_ds<0>, TKD::kSmemBytes) : hipSuccess,
+      kStoredDs ? aat::allow_lds(kernel_dk_ds<1>, TKD::kSmemBytes) : hipSuccess,
+      kStoredDs ? aat::allow_lds(kernel_dq_ds<DECAY, 0>, TQ::kSmemBytesDsOut) : hipSuccess,
+      kStoredDs ? aat::allow_lds(kernel_dq_ds<DECAY, 1>, TQ::kSmemBytesDsOut) : hipSuccess}};
+  for (hipError_t e : allowed)
     if (e != hipSuccess) return e;
   using H16 = aat::half_t;
   const H16 *Q = reinterpret_cast<const H16*>(q), *K = reinterpret_cast<const H16*>(k), *V = reinterpret_cast<const H16*>(v),
             *M = reinterpret_cast<const H16*>(mask), *G = reinterpret_cast<const H16*>(dO);
-  aat::MaskWalk walk;
-  const hipError_t scanned = aat::prepare_mask_walk(mask_mode, M, H, Seq_q, Seq_k, workspace, stream, &walk);
-  if (scanned != hipSuccess) return scanned;
-  const int causal = walk.causal;
-  kernel_dv<<<dim3(B * H * blocks_of(Seq_k), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
-      K, Q, G, M, r, reinterpret_cast<H16*>(dv), H, Seq_k, Seq_q, causal, nullptr, walk.extents, nullptr);
+  H16 *DQ = reinterpret_cast<H16*>(dq), *DK = reinterpret_cast<H16*>(dk), *DV = reinterpret_cast<H16*>(dv);
+  const int causal = DECAY ? 1 : walk.causal;
+  const int* extents = DECAY ? nullptr : walk.extents;
+  const bool whole_q = Seq_q % Br == 0, whole_k = Seq_k % Br == 0;
+  (whole_k ? kernel_dv<DECAY, 0> : kernel_dv<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_k), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
+      K, Q, G, M, r, DV, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr);
   if (room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k)) {{
     H16* ds = reinterpret_cast<H16*>(static_cast<char*>(workspace) + ds_offset(H, Seq_q, Seq_k));
-    kernel_dq_ds<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
-        G, V, K, M, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, causal, nullptr, walk.extents, ds);
-    kernel_dk_ds<<<dim3(B * H * ((Seq_k + kDkRows - 1) / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
-        Q, ds, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, causal, walk.extents, Br, Bc);
+    (whole_q ? kernel_dq_ds<DECAY, 0> : kernel_dq_ds<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
+        G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, ds);
+    (whole_q && Seq_k % kDkRows == 0 ? kernel_dk_ds<0> : kernel_dk_ds<1>)<<<dim3(B * H * ((Seq_k + kDkRows - 1) / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
+        Q, ds, DK, H, Seq_k, Seq_q, causal, extents, Br, Bc);
   }} else {{
-    kernel_dk<<<dim3(B * H * blocks_of(Seq_k), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
-        V, G, Q, M, r, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, causal, nullptr, walk.extents, nullptr);
-    kernel_dq<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
-        G, V, K, M, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, causal, nullptr, walk.extents, nullptr);
+    (whole_k ? kernel_dk<DECAY, 0> : kernel_dk<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_k), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
+        V, G, Q, M, r, DK, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr);
+    (whole_q ? kernel_dq<DECAY, 0> : kernel_dq<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
+        G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr);
   }}
   return hipGetLastError();
 }}
-// Decay-mask variant: the mask is gamma_h^(q + Seq_k - Seq_q - kv) below the diagonal, zero above it.
+hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* dO, float* r, aat_half* dq,
+                  aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, int mask_mode, void* workspace,
+                  size_t workspace_bytes, hipStream_t stream) {{
+  aat::MaskWalk walk;
+  const hipError_t scanned = aat::prepare_mask_walk(mask_mode, reinterpret_cast<const aat::half_t*>(mask), H, Seq_q, Seq_k,
+                                                    workspace, stream, &walk);
+  if (scanned != hipSuccess) return scanned;
+  return launch_passes<false>(q, k, v, mask, nullptr, dO, r, dq, dk, dv, B, H, Seq_q, Seq_k, walk, workspace, workspace_bytes, stream);
+}}
 hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* dO, float* r,
                         aat_half* dq, aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, void* workspace,
                         size_t workspace_bytes, hipStream_t stream) {{
-  static const hipError_t ok1 = aat::allow_lds(decay_dv, TV::kSmemBytes);
-  static const hipError_t ok2 = aat::allow_lds(decay_dk, TK::kSmemBytes);
-  static const hipError_t ok3 = aat::allow_lds(decay_dq, TQ::kSmemBytes);
-  static const hipError_t ok4 = kStoredDs ? aat::allow_lds(kernel_dk_ds, TKD::kSmemBytes) : hipSuccess;
-  static const hipError_t ok5 = kStoredDs ? aat::allow_lds(decay_dq_ds, TQ::kSmemBytesDsOut) : hipSuccess;
-  for (hipError_t e : {{ok1, ok2, ok3, ok4, ok5}})
-    if (e != hipSuccess) return e;
-  using H16 = aat::half_t;
-  const H16 *Q = reinterpret_cast<const H16*>(q), *K = reinterpret_cast<const H16*>(k), *V = reinterpret_cast<const H16*>(v),
-            *G = reinterpret_cast<const H16*>(dO);
-  decay_dv<<<dim3(B * H * blocks_of(Seq_k), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
-      K, Q, G, nullptr, r, reinterpret_cast<H16*>(dv), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, nullptr);
-  if (room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k)) {{
-    H16* ds = reinterpret_cast<H16*>(static_cast<char*>(workspace) + ds_offset(H, Seq_q, Seq_k));
-    decay_dq_ds<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
-        G, V, K, nullptr, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, ds);
-    kernel_dk_ds<<<dim3(B * H * ((Seq_k + kDkRows - 1) / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
-        Q, ds, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, 1, nullptr, Br, Bc);
-  }} else {{
-    decay_dk<<<dim3(B * H * blocks_of(Seq_k), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
-        V, G, Q, nullptr, r, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, nullptr);
-    decay_dq<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
-        G, V, K, nullptr, r, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, 1, log2_gamma, nullptr, nullptr);
-  }}
-  return hipGetLastError();
+  return launch_passes<true>(q, k, v, nullptr, log2_gamma, dO, r, dq, dk, dv, B, H, Seq_q, Seq_k, aat::MaskWalk(), workspace, workspace_bytes, stream);
 }}
 }}  // namespace
 

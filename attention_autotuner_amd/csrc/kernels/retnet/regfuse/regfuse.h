@@ -8,9 +8,11 @@
 // through LDS as a third DMA stream, and the normalisation is lazy (utils/retention.h).
 // `causal` promises a mask that is zero above the diagonal and only shortens the kv walk.
 //
-// seq_q is any multiple of 32, seq_k a multiple of Bc.  The 32-row groups the last row block of a head does not have repeat
-// its first group -- same loads, same arithmetic -- and are not stored: a select per mask copy and per group, nothing in the
-// loop.  (Where no 128-row tile divided the length the row blocks were 64 rows of two waves, with one buffer per stream.)
+// seq_k is a multiple of Bc, seq_q one of Br.  GEN: seq_q is any multiple of 32; the 32-row groups the last row block of a
+// head does not have repeat its first group -- same loads, same arithmetic -- and are not stored.  (Where no 128-row tile
+// divided the length the row blocks were 64 rows of two waves, with one buffer per stream.)  Every mask copy of
+// every tile pays a comparison and a 64-bit select of its source for it, so whole row blocks keep the form without (forward and
+// backward together at B4 H8 S2048 256/512: 538 us with the selects everywhere, 533 with none at whole blocks).
 #pragma once
 #include <type_traits>
 
@@ -51,7 +53,8 @@ struct RetFwdRegfuse {
 
 // DECAY: the mask is gamma_h^(q + diag - kv) below the diagonal and zero above it, built in registers
 // from lg2gamma[h] = log2(gamma_h); `mask` is not read and tiles above the diagonal are skipped.
-template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, bool DECAY = false>
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, int GEN = 0,
+          bool DECAY = false>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
                 const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H,
@@ -75,7 +78,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
-  const int Tr = (seq_q + Br - 1) / Br;
+  const int Tr = GEN ? (seq_q + Br - 1) / Br : seq_q / Br;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tr, rb = tile % Tr;
   if (causal || extents != nullptr) {             // a scanned mask is taken to be of the causal kind: later rows see more
@@ -84,7 +87,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
     rb = t.blk;
   }
   const int q0 = rb * Br;
-  const int rows = seq_q - q0 < Br ? seq_q - q0 : Br;      // of this block that exist
+  const int rows = GEN && seq_q - q0 < Br ? seq_q - q0 : Br;   // of this block that exist
   int n_tiles = seq_k / Bc;
   if (extents != nullptr) {                       // walk up to the last kv tile in which the mask has a non-zero entry
     int lo, hi, j_begin;
@@ -116,7 +119,7 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   int row_of[RT];                                 // where a group's rows start inside the block
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    const bool exists = wave * WM + rt * 32 < rows;
+    const bool exists = !GEN || wave * WM + rt * 32 < rows;
     groups += exists ? 1 : 0;
     row_of[rt] = exists ? wave * WM + rt * 32 : 0;
     load_q_frags<1, KS, Kd>(reinterpret_cast<h8(&)[1][KS]>(qf[rt]), q + ((size_t)bh * seq_q + q0 + row_of[rt] + n) * Kd + 8 * h);
@@ -147,7 +150,10 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   }
   auto issue_km = [&](int j, int par) {          // K tile j and mask tile j travel together
     kdma.issue(kg + (size_t)j * T::kKBytes, kbuf + (NSK == 2 ? par * T::kKBytes : 0), wave_base);
-    if constexpr (!DECAY) mdma.issue_rows(mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base, rows);
+    if constexpr (!DECAY) {
+      if constexpr (GEN) mdma.issue_rows(mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base, rows);
+      else mdma.issue(mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base);
+    }
   };
   if (n_tiles > 0) {
     issue_km(0, 0);
@@ -163,7 +169,8 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
     constexpr int KI = T::KDma::kIters, VI = T::VDma::kIters, MI = DECAY ? 0 : T::MDma::kIters;
     auto issue_km_one = [&](int j, int par, int i) {          // instruction i of the K copy followed by the mask copy
       if (i < KI) kdma.issue_one(i, kg + (size_t)j * T::kKBytes, kbuf + (NSK == 2 ? par * T::kKBytes : 0), wave_base);
-      else if constexpr (!DECAY) mdma.issue_one_of_rows(i - KI, mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base, rows);
+      else if constexpr (!DECAY && GEN) mdma.issue_one_of_rows(i - KI, mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base, rows);
+      else if constexpr (!DECAY) mdma.issue_one(i - KI, mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base);
     };
     // One loop body for both buffer parities: the parity is a run-time value that moves the operand addresses and the
     // copy destinations.

@@ -266,6 +266,21 @@ def test_resource_report_is_parsed_and_decides_what_the_tuner_times(tmp_path, mo
     assert any("flashattn_fwd_regfuse" in k["kernel"] for k in report)
 
 
+def test_whole_blocks_carry_no_selects_for_partial_ones():
+    """RetNet at lengths the row blocks divide: the kernels are built without the rebased mask copies of the general form, which
+    show in the scalar registers (dV 70, dQ with stored dS 74 at 256/512 before there was a general form)."""
+    cfg = gfx950_space.rule_ret_configs("ret_bwd", 256, 512)[-1]
+    assert (cfg.Br, cfg.Bc, cfg.ds_rows) == (128, 64, 128)
+    sgprs = {}
+    for k in codegen.resource_usage(codegen.compile_config(cfg, ARCH, timeout=600)):
+        flags, general = codegen.template_bools(k["kernel"]), codegen.general_form(k["kernel"])       # <..., GEN, DECAY, DS_OUT>
+        if flags == [False, False] and "ILi256ELi512E" in k["kernel"]:
+            sgprs["dv", general] = k["sgprs"]
+        if flags == [False, True]:
+            sgprs["dq", general] = k["sgprs"]
+    assert sgprs["dv", False] <= 70 < sgprs["dv", True] and sgprs["dq", False] <= 74 < sgprs["dq", True], sgprs
+
+
 def test_tune_skips_a_candidate_the_compiler_reports_as_spilling(tmp_path, monkeypatch):
     """The loop never times (here: never even loads) a library whose report shows a spilled working set."""
     from attention_autotuner_amd.benchmarks.tune import make_tensors
