@@ -255,9 +255,10 @@ class BaseTunner:
         _memo[self._memo_key()] = config
 
     # ---- what is not worth timing ----------------------------------------------------------------------
-    def _kernel_matters(self, mangled):
+    def _kernel_matters(self, mangled, config=None):
         """Whether a kernel of a candidate library is one this tuner's problem launches (a library holds
-        several variants: causal or not, decay mask or mask tensor)."""
+        several variants: causal or not, decay mask or mask tensor, whole tiles or any length).  ``config``: the
+        candidate; without it the lengths are taken to be whole tiles."""
         return True
 
     # A fitted costmodel.CostModel: tune() then times only its best-ranked candidates.  Subclasses name a model file
@@ -316,7 +317,7 @@ class BaseTunner:
         for res in results:
             if res.lib_name is None:
                 continue                                  # compile failed or timed out
-            spills = codegen.spilling_kernels(codegen.resource_usage(res.lib_name), self._kernel_matters)
+            spills = codegen.spilling_kernels(codegen.resource_usage(res.lib_name), lambda name: self._kernel_matters(name, res.config))
             if spills and os.environ.get("AAT_TUNE_SPILLS", "0") == "0":
                 # the compiler says this candidate keeps part of its working set in scratch memory: not worth timing
                 self.rejected_spills[res.config] = max(k.get("scratch_bytes", 0) for k in spills)

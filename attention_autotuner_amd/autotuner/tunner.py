@@ -49,11 +49,18 @@ class _ForwardTunner(BaseTunner):
     validate_register_fuse = _validate
     validate_shared_fuse = _validate
 
-    def _kernel_matters(self, mangled):
-        flags = codegen.template_bools(mangled)
-        if self.operation == "ret":                       # <..., DECAY>
-            return not flags or flags[-1] == bool(self.decay)
-        if "flashattn_fwd_regfuse" in mangled and len(flags) == 5:     # <..., PIPE, CAUSAL, SPLIT, PERSIST, PAIR>
+    def _kernel_matters(self, mangled, config=None):
+        flags, general = codegen.template_bools(mangled), codegen.general_form(mangled)
+        s = self.problem_shape
+        whole = config is None or s["Sq"] % config.Br == 0
+        if self.operation == "ret":                       # <..., GEN, DECAY>
+            return (not flags or flags[-1] == bool(self.decay)) and general in (None, not whole)
+        if "flashattn_fwd_regfuse" in mangled and len(flags) == 5:     # <..., GEN, PIPE, CAUSAL, SPLIT, PERSIST, PAIR>
+            # one general kernel, for both walks, in one part or in several; the others at whole tiles in one part
+            parts = 1 if config is None else gfx950_space.kv_parts(config, self.arch, s["B"], s["H"], s["Sq"], s["Sk"], self.causal)
+            whole = whole and (config is None or s["Sk"] % config.Bc == 0)
+            if general or parts > 1 or not whole:
+                return bool(general) and (parts > 1 or not whole) and flags[2] == (parts > 1)
             # the persistent and the paired variant are not launched from a build that spills (the wrapper asks the runtime)
             return flags[1] == bool(self.causal) and not flags[3] and not flags[4]
         if "flashattn_fwd_smemfuse" in mangled and flags:              # <..., CAUSAL>
@@ -128,9 +135,15 @@ class RetBwdTunner(BaseTunner):
             return gfx950_space.backward_valid(config, self.arch)
         return _foreign_space(self.arch).backward_valid(config, self.arch)
 
-    def _kernel_matters(self, mangled):                   # ret_bwd_chain<..., PASS, WPE, DECAY, DS_OUT>; the dK-from-dS kernel has no flags
-        flags = codegen.template_bools(mangled)
-        return len(flags) != 2 or flags[0] == bool(self.decay)
+    def _kernel_matters(self, mangled, config=None):      # ret_bwd_chain<..., PASS, WPE, GEN, DECAY, DS_OUT>; the dK-from-dS kernel has no flags
+        flags, general = codegen.template_bools(mangled), codegen.general_form(mangled)
+        whole_q = config is None or self.problem_shape["Sq"] % config.Br == 0
+        whole_k = config is None or self.problem_shape["Sk"] % config.Br == 0
+        if "ret_bwd_dk_from_ds" in mangled:
+            whole = whole_q and (config is None or not config.ds_rows or self.problem_shape["Sk"] % config.ds_rows == 0)
+        else:
+            whole = whole_q if "BwdPassE1E" in mangled else whole_k       # the row pass keeps query rows resident
+        return (len(flags) != 2 or flags[0] == bool(self.decay)) and general in (None, not whole)
 
     def tune(self, *a, **kw):
         if not _is_rocm(self.arch):
@@ -156,6 +169,11 @@ class AttnBwdTunner(BaseTunner):
 
     def validate_kernel(self, config):
         return gfx950_space.attn_backward_valid(config, self.arch)
+
+    def _kernel_matters(self, mangled, config=None):      # attn_bwd_chain<..., PASS, WPE, OUTS, GEN>
+        s = self.problem_shape
+        whole = config is None or (s["Sq"] % config.Br == 0 and s["Sk"] % config.Br == 0 and s["Sq"] % config.Bc == 0 and s["Sk"] % config.row_Bc == 0)
+        return codegen.general_form(mangled) in (None, not whole)
 
     def _ex_args(self):
         scale = self.softmax_scale

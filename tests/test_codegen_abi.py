@@ -266,6 +266,43 @@ def test_resource_report_is_parsed_and_decides_what_the_tuner_times(tmp_path, mo
     assert any("flashattn_fwd_regfuse" in k["kernel"] for k in report)
 
 
+def test_the_spill_gate_looks_at_the_form_a_problem_launches():
+    """Real reports of built libraries: whole tiles, partial tiles and a cut kv range launch different kernels of one library."""
+    from attention_autotuner_amd.autotuner import RetBwdTunner, RetTunner, AttnBwdTunner
+    from attention_autotuner_amd.benchmarks.tune import make_tensors
+
+    def looked_at(tuner, cfg):
+        names = [k["kernel"] for k in codegen.resource_usage(codegen.compile_config(cfg, ARCH, timeout=600))]
+        picked = [n for n in names if tuner._kernel_matters(n, cfg)]
+        return [(codegen.general_form(n), codegen.template_bools(n)) for n in picked if codegen.general_form(n) is not None]
+
+    cfg = gfx950_space.rule_configs(128, 128)[0]                                  # <..., GEN, PIPE, CAUSAL, SPLIT, PERSIST, PAIR>
+    for (b, h, sq, sk), causal, want in (((4, 32, 2048, 2048), False, (False, [False, False, False, False, False])),
+                                         ((4, 32, 2048, 2048), True, (False, [False, True, False, False, False])),
+                                         ((4, 32, 2080, 2080), False, (True, [False, True, False, False, False])),
+                                         ((4, 32, 2080, 2080), True, (True, [False, True, False, False, False])),
+                                         ((1, 8, 256, 16384), False, (True, [False, True, True, False, False])),
+                                         ((3, 12, 192, 4160), True, (True, [False, True, True, False, False]))):
+        tuner = AttnTunner(ARCH, make_tensors("attn", b, h, sq, sk, 128, 128, "meta"), causal=causal)
+        assert looked_at(tuner, cfg) == [want], (sq, sk, causal)
+    split = AttnConfig(128, 64, 128, 128, 128, 64, 2, 2, 256, True, waves_per_eu=2, kv_splits=8).set_fuse_type("register")
+    tuner = AttnTunner(ARCH, make_tensors("attn", 4, 32, 2048, 2048, 128, 128, "meta"))
+    assert looked_at(tuner, split) == [(True, [False, True, True, False, False])]
+    cfg = gfx950_space.rule_attn_backward_configs(128, 128)[1]
+    for s, general in ((2048, False), (1984, True)):
+        tuner = AttnBwdTunner(ARCH, make_tensors("attn_bwd", 1, 2, s, s, 128, 128, "meta"))
+        assert [g for g, _ in looked_at(tuner, cfg)] == [general] * 2, s
+    cfg = gfx950_space.rule_ret_configs("ret", 128, 128)[1]
+    for s, decay in ((2048, False), (1984, True)):
+        tuner = RetTunner(ARCH, make_tensors("ret", 1, 2, s, s, 128, 128, "meta"), decay=decay)
+        assert looked_at(tuner, cfg) == [(bool(s % cfg.Br), [decay])], s
+    cfg = gfx950_space.rule_ret_configs("ret_bwd", 256, 512)[-1]                  # <..., GEN, DECAY, DS_OUT>; 128 resident rows, dS stored
+    for (sq, sk), general in (((2048, 2048), {False}), ((1984, 1984), {True}), ((1984, 2048), {False, True})):
+        tuner = RetBwdTunner(ARCH, make_tensors("ret_bwd", 1, 2, sq, sk, 256, 512, "meta"), causal=True)
+        forms = looked_at(tuner, cfg)
+        assert {g for g, _ in forms} == general and len(forms) == 5 and not any(f and f[0] for _, f in forms), (sq, sk, forms)
+
+
 def test_whole_blocks_carry_no_selects_for_partial_ones():
     """RetNet at lengths the row blocks divide: the kernels are built without the rebased mask copies of the general form, which
     show in the scalar registers (dV 70, dQ with stored dS 74 at 256/512 before there was a general form)."""
