@@ -28,6 +28,7 @@ import re
 
 import numpy as np
 
+from ..arch import MI355X
 from . import gfx950_space
 from .configs import supported_configs
 
@@ -79,15 +80,15 @@ def backward_features(cfg, shape, causal=False):
     sds, sdq = getattr(cfg, "num_stages_ds", cfg.num_stages_qk), getattr(cfg, "num_stages_dq", cfg.num_stages_dv)
     bars_q = 2 if (sds == 1 or sdq == 1) else 1
     # dV: grid over kv blocks (x column slices where the output is cut), streams Sq / Bc query tiles
-    total += _chain_features(b * h * (sk // cfg.Br) * (cfg.D // dvb), half * sq / cfg.Bc + 0.5 * causal, cfg.Br, cfg.Bc, cfg.Kd, dvb, nw, per_cu, barriers=bars_v)
+    total += _chain_features(b * h * _blocks(sk, cfg.Br) * (cfg.D // dvb), half * sq / cfg.Bc + 0.5 * causal, cfg.Br, cfg.Bc, cfg.Kd, dvb, nw, per_cu, barriers=bars_v)
     # dQ: grid over query blocks, streams Sk / Bc kv tiles
-    total += _chain_features(b * h * (sq // cfg.Br), half * sk / cfg.Bc + 0.5 * causal, cfg.Br, cfg.Bc, cfg.D, cfg.Kd, nw, per_cu, barriers=bars_q)
+    total += _chain_features(b * h * _blocks(sq, cfg.Br), half * sk / cfg.Bc + 0.5 * causal, cfg.Br, cfg.Bc, cfg.D, cfg.Kd, nw, per_cu, barriers=bars_q)
     ds_rows = getattr(cfg, "ds_rows", 0)
     if ds_rows:                                           # dK = dS^T Q only: 64-row query tiles, 2 * ds_rows threads
-        total += _chain_features(b * h * (sk // ds_rows), half * sq / 64 + 0.5 * causal, ds_rows, 64, 0, cfg.Kd, ds_rows // 32, 2, barriers=1, mask_tiles=1)
+        total += _chain_features(b * h * _blocks(sk, ds_rows), half * sq / 64 + 0.5 * causal, ds_rows, 64, 0, cfg.Kd, ds_rows // 32, 2, barriers=1, mask_tiles=1)
         total[8] += b * h * sq * sk * 2 * 2 * half / 64.0 / CUS       # the dS round trip through memory (written once, read once)
     else:
-        total += _chain_features(b * h * (sk // cfg.Br), half * sq / cfg.Bc + 0.5 * causal, cfg.Br, cfg.Bc, cfg.D, cfg.Kd, nw, per_cu, barriers=bars_q)
+        total += _chain_features(b * h * _blocks(sk, cfg.Br), half * sq / cfg.Bc + 0.5 * causal, cfg.Br, cfg.Bc, cfg.D, cfg.Kd, nw, per_cu, barriers=bars_q)
     total[7] = 1.0
     return total
 
@@ -104,7 +105,7 @@ def attn_backward_features(cfg, shape, causal=False):
     def per_cu(wpe):
         return max(1, wpe * 4 // nw)
     total = np.zeros(len(ALL_FEATURES))
-    col_blocks, col_steps = b * h * (sk // cfg.Br), half * sq / cfg.Bc + 0.5 * causal
+    col_blocks, col_steps = b * h * _blocks(sk, cfg.Br), half * _blocks(sq, cfg.Bc) + 0.5 * causal
     if getattr(cfg, "col_split", 0):
         total += _chain_features(col_blocks, col_steps, cfg.Br, cfg.Bc, cfg.Kd, cfg.D, nw, per_cu(cfg.dv_waves_per_eu), barriers=1, mask_tiles=0)
         total += _chain_features(col_blocks, col_steps, cfg.Br, cfg.Bc, cfg.Kd + cfg.D, cfg.Kd, nw, per_cu(cfg.dk_waves_per_eu), barriers=1, mask_tiles=0)
@@ -112,7 +113,7 @@ def attn_backward_features(cfg, shape, causal=False):
         total += _chain_features(col_blocks, col_steps, cfg.Br, cfg.Bc, cfg.Kd + cfg.D, cfg.D + cfg.Kd, nw, per_cu(cfg.waves_per_eu), barriers=1, mask_tiles=0)
     row_bc = getattr(cfg, "row_Bc", cfg.Bc)
     row_wpe = getattr(cfg, "row_waves_per_eu", cfg.waves_per_eu)
-    total += _chain_features(b * h * (sq // cfg.Br), half * sk / row_bc + 0.5 * causal, cfg.Br, row_bc, cfg.Kd + cfg.D, cfg.Kd, nw, per_cu(row_wpe), barriers=1, mask_tiles=0)
+    total += _chain_features(b * h * _blocks(sq, cfg.Br), half * _blocks(sk, row_bc) + 0.5 * causal, cfg.Br, row_bc, cfg.Kd + cfg.D, cfg.Kd, nw, per_cu(row_wpe), barriers=1, mask_tiles=0)
     total[7] = 1.0
     return total
 
@@ -125,14 +126,29 @@ def features(cfg, shape, causal=False, names=FEATURES):
     return np.array([full[ALL_FEATURES.index(n)] for n in names])
 
 
+def _blocks(rows, tile):
+    return -(-rows // tile)                               # the last one may be partial
+
+
+def launched_parts(cfg, shape, causal=False):
+    """Into how many parts a launch cuts the kv range: what the library does with the problem, or what it did when a sample was
+    recorded (``recorded_parts``, set by the readers below)."""
+    recorded = getattr(cfg, "recorded_parts", 0)
+    if recorded:
+        return recorded
+    if getattr(cfg, "operation", "") != "attn" or cfg.fuse_type == "shared":
+        return 1
+    return gfx950_space.kv_parts(cfg, MI355X(), *shape, causal)
+
+
 def forward_features(cfg, shape, causal=False):
     b, h, sq, sk = shape
     nw = cfg.Nthreads // 64
-    splits = max(1, getattr(cfg, "kv_splits", 1))
-    n_blocks = b * h * (sq // cfg.Br) * splits
-    steps = sk / cfg.Bc / splits
+    splits = launched_parts(cfg, shape, causal)
+    n_blocks = b * h * _blocks(sq, cfg.Br) * splits
+    steps = _blocks(sk, cfg.Bc) / splits
     if causal:                                            # a row block walks the tiles up to its own diagonal
-        steps = (sk / cfg.Bc) * 0.5 + 0.5 * cfg.Br / cfg.Bc + 0.5
+        steps = (_blocks(sk, cfg.Bc) * 0.5 + 0.5 * cfg.Br / cfg.Bc + 0.5) / splits
     per_cu = gfx950_space.blocks_per_cu(cfg)
     lds_room = max(1, 160 * 1024 // max(1, gfx950_space.forward_lds_bytes(cfg)))
     per_cu = max(1, min(per_cu, lds_room))
@@ -237,8 +253,10 @@ def config_from_log_line(text, op, dim_qk, dim_v):
     return supported_configs[op].from_dict(fields)
 
 
-def samples_from_tuning_log(path, op, dim_qk, dim_v, shape, causal=False, failed=1e7):
-    """(cfg, shape, causal, ms) for every timed candidate in a ``profile_result_*.txt``."""
+def samples_from_tuning_log(path, op, dim_qk, dim_v, shape, causal=False, failed=1e7, parts_by_estimate=False):
+    """(cfg, shape, causal, ms) for every timed candidate in a ``profile_result_*.txt``.  ``parts_by_estimate``: the log is
+    of libraries that cut the kv range into as many parts as pay; the recorded runs this repository keeps are older, and
+    their launches were cut by ``kv_splits`` alone."""
     out = []
     with open(path) as f:
         lines = [l.rstrip("\n") for l in f]
@@ -250,7 +268,10 @@ def samples_from_tuning_log(path, op, dim_qk, dim_v, shape, causal=False, failed
         except ValueError:
             continue
         if ms < failed:
-            out.append((config_from_log_line(lines[i], op, dim_qk, dim_v), tuple(shape), bool(causal), ms))
+            cfg = config_from_log_line(lines[i], op, dim_qk, dim_v)
+            if not parts_by_estimate:
+                cfg.recorded_parts = 1 if causal else max(1, getattr(cfg, "kv_splits", 1))
+            out.append((cfg, tuple(shape), bool(causal), ms))
     return out
 
 
@@ -286,6 +307,8 @@ def samples_from_export(path, max_scratch_bytes=None):
             continue
         cfg = supported_configs[r["config"]["operation"]].from_dict(r["config"])
         (sq, sk, _, _), _, _, _, b, h = r["cost_model_config"]
+        if r.get("dispatches") == 1:                      # the split kernel comes with a merge: a launch of one kernel ran in one part
+            cfg.recorded_parts = 1
         out.append((cfg, (b, h, sq, sk), bool(r.get("causal", False)), float(r["cycles"])))
     return out
 

@@ -30,7 +30,7 @@ import tempfile
 import torch
 
 from ..arch import MI355X
-from ..autotuner import codegen, gfx950_space, library
+from ..autotuner import codegen, costmodel, gfx950_space, library
 from .tune import make_tensors
 
 TUNERS = {"attn": "AttnTunner", "ret": "RetTunner"}
@@ -63,10 +63,9 @@ def cost_model_tuple(cfg, dims):
 
 
 def dispatches_per_launch(cfg, dims, causal):
-    """Kernels one launch of ``cfg`` enqueues: a kv-splitting attention configuration runs its split kernel and the
-    merge (csrc/kernels/attention/regfuse/profile_code.py: ``split_applies``), everything else one kernel."""
-    ns = getattr(cfg, "kv_splits", 1)
-    return 2 if (cfg.operation == "attn" and ns > 1 and not causal and (dims[3] // cfg.Bc) % ns == 0) else 1
+    """Kernels one launch of ``cfg`` enqueues: an attention forward whose kv range is cut into parts runs its split
+    kernel and the merge (csrc/kernels/attention/regfuse/profile_code.py: ``kv_parts``), everything else one kernel."""
+    return 2 if costmodel.launched_parts(cfg, dims[:4], causal) > 1 else 1
 
 
 def scratch_bytes(cfg):

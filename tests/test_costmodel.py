@@ -266,3 +266,42 @@ def test_an_attention_model_file_still_loads_and_a_foreign_feature_set_does_not(
     assert m.names == costmodel.FEATURES
     with pytest.raises(ValueError):
         costmodel.CostModel.from_dict({"features": ["matrix", "moon_phase"], "weights": [1.0, 2.0]})
+
+
+def test_a_launch_counts_as_many_kernels_as_the_kv_range_has_parts():
+    """The exporter's dispatch count and the model's features follow the library's own choice (gfx950_space.kv_parts, which
+    test_codegen_abi.py holds against the library): a merge kernel wherever there is more than one part, causal walks too."""
+    from attention_autotuner_amd.autotuner import RetTunner, gfx950_space
+    from attention_autotuner_amd.benchmarks import export_costmodel_config as export
+    from attention_autotuner_amd.benchmarks.tune import make_tensors
+    arch, cut = MI355X(), 0
+    for dims, causal in (((1, 32, 256, 16384, 128, 128), False), ((3, 12, 192, 4160, 128, 128), True), ((4, 32, 2048, 2048, 128, 128), False)):
+        tuner = AttnTunner(arch, make_tensors("attn", *dims, "meta"), causal=causal)
+        for cfg in [c for c in tuner.get_tuned_configs() if tuner._fits_problem(c)]:
+            parts = 1 if cfg.fuse_type == "shared" else gfx950_space.kv_parts(cfg, arch, *dims[:4], causal)
+            assert export.dispatches_per_launch(cfg, dims, causal) == 1 + (parts > 1)
+            one, cut_up = (costmodel.forward_features(c, dims[:4], causal) for c in (_recorded(cfg, 1), cfg))
+            if parts > 1:                                 # the same matrix work, in shorter walks of more blocks
+                cut += 1
+                assert np.isclose(one[0], cut_up[0]) and np.array_equal(cut_up, costmodel.forward_features(_recorded(cfg, parts), dims[:4], causal))
+            else:
+                assert np.array_equal(one, cut_up)
+    assert cut > 100
+    ret = RetTunner(arch, make_tensors("ret", 1, 8, 256, 2048, 128, 128, "meta"))
+    assert {export.dispatches_per_launch(c, (1, 8, 256, 2048, 128, 128), False) for c in ret.get_tuned_configs()} == {1}
+
+
+def _recorded(cfg, parts):
+    again = type(cfg).from_dict(cfg.to_dict())
+    again.recorded_parts = parts
+    return again
+
+
+@pytest.mark.parametrize("op", ["attn", "attn_bwd", "ret_bwd"])
+def test_a_partial_block_counts_as_a_block(op):
+    """A row block over the last whole one costs what a whole one does, not nothing."""
+    from attention_autotuner_amd.autotuner import gfx950_space
+    cfg = {"attn": gfx950_space.rule_configs(128, 128)[0], "attn_bwd": gfx950_space.rule_attn_backward_configs(128, 128)[1],
+           "ret_bwd": gfx950_space.rule_ret_configs("ret_bwd", 256, 256)[1]}[op]
+    whole, ragged, less = (costmodel.features(cfg, (2, 64, s, s)) for s in (1280, 1216, 1152))
+    assert ragged[0] > less[0] and ragged[0] <= whole[0]
