@@ -194,10 +194,40 @@ def _shared_candidates(op, br, bc, dim_qk, dim_v, st_qk, st_v, nthreads, wpe):
 MIN_LENGTH = 32               # the register-fused forwards and both backwards take resident lengths that are multiples of this
 
 
-def _takes(seq, tile, step=MIN_LENGTH):
-    """Whether a kernel with tiles of ``tile`` rows runs a length of ``seq`` rows (None: any) without mostly idle tiles;
-    ``step``: what its lengths have to be multiples of."""
-    return not seq or seq % tile == 0 or (seq > tile and seq % step == 0)
+def _divides(tile, *seqs):
+    return all(not s or s % tile == 0 for s in seqs)
+
+
+# From this length on a last row block that is partial wastes less than the larger block gains.  Timed at 192 ... 1600 rows and 16
+# and 96 (batch, head)s, causal and not, against the 64-row shape that divides the lengths: at 1088 and 1600 rows the forwards
+# take 0.51 ... 0.97 of its time (attention 64/128, 128/192, 256/128, 128/256; RetNet 64/128, 256/128, 128/256) and the RetNet
+# backward 0.81 ... 0.94; at 320 rows both directions take 0.87 ... 1.6.  256-row blocks at lengths 128 divides take up to 1.5 times
+# the time of 128-row ones (640 rows), and a RetNet shape of them that spills 5.9 times (128/256), so only 128-row blocks may be partial.
+PARTIAL_FROM = 1024
+PARTIAL_ROWS = 128
+
+
+def _rounds(cfg, arch, b, h, seq):
+    return -(-b * h * -(-seq // cfg.Br) // (arch.compute_max_core * blocks_per_cu(cfg)))
+
+
+def _pick(candidates, fits, partial_pays=lambda whole, partial: True):
+    """The first of ``candidates`` (larger blocks first) for a length: one whose tiles divide it; where that is a block smaller than
+    PARTIAL_ROWS, a partial one of PARTIAL_ROWS that pays; where nothing divides the length, the smallest that takes it.
+    ``fits(cfg)``: 2 for whole tiles, 1 for partial ones, 0 for a length the kernel does not take; ``candidates`` may be a
+    generator of configurations that are all valid."""
+    candidates = list(candidates)
+    whole = next((c for c in candidates if fits(c) == 2), None)
+    if whole is not None and whole.Br >= PARTIAL_ROWS:
+        return whole
+    partial = next((c for c in candidates if c.Br == PARTIAL_ROWS and fits(c) == 1), None)
+    if whole is None:
+        return next((c for c in reversed(candidates) if fits(c)), None)
+    return partial if partial is not None and partial_pays(whole, partial) else whole
+
+
+def _long(*seqs):
+    return all(s and s >= PARTIAL_FROM for s in seqs)
 
 
 def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None, problem=None):
@@ -210,23 +240,31 @@ def default_forward_config(op, dim_qk, dim_v, arch, seq_q=None, seq_k=None, prob
             return cfg
     prefs = [(256, 64, 512, 2, 2, 2), (128, 64, 256, 2, 2, 2), (128, 64, 256, 1, 1, 2), (128, 64, 256, 1, 1, 1), (128, 32, 256, 1, 1, 1),
              (64, 32, 128, 1, 1, 1)]
-    if op == "ret" and dim_v == 512 and _takes(seq_q, 128) and _takes(seq_k, 64, 64):
+    if op == "ret" and dim_v == 512 and _divides(128, seq_q) and _divides(64, seq_k):
         # 32 rows x 512 columns per wave fill the 256 accumulation registers of a wave that has its SIMD to itself;
         # the RetNet kernel is written so that this builds without scratch, and at d_qk 256 it leads every mask mode
         cfg = RetConfig(128, 64, dim_qk, dim_v, dim_qk, 64, 1, 1, 1, 256, True, waves_per_eu=1)
         cfg.set_fuse_type("register")
         if forward_valid(cfg, arch):
             return cfg
-    for br, bc, nt, sq, sv, wpe in prefs:
-        if not _takes(seq_q, br) or not _takes(seq_k, bc, MIN_LENGTH if op == "attn" else bc):
-            continue
-        if op == "attn":
-            cfg = AttnConfig(br, bc, dim_qk, dim_v, dim_qk, bc, sq, sv, nt, True, waves_per_eu=wpe)
-        else:
-            cfg = RetConfig(br, bc, dim_qk, dim_v, dim_qk, bc, sq, sq, sv, nt, True, waves_per_eu=wpe)
-        cfg.set_fuse_type("register")
-        if forward_valid(cfg, arch) and not forward_likely_spills(cfg):
-            return cfg
+    def shapes():
+        for br, bc, nt, sq, sv, wpe in prefs:
+            if op == "attn":
+                cfg = AttnConfig(br, bc, dim_qk, dim_v, dim_qk, bc, sq, sv, nt, True, waves_per_eu=wpe)
+            else:
+                cfg = RetConfig(br, bc, dim_qk, dim_v, dim_qk, bc, sq, sq, sv, nt, True, waves_per_eu=wpe)
+            cfg.set_fuse_type("register")
+            if forward_valid(cfg, arch) and not forward_likely_spills(cfg):
+                yield cfg
+
+    def fits(cfg):
+        if _divides(cfg.Br, seq_q) and _divides(cfg.Bc, seq_k):
+            return 2
+        step = MIN_LENGTH if op == "attn" else cfg.Bc
+        return int(_divides(MIN_LENGTH, seq_q) and _divides(step, seq_k) and (not seq_q or seq_q > cfg.Br))
+    cfg = _pick(shapes(), fits, lambda whole, partial: _long(seq_q))
+    if cfg is not None:
+        return cfg
     # wide value heads: the LDS-fused kernel keeps the accumulator at Br*D/(64*waves) registers
     for br, bc, nt, w1n, w2n in ((128, 64, 512, 2, 8), (64, 64, 256, 2, 4)):
         if (seq_q and seq_q % br) or (seq_k and seq_k % bc):
@@ -419,14 +457,25 @@ def default_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, problem
              (64, 64, 128, 1, 1, 1))
     if dim_v == 512:            # measured at d_qk 256: 64-row streamed tiles with single buffers lead the three-buffer ring of 32-row tiles
         prefs = ((128, 64, 256, 1, 1, 1),) + prefs
-    for br, bc, nt, sy, sz, wpe in prefs:
-        if any(not _takes(s, br) or not _takes(s, bc, bc) for s in (seq_q, seq_k)):
-            continue
-        n = nt // WAVE
-        cfg = RetBwdConfig(br, bc, dim_qk, dim_v, n, n, n, n, nt, True, BlockKSmem=dim_qk, num_stages_qk=sy,
-                           num_stages_mask=sy, num_stages_dv=sz, num_stages_ds=sy, num_stages_dq=sz, waves_per_eu=wpe)
-        if backward_valid(cfg, arch):
-            return cfg
+    def shapes():
+        for br, bc, nt, sy, sz, wpe in prefs:
+            n = nt // WAVE
+            cfg = RetBwdConfig(br, bc, dim_qk, dim_v, n, n, n, n, nt, True, BlockKSmem=dim_qk, num_stages_qk=sy,
+                               num_stages_mask=sy, num_stages_dv=sz, num_stages_ds=sy, num_stages_dq=sz, waves_per_eu=wpe)
+            if backward_valid(cfg, arch):
+                yield cfg
+
+    def fits(cfg):
+        if not _divides(cfg.Bc, seq_q, seq_k):
+            return 0
+        return 2 if _divides(cfg.Br, seq_q, seq_k) else int(all(not s or s > cfg.Br for s in (seq_q, seq_k)) and _divides(MIN_LENGTH, seq_q, seq_k))
+
+    def partial_pays(whole, partial):
+        # 480 blocks of 64 rows are one round of two to a CU, the 288 blocks of 128 of the same problem are two of one: 1.6 times the time
+        return _long(seq_q, seq_k) and (problem is None or all(_rounds(partial, arch, *problem[:2], s) <= _rounds(whole, arch, *problem[:2], s) for s in (seq_q, seq_k)))
+    cfg = _pick(shapes(), fits, partial_pays)
+    if cfg is not None:
+        return cfg
     raise NoValidConfigError(f"no default ret_bwd configuration fits dim_qk={dim_qk} dim_v={dim_v} seq=({seq_q},{seq_k})")
 
 
@@ -560,19 +609,43 @@ def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, pr
         cfg = rule_attn_backward_config(dim_qk, dim_v, *problem[:2], seq_q, seq_k, problem[2])
         if cfg is not None:
             return cfg
-    for br, bc, nt, st, wpe in ((128, 32, 256, 3, 1), (128, 32, 256, 2, 1), (64, 32, 128, 3, 1), (64, 32, 128, 2, 1), (64, 32, 128, 2, 2)):
-        if any(not _takes(s, br) or not _takes(s, bc) for s in (seq_q, seq_k)):
-            continue
-        for row_wpe in ((2, wpe) if wpe == 1 else (wpe,)):            # the row kernel at two waves per SIMD where it fits
-            cfg = AttnBwdConfig(br, bc, dim_qk, dim_v, nt, st, waves_per_eu=wpe, row_waves_per_eu=row_wpe)
+    def shapes():
+        for br, bc, nt, st, wpe in ((128, 32, 256, 3, 1), (128, 32, 256, 2, 1), (64, 32, 128, 3, 1), (64, 32, 128, 2, 1), (64, 32, 128, 2, 2)):
+            for row_wpe in ((2, wpe) if wpe == 1 else (wpe,)):        # the row kernel at two waves per SIMD where it fits
+                cfg = AttnBwdConfig(br, bc, dim_qk, dim_v, nt, st, waves_per_eu=wpe, row_waves_per_eu=row_wpe)
+                if attn_backward_valid(cfg, arch):
+                    yield cfg
+
+    def split_shapes():                                               # ... or one column kernel per output
+        for br, bc, nt, st in ((128, 32, 256, 3), (128, 32, 256, 2), (64, 32, 128, 2)):
+            cfg = AttnBwdConfig(br, bc, dim_qk, dim_v, nt, st, waves_per_eu=1, col_split=1)
             if attn_backward_valid(cfg, arch):
-                return cfg
-    # head sizes whose dV and dK accumulators cannot share a wave: one column kernel per output
-    for br, bc, nt, st in ((128, 32, 256, 3), (128, 32, 256, 2), (64, 32, 128, 2)):
-        if any(not _takes(s, br) or not _takes(s, bc) for s in (seq_q, seq_k)):
-            continue
-        cfg = AttnBwdConfig(br, bc, dim_qk, dim_v, nt, st, waves_per_eu=1, col_split=1)
-        if attn_backward_valid(cfg, arch):
+                yield cfg
+
+    def fits(cfg):
+        if _divides(cfg.Br, seq_q, seq_k) and _divides(cfg.Bc, seq_q, seq_k):
+            return 2
+        return int(_divides(MIN_LENGTH, seq_q, seq_k) and all(not s or s > cfg.Br for s in (seq_q, seq_k)))
+
+    def partial_pays(whole, partial):
+        if problem is None:
+            return _long(seq_q, seq_k)
+        b, h, causal = problem
+        blocks = b * h * -(-seq_k // whole.Br)
+        if partial.col_split:
+            # d 256/512: a block of either size has its CU to itself, so one round less is what counts (96 heads of 192 rows 0.68, of 320
+            # rows 1.11 of the time; 16 of 1088 0.57), and in a causal walk, whose blocks differ in length, several rounds (96 of 1088 0.71,
+            # 16 of 1088 1.08)
+            per_round = arch.compute_max_core
+            return -(-b * h * -(-seq_k // partial.Br) // per_round) < -(-blocks // per_round) and (not causal or blocks > 2 * per_round)
+        # not causal: 0.90 ... 1.00 of the time from 1024 rows on.  Causal: 1.00 ... 1.07 at 64/128 and 256/128; 0.96 ... 1.00 at 128/192,
+        # where only the larger block lets the row kernel run two waves per SIMD
+        return _long(seq_q, seq_k) and _rounds(partial, arch, b, h, seq_k) <= _rounds(whole, arch, b, h, seq_k) and \
+            (not causal or partial.row_waves_per_eu > whole.row_waves_per_eu)
+    # head sizes whose dV and dK accumulators cannot share a wave have no shape of the first kind
+    for kind in (shapes, split_shapes):
+        cfg = _pick(kind(), fits, partial_pays)
+        if cfg is not None:
             return cfg
     raise NoValidConfigError(f"no default attn_bwd configuration fits dim_qk={dim_qk} dim_v={dim_v} seq=({seq_q},{seq_k})")
 

@@ -486,6 +486,25 @@ def test_a_fixed_kv_split_insists_on_its_room_only_where_its_parts_divide_the_ti
             assert (rc == -3) == refused, (sk, causal, rc)
 
 
+@pytest.mark.parametrize("op", ["attn", "ret", "attn_bwd", "ret_bwd"])
+def test_a_partial_block_is_taken_only_where_it_pays(op):
+    """Head sizes without a rule: tiles that divide a length come first, 128 rows that do not only from 1024 rows on."""
+    def pick(dqk, dv, s, problem=None):
+        fn = {"attn_bwd": gfx950_space.default_attn_backward_config, "ret_bwd": gfx950_space.default_backward_config}.get(op)
+        return fn(dqk, dv, ARCH, s, s, problem) if fn else gfx950_space.default_forward_config(op, dqk, dv, ARCH, s, s, problem)
+    for dqk, dv in ((64, 128), (128, 256), (256, 128)):
+        assert [pick(dqk, dv, s).Br for s in (64, 192, 320, 960)] == [64] * 4
+        assert [pick(dqk, dv, s).Br for s in (384, 640, 1152, 1408)] == [128] * 4
+        assert [pick(dqk, dv, s).Br for s in (1088, 1600, 2112)] == [128] * 3
+        if op in ("attn_bwd", "ret_bwd"):
+            # 30 heads of 1088 rows: 510 blocks of 64 rows are one round of two to a CU, 270 of 128 rows two of one
+            assert [pick(dqk, dv, 1088, (1, h, False)).Br for h in (16, 30)] == [128, 64]
+    if op == "attn_bwd":
+        assert [pick(256, 512, s, p).Br for s, p in ((192, (4, 24, False)), (320, (4, 24, False)), (1088, (2, 8, False)), (1088, (2, 8, True)), (1088, (4, 24, True)))] == \
+            [128, 64, 128, 64, 128]
+        assert [pick(dqk, dv, 1088, (2, 8, True)).Br for dqk, dv in ((64, 128), (256, 128), (128, 192))] == [64, 64, 128]
+
+
 def test_the_library_cuts_the_kv_range_as_the_tile_shape_rule_assumes():
     """gfx950_space.kv_parts and the library's own choice (kv_parts.h) are one estimate, written twice."""
     for d in (64, 128, 256):
