@@ -335,12 +335,34 @@ def kv_parts(cfg, arch, b, h, seq_q, seq_k, causal):
     return min(range(1, min(64, seq_k // 256) + 1), key=lambda p: forward_estimate_us(cfg, arch, b, h, seq_q, seq_k, causal, p))
 
 
+# All queries of a (batch, head) in one row block, 160 to 256 of them: every block reads K and V of its own from memory, once, and
+# what counts is how much of them it has in flight.  Blocks of eight waves have twice the copies of blocks of four under way, also
+# where half of their waves have no rows, and run at 4.1 ... 4.7 TB/s where the four waves do 3.2 ... 4.1 (d 192, 160 heads of 128
+# rows on 1536: 58.7 -> 46.2 us; 224 of 64 on 2176: 85.6 -> 72.8; d 256, 192 on 1024: 59.8 -> 50.7; inputs not in a cache, and 0.85
+# ... 1.05 of the time where they are).  The estimate sees matrix work only and puts both within 4 %.  Fewer than 192 blocks on
+# longer ranges are cut into parts by the smaller shapes, which is as good or better (d 192, 160 of 64 on 4160: 106.8 against
+# 111.2); over 256 of them are more than one round.  At d 128 the gain from memory (up to 14 %) is a loss of up to 6 % from a cache.
+STREAM_ROWS = 128
+STREAM_BLOCKS = (160, 192, 256)
+STREAM_KV = (1024, 2048)
+STREAM_WIDTH = 384
+
+
+def _streams_once(b, h, seq_q, seq_k):
+    least, any_range, most = STREAM_BLOCKS
+    return seq_q <= STREAM_ROWS and seq_k >= STREAM_KV[0] and least <= b * h <= most and (b * h >= any_range or seq_k <= STREAM_KV[1])
+
+
 def rule_forward_config(dim_qk, dim_v, arch, b, h, seq_q, seq_k, causal):
     """The tile shape for an attention forward problem nobody tuned, or None (head sizes or lengths the rule does not
-    cover): the one of RULE_SHAPES with the smallest estimate at the kv parts its library will take."""
+    cover): the one of RULE_SHAPES with the smallest estimate at the kv parts its library will take, the one of 256 rows and
+    eight waves where K and V stream through once (_streams_once)."""
     if seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
         return None
-    return min(rule_configs(dim_qk, dim_v), default=None,
+    shapes = rule_configs(dim_qk, dim_v)
+    if dim_qk + dim_v >= STREAM_WIDTH and _streams_once(b, h, seq_q, seq_k):
+        shapes = [c for c in shapes if c.Br == 256 and c.Nthreads == 512] or shapes
+    return min(shapes, default=None,
                key=lambda c: forward_estimate_us(c, arch, b, h, seq_q, seq_k, causal, kv_parts(c, arch, b, h, seq_q, seq_k, causal)))
 
 

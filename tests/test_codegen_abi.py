@@ -486,6 +486,18 @@ def test_a_fixed_kv_split_insists_on_its_room_only_where_its_parts_divide_the_ti
             assert (rc == -3) == refused, (sk, causal, rc)
 
 
+def test_few_rows_on_a_long_range_take_blocks_of_eight_waves():
+    """One row block per (batch, head) and a chip's worth of them: K and V stream through once."""
+    for d in (192, 256):
+        for b, h, sq, sk, wide in ((8, 20, 128, 1536, True), (8, 20, 128, 2048, True), (8, 20, 128, 2080, False), (6, 32, 64, 4160, True),
+                                   (8, 32, 128, 1024, True), (8, 32, 128, 992, False), (3, 53, 128, 1536, False), (7, 37, 128, 1536, False)):
+            for causal in (False, True):
+                cfg = gfx950_space.rule_forward_config(d, d, ARCH, b, h, sq, sk, causal)
+                assert (cfg.Nthreads == 512) == wide, (d, b, h, sq, sk, str(cfg))
+    assert gfx950_space.rule_forward_config(128, 128, ARCH, 8, 20, 128, 1536, True).Nthreads == 256
+    assert gfx950_space.rule_forward_config(192, 192, ARCH, 8, 20, 160, 1536, True) is not None
+
+
 @pytest.mark.parametrize("op", ["attn", "ret", "attn_bwd", "ret_bwd"])
 def test_a_partial_block_is_taken_only_where_it_pays(op):
     """Head sizes without a rule: tiles that divide a length come first, 128 rows that do not only from 1024 rows on."""
