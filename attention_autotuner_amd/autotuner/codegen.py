@@ -273,14 +273,18 @@ def template_bools(mangled):
     return [c == "1" for c in re.findall(r"Lb([01])E", m.group(1))] if m else []
 
 
-# Kernels with a form for lengths their tiles do not divide: where in the list of their integer template arguments it is chosen.
-GENERAL_FORM_ARG = {"flashattn_fwd_regfuse": 9, "attn_bwd_chain": 8, "ret_fwd_regfuse": 9, "ret_bwd_chain": 9, "ret_bwd_dk_from_ds": 6}
+# Kernels with a form for lengths their tiles do not divide: where in the list of their integer template arguments it is chosen,
+# or whether the kernel is that form.
+GENERAL_FORM = {"flashattn_fwd_regfuse": 9, "attn_bwd_chain": 8, "ret_fwd_regfuse": False, "ret_ragged_regfuse": True, "ret_bwd_chain": 9,
+                "ret_bwd_dk_from_ds": 6}
 
 
 def general_form(mangled):
     """Whether a mangled kernel name is the form for lengths its tiles do not divide; None for a kernel without such a form."""
-    for kernel, at in GENERAL_FORM_ARG.items():
+    for kernel, at in GENERAL_FORM.items():
         if f"{len(kernel)}{kernel}I" in mangled:
+            if isinstance(at, bool):
+                return at
             ints = re.findall(r"Li(\d+)E", mangled)
             return len(ints) > at and ints[at] != "0"
     return None

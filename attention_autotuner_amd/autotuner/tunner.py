@@ -53,7 +53,7 @@ class _ForwardTunner(BaseTunner):
         flags, general = codegen.template_bools(mangled), codegen.general_form(mangled)
         s = self.problem_shape
         whole = config is None or s["Sq"] % config.Br == 0
-        if self.operation == "ret":                       # <..., GEN, DECAY>
+        if self.operation == "ret":                       # <..., DECAY>
             return (not flags or flags[-1] == bool(self.decay)) and general in (None, not whole)
         if "flashattn_fwd_regfuse" in mangled and len(flags) == 5:     # <..., GEN, PIPE, CAUSAL, SPLIT, PERSIST, PAIR>
             # one general kernel, for both walks, in one part or in several; the others at whole tiles in one part

@@ -121,8 +121,8 @@ static void test_regfuse_retnet(const ProblemShape& ps, Tensors& t) {
   using T = aat::RetFwdRegfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM>;
   char name[128];
   std::snprintf(name, sizeof name, "regfuse  Br=%d Bc=%d thr=%d bufs=%d/%d/%d waves/SIMD=%d", Br, Bc, NT, NSK, NSV, NSM, WPE);
-  run_all_masks(name, ps, t, Br, Bc, NT, T::kSmemBytes, &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, 0, false>,
-                &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, 0, true>);
+  run_all_masks(name, ps, t, Br, Bc, NT, T::kSmemBytes, &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, false>,
+                &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, true>);
 }
 
 // LDS-fused: <Br, Bc, threads, K buffers, V buffers, mask buffers, waves along kv, waves along d, waves per SIMD>

@@ -87,8 +87,8 @@ struct RetBwdChain {
 // a dK kernel that reads them instead of evaluating them again (dk_from_ds.h).  Only the tiles of the walk are written.
 // GEN: resident lengths that are multiples of 32 and not of BX; the 32-row groups a last block does not have repeat its first
 // one (below).  Whole blocks keep the form without it, because every mask copy of every tile pays a comparison and a 64-bit
-// select for it: 78 scalar registers instead of 70 in the dV pass at 256/512, 86 instead of 74 in dQ + dS, and 538 us instead of
-// 533 for forward + backward at B4 H8 S2048.
+// select for it: 78 scalar registers instead of 70 in the dV pass at 256/512, 86 instead of 74 in dQ + dS, and 530 us instead of
+// 527 for forward + backward at B4 H8 S2048, timed in turn.
 template <int KX, int DZ, int DZB, int BX, int BY, int Nthreads, int NSY, int NSZ, BwdPass PASS, int WPE = 1,
           int GEN = 0, bool DECAY = false, bool DS_OUT = false>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))

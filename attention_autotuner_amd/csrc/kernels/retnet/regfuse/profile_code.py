@@ -21,14 +21,15 @@ constexpr int stages_mask = num_stages_mask < num_stages_qk ? num_stages_qk : nu
 
 using Traits = aat::RetFwdRegfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask>;
 constexpr int shared_mem = Traits::kSmemBytes;
-// GEN = 1: a query length the row blocks do not divide
-template <bool DECAY, int GEN> constexpr auto kernel_of = &aat::ret_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu, GEN, DECAY>;
+template <bool DECAY> constexpr auto kernel = &aat::ret_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu, DECAY>;
+// a query length the row blocks do not divide
+template <bool DECAY> constexpr auto kernel_ragged = &aat::ret_ragged_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu, DECAY>;
 
 bool lengths_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, Bc); }}
 int row_blocks(int Seq_q) {{ return (Seq_q + Br - 1) / Br; }}
 template <bool DECAY> hipError_t allow_kernels() {{
-  const hipError_t e = aat::allow_lds(kernel_of<DECAY, 0>, shared_mem);
-  return e != hipSuccess ? e : aat::allow_lds(kernel_of<DECAY, 1>, shared_mem);
+  const hipError_t e = aat::allow_lds(kernel<DECAY>, shared_mem);
+  return e != hipSuccess ? e : aat::allow_lds(kernel_ragged<DECAY>, shared_mem);
 }}
 
 hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* o, float* r, int B, int H,
@@ -39,7 +40,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_hal
   const hipError_t scanned = aat::prepare_mask_walk(mask_mode, reinterpret_cast<const aat::half_t*>(mask), H, Seq_q, Seq_k,
                                                     workspace, stream, &walk);
   if (scanned != hipSuccess) return scanned;
-  (Seq_q % Br == 0 ? kernel_of<false, 0> : kernel_of<false, 1>)<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
+  (Seq_q % Br == 0 ? kernel<false> : kernel_ragged<false>)<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<const aat::half_t*>(mask),
       reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, walk.causal, nullptr, walk.extents);
@@ -50,7 +51,7 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
                         int H, int Seq_q, int Seq_k, hipStream_t stream) {{
   static const hipError_t lds_ok = allow_kernels<true>();
   if (lds_ok != hipSuccess) return lds_ok;
-  (Seq_q % Br == 0 ? kernel_of<true, 0> : kernel_of<true, 1>)<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
+  (Seq_q % Br == 0 ? kernel<true> : kernel_ragged<true>)<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), nullptr, reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, 1,
       log2_gamma, nullptr);

@@ -8,11 +8,11 @@
 // through LDS as a third DMA stream, and the normalisation is lazy (utils/retention.h).
 // `causal` promises a mask that is zero above the diagonal and only shortens the kv walk.
 //
-// seq_k is a multiple of Bc, seq_q one of Br.  GEN: seq_q is any multiple of 32; the 32-row groups the last row block of a
+// seq_k is a multiple of Bc, seq_q one of Br.  GEN (ret_ragged_regfuse): seq_q is any multiple of 32; the 32-row groups the last row block of a
 // head does not have repeat its first group -- same loads, same arithmetic -- and are not stored.  (Where no 128-row tile
 // divided the length the row blocks were 64 rows of two waves, with one buffer per stream.)  Every mask copy of
 // every tile pays a comparison and a 64-bit select of its source for it, so whole row blocks keep the form without (forward and
-// backward together at B4 H8 S2048 256/512: 538 us with the selects everywhere, 533 with none at whole blocks).
+// backward together at B4 H8 S2048 256/512, timed in turn: 530 us with the selects everywhere, 527 with none at whole blocks).
 #pragma once
 #include <type_traits>
 
@@ -53,13 +53,10 @@ struct RetFwdRegfuse {
 
 // DECAY: the mask is gamma_h^(q + diag - kv) below the diagonal and zero above it, built in registers
 // from lg2gamma[h] = log2(gamma_h); `mask` is not read and tiles above the diagonal are skipped.
-template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, int GEN = 0,
-          bool DECAY = false>
-__global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
-                const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H,
-                int seq_k, int seq_q, int causal, const float* __restrict__ lg2gamma = nullptr,
-                const int* __restrict__ extents = nullptr) {
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE, int GEN, bool DECAY>
+AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
+                          const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H, int seq_k,
+                          int seq_q, int causal, const float* __restrict__ lg2gamma, const int* __restrict__ extents) {
   // One wave per SIMD: the output tile lives in the accumulation registers by number (utils/acc_file.h), the score
   // tile in vector registers through hand-written matrix instructions, and the compiler allocates the rest.
   constexpr bool kNumbered = WPE == 1;
@@ -332,6 +329,24 @@ ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, cons
   }
   store_o_tile<RT, DT, D, T::kOStride>(oacc, scale, smem + wave * WM * T::kOStride,
                                        o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane, 32, groups);
+}
+
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, bool DECAY = false>
+__global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
+                const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H,
+                int seq_k, int seq_q, int causal, const float* __restrict__ lg2gamma = nullptr,
+                const int* __restrict__ extents = nullptr) {
+  ret_fwd_walk<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM, WPE, 0, DECAY>(q, k, v, mask, o, r, H, seq_k, seq_q, causal, lg2gamma, extents);
+}
+
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, bool DECAY = false>
+__global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+ret_ragged_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
+                   const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H,
+                   int seq_k, int seq_q, int causal, const float* __restrict__ lg2gamma = nullptr,
+                   const int* __restrict__ extents = nullptr) {
+  ret_fwd_walk<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM, WPE, 1, DECAY>(q, k, v, mask, o, r, H, seq_k, seq_q, causal, lg2gamma, extents);
 }
 
 }  // namespace aat
