@@ -46,6 +46,15 @@ def persistent_graph_config():
     return AttnConfig(256, 128, 128, 128, 128, 128, 2, 2, 512, True, waves_per_eu=2).set_fuse_type("register")
 
 
+def ragged_row_group_configs():
+    """Two 32-row groups per wave on 32-row streams, for lengths at which a wave has one of them (the rule shapes of these
+    operators have one group per wave, or streams of 64 rows)."""
+    return [RetConfig(256, 32, 64, 64, 64, 32, 1, 1, 1, 256, True, waves_per_eu=2).set_fuse_type("register"),
+            RetConfig(256, 32, 128, 128, 128, 32, 2, 2, 2, 256, True, waves_per_eu=1).set_fuse_type("register"),
+            AttnBwdConfig(256, 32, 64, 64, 256, 2, waves_per_eu=1, row_waves_per_eu=1),
+            AttnBwdConfig(256, 64, 64, 64, 256, 2, waves_per_eu=1, row_waves_per_eu=1, row_Bc=64)]
+
+
 def ret_register_wide():
     """The register-fused RetNet forward at d_qk 256, d_v 512 (the reference has this variant,
     csrc/kernels/retnet/regfuse/regfuse.h:267-340): 256 output accumulators per lane."""
@@ -99,6 +108,7 @@ def parity_configs(arch=None):
     out.append(persistent_graph_config())
     out.append(ret_register_wide())
     out += ret_register_wide_buffered()
+    out += ragged_row_group_configs()
     out.append(ret_shared_wide_one_wave())
     for t in RET_BWD_STORED_DS:
         out += [ret_bwd_stored_ds_config(*t), ret_bwd_stored_ds_config(*t[:5], 0)]      # and the same passes without it

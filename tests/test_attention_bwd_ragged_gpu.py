@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import attention_autotuner_amd as aat
-from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space, prebuilt_extra
 from oracle import ref_op, tolerance
 
 pytestmark = pytest.mark.gpu
@@ -15,24 +15,43 @@ ARCH = aat.MI355X()
 SHAPES = [(1, 2, 32, 32), (2, 2, 96, 160), (1, 2, 288, 288), (1, 2, 160, 96), (1, 1, 64, 544), (1, 1, 416, 416)]
 
 
+def _check(problem, dqk, dv, causal, seed, cfgs):
+    b, h, sq, sk = problem
+    g = torch.Generator().manual_seed(seed)
+    q, k, v, do = (torch.randn(b, h, s, d, generator=g).half() for s, d in ((sq, dqk), (sk, dqk), (sk, dv), (sq, dv)))
+    o, lse = ref_op.attention_ref(q, k, v, None, causal, return_lse=True)
+    o = o.half()
+    want = ref_op.attention_bwd_ref(q, k, v, do, None, causal)
+    terms = ref_op.attention_bwd_rounding_bound(q, k, v, do, None, causal, o_stored=o)
+    for cfg in cfgs:
+        print(dqk, dv, causal, problem, cfg, flush=True)
+        out = [torch.full_like(t, 7.0, device="cuda") for t in (q, k, v)]
+        Runtime(ARCH, cfg).apply([q.cuda(), k.cuda(), v.cuda(), o.cuda(), do.cuda(), lse.cuda(), *out], softmax_scale=1 / math.sqrt(dqk), causal=causal)
+        torch.cuda.synchronize()
+        for name, got, ref, t in zip(("dq", "dk", "dv"), out, want, terms):
+            ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
+            assert ok, (name, worst, ratio)
+
+
 @pytest.mark.parametrize("d", sorted(p[0] for p in gfx950_space.ATTN_BWD_RULE))
 @pytest.mark.parametrize("causal", [False, True])
 def test_every_rule_shape_at_the_edges_of_its_tiles(d, causal):
-    for i, (b, h, sq, sk) in enumerate(SHAPES):
-        g = torch.Generator().manual_seed(300 + i)
-        q, k, v, do = (torch.randn(b, h, s, d, generator=g).half() for s in (sq, sk, sk, sq))
-        o, lse = ref_op.attention_ref(q, k, v, None, causal, return_lse=True)
-        o = o.half()
-        want = ref_op.attention_bwd_ref(q, k, v, do, None, causal)
-        terms = ref_op.attention_bwd_rounding_bound(q, k, v, do, None, causal, o_stored=o)
-        for cfg in gfx950_space.rule_attn_backward_configs(d, d):
-            print(d, causal, (b, h, sq, sk), cfg, flush=True)
-            out = [torch.full_like(t, 7.0, device="cuda") for t in (q, k, v)]
-            Runtime(ARCH, cfg).apply([q.cuda(), k.cuda(), v.cuda(), o.cuda(), do.cuda(), lse.cuda(), *out], softmax_scale=1 / math.sqrt(d), causal=causal)
-            torch.cuda.synchronize()
-            for name, got, ref, t in zip(("dq", "dk", "dv"), out, want, terms):
-                ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
-                assert ok, (name, worst, ratio)
+    for i, problem in enumerate(SHAPES):
+        _check(problem, d, d, causal, 300 + i, gfx950_space.rule_attn_backward_configs(d, d))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_two_row_groups_per_wave_and_one_column_kernel_per_output(causal):
+    """A wave of the last block may have one of its two row groups; with one column kernel per output both carry the general form."""
+    groups = [c for c in prebuilt_extra.ragged_row_group_configs() if c.operation == "attn_bwd"]
+    assert all(c.Br // (c.Nthreads // 64) == 64 for c in groups)
+    split = [prebuilt_extra.attn_bwd_split_config(*t) for t in prebuilt_extra.ATTN_BWD_SPLIT_TILES]
+    wide = [gfx950_space.default_attn_backward_config(256, 512, ARCH, s, s) for s in (96, 1344)]
+    assert all(c.col_split for c in split + wide)
+    for i, problem in enumerate([(1, 2, 96, 160), (1, 2, 288, 288), (2, 1, 160, 96)]):
+        _check(problem, 64, 64, causal, 330 + i, groups)
+        _check(problem, 128, 128, causal, 340 + i, split)
+        _check(problem, 256, 512, causal, 350 + i, wide)
 
 
 @pytest.mark.parametrize("d", sorted(p[0] for p in gfx950_space.ATTN_BWD_RULE))

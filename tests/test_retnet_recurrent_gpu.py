@@ -34,8 +34,8 @@ def _close(got, ref):
     assert err <= RTOL_OF_MAX * scale, (err, scale)
 
 
-# value slices of 64 and 128 dims, 64 and 128 key dims, few and many blocks (both launch shapes), ragged
-# chunk counts (odd number of 32-position chunks), a single chunk, more than 128 key dims (passes that add)
+# 64, 128 and more key dims, value dims that 128 does and does not divide, few and many chunks, an odd number of them, a single
+# one; all with few blocks, so the waves of a block split the key dims
 @pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(1, 2, 128, 128, 256), (1, 3, 64, 256, 96), (2, 1, 128, 64, 32),
                                                    (1, 2, 64, 64, 160), (2, 2, 64, 192, 64), (1, 2, 256, 64, 96),
                                                    (1, 1, 192, 128, 64)])
@@ -81,8 +81,21 @@ def test_many_blocks_take_the_wide_value_slice_and_agree_with_the_narrow_one():
     out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
     ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
     _close(out, ref)
-    narrow = aat.retnet_recurrent_fwd(q[:2].cuda(), k[:2].cuda(), v[:2].cuda(), decay.cuda())
-    _close(narrow, ref[:2])
+    # 64 of the value dims: 192 slices of 64 of them fit at once (two to a compute unit), 384 slices of 32 take two rounds
+    narrow = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v[:, :, :64].contiguous().cuda(), decay.cuda())
+    _close(narrow, ref[:, :, :64])
+
+
+# more than 128 key dims where 128-wide value slices fill the chip and the split blocks would take four rounds: passes over 128 and
+# 64 key dims, the second of which adds to the first one's output
+@pytest.mark.parametrize("kdim", [192, 256])
+def test_passes_over_the_key_dims_add_up(kdim):
+    q, k, v, decay = _inputs(12, 8, 32, kdim, 128, 64, -0.3, 1.2)
+    decay[0, 40] = 0.0
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(32):
+        _close(out[:, head], ref[:, head])
 
 
 def test_block_kdim_limits_the_contraction():
