@@ -18,7 +18,7 @@ class KernelLaunchError(RuntimeError):
     pass
 
 
-_ERRORS = {-2: "sequence lengths are not multiples of the configuration's tile (Br, Bc)",
+_ERRORS = {-2: "sequence lengths are not multiples of what the library takes: 32 where its row blocks and tiles may be partial, else the tile (Br, Bc)",
            -3: "workspace missing or too small"}
 
 

@@ -5,8 +5,9 @@
 // in one part, 35 us in three or six.  Every part costs a second kernel and a round trip of its fp32 output, so a problem
 // that fills the chip, or whose walk is short, stays in one part.
 //
-// The estimate below is the launch's time in microseconds, fitted on 3 700 launches of 37 tile shapes (d 64 ... 256, 26
-// problems, both walks, 1 ... 32 parts; mean error 12 %).  Over those launches the parts it picks are 2 % slower on the
+// The estimate below is the launch's time in microseconds, fitted on 3 700 launches of 38 tile shapes (d 64 ... 256, 26
+// problems, both walks, 1 ... 32 parts; mean error 12 % there).  It knows matrix work only: on 136 problems outside the fit it is
+// 7 to 25 % low, more where the stream from memory bounds a launch.  Over the launches of the fit the parts it picks are 2 % slower on the
 // mean than the best ones; the simplest rule, one block per CU, is 5 % and up to twice the time on long kv ranges, where
 // a second block per CU pays.  autotuner/gfx950_space.py holds the same estimate to choose between tile shapes.
 #pragma once

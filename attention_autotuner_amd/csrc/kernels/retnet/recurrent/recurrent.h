@@ -551,17 +551,16 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
 // rows of the output.  Q is read once per wave and feeds both contractions.
 //
 // Bound by fp32 MFMA like the kernel above; a slice of 32 repeats S^T in every block, so a chunk costs
-// (3 KD + 32) / (2 KD + 32 + KD / 4) of the work of a 128-wide slice, 1.27 to 1.36 times, against four times the blocks.
-// B2 H8 L1056 256/512, 256 blocks: 374 -> 144 us a call; at 2048 positions a chunk takes 3.4 us instead of 5.5 in each of
-// two passes, 2.9 us of them matrix instructions (100 of 64 cycles at 2.2 GHz).
+// (3 KD + 32) / (2 KD + 32 + KD / 4) of the work of a 128-wide slice, 1.27 times (KD 64) and 1.30 (KD 128), against four times the
+// blocks.  B4 H8 L2048 128/256, 256 blocks: 353 -> 145 us a call.
 // All key dims are contracted in one pass, so nothing is written twice and added.  K, Q, V and the factors are
 // double-buffered; S^T partials reuse the wave's own rows of the consumed Q tile.  The products D of the
 // decays, 4 KB per chunk of which a wave needs the rows of its group, skip LDS, which at KD 256 has no room for them.
 //
-// PRE: P itself comes from global memory in the same layout, made once per (batch, head) by retnet_recurrent_pmat below, for
-// callers with room for 4 KB per (batch, head, chunk).  That is a third of the matrix instructions of a block (32 of 100 at KD
-// 256) and the exchange of S^T, for one more read of q and k.  B2 H8 L1056 256/512: 136 -> 107 us a call; B4 H16 L2048
-// 192/256: 466 -> 371, 256/256: 447 -> 391.
+// PRE, taken beyond 128 key dims: P itself comes from global memory in the same layout, made once per (batch, head) by
+// retnet_recurrent_pmat above, 4 KB per (batch, head, chunk).  That is a third of the matrix instructions of a wave (32 of 100 at KD
+// 256: 68 x 64 cycles, 2.0 of 2.5 us a chunk) and the exchange of S^T, for one more read of q and k.  Whole calls, passes over 128 key
+// dims -> one pass without PRE -> with it: B2 H8 L1056 256/512 376 -> 119 -> 94 us; B4 H16 L2048 192/256: 609 -> 466 -> 371.
 template <int KD, int WK>
 struct RetRecurrentSplit {
   static constexpr int kChunk = 32;

@@ -13,7 +13,10 @@ DEFAULT_LOG_DIR = os.environ.get("AAT_LOG_DIR", os.path.join(_PKG, "logs"))
 # Octaves (BaseTunner.nearest_cached) within which a tuned problem's entry is taken before a built-in default that looks at the
 # whole problem (gfx950_space.covered_by_rule).
 # Attention forward, random problems: entries up to 3 octaves away run within 1 % of what the rule picks, entries 4 ... 12
-# octaves away are 9 % slower on the mean and up to 32 % (256-row blocks on 256 rows of 60 heads: 10.5 against 8.1 us).
+# octaves away are 9 % slower on the mean and up to 32 % (256-row blocks on 256 rows of 60 heads: 10.5 against 8.1 us).  The other
+# operators' rules were compared with the best of five to eight shapes (1 to 4 % slower on the mean, gfx950_space.py), not with
+# entries by distance; half the distance that is safe in the forward keeps an entry where it was tuned, one length or row count
+# off by less than a factor of three.
 NEAR_ENOUGH = 1.5
 
 

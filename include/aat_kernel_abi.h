@@ -13,8 +13,10 @@
  *   - q [B,H,Seq_q,Kd], k [B,H,Seq_k,Kd], v [B,H,Seq_k,D], o/dO [B,H,Seq_q,D] are IEEE fp16;
  *     mask [H,Seq_q,Seq_k] fp16; r [B,H,Seq_q] fp32; dqaccum [B,H,Seq_q,Kd] fp32, zero on entry;
  *   - Kd, D and the tile shape are baked into the library (see config_string());
- *   - Seq_q must be a multiple of the library's Br and Seq_k of its Bc; the register-fused attention forward takes any
- *     lengths that are multiples of 32;
+ *   - lengths: the register-fused attention forward and the attention backward take any multiples of 32; the register-fused
+ *     RetNet forward takes a Seq_q that is any multiple of 32 and a Seq_k that is a multiple of the library's Bc, the RetNet
+ *     backward takes lengths that are multiples of 32 and of its Bc; the LDS-fused forwards take a Seq_q that is a multiple of
+ *     Br and a Seq_k that is a multiple of Bc;
  *   - `profile*` launches the kernel repeatedly (one probe launch, then ceil(100 ms / t) launches) and
  *     returns the mean time of one launch in milliseconds, or -1 on any error;
  *   - `kernel_entry*` enqueues one launch and returns without synchronising.
@@ -23,7 +25,7 @@
  *   - the two reference-signature entry points keep the reference's argument ORDER, including the
  *     swapped (Seq_k, Seq_q) of kernel_entry, and its literal behaviour: softmax scale 0.125, no causal
  *     masking, null stream.  kernel_entry returns 0 on success (the reference always returns 0),
- *     a positive hipError_t on a launch failure, AAT_ERR_SHAPE for an indivisible shape;
+ *     a positive hipError_t on a launch failure, AAT_ERR_SHAPE for lengths the library does not take;
  *   - the *_ex entry points take (Seq_q, Seq_k) in that order plus a runtime softmax scale, a causal
  *     flag, an optional workspace and the stream to launch on (a hipStream_t passed as void*);
  *   - workspace_size() says how many bytes of workspace a problem needs (attention forward: 0 unless the kv
