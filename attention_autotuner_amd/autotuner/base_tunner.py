@@ -139,7 +139,7 @@ class BaseTunner:
         s = self.problem_shape
         need = int(lib.workspace_size(s["B"], s["H"], s["Sq"], s["Sk"]))
         if config is not None:
-            need = _wanted(config, need, s["B"], s["H"], s["Sq"], s["Sk"])
+            need = _wanted(config, need, s["B"], s["H"], s["Sq"], s["Sk"], self.decay)
         ws = torch.empty(need, dtype=torch.uint8, device=self.torch_array[0].device) if need else None
         return ws, need
 

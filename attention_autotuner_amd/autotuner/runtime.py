@@ -11,7 +11,7 @@ import os
 
 import torch
 
-from . import codegen, library
+from . import codegen, gfx950_space, library
 
 
 class KernelLaunchError(RuntimeError):
@@ -24,16 +24,19 @@ _ERRORS = {-2: "sequence lengths are not multiples of what the library takes: 32
 
 # A RetNet backward built with a stored dS asks for B*H*S_q*S_kv fp16 on top of the mask scan and works without them
 # (it then evaluates dS twice).  Beyond this many bytes the runtime does not grant the room on its own: a caller who
-# wants it there passes a workspace of workspace_size() bytes.
+# wants it there passes a workspace of workspace_size() bytes.  The same limit holds for the slots of a decay walk whose longest
+# blocks are walked in parts, which a call without the room walks in one piece.
 MAX_DS_BYTES = int(os.environ.get("AAT_MAX_DS_BYTES", 2 << 30))
 
 
-def _wanted(config, need, B, H, Sq, Sk):
+def _wanted(config, need, B, H, Sq, Sk, decay=False):
     """Bytes of workspace the runtime provides when the caller's is missing or too small."""
     ds_bytes = 2 * B * H * Sq * Sk
-    if getattr(config, "operation", "") == "ret_bwd" and getattr(config, "ds_rows", 0) and need >= ds_bytes > MAX_DS_BYTES:
-        return need - ds_bytes
-    return need
+    stored = getattr(config, "operation", "") == "ret_bwd" and getattr(config, "ds_rows", 0) and need >= ds_bytes
+    if stored and ds_bytes > MAX_DS_BYTES:
+        need, stored = need - ds_bytes, False
+    parts = gfx950_space.decay_parts_bytes(config, B, H, Sq, Sk, stored) if decay else 0
+    return need + (parts if parts <= MAX_DS_BYTES else 0)
 
 
 def _grown(workspace, need, device, keep):
@@ -92,9 +95,9 @@ class Runtime:
         lib = self._lib
         if lib is None:
             lib = self._lib = library.load(self._path(), op)
-        need = self._need.get((B, H, Sq, Sk))               # a property of the library and the problem: asked once
+        need = self._need.get((B, H, Sq, Sk, decay))        # a property of the library and the problem: asked once
         if need is None:
-            need = self._need[(B, H, Sq, Sk)] = _wanted(self.config, int(lib.workspace_size(B, H, Sq, Sk)), B, H, Sq, Sk)
+            need = self._need[(B, H, Sq, Sk, decay)] = _wanted(self.config, int(lib.workspace_size(B, H, Sq, Sk)), B, H, Sq, Sk, decay)
         if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
             workspace = _grown(workspace, need, q.device, keep=causal == "scanned")
         ws_ptr = workspace.data_ptr() if workspace is not None else None

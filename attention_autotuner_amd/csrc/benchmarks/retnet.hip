@@ -83,9 +83,10 @@ static void report(const char* what, const ProblemShape& ps, MaskKind m, const a
 
 static int g_failures = 0;
 
-template <class Plain, class Decay>
+// more: what the kernel takes behind the mask scan's ranges
+template <class Plain, class Decay, class... More>
 static void run_all_masks(const char* what, const ProblemShape& ps, Tensors& t, int Br, int Bc, int threads, int lds_bytes,
-                          Plain plain, Decay decay) {
+                          Plain plain, Decay decay, More... more) {
   if (ps.Sq % Br || ps.Sk % Bc) {
     std::printf("%-58s skipped: Sq %% %d or Sk %% %d\n", what, Br, Bc);
     return;
@@ -98,13 +99,13 @@ static void run_all_masks(const char* what, const ProblemShape& ps, Tensors& t, 
     const MaskArgs a = mask_args(t, m);
     auto launch = [&] {
       if (m == MaskKind::Decay) {
-        decay<<<grid, block, lds_bytes, 0>>>(t.q.dev, t.k.dev, t.v.dev, nullptr, t.o.dev, t.r.dev, ps.H, ps.Sk, ps.Sq, 1, a.log2_gamma, nullptr);
+        decay<<<grid, block, lds_bytes, 0>>>(t.q.dev, t.k.dev, t.v.dev, nullptr, t.o.dev, t.r.dev, ps.H, ps.Sk, ps.Sq, 1, a.log2_gamma, nullptr, more...);
         return;
       }
       aat::MaskWalk walk;
       HIP_OK(aat::prepare_mask_walk(a.walk_mode, a.mask, ps.H, ps.Sq, ps.Sk, a.workspace, 0, &walk));
       plain<<<grid, block, lds_bytes, 0>>>(t.q.dev, t.k.dev, t.v.dev, a.mask, t.o.dev, t.r.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr,
-                                           walk.extents);
+                                           walk.extents, more...);
     };
     HIP_OK(hipMemset(t.o.dev, 0xff, t.o.host.size() * sizeof(half_t)));
     launch();
@@ -122,7 +123,7 @@ static void test_regfuse_retnet(const ProblemShape& ps, Tensors& t) {
   char name[128];
   std::snprintf(name, sizeof name, "regfuse  Br=%d Bc=%d thr=%d bufs=%d/%d/%d waves/SIMD=%d", Br, Bc, NT, NSK, NSV, NSM, WPE);
   run_all_masks(name, ps, t, Br, Bc, NT, T::kSmemBytes, &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, false>,
-                &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, true>);
+                &aat::ret_fwd_regfuse<Kd, D, Br, Bc, NT, NSK, NSV, NSM, WPE, true>, aat::BlockParts());   // every block in one piece
 }
 
 // LDS-fused: <Br, Bc, threads, K buffers, V buffers, mask buffers, waves along kv, waves along d, waves per SIMD>

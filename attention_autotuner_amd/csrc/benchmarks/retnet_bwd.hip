@@ -142,17 +142,17 @@ static void test_retnet_bwd(const ProblemShape& ps, Tensors& t) {
     auto launch = [&] {
       if (m == MaskKind::Decay) {
         const float* lg = t.log2_gamma.dev;
-        dv_decay<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, nullptr, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr);
-        dk_decay<<<grid_k, block, TK::kSmemBytes, 0>>>(t.v.dev, t.dout.dev, t.q.dev, nullptr, t.r.dev, t.dk.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr);
-        dq_decay<<<grid_q, block, TQ::kSmemBytes, 0>>>(t.dout.dev, t.v.dev, t.k.dev, nullptr, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr);
+        dv_decay<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, nullptr, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr, aat::BlockParts());
+        dk_decay<<<grid_k, block, TK::kSmemBytes, 0>>>(t.v.dev, t.dout.dev, t.q.dev, nullptr, t.r.dev, t.dk.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr, aat::BlockParts());
+        dq_decay<<<grid_q, block, TQ::kSmemBytes, 0>>>(t.dout.dev, t.v.dev, t.k.dev, nullptr, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr, aat::BlockParts());
         return;
       }
       const int mode = m == MaskKind::Dense ? aat::kMaskDense : m == MaskKind::Causal ? aat::kMaskCausal : aat::kMaskScanned;
       aat::MaskWalk walk;
       HIP_OK(aat::prepare_mask_walk(mode, mask, ps.H, ps.Sq, ps.Sk, t.scan, 0, &walk));
-      dv_plain<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, mask, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr);
-      dk_plain<<<grid_k, block, TK::kSmemBytes, 0>>>(t.v.dev, t.dout.dev, t.q.dev, mask, t.r.dev, t.dk.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr);
-      dq_plain<<<grid_q, block, TQ::kSmemBytes, 0>>>(t.dout.dev, t.v.dev, t.k.dev, mask, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr);
+      dv_plain<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, mask, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr, aat::BlockParts());
+      dk_plain<<<grid_k, block, TK::kSmemBytes, 0>>>(t.v.dev, t.dout.dev, t.q.dev, mask, t.r.dev, t.dk.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr, aat::BlockParts());
+      dq_plain<<<grid_q, block, TQ::kSmemBytes, 0>>>(t.dout.dev, t.v.dev, t.k.dev, mask, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr, aat::BlockParts());
     };
     for (auto* x : {&t.dq, &t.dk, &t.dv}) HIP_OK(hipMemset(x->dev, 0xff, x->host.size() * sizeof(half_t)));
     launch();
@@ -204,17 +204,17 @@ static void test_retnet_bwd_stored_ds(const ProblemShape& ps, Tensors& t) {
     auto launch = [&] {
       if (m == MaskKind::Decay) {
         const float* lg = t.log2_gamma.dev;
-        dv_decay<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, nullptr, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr);
-        dq_decay<<<grid_q, block, TQ::kSmemBytesDsOut, 0>>>(t.dout.dev, t.v.dev, t.k.dev, nullptr, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, t.ds);
-        dk_ds<<<grid_k, kblock, TK::kSmemBytes, 0>>>(t.q.dev, t.ds, t.dk.dev, ps.H, ps.Sk, ps.Sq, 1, nullptr, Br, Bc);
+        dv_decay<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, nullptr, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, nullptr, aat::BlockParts());
+        dq_decay<<<grid_q, block, TQ::kSmemBytesDsOut, 0>>>(t.dout.dev, t.v.dev, t.k.dev, nullptr, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, 1, lg, nullptr, t.ds, aat::BlockParts());
+        dk_ds<<<grid_k, kblock, TK::kSmemBytes, 0>>>(t.q.dev, t.ds, t.dk.dev, ps.H, ps.Sk, ps.Sq, 1, nullptr, Br, Bc, aat::BlockParts());
         return;
       }
       const int mode = m == MaskKind::Dense ? aat::kMaskDense : m == MaskKind::Causal ? aat::kMaskCausal : aat::kMaskScanned;
       aat::MaskWalk walk;
       HIP_OK(aat::prepare_mask_walk(mode, mask, ps.H, ps.Sq, ps.Sk, t.scan, 0, &walk));
-      dv_plain<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, mask, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr);
-      dq_plain<<<grid_q, block, TQ::kSmemBytesDsOut, 0>>>(t.dout.dev, t.v.dev, t.k.dev, mask, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, t.ds);
-      dk_ds<<<grid_k, kblock, TK::kSmemBytes, 0>>>(t.q.dev, t.ds, t.dk.dev, ps.H, ps.Sk, ps.Sq, walk.causal, walk.extents, Br, Bc);
+      dv_plain<<<grid_v, block, TV::kSmemBytes, 0>>>(t.k.dev, t.q.dev, t.dout.dev, mask, t.r.dev, t.dv.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, nullptr, aat::BlockParts());
+      dq_plain<<<grid_q, block, TQ::kSmemBytesDsOut, 0>>>(t.dout.dev, t.v.dev, t.k.dev, mask, t.r.dev, t.dq.dev, ps.H, ps.Sk, ps.Sq, walk.causal, nullptr, walk.extents, t.ds, aat::BlockParts());
+      dk_ds<<<grid_k, kblock, TK::kSmemBytes, 0>>>(t.q.dev, t.ds, t.dk.dev, ps.H, ps.Sk, ps.Sq, walk.causal, walk.extents, Br, Bc, aat::BlockParts());
     };
     for (auto* x : {&t.dq, &t.dk, &t.dv}) HIP_OK(hipMemset(x->dev, 0xff, x->host.size() * sizeof(half_t)));
     HIP_OK(hipMemset(t.ds, 0x7f, (size_t)ps.B * ps.H * ps.Sq * ps.Sk * sizeof(half_t)));     // NaN patterns where nothing is written

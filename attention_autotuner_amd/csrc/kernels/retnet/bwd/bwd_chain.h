@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "../../utils/acc_file.h"
+#include "../../utils/block_parts.h"
 #include "../../utils/cdna4.h"
 #include "../../utils/mask_extents.h"
 #include "../../utils/retention.h"
@@ -83,6 +84,7 @@ struct RetBwdChain {
 // `causal` promises mask == 0 above the diagonal and only shortens the walk over streamed tiles.
 // DECAY: the mask is gamma_h^(q + diag - kv) below the diagonal and zero above it, built in registers
 // from lg2gamma[h] = log2(gamma_h); `mask` is not read and tiles above the diagonal are skipped.
+// Its longest blocks may be walked by several workgroups (utils/block_parts.h; one column slice per block then).
 // DS_OUT (row pass only): the fp16 E tiles (= dS) this pass forms are also written to ds_out (64 x 64 blocks, ds_layout.h), for
 // a dK kernel that reads them instead of evaluating them again (dk_from_ds.h).  Only the tiles of the walk are written.
 // GEN: resident lengths that are multiples of 32 and not of BX; the 32-row groups a last block does not have repeat its first
@@ -95,7 +97,7 @@ __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(W
 ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const half_t* __restrict__ z,
               const half_t* __restrict__ mask, const float* __restrict__ r, half_t* __restrict__ out, int H,
               int seq_k, int seq_q, int causal, const float* __restrict__ lg2gamma = nullptr,
-              const int* __restrict__ extents = nullptr, half_t* __restrict__ ds_out = nullptr) {
+              const int* __restrict__ extents = nullptr, half_t* __restrict__ ds_out = nullptr, BlockParts in_parts = {}) {
   static_assert(!DS_OUT || PASS == BwdPass::Row, "dS is written by the row pass");
   using T = RetBwdChain<KX, DZ, DZB, BX, BY, Nthreads, NSY, NSZ, PASS>;
   constexpr int RT = T::RT, NT = T::NT, KS = T::KS, DT = T::DT, NCY = T::NCY, NCZ = T::NCZ, NCM = T::NCM, WM = T::WM;
@@ -108,6 +110,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   constexpr bool kNumbered = WPE == 1 && RT == 1 && DT * 16 == 256;
   if constexpr (kNumbered) acc_claim_all();
   if constexpr (DECAY) causal = 1;
+  constexpr bool kParts = DECAY && parts_fit(RT, BY, WPE, 0);
   constexpr int PF = AAT_PF;
   constexpr bool COL = PASS == BwdPass::Col;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -124,7 +127,12 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   const int Tx = GEN ? (seq_x + BX - 1) / BX : seq_x / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
-  if (causal || extents != nullptr) {             // longest blocks first: the last query blocks, the first kv blocks
+  PartId id{};
+  if constexpr (kParts) {
+    id = causal_part(blockIdx.x, gridDim.x, Tx, !COL, in_parts);
+    bh = id.bh;
+    xb = id.blk;
+  } else if (causal || extents != nullptr) {      // longest blocks first: the last query blocks, the first kv blocks
     const TileId t = causal_tile(blockIdx.x, gridDim.x, Tx, !COL);
     bh = t.bh;
     xb = t.blk;
@@ -150,6 +158,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
       j_end = lim < j_end ? lim : j_end;
     }
   }
+  if constexpr (kParts) part_range(id, j_begin, j_end);
 
   const char* yg = reinterpret_cast<const char*>(y + (size_t)bh * seq_y * KX);
   const char* zg = reinterpret_cast<const char*>(z + ((size_t)bh * seq_y) * DZ + dz0);
@@ -497,8 +506,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   if constexpr (kNumbered) acc_settle();
   wait_vmcnt<0>();
   block_sync();
-  // the staging rows are DZB wide; the global rows are DZ wide
-  {
+  const auto finish = [&]() {                     // the staging rows are DZB wide; the global rows are DZ wide
     char* const ostage = smem + wave * WM * T::kOStride;
     half_t* og = out + ((size_t)bh * seq_x + x0 + wave * WM) * DZ + dz0;
     constexpr int kChunksPerRow = DZB / 8;
@@ -526,7 +534,18 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
       const u4v val = *reinterpret_cast<const u4v*>(ostage + row * T::kOStride + c * 16);
       *reinterpret_cast<u4v*>(reinterpret_cast<char*>(og) + (size_t)row * DZ * 2 + c * 16) = val;
     }
+  };
+  if constexpr (kParts) {
+    if (id.parts > 1) {                           // to the end in here: joined again, the two paths' accumulators cost scratch
+      float none[1];
+      bool last;
+      if constexpr (kNumbered) last = combine_parts_numbered<64, 0, Nthreads>(in_parts, id, none, smem);
+      else last = combine_parts<0, Nthreads, 4>(in_parts, id, acc, none, smem);
+      if (last) finish();
+      return;
+    }
   }
+  finish();
 }
 
 }  // namespace aat

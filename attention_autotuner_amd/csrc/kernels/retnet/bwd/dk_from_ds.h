@@ -20,6 +20,7 @@
 #pragma once
 #include <type_traits>
 
+#include "../../utils/block_parts.h"
 #include "../../utils/cdna4.h"
 #include "../../utils/mask_extents.h"
 #include "../../utils/tile_ops.h"
@@ -55,7 +56,7 @@ struct RetBwdDk {
 template <int Kd, int BX, int BY, int Nthreads, int NS, int WPE = 2, int GEN = 0>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, half_t* __restrict__ dk, int H,
-                   int seq_k, int seq_q, int causal, const int* __restrict__ extents, int wr_rows, int wr_cols) {
+                   int seq_k, int seq_q, int causal, const int* __restrict__ extents, int wr_rows, int wr_cols, BlockParts in_parts = {}) {
   using T = RetBwdDk<Kd, BX, BY, Nthreads, NS>;
   constexpr int DT = T::DT, KSTEPS = T::KSTEPS, NCZ = T::NCZ, NCS = T::NCS;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -68,10 +69,11 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   const int Tx = GEN ? (seq_k + BX - 1) / BX : seq_k / BX;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tx, xb = tile % Tx;
+  PartId id{};
   if (causal || extents != nullptr) {             // longest blocks first: the first kv blocks
-    const TileId t = causal_tile(blockIdx.x, gridDim.x, Tx, false);
-    bh = t.bh;
-    xb = t.blk;
+    id = causal_part(blockIdx.x, gridDim.x, Tx, false, in_parts);
+    bh = id.bh;
+    xb = id.blk;
   }
   const int x0 = xb * BX;
   const int cols = GEN && seq_k - x0 < BX ? seq_k - x0 : BX;   // kv rows of this block that exist, a multiple of 64
@@ -87,6 +89,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   } else if (causal) {                            // q tiles that reach kv >= x0:  q >= x0 - diag
     const int first = x0 - diag;
     j_begin = first <= 0 ? 0 : first / BY;
+    part_range(id, j_begin, j_end);
   }
   // walked downwards from the end of the sequence, like the column passes of the chained kernel
   const auto tile_of = [&](int j) { return j_begin + j_end - 1 - j; };
@@ -217,9 +220,17 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
 
   wait_vmcnt<0>();
   block_sync();
-  const float one[1] = {1.f};
-  store_o_tile<1, DT, Kd, T::kOStride>(acc, one, smem + wave * 32 * T::kOStride,
-                                       dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane, 32, !GEN || wave * 32 < cols ? 1 : 0);
+  const auto finish = [&]() {
+    const float one[1] = {1.f};
+    store_o_tile<1, DT, Kd, T::kOStride>(acc, one, smem + wave * 32 * T::kOStride,
+                                         dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane, 32, !GEN || wave * 32 < cols ? 1 : 0);
+  };
+  if (id.parts > 1) {                             // to the end in here: joined again, the two paths' accumulators cost 68 bytes of scratch
+    float none[1];
+    if (combine_parts<0, Nthreads, 4>(in_parts, id, acc, none, smem)) finish();
+    return;
+  }
+  finish();
 }
 
 }  // namespace aat

@@ -53,6 +53,38 @@ template <bool DECAY, int GEN> constexpr auto kernel_dq_ds = &aat::ret_bwd_chain
 template <int GEN> constexpr auto kernel_dk_ds = &aat::ret_bwd_dk_from_ds<Kd, kDkRows, kDkTile, kDkRows * 2, kDkStages, kDkWaves, GEN>;
 static_assert(!kStoredDs || Br % kDkTile == 0, "a query tile of the dK kernel lies inside one block of the row pass");
 
+// The longest blocks of a decay walk in parts (utils/block_parts.h), where the call has room for their slots behind its other
+// workspace.  The launches of a call follow each other and share the slots; each has counts of its own.
+constexpr bool kPartsFit = aat::parts_fit(RTv, Bc, waves_per_eu, 0);
+using PV = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DVB, Nthreads, 0, false>;
+using PQ = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, true>;
+using PK = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, false>;
+using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkRows * 2, 0, false, 270>;    // it streams dS and multiplies little
+struct BwdPlan {{
+  aat::PartsPlan dv, dq, dk;
+  aat::JobOrders<3> orders;
+  size_t counts, slots;
+}};
+BwdPlan plan_of(int B, int H, int Seq_q, int Seq_k, bool stored) {{
+  const long heads = (long)B * H;
+  BwdPlan p{{}};
+  const auto take = [](const auto& found, aat::PartsPlan& plan, aat::JobOrder& order) {{
+    plan = found.plan;
+    if (plan.split) order = found.order;
+  }};
+  constexpr int waves = Nthreads / 64;
+  const int row_lds = stored ? TQ::kSmemBytesDsOut : TQ::kSmemBytes;
+  if (D == DVB) take(PV::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TV::kSmemBytes)), p.dv, p.orders.of[0]);
+  take(PQ::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, row_lds)), p.dq, p.orders.of[1]);
+  if (stored) take(PKD::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(kDkRows / 32, kDkWaves, TKD::kSmemBytes)), p.dk, p.orders.of[2]);
+  else take(PK::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TK::kSmemBytes)), p.dk, p.orders.of[2]);
+  const size_t dk = stored ? PKD::slot_bytes(heads, p.dk) : PK::slot_bytes(heads, p.dk);
+  const size_t dv = PV::slot_bytes(heads, p.dv), dq = PQ::slot_bytes(heads, p.dq);
+  p.slots = dv > dq ? (dv > dk ? dv : dk) : (dq > dk ? dq : dk);
+  p.counts = aat::count_bytes(heads, p.dv) + aat::count_bytes(heads, p.dq) + aat::count_bytes(heads, p.dk);
+  return p;
+}}
+
 bool bwd_shape_ok(int B, int H, int Seq_q, int Seq_k) {{
   // every sequence length plays both roles: resident rows (any multiple of 32) in one pass, streamed rows in another
   return aat::shape_ok(B, H, Seq_q, Seq_k, 32, 32) && aat::shape_ok(B, H, Seq_q, Seq_k, Bc, Bc);
@@ -100,19 +132,44 @@ template <bool DECAY> hipError_t launch_passes(aat_half* q, aat_half* k, aat_hal
   const int causal = DECAY ? 1 : walk.causal;
   const int* extents = DECAY ? nullptr : walk.extents;
   const bool whole_q = Seq_q % Br == 0, whole_k = Seq_k % Br == 0;
-  (whole_k ? kernel_dv<DECAY, 0> : kernel_dv<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_k), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
-      K, Q, G, M, r, DV, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr);
-  if (room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k)) {{
+  const bool stored = room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k);
+  aat::BlockParts dv_parts, dq_parts, dk_parts;
+  if constexpr (DECAY) {{
+    const BwdPlan plan = plan_of(B, H, Seq_q, Seq_k, stored);
+    const size_t at = stored ? ws_bytes_needed(B, H, Seq_q, Seq_k) : ds_offset(H, Seq_q, Seq_k);
+    if (plan.slots > 0 && workspace != nullptr && workspace_bytes >= at + plan.counts + 3 * aat::kOrderBytes + plan.slots) {{
+      char* const room = static_cast<char*>(workspace) + at;
+      uint16_t* const order = reinterpret_cast<uint16_t*>(room + plan.counts);
+      float* const slots = reinterpret_cast<float*>(room + plan.counts + 3 * aat::kOrderBytes);
+      const int n = (int)(plan.counts / sizeof(uint32_t));
+      aat::prepare_parts<3><<<dim3((n + aat::kMostJobs - 1) / aat::kMostJobs), dim3(aat::kMostJobs), 0, stream>>>(
+          reinterpret_cast<uint32_t*>(room), n,
+          plan.orders, order);
+      size_t counted = 0;
+      const auto take = [&](const aat::PartsPlan& p, int launch) {{
+        const aat::BlockParts b{{p.split, p.parts, slots, reinterpret_cast<uint32_t*>(room + counted), order + launch * aat::kMostJobs}};
+        counted += aat::count_bytes((long)B * H, p);
+        return b;
+      }};
+      dv_parts = take(plan.dv, 0);
+      dq_parts = take(plan.dq, 1);
+      dk_parts = take(plan.dk, 2);
+    }}
+  }}
+  const auto grid = [&](int blocks, const aat::BlockParts& p) {{ return (unsigned)(B * H * (blocks + p.split * (p.parts - 1))); }};
+  (whole_k ? kernel_dv<DECAY, 0> : kernel_dv<DECAY, 1>)<<<dim3(grid(blocks_of(Seq_k), dv_parts), D / DVB), dim3(Nthreads), TV::kSmemBytes, stream>>>(
+      K, Q, G, M, r, DV, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr, dv_parts);
+  if (stored) {{
     H16* ds = reinterpret_cast<H16*>(static_cast<char*>(workspace) + ds_offset(H, Seq_q, Seq_k));
-    (whole_q ? kernel_dq_ds<DECAY, 0> : kernel_dq_ds<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
-        G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, ds);
-    (whole_q && Seq_k % kDkRows == 0 ? kernel_dk_ds<0> : kernel_dk_ds<1>)<<<dim3(B * H * ((Seq_k + kDkRows - 1) / kDkRows)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
-        Q, ds, DK, H, Seq_k, Seq_q, causal, extents, Br, Bc);
+    (whole_q ? kernel_dq_ds<DECAY, 0> : kernel_dq_ds<DECAY, 1>)<<<dim3(grid(blocks_of(Seq_q), dq_parts), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
+        G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, ds, dq_parts);
+    (whole_q && Seq_k % kDkRows == 0 ? kernel_dk_ds<0> : kernel_dk_ds<1>)<<<dim3(grid((Seq_k + kDkRows - 1) / kDkRows, dk_parts)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
+        Q, ds, DK, H, Seq_k, Seq_q, causal, extents, Br, Bc, dk_parts);
   }} else {{
-    (whole_k ? kernel_dk<DECAY, 0> : kernel_dk<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_k), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
-        V, G, Q, M, r, DK, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr);
-    (whole_q ? kernel_dq<DECAY, 0> : kernel_dq<DECAY, 1>)<<<dim3(B * H * blocks_of(Seq_q), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
-        G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr);
+    (whole_k ? kernel_dk<DECAY, 0> : kernel_dk<DECAY, 1>)<<<dim3(grid(blocks_of(Seq_k), dk_parts), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(
+        V, G, Q, M, r, DK, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr, dk_parts);
+    (whole_q ? kernel_dq<DECAY, 0> : kernel_dq<DECAY, 1>)<<<dim3(grid(blocks_of(Seq_q), dq_parts), Kd / DKB), dim3(Nthreads), TQ::kSmemBytes, stream>>>(
+        G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, nullptr, dq_parts);
   }}
   return hipGetLastError();
 }}

@@ -25,6 +25,10 @@ template <bool DECAY> constexpr auto kernel = &aat::ret_fwd_regfuse<Kd, D, Br, B
 // a query length the row blocks do not divide
 template <bool DECAY> constexpr auto kernel_ragged = &aat::ret_ragged_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu, DECAY>;
 
+// The longest blocks of a decay walk in parts (utils/block_parts.h), where the call has room for their slots behind workspace_size().
+using Parts = aat::PartsLaunch<aat::parts_fit(Traits::RT, Bc, waves_per_eu, Kd + D), Br, Bc, Kd + D, D, Nthreads, Traits::RT, true>;
+constexpr int kBlocksPerCu = aat::blocks_per_cu(Nthreads / 64, waves_per_eu, shared_mem);
+
 bool lengths_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, Bc); }}
 int row_blocks(int Seq_q) {{ return (Seq_q + Br - 1) / Br; }}
 template <bool DECAY> hipError_t allow_kernels() {{
@@ -43,18 +47,32 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_hal
   (Seq_q % Br == 0 ? kernel<false> : kernel_ragged<false>)<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<const aat::half_t*>(mask),
-      reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, walk.causal, nullptr, walk.extents);
+      reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, walk.causal, nullptr, walk.extents, aat::BlockParts());
   return hipGetLastError();
 }}
 // Decay-mask variant: the mask is gamma_h^(q + Seq_k - Seq_q - kv) below the diagonal, zero above it.
 hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r, int B,
-                        int H, int Seq_q, int Seq_k, hipStream_t stream) {{
+                        int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes, hipStream_t stream) {{
   static const hipError_t lds_ok = allow_kernels<true>();
   if (lds_ok != hipSuccess) return lds_ok;
-  (Seq_q % Br == 0 ? kernel<true> : kernel_ragged<true>)<<<dim3(B * H * row_blocks(Seq_q)), dim3(Nthreads), shared_mem, stream>>>(
+  const auto& found = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
+  const aat::PartsPlan& plan = found.plan;
+  const size_t at = workspace_size(B, H, Seq_q, Seq_k), counts = aat::count_bytes((long)B * H, plan);
+  aat::BlockParts in_parts;
+  if (plan.split > 0 && workspace != nullptr && workspace_bytes >= at + counts + aat::kOrderBytes + Parts::slot_bytes((long)B * H, plan)) {{
+    char* const room = static_cast<char*>(workspace) + at;
+    uint32_t* const arrived = reinterpret_cast<uint32_t*>(room);
+    uint16_t* const order = reinterpret_cast<uint16_t*>(room + counts);
+    const int n = B * H * plan.split;
+    aat::prepare_parts<1><<<dim3((n + aat::kMostJobs - 1) / aat::kMostJobs), dim3(aat::kMostJobs), 0, stream>>>(
+        arrived, n, {{found.order}}, order);
+    in_parts = {{plan.split, plan.parts, reinterpret_cast<float*>(room + counts + aat::kOrderBytes), arrived, order}};
+  }}
+  const int jobs = row_blocks(Seq_q) + in_parts.split * (in_parts.parts - 1);
+  (Seq_q % Br == 0 ? kernel<true> : kernel_ragged<true>)<<<dim3(B * H * jobs), dim3(Nthreads), shared_mem, stream>>>(
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), nullptr, reinterpret_cast<aat::half_t*>(o), r, H, Seq_k, Seq_q, 1,
-      log2_gamma, nullptr);
+      log2_gamma, nullptr, in_parts);
   return hipGetLastError();
 }}
 }}  // namespace
@@ -98,15 +116,15 @@ extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* mas
 
 decay_entry = r"""
 extern "C" float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
-                               int B, int H, int Seq_q, int Seq_k, void*, size_t, void* stream) {{
+                               int B, int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes, void* stream) {{
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return aat::timed_mean_ms(s, [&] {{ return launch_decay(q, k, v, log2_gamma, o, r, B, H, Seq_q, Seq_k, s); }});
+  return aat::timed_mean_ms(s, [&] {{ return launch_decay(q, k, v, log2_gamma, o, r, B, H, Seq_q, Seq_k, workspace, workspace_bytes, s); }});
 }}
 extern "C" int kernel_entry_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
-                                  int B, int H, int Seq_q, int Seq_k, void*, size_t, void* stream) {{
+                                  int B, int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes, void* stream) {{
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return AAT_ERR_SHAPE;
-  return (int)launch_decay(q, k, v, log2_gamma, o, r, B, H, Seq_q, Seq_k, static_cast<hipStream_t>(stream));
+  return (int)launch_decay(q, k, v, log2_gamma, o, r, B, H, Seq_q, Seq_k, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }}
 """
 

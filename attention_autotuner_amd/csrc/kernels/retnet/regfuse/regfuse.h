@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "../../utils/acc_file.h"
+#include "../../utils/block_parts.h"
 #include "../../utils/cdna4.h"
 #include "../../utils/mask_extents.h"
 #include "../../utils/retention.h"
@@ -52,11 +53,13 @@ struct RetFwdRegfuse {
 };
 
 // DECAY: the mask is gamma_h^(q + diag - kv) below the diagonal and zero above it, built in registers
-// from lg2gamma[h] = log2(gamma_h); `mask` is not read and tiles above the diagonal are skipped.
+// from lg2gamma[h] = log2(gamma_h); `mask` is not read and tiles above the diagonal are skipped.  Its longest blocks may be
+// walked by several workgroups (utils/block_parts.h): a part's slot holds its O times r_ref and its |S| sums.
 template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE, int GEN, bool DECAY>
 AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
                           const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H, int seq_k,
-                          int seq_q, int causal, const float* __restrict__ lg2gamma, const int* __restrict__ extents) {
+                          int seq_q, int causal, const float* __restrict__ lg2gamma, const int* __restrict__ extents,
+                          const BlockParts& in_parts) {
   // One wave per SIMD: the output tile lives in the accumulation registers by number (utils/acc_file.h), the score
   // tile in vector registers through hand-written matrix instructions, and the compiler allocates the rest.
   constexpr bool kNumbered = WPE == 1;
@@ -64,6 +67,7 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
   if constexpr (DECAY) causal = 1;
   using T = RetFwdRegfuse<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM>;
   constexpr int RT = T::RT, NT = T::NT, KS = T::KS, DT = T::DT, NCK = T::NCK, NCV = T::NCV, NCM = T::NCM, WM = T::WM;
+  constexpr bool kParts = DECAY && parts_fit(RT, Bc, WPE, Kd + D);
   constexpr int PF = AAT_PF;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   char* const kbuf = smem;
@@ -78,7 +82,12 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
   const int Tr = GEN ? (seq_q + Br - 1) / Br : seq_q / Br;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   int bh = tile / Tr, rb = tile % Tr;
-  if (causal || extents != nullptr) {             // a scanned mask is taken to be of the causal kind: later rows see more
+  PartId id{};
+  if constexpr (kParts) {
+    id = causal_part(blockIdx.x, gridDim.x, Tr, true, in_parts);
+    bh = id.bh;
+    rb = id.blk;
+  } else if (causal || extents != nullptr) {      // a scanned mask is taken to be of the causal kind: later rows see more
     const TileId t = causal_tile(blockIdx.x, gridDim.x, Tr, true);
     bh = t.bh;
     rb = t.blk;
@@ -95,6 +104,8 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
     const int lim = last < 0 ? 0 : last / Bc + 1;
     n_tiles = lim < n_tiles ? lim : n_tiles;
   }
+  int j_begin = 0;
+  if constexpr (kParts) part_range(id, j_begin, n_tiles);
 
   const char* kg = reinterpret_cast<const char*>(k + (size_t)bh * seq_k * Kd);
   const char* vg = reinterpret_cast<const char*>(v + (size_t)bh * seq_k * D);
@@ -152,9 +163,9 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
       else mdma.issue(mg + (size_t)j * Bc * 2, mbuf + (NSM == 2 ? par * T::kMBytes : 0), wave_base);
     }
   };
-  if (n_tiles > 0) {
-    issue_km(0, 0);
-    if constexpr (NSV == 2) vdma.issue(vg, vbuf, wave_base);
+  if (n_tiles > j_begin) {
+    issue_km(j_begin, 0);
+    if constexpr (NSV == 2) vdma.issue(vg + (size_t)j_begin * T::kVBytes, vbuf, wave_base);
   }
 
   if constexpr (kNumbered) {
@@ -172,7 +183,7 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
     // One loop body for both buffer parities: the parity is a run-time value that moves the operand addresses and the
     // copy destinations.
     int par = 0;
-    for (int j = 0; j < n_tiles; ++j) {
+    for (int j = j_begin; j < n_tiles; ++j) {
       const bool more = (j + 1 < n_tiles);
       // (A) K_j, mask_j (and with two V buffers V_j) have landed; every wave is past iteration j-1.
       wait_vmcnt<0>();
@@ -249,6 +260,20 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
     acc_settle();
     wait_vmcnt<0>();
     block_sync();
+    if constexpr (kParts) {
+      if (id.parts > 1) {
+        float sums[RT];
+        static_for<RT>([&](auto rt_tag) {
+          constexpr int rt = decltype(rt_tag)::value;
+          acc_scale<16 * rt * DT, 16 * DT>(row[rt].r_ref);     // every part on the same footing
+          row[rt].r_ref = 1.f;
+          sums[rt] = row[rt].big_r;
+        });
+        if (!combine_parts_numbered<4 * RT * DT, RT, Nthreads>(in_parts, id, sums, smem)) return;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) row[rt].big_r = sums[rt];
+      }
+    }
     float scale[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -312,7 +337,7 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
   };
   using P0 = std::integral_constant<int, 0>;
   using P1 = std::integral_constant<int, 1>;
-  for (int j = 0; j < n_tiles; j += 2) {
+  for (int j = j_begin; j < n_tiles; j += 2) {
     kv_tile(j, P0{});
     if (j + 1 < n_tiles) kv_tile(j + 1, P1{});
   }
@@ -320,15 +345,37 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
   // ---- epilogue -------------------------------------------------------------------------------------
   wait_vmcnt<0>();
   block_sync();
-  float scale[RT];
+  const auto finish = [&]() {
+    float scale[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const float r_fin = fmaxf(row[rt].big_r, 1.0f);
-    scale[rt] = row[rt].r_ref * fast_rcp(r_fin);
-    if (h == 0 && rt < groups) r[(size_t)bh * seq_q + q0 + wave * WM + rt * 32 + n] = r_fin;
+    for (int rt = 0; rt < RT; ++rt) {
+      const float r_fin = fmaxf(row[rt].big_r, 1.0f);
+      scale[rt] = row[rt].r_ref * fast_rcp(r_fin);
+      if (h == 0 && rt < groups) r[(size_t)bh * seq_q + q0 + wave * WM + rt * 32 + n] = r_fin;
+    }
+    store_o_tile<RT, DT, D, T::kOStride>(oacc, scale, smem + wave * WM * T::kOStride,
+                                         o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane, 32, groups);
+  };
+  if constexpr (kParts) {
+    if (id.parts > 1) {                           // to the end in here: joined again, the two paths' accumulators cost scratch
+      float sums[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) oacc[rt][dt][e] *= row[rt].r_ref;
+        row[rt].r_ref = 1.f;
+        sums[rt] = row[rt].big_r;
+      }
+      if (!combine_parts<RT, Nthreads, 4>(in_parts, id, oacc, sums, smem)) return;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) row[rt].big_r = sums[rt];
+      finish();
+      return;
+    }
   }
-  store_o_tile<RT, DT, D, T::kOStride>(oacc, scale, smem + wave * WM * T::kOStride,
-                                       o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane, 32, groups);
+  finish();
 }
 
 template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, bool DECAY = false>
@@ -336,8 +383,8 @@ __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(W
 ret_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
                 const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H,
                 int seq_k, int seq_q, int causal, const float* __restrict__ lg2gamma = nullptr,
-                const int* __restrict__ extents = nullptr) {
-  ret_fwd_walk<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM, WPE, 0, DECAY>(q, k, v, mask, o, r, H, seq_k, seq_q, causal, lg2gamma, extents);
+                const int* __restrict__ extents = nullptr, BlockParts in_parts = {}) {
+  ret_fwd_walk<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM, WPE, 0, DECAY>(q, k, v, mask, o, r, H, seq_k, seq_q, causal, lg2gamma, extents, in_parts);
 }
 
 template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int NSM, int WPE = 1, bool DECAY = false>
@@ -345,8 +392,8 @@ __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(W
 ret_ragged_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
                    const half_t* __restrict__ mask, half_t* __restrict__ o, float* __restrict__ r, int H,
                    int seq_k, int seq_q, int causal, const float* __restrict__ lg2gamma = nullptr,
-                   const int* __restrict__ extents = nullptr) {
-  ret_fwd_walk<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM, WPE, 1, DECAY>(q, k, v, mask, o, r, H, seq_k, seq_q, causal, lg2gamma, extents);
+                   const int* __restrict__ extents = nullptr, BlockParts in_parts = {}) {
+  ret_fwd_walk<Kd, D, Br, Bc, Nthreads, NSK, NSV, NSM, WPE, 1, DECAY>(q, k, v, mask, o, r, H, seq_k, seq_q, causal, lg2gamma, extents, in_parts);
 }
 
 }  // namespace aat

@@ -105,7 +105,9 @@ int kernel_entry_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_h
  * log2_gamma [H] fp32 holds log2(gamma_h), 0.5 <= gamma_h <= 1.  Tiles above the diagonal are skipped.
  * No counterpart in the reference, which always streams the [H,Seq_q,Seq_k] tensor
  * (python/ops/retnet_interface.py:26-31) and lists "causal config" and the mask stream's cost as open
- * items (README.md:102-114). */
+ * items (README.md:102-114).  Given more workspace than workspace_size(), the longest blocks of a problem that leaves the chip
+ * partly idle are walked by several workgroups whose sums meet in it (csrc/kernels/utils/block_parts.h; how much more:
+ * decay_parts_bytes in autotuner/gfx950_space.py); given less, every block is walked in one piece. */
 float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
                     int B, int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes,
                     void* stream);
@@ -132,7 +134,7 @@ float profile_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half
 int kernel_entry_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_half* dO, float* r,
                     aat_half* dq, aat_half* dk, aat_half* dv, float* dqaccum, int B, int H, int Seq_q,
                     int Seq_k, int causal, void* workspace, size_t workspace_bytes, void* stream);
-/* Decay-mask variant of the backward (see the forward's profile_decay); no dqaccum argument. */
+/* Decay-mask variant of the backward (see the forward's profile_decay, also for the workspace); no dqaccum argument. */
 float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* dO, float* r,
                     aat_half* dq, aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k,
                     void* workspace, size_t workspace_bytes, void* stream);

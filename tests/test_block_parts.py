@@ -1,0 +1,70 @@
+"""Blocks of a causal walk in parts: the plan the libraries make and the room the runtime provides for it are the same arithmetic,
+and a plan's jobs are every part of every block once, longest first."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+from attention_autotuner_amd.arch import MI355X
+from attention_autotuner_amd.autotuner import codegen, gfx950_space
+
+SOURCE = r"""
+#include <hip/hip_runtime.h>
+#include "kernels/utils/block_parts.h"
+extern "C" int plan(long heads, int T, const int* walks, double tile_us, double places, int waves, size_t slot, int* split, int* parts, int* jobs) {
+  const auto walk = [=](int t) { return walks[t]; };
+  const aat::PartsPlan p = aat::plan_parts(heads, T, walk, aat::PartsCost{tile_us, places, waves, slot});
+  *split = p.split;
+  *parts = p.parts;
+  return aat::each_job(T, p, walk, [&](int n, int rank, int part) { jobs[n] = 8 * rank + (part < 0 ? 0 : part); });
+}
+extern "C" void walks(int rows, int T, int Br, int Bc, int Seq_q, int Seq_k, int* out) {
+  for (int t = 0; t < T; ++t) out[t] = rows ? aat::row_walk(t, Br, Bc, Seq_q, Seq_k) : aat::col_walk(t, Br, Bc, Seq_q, Seq_k);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    work = tmp_path_factory.mktemp("parts")
+    src, out = str(work / "plan.hip"), str(work / "plan.so")
+    with open(src, "w") as f:
+        f.write(SOURCE)
+    subprocess.run(codegen.hipcc_command(src, out, MI355X()), check=True, capture_output=True, cwd=str(work))
+    return ctypes.CDLL(out)
+
+
+def test_the_plan_and_its_room_agree_and_the_jobs_are_complete(lib):
+    rng = random.Random(5)
+    cut = 0
+    for _ in range(150):
+        br, bc, waves = rng.choice(((128, 64, 4), (64, 64, 2), (64, 32, 2), (128, 32, 4)))
+        sq, sk = 64 * rng.randint(1, 64), 64 * rng.randint(1, 64)
+        heads, rows, per_cu = rng.randint(1, 96), rng.randint(0, 1), rng.choice((1, 2, 4))
+        cols, width = rng.choice(((64, 128), (128, 256), (256, 512), (256, 768), (512, 768)))
+        want = gfx950_space._walks(bool(rows), br, bc, sq, sk)
+        T = len(want)
+        got = (ctypes.c_int * T)()
+        lib.walks(rows, T, br, bc, sq, sk, got)
+        assert list(got) == want, (rows, br, bc, sq, sk)
+        tile, slot = 2.0 * br * bc * width / 4.5e6, br * cols * 4
+        split, parts = gfx950_space.plan_parts(heads, want, tile, 256.0 * per_cu, waves, slot)
+        c_split, c_parts, jobs = ctypes.c_int(), ctypes.c_int(), (ctypes.c_int * (T * gfx950_space.MOST_PARTS))()
+        n = lib.plan(ctypes.c_long(heads), T, got, ctypes.c_double(tile), ctypes.c_double(256.0 * per_cu), waves, ctypes.c_size_t(slot),
+                     ctypes.byref(c_split), ctypes.byref(c_parts), jobs)
+        assert (c_split.value, c_parts.value) == (split, parts)
+        assert sorted(jobs[:n]) == sorted([8 * t + p for t in range(split) for p in range(parts)] + [8 * t for t in range(split, T)])
+        lengths = [want[j >> 3] / (parts if j >> 3 < split else 1) for j in jobs[:n]]
+        assert all(a >= b - 1e-9 for a, b in zip(lengths, lengths[1:]))
+        assert n <= gfx950_space.MOST_JOBS or split == 0
+        cut += split > 0
+    assert 20 <= cut <= 130
+
+
+def test_shares_cover_the_walk():
+    for n in range(0, 40):
+        for parts in (2, 3, 4):
+            cuts = [n * p // parts for p in range(parts + 1)]           # part_range
+            assert cuts[0] == 0 and cuts[-1] == n and all(b - a in (n // parts, n // parts + 1) for a, b in zip(cuts, cuts[1:]))

@@ -1,0 +1,46 @@
+"""RetNet with decay rates where the longest blocks are walked by several workgroups: lengths at which the library cuts, ragged and
+with either side the longer one, against the oracle's exact form under the rounded-operand rule of oracle/tolerance.py; the order in
+which the parts arrive must not show."""
+import pytest
+import torch
+
+import attention_autotuner_amd as aat
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from test_retnet_ragged_gpu import _check, _problem
+
+pytestmark = pytest.mark.gpu
+ARCH = aat.MI355X()
+SHAPES = [(1, 2, 1088, 1088), (1, 3, 1024, 1344), (2, 1, 1344, 1024)]
+
+
+def _configs(dqk, dv, problem):
+    b, h, sq, sk = problem
+    return (gfx950_space.rule_ret_config("ret", dqk, dv, b, h, sq, sk, True), gfx950_space.rule_ret_config("ret_bwd", dqk, dv, b, h, sq, sk, True))
+
+
+@pytest.mark.parametrize("dqk,dv", sorted(gfx950_space.RET_RULE))
+def test_blocks_in_parts_against_the_oracle(dqk, dv):
+    cut = 0
+    for i, problem in enumerate(SHAPES):
+        fwd, bwd = _configs(dqk, dv, problem)
+        cut += (gfx950_space.decay_parts_bytes(fwd, *problem) > 0) + (gfx950_space.decay_parts_bytes(bwd, *problem, stored_ds=bwd.ds_rows > 0) > 0)
+        _check(problem, dqk, dv, "decay", 900 + i, [fwd], [bwd])
+    assert cut >= 2 or dqk == 64, "nothing was cut"          # a walk of 17 tiles of 64 columns is not worth an exchange
+
+
+@pytest.mark.parametrize("dqk,dv", [(64, 64), (128, 128), (256, 512)])
+def test_parts_give_the_same_bits_every_time(dqk, dv):
+    problem = b, h, sq, sk = 1, 4, 2112, 2112
+    q, k, v, do, _, lg = (t.cuda() for t in _problem(1, 4, sq, sk, dqk, dv, "decay", 31))
+    fwd, bwd = (Runtime(ARCH, c) for c in _configs(dqk, dv, problem))
+    assert gfx950_space.decay_parts_bytes(bwd.config, *problem, stored_ds=bwd.config.ds_rows > 0) > 0
+    first = None
+    for _ in range(5):
+        o, r = torch.full_like(do, 7.0), torch.full((b, h, sq), 7.0, device="cuda")
+        grads = [torch.full_like(t, 7.0) for t in (q, k, v)]
+        fwd.apply([q, k, v, lg, o, r], decay=True)
+        bwd.apply([q, k, v, lg, do, r, *grads], decay=True)
+        torch.cuda.synchronize()
+        outs = [o, r, *grads]
+        first = first or outs
+        assert all(torch.equal(a, x) for a, x in zip(first, outs))
