@@ -2,9 +2,9 @@
 
 The reference has no such wrapper (its attention operator's ``backward`` is empty, reference
 python/ops/attention_interface.py:37-58); the layout follows its RetNet backward wrapper
-(csrc/kernels/retnet/bwd/profile_code.py:1-119).  One library launches three kernels: the preparation
-pass (delta = rowsum(dO * O), lse in base-2 units, both into the workspace), the column kernel (dV, dK)
-and the row kernel (dQ); with ``col_split`` the column kernel runs twice, once per output.
+(csrc/kernels/retnet/bwd/profile_code.py:1-119).  One library launches two kernels: the row kernel (dQ), which also
+leaves delta = rowsum(dO * O) and lse in base-2 units in the workspace, and the column kernel (dV, dK), which reads them;
+with ``col_split`` the column kernel runs twice, once per output.
 """
 
 global_vars = r"""
@@ -66,20 +66,18 @@ template <int GEN> hipError_t launch_kernels(aat_half* q, aat_half* k, aat_half*
   const int rows = B * H * Seq_q;
   float* lse2 = static_cast<float*>(workspace);
   float* delta = lse2 + rows;
-  constexpr int rows_per_block = aat::attn_bwd_prepare_rows_per_block<D>();
-  aat::attn_bwd_prepare<D><<<dim3((rows + rows_per_block - 1) / rows_per_block), dim3(256), 0, stream>>>(O, G, lse, lse2, delta, rows);
   const float c2 = softmax_scale * 1.4426950408889634f;
+  kernel_row<GEN><<<dim3(B * H * blocks_of(Seq_q)), dim3(Nthreads), TR::kSmemBytes, stream>>>(
+      Q, G, K, V, O, lse, lse2, delta, nullptr, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #if AAT_COL_SPLIT
   kernel_dv<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
-      K, V, Q, G, lse2, delta, reinterpret_cast<H16*>(dv), nullptr, H, Seq_k, Seq_q, c2, softmax_scale, causal);
+      K, V, Q, G, nullptr, nullptr, lse2, delta, reinterpret_cast<H16*>(dv), nullptr, H, Seq_k, Seq_q, c2, softmax_scale, causal);
   kernel_dk<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
-      K, V, Q, G, lse2, delta, nullptr, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
+      K, V, Q, G, nullptr, nullptr, lse2, delta, nullptr, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #else
   kernel_col<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
-      K, V, Q, G, lse2, delta, reinterpret_cast<H16*>(dv), reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
+      K, V, Q, G, nullptr, nullptr, lse2, delta, reinterpret_cast<H16*>(dv), reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #endif
-  kernel_row<GEN><<<dim3(B * H * blocks_of(Seq_q)), dim3(Nthreads), TR::kSmemBytes, stream>>>(
-      Q, G, K, V, lse2, delta, nullptr, reinterpret_cast<H16*>(dq), H, Seq_k, Seq_q, c2, softmax_scale, causal);
   return hipGetLastError();
 }}
 hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* dO, float* lse, aat_half* dq,
