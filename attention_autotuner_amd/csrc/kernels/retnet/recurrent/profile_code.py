@@ -54,22 +54,31 @@ hipError_t launch_one(const float* q, const float* k, const float* v, const char
   return hipGetLastError();
 }}
 
+void launch_factors(const float* decay, char* factors, int heads, int l, hipStream_t stream) {{
+  // one chunk per wave up to 256 chunks; more blocks per head would walk the same long chain of decays once more each
+  const int parts = std::min(16, (l / 32 + aat::kRecFactorWaves - 1) / aat::kRecFactorWaves);
+  aat::retnet_recurrent_factors<<<dim3(heads, parts), dim3(aat::kRecFactorThreads), (size_t)(l / 32) * 8, stream>>>(decay, factors, l);
+}}
+
 // Beyond 128 key dims the workspace has an output-sized buffer for the passes (at least 64 value dims: 8 KB per (batch, head,
 // chunk)), which holds P here.
 template <int KD, int WK>
-hipError_t launch_split(const float* q, const float* k, const float* v, const char* factors, char* room, float* out, int batch,
-                        int heads, int kdim, int vdim, int l, hipStream_t stream) {{
+hipError_t launch_split(const float* q, const float* k, const float* v, const float* decay, char* factors, char* room, float* out,
+                        int batch, int heads, int kdim, int vdim, int l, hipStream_t stream) {{
   using T = aat::RetRecurrentSplit<KD, WK>;
   constexpr bool kPre = KD > 128;
   const auto kernel = &aat::retnet_recurrent_split_kernel<KD, WK, kPre>;
   static const hipError_t ok = aat::allow_lds(kernel, T::kSmemBytes);
   if (ok != hipSuccess) return ok;
   if constexpr (kPre) {{
-    aat::retnet_recurrent_pmat<KD><<<dim3((unsigned)batch * heads * (l / 32)), dim3(256), 0, stream>>>(q, k, factors, room, heads,
-                                                                                               kdim, l);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    const int parts = std::min(32, (l / 32 + 3) / 4);                  // a chunk per wave up to 128 chunks
+    aat::retnet_recurrent_pmat<KD><<<dim3((unsigned)heads * parts + (unsigned)batch * heads * (l / 32)), dim3(256),
+                                     (size_t)(l / 32) * 8, stream>>>(q, k, decay, factors, room, heads, parts, kdim, l);
+  }} else {{
+    launch_factors(decay, factors, heads, l, stream);
   }}
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
   kernel<<<dim3((unsigned)batch * heads * (vdim / 32)), dim3(T::kThreads), T::kSmemBytes, stream>>>(q, k, v, factors, room, out,
                                                                                              heads, kdim, vdim, l);
   return hipGetLastError();
@@ -93,27 +102,25 @@ bool split_pays(long bh, int vdim, int block_kdim, bool wide) {{
   return split < passes + add;
 }}
 
-// Two launches: the decay factors of every (head, chunk), then the scan.  A value slice of 128 dims per
+// Two launches: the decay factors of every (head, chunk), beyond 128 key dims in the launch that makes P, then the scan.  A value slice of 128 dims per
 // block halves the traffic of q and k; where it would leave most of the compute units without a block or vdim does not
 // allow it, 64 key dims take slices of 64 and more of them the split kernel, which split_pays() may choose elsewhere too.
 hipError_t launch(const float* q, const float* k, const float* v, const float* decay, float* out, int batch, int heads,
                   int kdim, int vdim, int l, int block_kdim, char* workspace, hipStream_t stream) {{
   char* factors = workspace;
   float* part = reinterpret_cast<float*>(workspace + (factor_bytes(heads, l) + 255) / 256 * 256);
-  // one chunk per wave up to 256 chunks; more blocks per head would walk the same long chain of decays once more each
-  const int parts = std::min(16, (l / 32 + aat::kRecFactorWaves - 1) / aat::kRecFactorWaves);
-  aat::retnet_recurrent_factors<<<dim3(heads, parts), dim3(aat::kRecFactorThreads), (size_t)(l / 32) * 8, stream>>>(decay, factors, l);
-  hipError_t e = hipGetLastError();
   char* const room = reinterpret_cast<char*>(part);
   const bool wide = vdim % 128 == 0 && (long)batch * heads * (vdim / 128) >= 192;
-  if (e == hipSuccess && split_pays((long)batch * heads, vdim, block_kdim, wide)) {{
+  if (split_pays((long)batch * heads, vdim, block_kdim, wide)) {{
     switch (block_kdim) {{
-      case 64: return launch_split<64, 2>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
-      case 128: return launch_split<128, 4>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
-      case 192: return launch_split<192, 3>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
-      default: return launch_split<256, 4>(q, k, v, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 64: return launch_split<64, 2>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 128: return launch_split<128, 4>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 192: return launch_split<192, 3>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      default: return launch_split<256, 4>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
     }}
   }}
+  launch_factors(decay, factors, heads, l, stream);
+  hipError_t e = hipGetLastError();
   for (int kd0 = 0; kd0 < block_kdim && e == hipSuccess; ) {{
     const int kd = block_kdim - kd0 >= 128 ? 128 : 64;                 // key dims of this pass
     const float* qp = q + (size_t)kd0 * l;                             // rows kd0.. of every (batch, head) slice

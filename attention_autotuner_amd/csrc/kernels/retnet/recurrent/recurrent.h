@@ -89,24 +89,22 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
 constexpr int kRecFactorBytes = 5120;
 constexpr int kRecFactorW = 4096, kRecFactorPnl = 4224, kRecFactorFlag = 4352;
 
-// decay [H][L] -> factors [H][L/32][kRecFactorBytes].  Grid (H, parts of the sequence), kRecFactorThreads threads, 8 bytes of
-// dynamic LDS per chunk.  A head's chunks are shared out over the blocks of its row and the waves of a block.  Each block
+// decay [H][L] -> factors [H][L/32][kRecFactorBytes], for part `part` of `parts` of head `head`'s sequence, by a block of
+// WAVES waves with 8 bytes of dynamic LDS per chunk.  WITH_D: the D of the records too.  A head's chunks are shared out over the blocks of its row and the waves of a block.  Each block
 // walks lambda from the first chunk to its own last one by itself (a product per thread and chunk, then one wave chains
 // them); lambda is known before a record is written, so a record is written once.
 //
 // Bound by latency: a load, the walk (one dependent multiplication and comparison per chunk), a load and 32 products, a store.
-constexpr int kRecFactorThreads = 1024;
-constexpr int kRecFactorWaves = kRecFactorThreads / 64;
-__global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(const float* __restrict__ decay,
-                                                                              char* __restrict__ factors, int L) {
+template <int WAVES, bool WITH_D>
+AAT_DEV void rec_factor_records(const float* __restrict__ decay, char* __restrict__ factors, int L, int head, int part, int parts) {
   extern __shared__ __align__(16) float fsm[];     // per chunk: A, then lambda before the chunk; and A lambda
   const int lane = threadIdx.x & 63, n = lane & 31, hi = lane >> 5, nchunk = L / 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int per_block = (nchunk + gridDim.y - 1) / gridDim.y;
-  const int first = blockIdx.y * per_block, last = min(nchunk, first + per_block);
+  const int per_block = (nchunk + parts - 1) / parts;
+  const int first = part * per_block, last = min(nchunk, first + per_block);
   if (first >= last) return;
-  const float* const dh = decay + (size_t)blockIdx.x * L;
-  for (int c = threadIdx.x; c < last; c += kRecFactorThreads) {
+  const float* const dh = decay + (size_t)head * L;
+  for (int c = threadIdx.x; c < last; c += WAVES * 64) {
     typedef f4v f4v_dword __attribute__((aligned(4)));                    // decay may start at any float
     const f4v_dword* p = reinterpret_cast<const f4v_dword*>(dh + (size_t)c * 32);
     f4v x[8];
@@ -138,9 +136,9 @@ __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(co
     }
   }
   __syncthreads();
-  for (int c = first + wave; c < last; c += kRecFactorWaves) {
+  for (int c = first + wave; c < last; c += WAVES) {
     const float* dg = dh + (size_t)c * 32;
-    char* rec = factors + ((size_t)blockIdx.x * nchunk + c) * kRecFactorBytes;
+    char* rec = factors + ((size_t)head * nchunk + c) * kRecFactorBytes;
     const float lam = fsm[2 * c], lam_new = fsm[2 * c + 1], mag = __builtin_fabsf(lam_new);
     const bool rescale = !(mag >= 0x1p-40f && mag <= 0x1p40f);
     const float inv = rescale ? 1.f : 1.f / lam_new;
@@ -157,7 +155,7 @@ __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(co
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       f4v x = {dsel[4 * g], dsel[4 * g + 1], dsel[4 * g + 2], dsel[4 * g + 3]};
-      *reinterpret_cast<f4v*>(rec + g * 1024 + lane * 16) = x;
+      if constexpr (WITH_D) *reinterpret_cast<f4v*>(rec + g * 1024 + lane * 16) = x;
       if (n == 0) {
         f4v y = {wsel[4 * g] * inv, wsel[4 * g + 1] * inv, wsel[4 * g + 2] * inv, wsel[4 * g + 3] * inv};
         *reinterpret_cast<f4v*>(rec + kRecFactorW + hi * 64 + g * 16) = y;
@@ -169,6 +167,14 @@ __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(co
       *reinterpret_cast<float*>(rec + kRecFactorFlag + 4) = lam_new;
     }
   }
+}
+
+// Grid (H, parts of the sequence).
+constexpr int kRecFactorThreads = 1024;
+constexpr int kRecFactorWaves = kRecFactorThreads / 64;
+__global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(const float* __restrict__ decay,
+                                                                              char* __restrict__ factors, int L) {
+  rec_factor_records<kRecFactorWaves, true>(decay, factors, L, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
 template <int KD, int DVS>
@@ -511,14 +517,24 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
 // P of every (batch, head, chunk) for the kernel below, as C registers: [B*H][L/32][g][lane][e], 4 KB per chunk.  One block
 // per chunk; its waves split the key dims, read q and k straight from memory (rows of 128 bytes, each used once) and wave w adds
 // up row group w and multiplies it by D.  Bound by the read of q and k.
+//
+// The first heads * parts blocks of the launch make the records of the decay factors instead, 8 bytes of dynamic LDS per chunk
+// (the kernel below waits for both anyway): D, which P needs, depends on its own chunk only, and every wave forms its 8 rows
+// while its loads are under way, in the order of the records.  B2 H8 L1056 256/512: 94.4 us a call with a
+// launch of its own for the records (5.6 us and the gap behind it), 88.6 like this.
 template <int KD>
 __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __restrict__ q, const float* __restrict__ k,
-                                                             const char* __restrict__ factors, char* __restrict__ pmat,
-                                                             int heads, int kdim, int L) {
+                                                             const float* __restrict__ decay, char* __restrict__ factors,
+                                                             char* __restrict__ pmat, int heads, int parts, int kdim, int L) {
   __shared__ __align__(16) f4v part[4][4][64];
+  const int records = heads * parts;
+  if ((int)blockIdx.x < records) {
+    rec_factor_records<4, false>(decay, factors, L, blockIdx.x / parts, blockIdx.x % parts, parts);
+    return;
+  }
   const int lane = threadIdx.x & 63, n = lane & 31, hi = lane >> 5, nchunk = L / 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tile = xcd_remap(blockIdx.x, gridDim.x), bh = tile / nchunk, c = tile % nchunk;
+  const int tile = xcd_remap(blockIdx.x - records, gridDim.x - records), bh = tile / nchunk, c = tile % nchunk;
   constexpr int kRows = KD / 4;                       // key dims of one wave
   const size_t at = ((size_t)bh * kdim + wave * kRows + hi) * L + (size_t)c * 32 + n;
   const float *qp = q + at, *kp = k + at;
@@ -529,6 +545,22 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
     qx[i] = qp[(size_t)2 * i * L];
   }
   sched_fence();                                      // all loads in flight before the first product
+  const float* const dg = decay + (size_t)(bh % heads) * L + (size_t)c * 32;
+  f4v dsel = {0.f, 0.f, 0.f, 0.f};                    // D of rows 8 wave + 4 hi + e
+  float d = 0.f;
+#pragma unroll
+  for (int g = 3; g >= 0; --g) {
+    f4v rows[2];
+#pragma unroll
+    for (int i = 7; i >= 0; --i) {
+      const int m = 8 * g + i;
+      if (m < 31) d *= dg[m + 1];
+      d = (m == n) ? 1.f : d;
+      rows[i >> 2][i & 3] = d;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dsel[e] = g == wave ? (hi ? rows[1][e] : rows[0][e]) : dsel[e];
+  }
   f16v sp = zero16();
 #pragma unroll
   for (int i = 0; i < kRows / 2; ++i) sp = mfma_32x32x2_f32(kx[i], qx[i], sp);
@@ -538,7 +570,7 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
   f4v x = part[0][wave][lane];
 #pragma unroll
   for (int t = 1; t < 4; ++t) x += part[t][wave][lane];
-  x *= *reinterpret_cast<const f4v*>(factors + ((size_t)(bh % heads) * nchunk + c) * kRecFactorBytes + wave * 1024 + lane * 16);
+  x *= dsel;
   *reinterpret_cast<f4v*>(pmat + ((size_t)bh * nchunk + c) * 4096 + wave * 1024 + lane * 16) = x;
 }
 

@@ -220,6 +220,20 @@ def test_decay_factors_over_blocks(seqlen):
         _close(out[:, head], ref[:, head])
 
 
+# beyond 128 key dims the launch that makes P makes the records too, in blocks of four waves: a single part, a second one with a
+# single chunk, several chunks per wave in as many parts as a launch has and a short last part
+@pytest.mark.parametrize("kdim,seqlen", [(192, 4 * 32), (256, 5 * 32), (256, 131 * 32), (192, 259 * 32)])
+def test_decay_factors_beside_the_products_of_q_and_k(kdim, seqlen):
+    q, k, v, decay = _inputs(13, 2, 2, kdim, 64, seqlen, 0.8, 1.0)
+    decay[1, ::97] = -1.5
+    decay[1, seqlen - 40] = 0.0
+    shifted = torch.zeros(2 * seqlen + 1, device="cuda")[1:].view(2, seqlen).copy_(decay)
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), shifted)
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(2):
+        _close(out[:, head], ref[:, head])
+
+
 def test_graph_capture_replays():
     """The extended entry point allocates nothing and launches two kernels: a captured graph of it replays
     correctly with eager work and synchronisations in between, and follows new inputs written in place."""
