@@ -79,6 +79,39 @@ struct RetBwdChain {
   static constexpr int kSmemBytesDsOut = (kMainBytes + kDsStageBytes > kEpiBytes) ? kMainBytes + kDsStageBytes : kEpiBytes;
 };
 
+// The end of a block: the wave's output tile through its staging rows to memory.  A function and no lambda: a closure over the
+// whole kernel left the forms that are never walked in parts with 20 and 24 bytes of scratch a lane where they have none (the
+// row passes of ret_bwd at 256/256 in blocks of 256 rows, dense mask, GEN).
+template <class T, int DZ, int DZB, bool NUMBERED>
+AAT_DEV void store_chain_tile(const f16v (&acc)[T::RT][T::DT], char* ostage, half_t* og, int lane, int groups) {
+  constexpr int DT = T::DT, kChunksPerRow = DZB / 8;    // the staging rows are DZB wide; the global rows are DZ wide
+  const int n = lane & 31, h = lane >> 5;
+  static_for<T::RT * DT>([&](auto i_tag) {
+    constexpr int rt = decltype(i_tag)::value / DT, dt = decltype(i_tag)::value % DT;
+    f16v blk;
+    if constexpr (NUMBERED) blk = acc_read16<16 * (rt * DT + dt)>();
+    else blk = acc[rt][dt];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const h2 a = pack_rne(blk[4 * g], blk[4 * g + 1]);
+      const h2 b = pack_rne(blk[4 * g + 2], blk[4 * g + 3]);
+      h4 w;
+      w[0] = a[0]; w[1] = a[1]; w[2] = b[0]; w[3] = b[1];
+      *reinterpret_cast<h4*>(ostage + (rt * 32 + n) * T::kOStride + (32 * dt + 8 * g + 4 * h) * 2) = w;
+    }
+  });
+  wait_lgkm0();
+  constexpr int kChunks = T::WM * kChunksPerRow;
+#pragma unroll
+  for (int t = 0; t < kChunks / 64; ++t) {
+    if (t * 64 / (32 * kChunksPerRow) >= groups) break;
+    const int idx = t * 64 + lane;
+    const int row = idx / kChunksPerRow, c = idx % kChunksPerRow;
+    const u4v val = *reinterpret_cast<const u4v*>(ostage + row * T::kOStride + c * 16);
+    *reinterpret_cast<u4v*>(reinterpret_cast<char*>(og) + (size_t)row * DZ * 2 + c * 16) = val;
+  }
+}
+
 // x, y, z, out: [B*H, S, width] fp16 with S = seq_x for x/out and seq_y for y/z; mask [H, seq_q, seq_k];
 // r [B*H, seq_q].  For COL passes seq_x = seq_k, seq_y = seq_q; for the ROW pass the other way round.
 // `causal` promises mask == 0 above the diagonal and only shortens the walk over streamed tiles.
@@ -506,46 +539,19 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
   if constexpr (kNumbered) acc_settle();
   wait_vmcnt<0>();
   block_sync();
-  const auto finish = [&]() {                     // the staging rows are DZB wide; the global rows are DZ wide
-    char* const ostage = smem + wave * WM * T::kOStride;
-    half_t* og = out + ((size_t)bh * seq_x + x0 + wave * WM) * DZ + dz0;
-    constexpr int kChunksPerRow = DZB / 8;
-    static_for<RT * DT>([&](auto i_tag) {
-      constexpr int rt = decltype(i_tag)::value / DT, dt = decltype(i_tag)::value % DT;
-      f16v blk;
-      if constexpr (kNumbered) blk = acc_read16<16 * (rt * DT + dt)>();
-      else blk = acc[rt][dt];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const h2 a = pack_rne(blk[4 * g], blk[4 * g + 1]);
-        const h2 b = pack_rne(blk[4 * g + 2], blk[4 * g + 3]);
-        h4 w;
-        w[0] = a[0]; w[1] = a[1]; w[2] = b[0]; w[3] = b[1];
-        *reinterpret_cast<h4*>(ostage + (rt * 32 + n) * T::kOStride + (32 * dt + 8 * g + 4 * h) * 2) = w;
-      }
-    });
-    wait_lgkm0();
-    constexpr int kChunks = WM * kChunksPerRow;
-#pragma unroll
-    for (int t = 0; t < kChunks / 64; ++t) {
-      if (t * 64 / (32 * kChunksPerRow) >= groups) break;
-      const int idx = t * 64 + lane;
-      const int row = idx / kChunksPerRow, c = idx % kChunksPerRow;
-      const u4v val = *reinterpret_cast<const u4v*>(ostage + row * T::kOStride + c * 16);
-      *reinterpret_cast<u4v*>(reinterpret_cast<char*>(og) + (size_t)row * DZ * 2 + c * 16) = val;
-    }
-  };
+  char* const ostage = smem + wave * WM * T::kOStride;
+  half_t* const og = out + ((size_t)bh * seq_x + x0 + wave * WM) * DZ + dz0;
   if constexpr (kParts) {
     if (id.parts > 1) {                           // to the end in here: joined again, the two paths' accumulators cost scratch
       float none[1];
       bool last;
       if constexpr (kNumbered) last = combine_parts_numbered<64, 0, Nthreads>(in_parts, id, none, smem);
       else last = combine_parts<0, Nthreads, 4>(in_parts, id, acc, none, smem);
-      if (last) finish();
+      if (last) store_chain_tile<T, DZ, DZB, kNumbered>(acc, ostage, og, lane, groups);
       return;
     }
   }
-  finish();
+  store_chain_tile<T, DZ, DZB, kNumbered>(acc, ostage, og, lane, groups);
 }
 
 }  // namespace aat

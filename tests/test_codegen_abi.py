@@ -318,6 +318,16 @@ def test_whole_blocks_carry_no_selects_for_partial_ones():
     assert sgprs["dv", False] <= 70 < sgprs["dv", True] and sgprs["dq", False] <= 74 < sgprs["dq", True], sgprs
 
 
+def test_forms_that_are_never_walked_in_parts_pay_no_scratch_for_the_others():
+    """The row passes of the 256-row backward at 256/256 at ragged lengths, with a mask tensor: 246 vector registers, no scratch."""
+    cfg = [c for c in gfx950_space.rule_ret_configs("ret_bwd", 256, 256) if c.Br == 256]
+    assert len(cfg) == 1
+    report = codegen.resource_usage(codegen.compile_config(cfg[0], ARCH, timeout=600))
+    # <KX, DZ, DZB, BX, BY, threads, NSY, NSZ, pass (1: row), waves per SIMD, GEN, DECAY, DS_OUT>
+    picked = [k for k in report if re.search(r"13ret_bwd_chain.*BwdPassE1ELi1ELi1ELb0ELb[01]EEEv", k["kernel"])]
+    assert [k["scratch_bytes"] for k in picked] == [0, 0]
+
+
 def test_tune_skips_a_candidate_the_compiler_reports_as_spilling(tmp_path, monkeypatch):
     """The loop never times (here: never even loads) a library whose report shows a spilled working set."""
     from attention_autotuner_amd.benchmarks.tune import make_tensors
