@@ -25,7 +25,8 @@ _ERRORS = {-2: "sequence lengths are not multiples of what the library takes: 32
 # A RetNet backward built with a stored dS asks for B*H*S_q*S_kv fp16 on top of the mask scan and works without them
 # (it then evaluates dS twice).  Beyond this many bytes the runtime does not grant the room on its own: a caller who
 # wants it there passes a workspace of workspace_size() bytes.  The same limit holds for the slots of a decay walk whose longest
-# blocks are walked in parts, which a call without the room walks in one piece.
+# blocks are walked in parts, which a call without the room walks in one piece: also where a caller's workspace has the
+# bytes of workspace_size() and no more, which is used as it is.
 MAX_DS_BYTES = int(os.environ.get("AAT_MAX_DS_BYTES", 2 << 30))
 
 
@@ -95,11 +96,13 @@ class Runtime:
         lib = self._lib
         if lib is None:
             lib = self._lib = library.load(self._path(), op)
-        need = self._need.get((B, H, Sq, Sk, decay))        # a property of the library and the problem: asked once
-        if need is None:
-            need = self._need[(B, H, Sq, Sk, decay)] = _wanted(self.config, int(lib.workspace_size(B, H, Sq, Sk)), B, H, Sq, Sk, decay)
-        if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-            workspace = _grown(workspace, need, q.device, keep=causal == "scanned")
+        needs = self._need.get((B, H, Sq, Sk, decay))       # a property of the library and the problem: asked once
+        if needs is None:
+            size = int(lib.workspace_size(B, H, Sq, Sk))
+            # what a caller's workspace has to hold to be used as it is, what is provided otherwise
+            needs = self._need[(B, H, Sq, Sk, decay)] = (_wanted(self.config, size, B, H, Sq, Sk), _wanted(self.config, size, B, H, Sq, Sk, decay))
+        if needs[1] and (workspace is None or workspace.numel() * workspace.element_size() < needs[0]):
+            workspace = _grown(workspace, needs[1], q.device, keep=causal == "scanned")
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
         if op in library.SCALED_OPS:

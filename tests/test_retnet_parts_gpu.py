@@ -6,6 +6,7 @@ import torch
 
 import attention_autotuner_amd as aat
 from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from oracle import ref_op, tolerance
 from test_retnet_ragged_gpu import _check, _problem
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +45,40 @@ def test_parts_give_the_same_bits_every_time(dqk, dv):
         outs = [o, r, *grads]
         first = first or outs
         assert all(torch.equal(a, x) for a, x in zip(first, outs))
+
+
+@pytest.mark.parametrize("op", ["ret", "ret_bwd"])
+def test_a_workspace_of_workspace_size_bytes_is_used_as_it_is(op):
+    """... with nothing allocated beside it, every block walked in one piece, and the bytes behind it left alone; results against
+    the oracle's.  One that is larger by the room for the parts is used too."""
+    problem = b, h, sq, sk = 1, 2, 1088, 1088
+    dqk, dv = 256, 512
+    q, k, v, do, mask, lg = _problem(b, h, sq, sk, dqk, dv, "decay", 37)
+    rt = Runtime(ARCH, _configs(dqk, dv, problem)[op == "ret_bwd"])
+    size, guard = rt.workspace_size(*problem), 1 << 26
+    qc, kc, vc, dc = (t.cuda() for t in (q, k, v, do))
+    o_want, r_want = ref_op.retnet_ref(q, k, v, mask, return_r=True)
+    r_want = r_want.reshape(b, h, sq)
+    if op == "ret":
+        s = (q.float() @ k.float().transpose(-1, -2)) * mask.float()
+        want, terms = [o_want], [(s.abs() / s.abs().sum(-1, keepdim=True).clamp(min=1.0)) @ v.float().abs()]
+        out, r = [torch.full_like(dc, 7.0)], torch.full((b, h, sq), 7.0, device="cuda")
+        arrays = [qc, kc, vc, lg.cuda(), out[0], r]
+    else:
+        want, terms = ref_op.retnet_bwd_ref(q, k, v, mask, do), ref_op.retnet_bwd_rounding_bound(q, k, v, mask, do)
+        out = [torch.full_like(t, 7.0) for t in (qc, kc, vc)]
+        arrays = [qc, kc, vc, lg.cuda(), dc, r_want.cuda(), *out]
+    room = torch.full((size + guard,), 0x5a, dtype=torch.uint8, device="cuda")
+    rt.apply(arrays, decay=True, workspace=room[:size])                    # the library is loaded
+    for workspace in (room[:size], room):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        rt.apply(arrays, decay=True, workspace=workspace)
+        torch.cuda.synchronize()
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+        untouched = bool((room[size:] == 0x5a).all())
+        assert untouched == (workspace is not room)                       # the parts' counts, order and slots lie there
+        for got, ref, t in zip(out, want, terms):
+            ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
+            assert ok, (worst, ratio)
+            got.fill_(7.0)
