@@ -62,22 +62,17 @@ using PK = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, false>;
 using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkRows * 2, 0, false, 270>;    // it streams dS and multiplies little
 struct BwdPlan {{
   aat::PartsPlan dv, dq, dk;
-  aat::JobOrders<3> orders;
   size_t counts, slots;
 }};
 BwdPlan plan_of(int B, int H, int Seq_q, int Seq_k, bool stored) {{
   const long heads = (long)B * H;
-  BwdPlan p{{}};
-  const auto take = [](const auto& found, aat::PartsPlan& plan, aat::JobOrder& order) {{
-    plan = found.plan;
-    if (plan.split) order = found.order;
-  }};
   constexpr int waves = Nthreads / 64;
   const int row_lds = stored ? TQ::kSmemBytesDsOut : TQ::kSmemBytes;
-  if (D == DVB) take(PV::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TV::kSmemBytes)), p.dv, p.orders.of[0]);
-  take(PQ::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, row_lds)), p.dq, p.orders.of[1]);
-  if (stored) take(PKD::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(kDkRows / 32, kDkWaves, TKD::kSmemBytes)), p.dk, p.orders.of[2]);
-  else take(PK::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TK::kSmemBytes)), p.dk, p.orders.of[2]);
+  BwdPlan p{{}};
+  if (D == DVB) p.dv = PV::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TV::kSmemBytes));
+  p.dq = PQ::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, row_lds));
+  p.dk = stored ? PKD::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(kDkRows / 32, kDkWaves, TKD::kSmemBytes))
+                : PK::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TK::kSmemBytes));
   const size_t dk = stored ? PKD::slot_bytes(heads, p.dk) : PK::slot_bytes(heads, p.dk);
   const size_t dv = PV::slot_bytes(heads, p.dv), dq = PQ::slot_bytes(heads, p.dq);
   p.slots = dv > dq ? (dv > dk ? dv : dk) : (dq > dk ? dq : dk);
@@ -135,16 +130,21 @@ template <bool DECAY> hipError_t launch_passes(aat_half* q, aat_half* k, aat_hal
   const bool stored = room_for_ds(workspace, workspace_bytes, B, H, Seq_q, Seq_k);
   aat::BlockParts dv_parts, dq_parts, dk_parts;
   if constexpr (DECAY) {{
-    const BwdPlan plan = plan_of(B, H, Seq_q, Seq_k, stored);
     const size_t at = stored ? ws_bytes_needed(B, H, Seq_q, Seq_k) : ds_offset(H, Seq_q, Seq_k);
-    if (plan.slots > 0 && workspace != nullptr && workspace_bytes >= at + plan.counts + 3 * aat::kOrderBytes + plan.slots) {{
+    BwdPlan plan{{}};
+    if (workspace != nullptr && workspace_bytes > at + 3 * aat::kOrderBytes) plan = plan_of(B, H, Seq_q, Seq_k, stored);   // else no room for any parts
+    if (plan.slots > 0 && workspace_bytes >= at + plan.counts + 3 * aat::kOrderBytes + plan.slots) {{
       char* const room = static_cast<char*>(workspace) + at;
       uint16_t* const order = reinterpret_cast<uint16_t*>(room + plan.counts);
       float* const slots = reinterpret_cast<float*>(room + plan.counts + 3 * aat::kOrderBytes);
       const int n = (int)(plan.counts / sizeof(uint32_t));
+      aat::JobOrders<3> orders{{}};
+      PV::put_order(plan.dv, Seq_q, Seq_k, orders.of[0]);
+      PQ::put_order(plan.dq, Seq_q, Seq_k, orders.of[1]);
+      if (stored) PKD::put_order(plan.dk, Seq_q, Seq_k, orders.of[2]);
+      else PK::put_order(plan.dk, Seq_q, Seq_k, orders.of[2]);
       aat::prepare_parts<3><<<dim3((n + aat::kMostJobs - 1) / aat::kMostJobs), dim3(aat::kMostJobs), 0, stream>>>(
-          reinterpret_cast<uint32_t*>(room), n,
-          plan.orders, order);
+          reinterpret_cast<uint32_t*>(room), n, orders, order);
       size_t counted = 0;
       const auto take = [&](const aat::PartsPlan& p, int launch) {{
         const aat::BlockParts b{{p.split, p.parts, slots, reinterpret_cast<uint32_t*>(room + counted), order + launch * aat::kMostJobs}};

@@ -55,18 +55,22 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
                         int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes, hipStream_t stream) {{
   static const hipError_t lds_ok = allow_kernels<true>();
   if (lds_ok != hipSuccess) return lds_ok;
-  const auto& found = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
-  const aat::PartsPlan& plan = found.plan;
-  const size_t at = workspace_size(B, H, Seq_q, Seq_k), counts = aat::count_bytes((long)B * H, plan);
+  const size_t at = workspace_size(B, H, Seq_q, Seq_k);
   aat::BlockParts in_parts;
-  if (plan.split > 0 && workspace != nullptr && workspace_bytes >= at + counts + aat::kOrderBytes + Parts::slot_bytes((long)B * H, plan)) {{
-    char* const room = static_cast<char*>(workspace) + at;
-    uint32_t* const arrived = reinterpret_cast<uint32_t*>(room);
-    uint16_t* const order = reinterpret_cast<uint16_t*>(room + counts);
-    const int n = B * H * plan.split;
-    aat::prepare_parts<1><<<dim3((n + aat::kMostJobs - 1) / aat::kMostJobs), dim3(aat::kMostJobs), 0, stream>>>(
-        arrived, n, {{found.order}}, order);
-    in_parts = {{plan.split, plan.parts, reinterpret_cast<float*>(room + counts + aat::kOrderBytes), arrived, order}};
+  if (workspace != nullptr && workspace_bytes > at + aat::kOrderBytes) {{               // else there is no room for any parts
+    const aat::PartsPlan plan = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
+    const size_t counts = aat::count_bytes((long)B * H, plan);
+    if (plan.split > 0 && workspace_bytes >= at + counts + aat::kOrderBytes + Parts::slot_bytes((long)B * H, plan)) {{
+      char* const room = static_cast<char*>(workspace) + at;
+      uint32_t* const arrived = reinterpret_cast<uint32_t*>(room);
+      uint16_t* const order = reinterpret_cast<uint16_t*>(room + counts);
+      const int n = B * H * plan.split;
+      aat::JobOrders<1> orders{{}};
+      Parts::put_order(plan, Seq_q, Seq_k, orders.of[0]);
+      aat::prepare_parts<1><<<dim3((n + aat::kMostJobs - 1) / aat::kMostJobs), dim3(aat::kMostJobs), 0, stream>>>(
+          arrived, n, orders, order);
+      in_parts = {{plan.split, plan.parts, reinterpret_cast<float*>(room + counts + aat::kOrderBytes), arrived, order}};
+    }}
   }}
   const int jobs = row_blocks(Seq_q) + in_parts.split * (in_parts.parts - 1);
   (Seq_q % Br == 0 ? kernel<true> : kernel_ragged<true>)<<<dim3(B * H * jobs), dim3(Nthreads), shared_mem, stream>>>(

@@ -10,6 +10,8 @@
 // RetNet with decay rates: B2 H8 S2112 256/512 (272 blocks of 128 rows, one to a compute unit) forward 99 -> 88 us, forward and
 // backward 365 -> 319; B1 H8 S2048 256/512 104 -> 68 and 327 -> 220; B1 H4 S4096 128/128 81 -> 47 and 313 -> 206.
 #pragma once
+#include <mutex>
+
 #include "acc_file.h"
 #include "cdna4.h"
 
@@ -304,26 +306,55 @@ template <class Length> inline PartsPlan plan_parts(long heads, int T, Length&& 
   return best;
 }
 
-// One kind of launch of a library (FIT: its kernel can): its plan and the order of its jobs, found once per problem and thread.  MEMORY: by how much
-// the launch's tiles are slower than their matrix work (percent).
-template <bool FIT, int Br, int Bc, int Width, int Cols, int Nthreads, int Extra, bool ROWS, int MEMORY = 100>
-struct PartsLaunch {
-  static constexpr size_t kSlotBytes = part_floats<Br * Cols / (4 * Nthreads), Extra, Nthreads>() * sizeof(float);
-  struct Found {
+// The plans of the problems that a kind of launch met last, for all threads: 256 of them in sets of four, 10 KB.  A search takes
+// 1.6 us of the call at 512 rows, 9 at 1024, 21 at 2048, 50 at 4096 (forward), so a loop over a few dozen lengths must not
+// search for one of them twice.
+class PlanMemory {
+  struct Entry {
     long heads = 0;
     int Seq_q = 0, Seq_k = 0, blocks_per_cu = 0;
     PartsPlan plan;
-    JobOrder order;
   };
-  static const Found& find(long heads, int Seq_q, int Seq_k, int blocks_per_cu) {
-    static thread_local Found f;
-    if (f.heads == heads && f.Seq_q == Seq_q && f.Seq_k == Seq_k && f.blocks_per_cu == blocks_per_cu) return f;
-    const int T = ((ROWS ? Seq_q : Seq_k) + Br - 1) / Br;
-    const auto walk = [=](int rank) { return ROWS ? row_walk(rank, Br, Bc, Seq_q, Seq_k) : col_walk(rank, Br, Bc, Seq_q, Seq_k); };
-    const PartsCost cost{MEMORY / 100.0 * 2.0 * Br * Bc * Width / 4.5e6, 256.0 * blocks_per_cu, Nthreads / 64, kSlotBytes};
-    f = Found{heads, Seq_q, Seq_k, blocks_per_cu, FIT ? plan_parts(heads, T, walk, cost) : PartsPlan{}, JobOrder{}};
-    if (f.plan.split) each_job(T, f.plan, walk, [&](int n, int rank, int part) { f.order.job[n] = (uint16_t)(8 * rank + (part < 0 ? 0 : part)); });
-    return f;
+  static constexpr int kSets = 64, kWays = 4;
+  Entry entry_[kSets][kWays];
+  unsigned next_[kSets] = {};
+  std::mutex guard_;
+
+ public:
+  template <class Search> PartsPlan get(long heads, int Seq_q, int Seq_k, int blocks_per_cu, Search&& search) {
+    const unsigned long mixed = (((unsigned long)heads * 0x9e3779b97f4a7c15ul + Seq_q) * 0x9e3779b97f4a7c15ul + Seq_k) * 0x9e3779b97f4a7c15ul;
+    const int set = (int)(mixed >> 58);
+    {
+      std::lock_guard<std::mutex> lock(guard_);
+      for (const Entry& e : entry_[set])
+        if (e.heads == heads && e.Seq_q == Seq_q && e.Seq_k == Seq_k && e.blocks_per_cu == blocks_per_cu) return e.plan;
+    }
+    const PartsPlan plan = search();
+    std::lock_guard<std::mutex> lock(guard_);
+    entry_[set][next_[set]++ % kWays] = {heads, Seq_q, Seq_k, blocks_per_cu, plan};
+    return plan;
+  }
+};
+
+// One kind of launch of a library (FIT: its kernel can): its plan, found once per problem, and the order of the plan's jobs.  MEMORY:
+// by how much the launch's tiles are slower than their matrix work (percent).
+template <bool FIT, int Br, int Bc, int Width, int Cols, int Nthreads, int Extra, bool ROWS, int MEMORY = 100>
+struct PartsLaunch {
+  static constexpr size_t kSlotBytes = part_floats<Br * Cols / (4 * Nthreads), Extra, Nthreads>() * sizeof(float);
+  static int blocks(int Seq_q, int Seq_k) { return ((ROWS ? Seq_q : Seq_k) + Br - 1) / Br; }
+  static auto walk(int Seq_q, int Seq_k) {
+    return [=](int rank) { return ROWS ? row_walk(rank, Br, Bc, Seq_q, Seq_k) : col_walk(rank, Br, Bc, Seq_q, Seq_k); };
+  }
+  static PartsPlan find(long heads, int Seq_q, int Seq_k, int blocks_per_cu) {
+    if (!FIT) return {};
+    static PlanMemory known;
+    return known.get(heads, Seq_q, Seq_k, blocks_per_cu, [=] {
+      const PartsCost cost{MEMORY / 100.0 * 2.0 * Br * Bc * Width / 4.5e6, 256.0 * blocks_per_cu, Nthreads / 64, kSlotBytes};
+      return plan_parts(heads, blocks(Seq_q, Seq_k), walk(Seq_q, Seq_k), cost);
+    });
+  }
+  static void put_order(const PartsPlan& p, int Seq_q, int Seq_k, JobOrder& order) {
+    if (p.split) each_job(blocks(Seq_q, Seq_k), p, walk(Seq_q, Seq_k), [&](int n, int rank, int part) { order.job[n] = (uint16_t)(8 * rank + (part < 0 ? 0 : part)); });
   }
   static size_t slot_bytes(long heads, const PartsPlan& p) { return (size_t)heads * p.split * (p.split ? p.parts : 0) * kSlotBytes; }
 };

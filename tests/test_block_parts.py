@@ -23,6 +23,17 @@ extern "C" int plan(long heads, int T, const int* walks, double tile_us, double 
 extern "C" void walks(int rows, int T, int Br, int Bc, int Seq_q, int Seq_k, int* out) {
   for (int t = 0; t < T; ++t) out[t] = rows ? aat::row_walk(t, Br, Bc, Seq_q, Seq_k) : aat::col_walk(t, Br, Bc, Seq_q, Seq_k);
 }
+// how often plans are searched for where the problems (heads, Seq_q, Seq_k, blocks per CU) come in this order, by one launch's memory
+extern "C" int searches(const int* problems, int n) {
+  static aat::PlanMemory known;
+  int count = 0;
+  for (int i = 0; i < n; ++i) {
+    const int* p = problems + 4 * i;
+    const aat::PartsPlan got = known.get(p[0], p[1], p[2], p[3], [&] { ++count; return aat::PartsPlan{p[1] / 64, 1 + p[2] / 64}; });
+    if (got.split != p[1] / 64 || got.parts != 1 + p[2] / 64) return -1;
+  }
+  return count;
+}
 """
 
 
@@ -68,3 +79,10 @@ def test_shares_cover_the_walk():
         for parts in (2, 3, 4):
             cuts = [n * p // parts for p in range(parts + 1)]           # part_range
             assert cuts[0] == 0 and cuts[-1] == n and all(b - a in (n // parts, n // parts + 1) for a, b in zip(cuts, cuts[1:]))
+
+
+def test_lengths_in_turn_are_searched_for_once(lib):
+    lengths = [64 * i for i in range(1, 65)]
+    problems = [(h, s, s, 1) for _ in range(3) for s in lengths for h in (8, 32)] + [(8, 64, 128, 1), (8, 64, 128, 2), (8, 64, 128, 1)] * 5
+    flat = (ctypes.c_int * (4 * len(problems)))(*[x for p in problems for x in p])
+    assert 128 + 2 <= lib.searches(flat, len(problems)) <= 128 + 2 + 16          # sets of four: a few problems push each other out
