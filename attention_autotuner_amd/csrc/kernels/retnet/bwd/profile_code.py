@@ -132,7 +132,7 @@ template <bool DECAY> hipError_t launch_passes(aat_half* q, aat_half* k, aat_hal
   if constexpr (DECAY) {{
     const size_t at = stored ? ws_bytes_needed(B, H, Seq_q, Seq_k) : ds_offset(H, Seq_q, Seq_k);
     BwdPlan plan{{}};
-    if (workspace != nullptr && workspace_bytes > at + 3 * aat::kOrderBytes) plan = plan_of(B, H, Seq_q, Seq_k, stored);   // else no room for any parts
+    if (aat::parts_room(workspace, workspace_bytes, at)) plan = plan_of(B, H, Seq_q, Seq_k, stored);
     if (plan.slots > 0 && workspace_bytes >= at + plan.counts + 3 * aat::kOrderBytes + plan.slots) {{
       char* const room = static_cast<char*>(workspace) + at;
       uint16_t* const order = reinterpret_cast<uint16_t*>(room + plan.counts);

@@ -57,7 +57,7 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
   if (lds_ok != hipSuccess) return lds_ok;
   const size_t at = workspace_size(B, H, Seq_q, Seq_k);
   aat::BlockParts in_parts;
-  if (workspace != nullptr && workspace_bytes > at + aat::kOrderBytes) {{               // else there is no room for any parts
+  if (aat::parts_room(workspace, workspace_bytes, at)) {{
     const aat::PartsPlan plan = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
     const size_t counts = aat::count_bytes((long)B * H, plan);
     if (plan.split > 0 && workspace_bytes >= at + counts + aat::kOrderBytes + Parts::slot_bytes((long)B * H, plan)) {{

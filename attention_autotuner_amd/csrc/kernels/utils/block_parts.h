@@ -361,5 +361,10 @@ struct PartsLaunch {
 // The room of a call: its launches' counts, in units of 256 bytes, their orders, the slots.
 inline size_t count_bytes(long heads, const PartsPlan& p) { return ((size_t)heads * p.split * sizeof(uint32_t) + 255) / 256 * 256; }
 constexpr size_t kOrderBytes = sizeof(JobOrder);
+// Whether a workspace of `bytes` may hold them behind its first `at` bytes (a multiple of 256): counts take atomic additions and
+// slots pairs of floats, so one that starts off a boundary of eight bytes, which a call without parts never looks at, does not.
+inline bool parts_room(const void* workspace, size_t bytes, size_t at) {
+  return workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 8 == 0 && bytes > at + kOrderBytes;
+}
 
 }  // namespace aat

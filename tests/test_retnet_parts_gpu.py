@@ -50,7 +50,8 @@ def test_parts_give_the_same_bits_every_time(dqk, dv):
 @pytest.mark.parametrize("op", ["ret", "ret_bwd"])
 def test_a_workspace_of_workspace_size_bytes_is_used_as_it_is(op):
     """... with nothing allocated beside it, every block walked in one piece, and the bytes behind it left alone; results against
-    the oracle's.  One that is larger by the room for the parts is used too."""
+    the oracle's.  So is a larger one that starts off a boundary of eight bytes; any other one that has room for the parts is used
+    for them too."""
     problem = b, h, sq, sk = 1, 2, 1088, 1088
     dqk, dv = 256, 512
     q, k, v, do, mask, lg = _problem(b, h, sq, sk, dqk, dv, "decay", 37)
@@ -70,13 +71,13 @@ def test_a_workspace_of_workspace_size_bytes_is_used_as_it_is(op):
         arrays = [qc, kc, vc, lg.cuda(), dc, r_want.cuda(), *out]
     room = torch.full((size + guard,), 0x5a, dtype=torch.uint8, device="cuda")
     rt.apply(arrays, decay=True, workspace=room[:size])                    # the library is loaded
-    for workspace in (room[:size], room):
+    for workspace in (room[:size], room[4:], room):
         torch.cuda.synchronize()
         before = torch.cuda.memory_stats()["allocation.all.allocated"]
         rt.apply(arrays, decay=True, workspace=workspace)
         torch.cuda.synchronize()
         assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
-        untouched = bool((room[size:] == 0x5a).all())
+        untouched = bool((room[size + 4:] == 0x5a).all())
         assert untouched == (workspace is not room)                       # the parts' counts, order and slots lie there
         for got, ref, t in zip(out, want, terms):
             ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
