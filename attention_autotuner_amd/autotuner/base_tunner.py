@@ -135,11 +135,11 @@ class BaseTunner:
         """(tensor or None, bytes): the workspace the runtime would grant ``config`` for this problem -- a stored dS
         beyond the runtime's limit is withheld there too, so what is timed is what will be launched.  Raises
         torch.cuda.OutOfMemoryError like any allocation."""
-        from .runtime import _wanted
+        from .runtime import _provided
         s = self.problem_shape
         need = int(lib.workspace_size(s["B"], s["H"], s["Sq"], s["Sk"]))
         if config is not None:
-            need = _wanted(config, need, s["B"], s["H"], s["Sq"], s["Sk"], self.decay)
+            need = _provided(lib, config, need, s["B"], s["H"], s["Sq"], s["Sk"], self.decay)
         ws = torch.empty(need, dtype=torch.uint8, device=self.torch_array[0].device) if need else None
         return ws, need
 

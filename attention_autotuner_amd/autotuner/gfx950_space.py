@@ -756,96 +756,3 @@ def rule_ret_config(op, dim_qk, dim_v, b, h, seq_q, seq_k, skips):
         return None
     few, line, many = walks["skip" if skips else "dense"]
     return _ret_config(op, dim_qk, dim_v, few if b * h * (seq_q if op == "ret" else seq_k) // 64 <= line else many)
-
-
-# ---- RetNet decay walks: blocks in parts -------------------------------------------------------------------
-# The room a decay call's longest blocks need to be walked in parts, behind its other workspace: the arithmetic of
-# csrc/kernels/utils/block_parts.h, where the reasons are.  A library that finds less room there walks every block in one piece.
-MOST_PARTS, MOST_JOBS = 4, 256
-
-
-def _parts_estimate_us(heads, lengths, split, parts, tile_us, places, waves, slot):
-    alone, exchange = 4.2 / waves * tile_us, 6.5 + 1.3 * slot / 131072.0
-    cut = [-(-n // parts) * alone + exchange for n in lengths[:split] for _ in range(parts)]
-    # the library merges the two falling sequences by walk length; ties between a part and a whole block go to the part
-    order, whole = [], split
-    for rank in range(split):
-        while whole < len(lengths) and lengths[rank] < parts * lengths[whole]:
-            order.append(lengths[whole] * alone)
-            whole += 1
-        order += cut[rank * parts:(rank + 1) * parts]
-    order += [n * alone for n in lengths[whole:]]
-    row = int(places / heads) if places > heads else 1
-    chain = max(order)
-    if len(order) > row and order[row] > 0.0:
-        chain = max(chain, order[row - 1] + order[row])
-    work = 1.14 * sum(lengths) * tile_us * heads / 256.0 + split * parts * exchange * heads / places
-    return max(work, chain) + (4.5 + 0.22e-6 * heads * split * parts * slot if split else 0.0)
-
-
-def plan_parts(heads, lengths, tile_us, places, waves, slot):
-    """(split, parts) for ``heads`` heads of blocks that walk ``lengths`` tiles, longest first."""
-    cost, total = (tile_us, places, waves, slot), len(lengths)
-    best, least, step = (0, 1), 0.95 * _parts_estimate_us(heads, lengths, 0, 1, *cost), max(1, total // 16)
-    for parts in range(2, MOST_PARTS + 1):
-        for split in range(step, total + 1, step):
-            if lengths[split - 1] < 2 * parts or total + split * (parts - 1) > MOST_JOBS:
-                break
-            us = _parts_estimate_us(heads, lengths, split, parts, *cost)
-            if us < least:
-                least, best = us, (split, parts)
-    return best
-
-
-def _walks(rows, br, bc, seq_q, seq_k):
-    diag = seq_k - seq_q
-    if rows:
-        firsts = range((-(-seq_q // br) - 1) * br, -1, -br)
-        return [max(0, min(seq_k // bc, (min(q0 + br, seq_q) - 1 + diag) // bc + 1)) for q0 in firsts]
-    return [max(0, seq_q // bc - max(0, k0 - diag) // bc) for k0 in range(0, seq_k, br)]
-
-
-def _parts_launch(heads, rows, seq_q, seq_k, br, bc, width, cols, threads, extra, per_cu, memory=1.0):
-    """(bytes of counts and order, bytes of slots) of one launch."""
-    slot = (br * cols + extra * threads) * 4
-    split, parts = plan_parts(heads, _walks(rows, br, bc, seq_q, seq_k), memory * 2.0 * br * bc * width / 4.5e6, 256.0 * per_cu, threads // WAVE, slot)
-    return -(-heads * split * 4 // 256) * 256 + 2 * MOST_JOBS, heads * split * parts * slot
-
-
-def _per_cu(waves, wpe, lds):
-    return max(1, min(wpe * 4 // waves, 160 * 1024 // lds))
-
-
-def decay_parts_bytes(cfg, b, h, seq_q, seq_k, stored_ds=False):
-    """Bytes behind the workspace of a RetNet decay call (``stored_ds``: of a backward that is granted the room for dS)."""
-    heads, waves = b * h, _waves(cfg)
-    fit = rows_per_wave(cfg) == MFMA_M and cfg.Bc <= 64 and (cfg.waves_per_eu == 1 or (cfg.operation == "ret" and cfg.Kd + cfg.D <= 256))
-    if cfg.operation == "ret":
-        if cfg.fuse_type != "register" or not fit:
-            return 0
-        ahead, slots = _parts_launch(heads, True, seq_q, seq_k, cfg.Br, cfg.Bc, cfg.Kd + cfg.D, cfg.D, cfg.Nthreads,
-                                     cfg.Br // waves // 32, _per_cu(waves, cfg.waves_per_eu, forward_lds_bytes(cfg)))
-        return ahead + slots if slots else 0
-    def lds(kx, dzb, sy, sz, staged):
-        main = sy * (cfg.Bc * kx * 2 + cfg.Br * cfg.Bc * 2) + sz * cfg.Bc * dzb * 2
-        return max(main + (cfg.Br * (cfg.Bc * 2 + 16) if staged else 0), cfg.Br * (dzb * 2 + 16))
-    width, dvb, launches = cfg.Kd + cfg.D, backward_dv_cols(cfg), []
-    shape = (cfg.Br, cfg.Bc, width)
-    if dvb == cfg.D and fit:
-        launches.append(_parts_launch(heads, False, seq_q, seq_k, *shape, dvb, cfg.Nthreads, 0,
-                                      _per_cu(waves, cfg.waves_per_eu, lds(cfg.Kd, dvb, cfg.num_stages_qk, cfg.num_stages_dv, False))))
-    else:
-        launches.append((2 * MOST_JOBS, 0))
-    chained = lds(cfg.D, cfg.Kd, cfg.num_stages_ds, cfg.num_stages_dq, stored_ds)
-    launches.append(_parts_launch(heads, True, seq_q, seq_k, *shape, cfg.Kd, cfg.Nthreads, 0, _per_cu(waves, cfg.waves_per_eu, chained))
-                    if fit else (2 * MOST_JOBS, 0))
-    if stored_ds:
-        rows = cfg.ds_rows
-        dk = max(2 * (DS_TILE * cfg.Kd * 2 + DS_TILE * rows * 2), rows * (cfg.Kd * 2 + 16))
-        launches.append(_parts_launch(heads, False, seq_q, seq_k, rows, DS_TILE, cfg.Kd, cfg.Kd, rows * 2, 0, _per_cu(rows // 32, 2, dk), 2.7))
-    elif fit:
-        launches.append(_parts_launch(heads, False, seq_q, seq_k, *shape, cfg.Kd, cfg.Nthreads, 0, _per_cu(waves, cfg.waves_per_eu, chained)))
-    else:
-        launches.append((2 * MOST_JOBS, 0))
-    slots = max(s for _, s in launches)
-    return sum(c for c, _ in launches) + slots if slots else 0

@@ -46,6 +46,9 @@ def _bind(lib, op):
         lib.profile_decay.argtypes = [_VP] * nd + [_I] * 4 + [_VP, _SZ, _VP]
         lib.kernel_entry_decay.restype = _I
         lib.kernel_entry_decay.argtypes = [_VP] * nd + [_I] * 4 + [_VP, _SZ, _VP]
+        if hasattr(lib, "decay_workspace_size"):
+            lib.decay_workspace_size.restype = _SZ
+            lib.decay_workspace_size.argtypes = [_I] * 4 + [_SZ]
     lib.profile_ex.restype = _F
     lib.profile_ex.argtypes = ptrs + [_I] * 4 + tail
     lib.kernel_entry_ex.restype = _I

@@ -11,7 +11,7 @@ import os
 
 import torch
 
-from . import codegen, gfx950_space, library
+from . import codegen, library
 
 
 class KernelLaunchError(RuntimeError):
@@ -30,14 +30,18 @@ _ERRORS = {-2: "sequence lengths are not multiples of what the library takes: 32
 MAX_DS_BYTES = int(os.environ.get("AAT_MAX_DS_BYTES", 2 << 30))
 
 
-def _wanted(config, need, B, H, Sq, Sk, decay=False):
-    """Bytes of workspace the runtime provides when the caller's is missing or too small."""
+def _wanted(config, need, B, H, Sq, Sk):
+    """Bytes of workspace a caller's has to hold to be used as it is, of the ``need`` the library reports."""
     ds_bytes = 2 * B * H * Sq * Sk
-    stored = getattr(config, "operation", "") == "ret_bwd" and getattr(config, "ds_rows", 0) and need >= ds_bytes
-    if stored and ds_bytes > MAX_DS_BYTES:
-        need, stored = need - ds_bytes, False
-    parts = gfx950_space.decay_parts_bytes(config, B, H, Sq, Sk, stored) if decay else 0
-    return need + (parts if parts <= MAX_DS_BYTES else 0)
+    if getattr(config, "operation", "") == "ret_bwd" and getattr(config, "ds_rows", 0) and need >= ds_bytes > MAX_DS_BYTES:
+        return need - ds_bytes
+    return need
+
+
+def _provided(lib, config, need, B, H, Sq, Sk, decay):
+    """Bytes of workspace the runtime provides when the caller's is missing or too small."""
+    ask = getattr(lib, "decay_workspace_size", None) if decay else None      # a library built before there were parts has none
+    return int(ask(B, H, Sq, Sk, MAX_DS_BYTES)) if ask is not None else _wanted(config, need, B, H, Sq, Sk)
 
 
 def _grown(workspace, need, device, keep):
@@ -99,8 +103,8 @@ class Runtime:
         needs = self._need.get((B, H, Sq, Sk, decay))       # a property of the library and the problem: asked once
         if needs is None:
             size = int(lib.workspace_size(B, H, Sq, Sk))
-            # what a caller's workspace has to hold to be used as it is, what is provided otherwise
-            needs = self._need[(B, H, Sq, Sk, decay)] = (_wanted(self.config, size, B, H, Sq, Sk), _wanted(self.config, size, B, H, Sq, Sk, decay))
+            needs = self._need[(B, H, Sq, Sk, decay)] = (_wanted(self.config, size, B, H, Sq, Sk),
+                                                         _provided(lib, self.config, size, B, H, Sq, Sk, decay))
         if needs[1] and (workspace is None or workspace.numel() * workspace.element_size() < needs[0]):
             workspace = _grown(workspace, needs[1], q.device, keep=causal == "scanned")
         ws_ptr = workspace.data_ptr() if workspace is not None else None

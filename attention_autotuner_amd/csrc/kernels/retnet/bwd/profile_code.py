@@ -63,6 +63,7 @@ using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkRows * 2, 0, fal
 struct BwdPlan {{
   aat::PartsPlan dv, dq, dk;
   size_t counts, slots;
+  size_t bytes() const {{ return slots ? counts + 3 * aat::kOrderBytes + slots : 0; }}
 }};
 BwdPlan plan_of(int B, int H, int Seq_q, int Seq_k, bool stored) {{
   const long heads = (long)B * H;
@@ -133,7 +134,7 @@ template <bool DECAY> hipError_t launch_passes(aat_half* q, aat_half* k, aat_hal
     const size_t at = stored ? ws_bytes_needed(B, H, Seq_q, Seq_k) : ds_offset(H, Seq_q, Seq_k);
     BwdPlan plan{{}};
     if (aat::parts_room(workspace, workspace_bytes, at)) plan = plan_of(B, H, Seq_q, Seq_k, stored);
-    if (plan.slots > 0 && workspace_bytes >= at + plan.counts + 3 * aat::kOrderBytes + plan.slots) {{
+    if (plan.slots > 0 && workspace_bytes >= at + plan.bytes()) {{
       char* const room = static_cast<char*>(workspace) + at;
       uint16_t* const order = reinterpret_cast<uint16_t*>(room + plan.counts);
       float* const slots = reinterpret_cast<float*>(room + plan.counts + 3 * aat::kOrderBytes);
@@ -232,6 +233,13 @@ extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* mas
 """
 
 decay_entry = r"""
+extern "C" size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most) {{
+  if (!bwd_shape_ok(B, H, Seq_q, Seq_k)) return workspace_size(B, H, Seq_q, Seq_k);
+  const size_t scan = ds_offset(H, Seq_q, Seq_k), ds = ws_bytes_needed(B, H, Seq_q, Seq_k) - scan;
+  const bool stored = ds > 0 && ds <= most;
+  const size_t at = stored ? scan + ds : scan, room = plan_of(B, H, Seq_q, Seq_k, stored).bytes();
+  return room <= most ? at + room : at;
+}}
 extern "C" float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* dO, float* r,
                                aat_half* dq, aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, void* workspace,
                                size_t workspace_bytes, void* stream) {{

@@ -29,6 +29,11 @@ template <bool DECAY> constexpr auto kernel_ragged = &aat::ret_ragged_regfuse<Kd
 using Parts = aat::PartsLaunch<aat::parts_fit(Traits::RT, Bc, waves_per_eu, Kd + D), Br, Bc, Kd + D, D, Nthreads, Traits::RT, true>;
 constexpr int kBlocksPerCu = aat::blocks_per_cu(Nthreads / 64, waves_per_eu, shared_mem);
 
+// ... their counts, their order and their slots
+size_t parts_bytes(int B, int H, const aat::PartsPlan& p) {{
+  return p.split ? aat::count_bytes((long)B * H, p) + aat::kOrderBytes + Parts::slot_bytes((long)B * H, p) : 0;
+}}
+
 bool lengths_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, Bc); }}
 int row_blocks(int Seq_q) {{ return (Seq_q + Br - 1) / Br; }}
 template <bool DECAY> hipError_t allow_kernels() {{
@@ -60,7 +65,7 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
   if (aat::parts_room(workspace, workspace_bytes, at)) {{
     const aat::PartsPlan plan = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
     const size_t counts = aat::count_bytes((long)B * H, plan);
-    if (plan.split > 0 && workspace_bytes >= at + counts + aat::kOrderBytes + Parts::slot_bytes((long)B * H, plan)) {{
+    if (plan.split > 0 && workspace_bytes >= at + parts_bytes(B, H, plan)) {{
       char* const room = static_cast<char*>(workspace) + at;
       uint32_t* const arrived = reinterpret_cast<uint32_t*>(room);
       uint16_t* const order = reinterpret_cast<uint16_t*>(room + counts);
@@ -119,6 +124,12 @@ extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* mas
 """
 
 decay_entry = r"""
+extern "C" size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most) {{
+  const size_t at = workspace_size(B, H, Seq_q, Seq_k);
+  if (!lengths_ok(B, H, Seq_q, Seq_k)) return at;
+  const size_t room = parts_bytes(B, H, Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu));
+  return room <= most ? at + room : at;
+}}
 extern "C" float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
                                int B, int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes, void* stream) {{
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return -1.f;

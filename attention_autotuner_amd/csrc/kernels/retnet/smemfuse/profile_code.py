@@ -91,6 +91,7 @@ extern "C" int kernel_entry(aat_half* q, aat_half* k, aat_half* v, aat_half* mas
 """
 
 decay_entry = r"""
+extern "C" size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t) {{ return workspace_size(B, H, Seq_q, Seq_k); }}   // no parts here
 extern "C" float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
                                int B, int H, int Seq_q, int Seq_k, void*, size_t, void* stream) {{
   if (!aat::shape_ok(B, H, Seq_q, Seq_k, Br, Bc)) return -1.f;

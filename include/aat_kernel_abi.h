@@ -107,7 +107,7 @@ int kernel_entry_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_h
  * (python/ops/retnet_interface.py:26-31) and lists "causal config" and the mask stream's cost as open
  * items (README.md:102-114).  Given more workspace than workspace_size(), the longest blocks of a problem that leaves the chip
  * partly idle are walked by several workgroups whose sums meet in it (csrc/kernels/utils/block_parts.h; how much more:
- * decay_parts_bytes in autotuner/gfx950_space.py); given less, every block is walked in one piece. */
+ * decay_workspace_size() below); given less, every block is walked in one piece. */
 float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,
                     int B, int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes,
                     void* stream);
@@ -195,6 +195,14 @@ float retnet_recurrent_profile(const float* q, const float* k, const float* v, c
 #define AAT_RECURRENT_NOALLOC_MAX_RECORDS 3072
 int retnet_recurrent_fwd_noalloc(const float* q, const float* k, const float* v, const float* decay, float* out,
                                  int batch, int heads, int kdim, int vdim, int l, int block_kdim, void* stream);
+#endif
+
+#if defined(AAT_OP_RET) || defined(AAT_OP_RET_BWD)
+/* Bytes of workspace that a decay call (profile_decay, kernel_entry_decay) of this problem makes use of: what workspace_size()
+ * reports and, where walking the longest blocks in parts pays, the parts' room behind it.  A stored dS and the parts' room are
+ * optional; each is left out where it takes more than `most` bytes, so SIZE_MAX asks for everything and 0 for neither.  Results
+ * with and without the parts differ by the order of fp32 additions. */
+size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most);
 #endif
 
 #ifdef __cplusplus

@@ -1,5 +1,5 @@
-"""Blocks of a causal walk in parts: the plan the libraries make and the room the runtime provides for it are the same arithmetic,
-and a plan's jobs are every part of every block once, longest first."""
+"""Blocks of a causal walk in parts, on the host: a plan's jobs are every part of every block once, longest first; plans are searched
+for once; the libraries report the room their plans take."""
 import ctypes
 import os
 import random
@@ -8,7 +8,10 @@ import subprocess
 import pytest
 
 from attention_autotuner_amd.arch import MI355X
-from attention_autotuner_amd.autotuner import codegen, gfx950_space
+from attention_autotuner_amd.autotuner import codegen, gfx950_space, library, runtime
+
+MOST_PARTS, MOST_JOBS, ORDER_BYTES = 4, 256, 512
+RULE = [(op, d, c) for op in ("ret", "ret_bwd") for d in sorted(gfx950_space.RET_RULE) for c in gfx950_space.rule_ret_configs(op, *d)]
 
 SOURCE = r"""
 #include <hip/hip_runtime.h>
@@ -47,7 +50,16 @@ def lib(tmp_path_factory):
     return ctypes.CDLL(out)
 
 
-def test_the_plan_and_its_room_agree_and_the_jobs_are_complete(lib):
+def _walks(rows, br, bc, seq_q, seq_k):
+    """Tiles a block walks below the diagonal kv <= q + seq_k - seq_q, the longest block first."""
+    diag = seq_k - seq_q
+    if rows:
+        firsts = range((-(-seq_q // br) - 1) * br, -1, -br)
+        return [max(0, min(seq_k // bc, (min(q0 + br, seq_q) - 1 + diag) // bc + 1)) for q0 in firsts]
+    return [max(0, seq_q // bc - max(0, k0 - diag) // bc) for k0 in range(0, seq_k, br)]
+
+
+def test_the_jobs_of_a_plan_are_complete_and_longest_first(lib):
     rng = random.Random(5)
     cut = 0
     for _ in range(150):
@@ -55,23 +67,61 @@ def test_the_plan_and_its_room_agree_and_the_jobs_are_complete(lib):
         sq, sk = 64 * rng.randint(1, 64), 64 * rng.randint(1, 64)
         heads, rows, per_cu = rng.randint(1, 96), rng.randint(0, 1), rng.choice((1, 2, 4))
         cols, width = rng.choice(((64, 128), (128, 256), (256, 512), (256, 768), (512, 768)))
-        want = gfx950_space._walks(bool(rows), br, bc, sq, sk)
+        want = _walks(bool(rows), br, bc, sq, sk)
         T = len(want)
         got = (ctypes.c_int * T)()
         lib.walks(rows, T, br, bc, sq, sk, got)
         assert list(got) == want, (rows, br, bc, sq, sk)
         tile, slot = 2.0 * br * bc * width / 4.5e6, br * cols * 4
-        split, parts = gfx950_space.plan_parts(heads, want, tile, 256.0 * per_cu, waves, slot)
-        c_split, c_parts, jobs = ctypes.c_int(), ctypes.c_int(), (ctypes.c_int * (T * gfx950_space.MOST_PARTS))()
+        c_split, c_parts, jobs = ctypes.c_int(), ctypes.c_int(), (ctypes.c_int * (T * MOST_PARTS))()
         n = lib.plan(ctypes.c_long(heads), T, got, ctypes.c_double(tile), ctypes.c_double(256.0 * per_cu), waves, ctypes.c_size_t(slot),
                      ctypes.byref(c_split), ctypes.byref(c_parts), jobs)
-        assert (c_split.value, c_parts.value) == (split, parts)
+        split, parts = c_split.value, c_parts.value
         assert sorted(jobs[:n]) == sorted([8 * t + p for t in range(split) for p in range(parts)] + [8 * t for t in range(split, T)])
         lengths = [want[j >> 3] / (parts if j >> 3 < split else 1) for j in jobs[:n]]
         assert all(a >= b - 1e-9 for a, b in zip(lengths, lengths[1:]))
-        assert n <= gfx950_space.MOST_JOBS or split == 0
+        assert split == 0 or (n <= MOST_JOBS and want[split - 1] >= 2 * parts)
         cut += split > 0
     assert 20 <= cut <= 130
+
+
+@pytest.mark.parametrize("op", ["ret", "ret_bwd"])
+def test_the_libraries_report_the_room_of_their_parts(op):
+    rng, cut = random.Random(7), 0
+    for _, d, cfg in (r for r in RULE if r[0] == op):
+        loaded = library.load(codegen.compile_config(cfg, MI355X(), timeout=600), op)
+        for _ in range(40):
+            b, h, sq = rng.randint(1, 4), rng.choice((1, 2, 3, 4, 8, 12)), 64 * rng.randint(1, 48)
+            sk = rng.choice((sq, 64 * rng.randint(1, 48)))
+            problem, heads = (b, h, sq, sk), b * h
+            least, most = loaded.decay_workspace_size(*problem, 0), loaded.decay_workspace_size(*problem, ctypes.c_size_t(-1).value)
+            ds = 2 * b * h * sq * sk if loaded.workspace_size(*problem) >= 2 * b * h * sq * sk and getattr(cfg, "ds_rows", 0) else 0
+            assert least == loaded.workspace_size(*problem) - ds and most >= loaded.workspace_size(*problem)
+            # counts are whole units of 256 bytes, each launch has an order, slots hold the resident rows of a block in fp32
+            for stored in {0, ds}:
+                total = loaded.decay_workspace_size(*problem, max(ds, 1 << 40)) if stored == ds else loaded.decay_workspace_size(*problem, ds - 1)
+                room = total - least - stored
+                if room > 0:
+                    launches = 1 if op == "ret" else 3
+                    assert room % 256 == 0 and room > launches * ORDER_BYTES + heads * 2 * 64 * cfg.Kd * 4
+                    assert loaded.decay_workspace_size(*problem, max(stored, room)) in (total, least + ds + room)
+                    cut += 1
+        assert loaded.decay_workspace_size(1, 1, 16, 16, 1 << 40) == loaded.workspace_size(1, 1, 16, 16)      # no length it takes
+    assert cut > 40
+
+
+def test_a_library_without_the_question_is_asked_for_its_workspace_size():
+    class Old:
+        pass
+    cfg = next(c for op, d, c in RULE if op == "ret_bwd" and c.ds_rows)
+    assert runtime._provided(Old(), cfg, 4096, 1, 8, 512, 512, True) == 4096
+
+    class New:
+        def decay_workspace_size(self, *problem_and_limit):
+            assert problem_and_limit == (1, 8, 512, 512, runtime.MAX_DS_BYTES)
+            return 9999
+    assert runtime._provided(New(), cfg, 4096, 1, 8, 512, 512, True) == 9999
+    assert runtime._provided(New(), cfg, 4096, 1, 8, 512, 512, False) == 4096
 
 
 def test_shares_cover_the_walk():

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import attention_autotuner_amd as aat
-from attention_autotuner_amd.autotuner import Runtime, gfx950_space
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space, library
 from oracle import ref_op, tolerance
 from test_retnet_ragged_gpu import _check, _problem
 
@@ -19,12 +19,17 @@ def _configs(dqk, dv, problem):
     return (gfx950_space.rule_ret_config("ret", dqk, dv, b, h, sq, sk, True), gfx950_space.rule_ret_config("ret_bwd", dqk, dv, b, h, sq, sk, True))
 
 
+def _cuts(rt, problem):
+    lib = library.load(rt._path(), rt.config.operation)
+    return lib.decay_workspace_size(*problem, 1 << 40) > lib.workspace_size(*problem)
+
+
 @pytest.mark.parametrize("dqk,dv", sorted(gfx950_space.RET_RULE))
 def test_blocks_in_parts_against_the_oracle(dqk, dv):
     cut = 0
     for i, problem in enumerate(SHAPES):
         fwd, bwd = _configs(dqk, dv, problem)
-        cut += (gfx950_space.decay_parts_bytes(fwd, *problem) > 0) + (gfx950_space.decay_parts_bytes(bwd, *problem, stored_ds=bwd.ds_rows > 0) > 0)
+        cut += sum(_cuts(Runtime(ARCH, cfg), problem) for cfg in (fwd, bwd))
         _check(problem, dqk, dv, "decay", 900 + i, [fwd], [bwd])
     assert cut >= 2 or dqk == 64, "nothing was cut"          # a walk of 17 tiles of 64 columns is not worth an exchange
 
@@ -34,7 +39,7 @@ def test_parts_give_the_same_bits_every_time(dqk, dv):
     problem = b, h, sq, sk = 1, 4, 2112, 2112
     q, k, v, do, _, lg = (t.cuda() for t in _problem(1, 4, sq, sk, dqk, dv, "decay", 31))
     fwd, bwd = (Runtime(ARCH, c) for c in _configs(dqk, dv, problem))
-    assert gfx950_space.decay_parts_bytes(bwd.config, *problem, stored_ds=bwd.config.ds_rows > 0) > 0
+    assert _cuts(bwd, problem)
     first = None
     for _ in range(5):
         o, r = torch.full_like(do, 7.0), torch.full((b, h, sq), 7.0, device="cuda")
