@@ -546,7 +546,7 @@ ret_bwd_chain(const half_t* __restrict__ x, const half_t* __restrict__ y, const 
       float none[1];
       bool last;
       if constexpr (kNumbered) last = combine_parts_numbered<64, 0, Nthreads>(in_parts, id, none, smem);
-      else last = combine_parts<0, Nthreads, 4>(in_parts, id, acc, none, smem);
+      else last = combine_parts<0, Nthreads>(in_parts, id, acc, none, smem);
       if (last) store_chain_tile<T, DZ, DZB, kNumbered>(acc, ostage, og, lane, groups);
       return;
     }

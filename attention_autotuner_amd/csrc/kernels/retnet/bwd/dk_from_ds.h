@@ -227,7 +227,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   };
   if (id.parts > 1) {                             // to the end in here: joined again, the two paths' accumulators cost 68 bytes of scratch
     float none[1];
-    if (combine_parts<0, Nthreads, 4>(in_parts, id, acc, none, smem)) finish();
+    if (combine_parts<0, Nthreads>(in_parts, id, acc, none, smem)) finish();
     return;
   }
   finish();

@@ -56,10 +56,10 @@ static_assert(!kStoredDs || Br % kDkTile == 0, "a query tile of the dK kernel li
 // The longest blocks of a decay walk in parts (utils/block_parts.h), where the call has room for their slots behind its other
 // workspace.  The launches of a call follow each other and share the slots; each has counts of its own.
 constexpr bool kPartsFit = aat::parts_fit(RTv, Bc, waves_per_eu, 0);
-using PV = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DVB, Nthreads, 0, false>;
-using PQ = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, true>;
-using PK = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, false>;
-using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkRows * 2, 0, false, 270>;    // it streams dS and multiplies little
+using PV = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DVB, Nthreads, 0, false, DVB == 512>;
+using PQ = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, true, DKB == 512>;
+using PK = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, false, DKB == 512>;
+using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkRows * 2, 0, false, false, 109>;    // it streams dS as well
 struct BwdPlan {{
   aat::PartsPlan dv, dq, dk;
   size_t counts, slots;
@@ -74,6 +74,7 @@ BwdPlan plan_of(int B, int H, int Seq_q, int Seq_k, bool stored) {{
   p.dq = PQ::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, row_lds));
   p.dk = stored ? PKD::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(kDkRows / 32, kDkWaves, TKD::kSmemBytes))
                 : PK::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TK::kSmemBytes));
+  if (p.dv.gain_us + p.dq.gain_us + p.dk.gain_us < aat::kPrepareUs) return BwdPlan{{}};
   const size_t dk = stored ? PKD::slot_bytes(heads, p.dk) : PK::slot_bytes(heads, p.dk);
   const size_t dv = PV::slot_bytes(heads, p.dv), dq = PQ::slot_bytes(heads, p.dq);
   p.slots = dv > dq ? (dv > dk ? dv : dk) : (dq > dk ? dq : dk);

@@ -26,9 +26,13 @@ template <bool DECAY> constexpr auto kernel = &aat::ret_fwd_regfuse<Kd, D, Br, B
 template <bool DECAY> constexpr auto kernel_ragged = &aat::ret_ragged_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, stages_mask, waves_per_eu, DECAY>;
 
 // The longest blocks of a decay walk in parts (utils/block_parts.h), where the call has room for their slots behind workspace_size().
-using Parts = aat::PartsLaunch<aat::parts_fit(Traits::RT, Bc, waves_per_eu, Kd + D), Br, Bc, Kd + D, D, Nthreads, Traits::RT, true>;
+using Parts = aat::PartsLaunch<aat::parts_fit(Traits::RT, Bc, waves_per_eu, Kd + D), Br, Bc, Kd + D, D, Nthreads, Traits::RT, true, waves_per_eu == 1>;
 constexpr int kBlocksPerCu = aat::blocks_per_cu(Nthreads / 64, waves_per_eu, shared_mem);
 
+aat::PartsPlan plan_of(int B, int H, int Seq_q, int Seq_k) {{
+  const aat::PartsPlan p = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
+  return p.gain_us >= aat::kPrepareUs ? p : aat::PartsPlan();
+}}
 // ... their counts, their order and their slots
 size_t parts_bytes(int B, int H, const aat::PartsPlan& p) {{
   return p.split ? aat::count_bytes((long)B * H, p) + aat::kOrderBytes + Parts::slot_bytes((long)B * H, p) : 0;
@@ -63,7 +67,7 @@ hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2
   const size_t at = workspace_size(B, H, Seq_q, Seq_k);
   aat::BlockParts in_parts;
   if (aat::parts_room(workspace, workspace_bytes, at)) {{
-    const aat::PartsPlan plan = Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu);
+    const aat::PartsPlan plan = plan_of(B, H, Seq_q, Seq_k);
     const size_t counts = aat::count_bytes((long)B * H, plan);
     if (plan.split > 0 && workspace_bytes >= at + parts_bytes(B, H, plan)) {{
       char* const room = static_cast<char*>(workspace) + at;
@@ -127,7 +131,7 @@ decay_entry = r"""
 extern "C" size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most) {{
   const size_t at = workspace_size(B, H, Seq_q, Seq_k);
   if (!lengths_ok(B, H, Seq_q, Seq_k)) return at;
-  const size_t room = parts_bytes(B, H, Parts::find((long)B * H, Seq_q, Seq_k, kBlocksPerCu));
+  const size_t room = parts_bytes(B, H, plan_of(B, H, Seq_q, Seq_k));
   return room <= most ? at + room : at;
 }}
 extern "C" float profile_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r,

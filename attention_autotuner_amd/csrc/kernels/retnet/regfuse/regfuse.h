@@ -368,7 +368,7 @@ AAT_DEV void ret_fwd_walk(const half_t* __restrict__ q, const half_t* __restrict
         row[rt].r_ref = 1.f;
         sums[rt] = row[rt].big_r;
       }
-      if (!combine_parts<RT, Nthreads, 4>(in_parts, id, oacc, sums, smem)) return;
+      if (!combine_parts<RT, Nthreads>(in_parts, id, oacc, sums, smem)) return;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) row[rt].big_r = sums[rt];
       finish();

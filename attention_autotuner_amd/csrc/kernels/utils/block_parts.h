@@ -7,9 +7,12 @@
 // last adds the slots up in the order of the parts (so the sum does not depend on which one that is) and finishes the block.
 // Nobody waits for anybody: a part that is not the last one to arrive ends.
 //
-// RetNet with decay rates: B2 H8 S2112 256/512 (272 blocks of 128 rows, one to a compute unit) forward 99 -> 88 us, forward and
-// backward 365 -> 319; B1 H8 S2048 256/512 104 -> 68 and 327 -> 220; B1 H4 S4096 128/128 81 -> 47 and 313 -> 206.
+// RetNet with decay rates, kernel time of forward and backward, the launches that prepare the parts included: B2 H8 S2112 256/512
+// (272 blocks of 128 rows, one to a compute unit) 328 -> 300 us, B1 H8 S2112 256/512 317 -> 228, B1 H4 S4096 128/128 309 -> 190.
 #pragma once
+#include <algorithm>
+#include <functional>
+#include <initializer_list>
 #include <mutex>
 
 #include "acc_file.h"
@@ -97,6 +100,9 @@ AAT_DEV bool last_to_arrive(uint32_t* arrived, int parts, uint32_t* word) {
   return last;
 }
 
+// Quads whose loads are in flight together: those of numbered accumulators are read into registers the walk no longer needs.
+constexpr int parts_at_once(int quads, bool numbered) { return !numbered ? 4 : quads % 16 == 0 ? 16 : 8; }
+
 // Adds the slots of a block up, part 0 first.  get(q) is quad q of the own accumulators (read instead of the own slot),
 // put(q, sum) takes the sums.  AT quads at a time: that many loads are in flight per wave.
 template <int QUADS, int NT, int AT, class Get, class Put>
@@ -167,7 +173,7 @@ AAT_DEV bool combine_parts_numbered(const BlockParts& p, const PartId& id, float
 #pragma unroll
   for (int i = 0; i < EXTRA; ++i) __hip_atomic_store(own + (4 * QUADS + i) * NT + threadIdx.x, extra[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (!last_to_arrive(p.arrived + id.place, id.parts, reinterpret_cast<uint32_t*>(lds))) return false;
-  sum_parts<QUADS, NT, QUADS % 16 == 0 ? 16 : 8>(block, kSlot, id, get, [&](auto q_tag, const f4v& sum) {
+  sum_parts<QUADS, NT, parts_at_once(QUADS, true)>(block, kSlot, id, get, [&](auto q_tag, const f4v& sum) {
     static_for<4>([&](auto e_tag) {
       constexpr int E = decltype(e_tag)::value;
       const float t = sum[E];
@@ -178,8 +184,8 @@ AAT_DEV bool combine_parts_numbered(const BlockParts& p, const PartId& id, float
   return true;
 }
 
-// The same for an output tile the compiler allocates.  AT: quads in flight, fewer where several waves share a SIMD.
-template <int EXTRA, int NT, int AT, int RT, int DT>
+// The same for an output tile the compiler allocates.
+template <int EXTRA, int NT, int RT, int DT>
 AAT_DEV bool combine_parts(const BlockParts& p, const PartId& id, f16v (&acc)[RT][DT], float (&extra)[EXTRA > 0 ? EXTRA : 1], char* lds) {
   constexpr int QUADS = 4 * RT * DT;
   constexpr size_t kSlot = part_floats<QUADS, EXTRA, NT>();
@@ -193,7 +199,7 @@ AAT_DEV bool combine_parts(const BlockParts& p, const PartId& id, f16v (&acc)[RT
 #pragma unroll
   for (int i = 0; i < EXTRA; ++i) __hip_atomic_store(own + (4 * QUADS + i) * NT + threadIdx.x, extra[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (!last_to_arrive(p.arrived + id.place, id.parts, reinterpret_cast<uint32_t*>(lds))) return false;
-  sum_parts<QUADS, NT, AT>(block, kSlot, id, get, [&](auto q_tag, const f4v& sum) {
+  sum_parts<QUADS, NT, parts_at_once(QUADS, false)>(block, kSlot, id, get, [&](auto q_tag, const f4v& sum) {
     constexpr int Q = decltype(q_tag)::value, R = Q / 4 / DT, C = Q / 4 % DT, V = 4 * (Q % 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[R][C][V + e] = sum[e];
@@ -241,6 +247,7 @@ constexpr int blocks_per_cu(int waves, int waves_per_eu, int lds_bytes) {
 
 struct PartsPlan {
   int split = 0, parts = 1;
+  float gain_us = 0.f;                   // by the estimate
 };
 constexpr int kMostParts = 4;
 
@@ -258,57 +265,123 @@ template <class Length, class Job> inline int each_job(int T, const PartsPlan& p
   return n;
 }
 
-// What a launch of `heads` heads of T blocks takes, in microseconds: the larger of the whole work at the rate of a full chip and
-// of the longest chain of jobs, and what goes through memory between the parts.  A tile of one block takes `tile_us` of a CU's
-// matrix time, 4.2 / waves of that where the block is alone on its CU; a part waits 6.5 us and the time of its slot for its
-// arrival and the sum; slots move at 4.5 TB/s, written and read.  Fitted on 290 launches of 9 problems (d 64 ... 512, 96 ... 528
-// blocks, 0 ... all of them in 2 ... 4 parts; 14 % off on the mean).  With the plan it picks a problem is within 3 % of the best
-// measured one (B1 H4 S4096 d 128 with the 64-row shapes: forward 77 -> 43 us, backward 233 -> 142; B1 H8 S2048 256/512 100 -> 66 and
-// 224 -> 150), 8 to 22 % where it cuts a few too many; it cuts nothing where the best plan gains less than 10 % (walks of 8 tiles).
+// What a launch takes, in microseconds: its jobs handed out in their order to the places of an XCD, as the hardware does.  A tile
+// of one block takes `tile_us` of a CU's matrix time, 3.95 / waves of that where the block is alone on its CU, 1.15 times its
+// share of the CU beside others.  A part waits 8 us for every 128 KB of its slot to be where the device sees them; the last one
+// reads every other slot in `rounds` of loads, 0.3 us each and 2 us for every 32 KB of a wave.
+//
+// Fitted on 1740 launches (d 64 ... 512, 1 ... 48 heads, 512 ... 4096 rows; forward, dV, dQ and dK), each timed whole and in up to 24
+// plans.  Over the 870 calls they belong to, the plans it picks take 0.904 of the time without any, the launches that prepare them
+// included, the best measured ones 0.882; 7 calls run longer than whole by more than 3 %, the worst by 8.  An estimate from the
+// longest block and the mean work alone, which this one replaces, reached 0.942 and made 121 calls longer by more than 2 %, the worst
+// by 43 (B1 H4 S512 256/512 forward and backward 108 us whole, 134 in its parts; B2 H8 S1088 192/192 119 and 138): short walks lose
+// to the exchange, and where the head count is no multiple of 8 an XCD holds the longest jobs of a head or the shortest, so that
+// cutting a few blocks may leave it more long jobs than places.
 struct PartsCost {
-  double tile_us, places;
-  int waves;
+  double tile_us;
+  int waves, blocks_per_cu, rounds;
   size_t slot_bytes;
 };
-template <class Length> inline double parts_estimate_us(long heads, int T, const PartsPlan& p, Length&& length, const PartsCost& c) {
-  const double alone = 4.2 / c.waves * c.tile_us, exchange = 6.5 + 1.3 * c.slot_bytes / 131072.0;
-  const int row = c.places > heads ? (int)(c.places / heads) : 1;         // jobs of a head the chip holds at once
-  double tiles = 0., longest = 0., last = 0., next = 0.;
-  each_job(T, p, length, [&](int n, int rank, int part) {
-    const int walk = part < 0 ? length(rank) : (length(rank) + p.parts - 1) / p.parts;
-    const double us = walk * alone + (part < 0 ? 0. : exchange);
-    tiles += part < 0 ? walk : (double)length(rank) / p.parts;
-    if (us > longest) longest = us;
-    if (n == row - 1) last = us;
-    if (n == row) next = us;                                              // starts where the shortest of the first ones ends
-  });
-  const double chain = next > 0. && last + next > longest ? last + next : longest;
-  const double work = 1.14 * tiles * c.tile_us * heads / 256.0 + (double)p.split * p.parts * exchange * heads / c.places;
-  return (work > chain ? work : chain) + (p.split ? 4.5 + 0.22e-6 * heads * p.split * p.parts * c.slot_bytes : 0.);
+constexpr int kXcds = 8, kXcdCus = 32;
+struct PartsTimes {
+  float tile, alone;                     // of a tile: at the rate of a full CU, of a block that has its CU to itself
+  float store, read;                     // of a part: its slot; of the last one: the others' slots
+  PartsTimes(const PartsCost& c, int parts)
+      : tile((float)c.tile_us), alone(3.95f / c.waves * tile), store(parts > 1 ? 8.f / 131072.f * c.slot_bytes : 0.f),
+        read((parts - 1) * (0.3f * c.rounds + 2.f / 32768.f * c.slot_bytes / c.waves)) {}
+};
+
+// The time of `count` jobs, job(i) the i-th of them, on one XCD.
+struct PartsJob {
+  float us;
+  int walk;
+};
+template <class At> inline float xcd_us(int count, const PartsCost& c, const PartsTimes& t, At&& job) {
+  constexpr int kMostPlaces = 256;
+  const int room = kXcdCus * c.blocks_per_cu, places = room < kMostPlaces ? room : kMostPlaces;
+  float end[kMostPlaces];                // when the places are free again, a heap with the first one in front
+  float total = 0.f, last = 0.f;
+  long tiles = 0;
+  int used = 0;
+  for (int i = 0; i < count; ++i) {
+    const PartsJob j = job(i);
+    total += j.us;
+    tiles += j.walk;
+    if (used < places) {
+      end[used++] = j.us;
+      std::push_heap(end, end + used, std::greater<float>());
+      last = j.us > last ? j.us : last;
+    } else {
+      std::pop_heap(end, end + places, std::greater<float>());
+      const float done = end[places - 1] += j.us;
+      std::push_heap(end, end + places, std::greater<float>());
+      last = done > last ? done : last;
+    }
+  }
+  if (total <= 0.f) return 0.f;
+  const float sharing = count <= kXcdCus ? 1.f : (float)count / kXcdCus < c.blocks_per_cu ? (float)count / kXcdCus : (float)c.blocks_per_cu;
+  const float beside = 1.15f * t.tile * sharing, busy = total / (places * last);
+  if (beside <= t.alone) return last;
+  return last * (1.f + (beside / t.alone - 1.f) * (busy < 1.f ? busy : 1.f) * (tiles * t.alone / total));
 }
 
-// The plan with the smallest estimate; cutting has to gain a twentieth.  autotuner/gfx950_space.py holds the same arithmetic, to
-// provide the room.
+template <class Length> inline float parts_estimate_us(long heads, int T, const PartsPlan& p, Length&& length, const PartsCost& c) {
+  const PartsTimes t(c, p.parts);
+  PartsJob head[kMostJobs];
+  const int n = each_job(T, p, length, [&](int i, int rank, int part) {
+    const int walk = part < 0 ? length(rank) : (length(rank) + p.parts - 1) / p.parts;
+    head[i] = {2.3f + walk * t.alone + (part < 0 ? 0.f : t.store) + (part == p.parts - 1 ? t.read : 0.f), walk};
+  });
+  // which jobs an XCD gets, in their order: as causal_tile deals them out
+  const long grid = n * heads, each = grid / kXcds;
+  float us = 0.f;
+  const auto take = [&](float one) { us = one > us ? one : us; };
+  if (grid % kXcds != 0) {                               // every eighth of all
+    for (int first = 0; first < (heads < 4 ? 1 : 4); first += 3)
+      take(xcd_us((int)((grid - first + kXcds - 1) / kXcds), c, t, [&](int i) { return head[(first + (long)i * kXcds) % n]; }));
+  } else if (heads % kXcds == 0) {                       // its heads side by side
+    take(xcd_us((int)each, c, t, [&](int i) { return head[i / (heads / kXcds)]; }));
+  } else {                                               // a piece of the row of all heads
+    for (int x = 0; x < kXcds && (x == 0 || x * each % n != 0); ++x)
+      take(xcd_us((int)each, c, t, [&](int i) { return head[(x * each + i) % n]; }));
+  }
+  return 6.4f + us;
+}
+
+// The plan with the smallest estimate; cutting has to gain a twentieth, and a fifth where the pieces of several heads share an XCD and
+// the estimate is least sure (with a twentieth six of 280 such calls lost 3 % and more, up to 17, with a fifth one).  No plan: beyond two rounds of blocks, which even out by
+// themselves; where a part saves less of its block's walk than its exchange takes; where the jobs could not be dealt out to the
+// XCDs by heads any more (all of K and V in every L2: B1 H10 S3008 192/192 forward 74 us whole, 96 in such a plan).
 template <class Length> inline PartsPlan plan_parts(long heads, int T, Length&& length, const PartsCost& c) {
   PartsPlan best;
-  double least = 0.95 * parts_estimate_us(heads, T, best, length, c);
-  const int step = T < 16 ? 1 : T / 16;
+  if (T > kMostJobs || heads * T > 2l * kXcds * kXcdCus * c.blocks_per_cu) return best;
+  const float whole = parts_estimate_us(heads, T, best, length, c);
+  float least = (heads > kXcds && heads % kXcds != 0 ? 0.8f : 0.95f) * whole;
   for (int parts = 2; parts <= kMostParts; ++parts) {
-    for (int split = step; split <= T; split += step) {
-      if (length(split - 1) < 2 * parts || T + split * (parts - 1) > kMostJobs) break;     // shares of two tiles at least
-      const double us = parts_estimate_us(heads, T, {split, parts}, length, c);
+    const PartsTimes t(c, parts);
+    int split = 0;
+    for (const int sixteenths : {1, 2, 3, 4, 6, 8, 10, 12}) {
+      const int next = (T * sixteenths + 8) / 16 > 1 ? (T * sixteenths + 8) / 16 : 1;
+      if (next == split) continue;
+      split = next;
+      const int jobs = T + split * (parts - 1);
+      if (length(split - 1) < 2 * parts || jobs > kMostJobs) break;                        // shares of two tiles at least
+      if (length(split - 1) * t.alone * (parts - 1) < parts * (t.store + t.read)) break;
+      if (heads >= kXcds && heads * T % kXcds == 0 && heads * jobs % kXcds != 0) continue;
+      const float us = parts_estimate_us(heads, T, {split, parts}, length, c);
       if (us < least) {
         least = us;
-        best = {split, parts};
+        best = {split, parts, whole - us};
       }
     }
   }
   return best;
 }
+// What the plans of a call have to gain together for the launch that prepares them (5 us and the gap behind it).
+constexpr float kPrepareUs = 7.f;
 
 // The plans of the problems that a kind of launch met last, for all threads: 256 of them in sets of four, 10 KB.  A search takes
-// 1.6 us of the call at 512 rows, 9 at 1024, 21 at 2048, 50 at 4096 (forward), so a loop over a few dozen lengths must not
-// search for one of them twice.
+// 1 to 300 us of the call, so a loop over a few dozen lengths must not search for one of them twice.
 class PlanMemory {
   struct Entry {
     long heads = 0;
@@ -337,10 +410,11 @@ class PlanMemory {
 };
 
 // One kind of launch of a library (FIT: its kernel can): its plan, found once per problem, and the order of the plan's jobs.  MEMORY:
-// by how much the launch's tiles are slower than their matrix work (percent).
-template <bool FIT, int Br, int Bc, int Width, int Cols, int Nthreads, int Extra, bool ROWS, int MEMORY = 100>
+// by how much the launch's tiles are slower than their matrix work (percent).  NUMBERED: the kernel's output tile is in numbered registers.
+template <bool FIT, int Br, int Bc, int Width, int Cols, int Nthreads, int Extra, bool ROWS, bool NUMBERED, int MEMORY = 100>
 struct PartsLaunch {
-  static constexpr size_t kSlotBytes = part_floats<Br * Cols / (4 * Nthreads), Extra, Nthreads>() * sizeof(float);
+  static constexpr int kQuads = Br * Cols / (4 * Nthreads);
+  static constexpr size_t kSlotBytes = part_floats<kQuads, Extra, Nthreads>() * sizeof(float);
   static int blocks(int Seq_q, int Seq_k) { return ((ROWS ? Seq_q : Seq_k) + Br - 1) / Br; }
   static auto walk(int Seq_q, int Seq_k) {
     return [=](int rank) { return ROWS ? row_walk(rank, Br, Bc, Seq_q, Seq_k) : col_walk(rank, Br, Bc, Seq_q, Seq_k); };
@@ -349,7 +423,7 @@ struct PartsLaunch {
     if (!FIT) return {};
     static PlanMemory known;
     return known.get(heads, Seq_q, Seq_k, blocks_per_cu, [=] {
-      const PartsCost cost{MEMORY / 100.0 * 2.0 * Br * Bc * Width / 4.5e6, 256.0 * blocks_per_cu, Nthreads / 64, kSlotBytes};
+      const PartsCost cost{MEMORY / 100.0 * 2.0 * Br * Bc * Width / 4.5e6, Nthreads / 64, blocks_per_cu, kQuads / parts_at_once(kQuads, NUMBERED), kSlotBytes};
       return plan_parts(heads, blocks(Seq_q, Seq_k), walk(Seq_q, Seq_k), cost);
     });
   }

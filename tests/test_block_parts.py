@@ -16,9 +16,9 @@ RULE = [(op, d, c) for op in ("ret", "ret_bwd") for d in sorted(gfx950_space.RET
 SOURCE = r"""
 #include <hip/hip_runtime.h>
 #include "kernels/utils/block_parts.h"
-extern "C" int plan(long heads, int T, const int* walks, double tile_us, double places, int waves, size_t slot, int* split, int* parts, int* jobs) {
+extern "C" int plan(long heads, int T, const int* walks, double tile_us, int waves, int blocks_per_cu, int rounds, size_t slot, int* split, int* parts, int* jobs) {
   const auto walk = [=](int t) { return walks[t]; };
-  const aat::PartsPlan p = aat::plan_parts(heads, T, walk, aat::PartsCost{tile_us, places, waves, slot});
+  const aat::PartsPlan p = aat::plan_parts(heads, T, walk, aat::PartsCost{tile_us, waves, blocks_per_cu, rounds, slot});
   *split = p.split;
   *parts = p.parts;
   return aat::each_job(T, p, walk, [&](int n, int rank, int part) { jobs[n] = 8 * rank + (part < 0 ? 0 : part); });
@@ -65,7 +65,7 @@ def test_the_jobs_of_a_plan_are_complete_and_longest_first(lib):
     for _ in range(150):
         br, bc, waves = rng.choice(((128, 64, 4), (64, 64, 2), (64, 32, 2), (128, 32, 4)))
         sq, sk = 64 * rng.randint(1, 64), 64 * rng.randint(1, 64)
-        heads, rows, per_cu = rng.randint(1, 96), rng.randint(0, 1), rng.choice((1, 2, 4))
+        heads, rows, per_cu = rng.randint(1, 32), rng.randint(0, 1), rng.choice((1, 2, 4))
         cols, width = rng.choice(((64, 128), (128, 256), (256, 512), (256, 768), (512, 768)))
         want = _walks(bool(rows), br, bc, sq, sk)
         T = len(want)
@@ -74,7 +74,7 @@ def test_the_jobs_of_a_plan_are_complete_and_longest_first(lib):
         assert list(got) == want, (rows, br, bc, sq, sk)
         tile, slot = 2.0 * br * bc * width / 4.5e6, br * cols * 4
         c_split, c_parts, jobs = ctypes.c_int(), ctypes.c_int(), (ctypes.c_int * (T * MOST_PARTS))()
-        n = lib.plan(ctypes.c_long(heads), T, got, ctypes.c_double(tile), ctypes.c_double(256.0 * per_cu), waves, ctypes.c_size_t(slot),
+        n = lib.plan(ctypes.c_long(heads), T, got, ctypes.c_double(tile), waves, per_cu, br * cols // (256 * waves) // 4, ctypes.c_size_t(slot),
                      ctypes.byref(c_split), ctypes.byref(c_parts), jobs)
         split, parts = c_split.value, c_parts.value
         assert sorted(jobs[:n]) == sorted([8 * t + p for t in range(split) for p in range(parts)] + [8 * t for t in range(split, T)])
@@ -108,6 +108,25 @@ def test_the_libraries_report_the_room_of_their_parts(op):
                     cut += 1
         assert loaded.decay_workspace_size(1, 1, 16, 16, 1 << 40) == loaded.workspace_size(1, 1, 16, 16)      # no length it takes
     assert cut > 40
+
+
+# Problems measured whole and in the parts an estimate without the exchange's cost and the XCDs' shares of the jobs picked
+@pytest.mark.parametrize("op,dqk,dv,b,h,s,pays", [
+    ("ret_bwd", 192, 192, 1, 8, 832, False),       # 69 us whole, 90 in parts
+    ("ret_bwd", 256, 256, 4, 8, 1088, False),
+    ("ret", 256, 512, 1, 4, 512, False),           # 28.6, 35.6
+    ("ret", 256, 512, 5, 4, 1344, False),          # 64.4, 87.8
+    ("ret", 192, 192, 1, 10, 3008, False),         # 73.9, 95.7
+    ("ret", 128, 128, 1, 4, 4096, True),           # 80, 47
+    ("ret_bwd", 128, 128, 1, 4, 4096, True),       # 238, 173
+    ("ret_bwd", 64, 64, 1, 2, 4096, True),
+    ("ret", 256, 512, 1, 8, 2048, True),           # 101, 64
+    ("ret_bwd", 256, 512, 2, 8, 2112, True)])      # 257, 211
+def test_only_what_pays_is_cut(op, dqk, dv, b, h, s, pays):
+    cfg = gfx950_space.rule_ret_config(op, dqk, dv, b, h, s, s, True)
+    loaded = library.load(codegen.compile_config(cfg, MI355X(), timeout=600), op)
+    whole = loaded.workspace_size(b, h, s, s)
+    assert (loaded.decay_workspace_size(b, h, s, s, 1 << 40) > whole) == pays
 
 
 def test_a_library_without_the_question_is_asked_for_its_workspace_size():
