@@ -106,7 +106,13 @@ class Runtime:
             needs = self._need[(B, H, Sq, Sk, decay)] = (_wanted(self.config, size, B, H, Sq, Sk),
                                                          _provided(lib, self.config, size, B, H, Sq, Sk, decay))
         if needs[1] and (workspace is None or workspace.numel() * workspace.element_size() < needs[0]):
-            workspace = _grown(workspace, needs[1], q.device, keep=causal == "scanned")
+            try:
+                workspace = _grown(workspace, needs[1], q.device, keep=causal == "scanned")
+            except torch.cuda.OutOfMemoryError:
+                if needs[0] == needs[1]:
+                    raise
+                # no memory for the parts of a decay walk: the blocks are walked in one piece
+                workspace = _grown(workspace, needs[0], q.device, keep=False) if needs[0] else None
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
         if op in library.SCALED_OPS:

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import attention_autotuner_amd as aat
-from attention_autotuner_amd.autotuner import Runtime, gfx950_space, library
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space, library, runtime
 from oracle import ref_op, tolerance
 from test_retnet_ragged_gpu import _check, _problem
 
@@ -88,3 +88,24 @@ def test_a_workspace_of_workspace_size_bytes_is_used_as_it_is(op):
             ok, worst, ratio = tolerance.check_rounded_operand(got, ref, t)
             assert ok, (worst, ratio)
             got.fill_(7.0)
+
+
+def test_without_memory_for_the_parts_blocks_are_walked_in_one_piece(monkeypatch):
+    problem = b, h, sq, sk = 1, 2, 1088, 1088
+    q, k, v, _, _, lg = (t.cuda() for t in _problem(b, h, sq, sk, 256, 512, "decay", 41))
+    rt = Runtime(ARCH, _configs(256, 512, problem)[0])
+    assert _cuts(rt, problem)
+    o, r = torch.empty(b, h, sq, 512, device="cuda", dtype=torch.float16), torch.empty(b, h, sq, device="cuda")
+    rt.apply([q, k, v, lg, o, r], decay=True, workspace=torch.empty(rt.workspace_size(*problem), dtype=torch.uint8, device="cuda"))
+    whole, grown, asked = o.clone(), runtime._grown, []
+
+    def no_memory(workspace, need, device, keep):
+        asked.append(need)
+        if need > rt.workspace_size(*problem):
+            raise torch.cuda.OutOfMemoryError("no room")
+        return grown(workspace, need, device, keep)
+    monkeypatch.setattr(runtime, "_grown", no_memory)
+    o.fill_(7.0)
+    rt.apply([q, k, v, lg, o, r], decay=True)
+    torch.cuda.synchronize()
+    assert torch.equal(o, whole) and asked[0] > asked[1] == rt.workspace_size(*problem)
