@@ -53,7 +53,7 @@ AAT_DEV PartId causal_part(int wg, int grid, int T, bool last_is_longest, const 
 }
 
 // The share of [begin, end) that is this part's: every part of a block computes the same cuts.
-AAT_DEV void part_range(const PartId& id, int& begin, int& end) {
+__host__ __device__ inline void part_range(const PartId& id, int& begin, int& end) {
   const int n = end > begin ? end - begin : 0, first = begin;
   begin = first + n * id.part / id.parts;
   end = first + n * (id.part + 1) / id.parts;

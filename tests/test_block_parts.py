@@ -23,6 +23,7 @@ extern "C" int plan(long heads, int T, const int* walks, double tile_us, int wav
   *parts = p.parts;
   return aat::each_job(T, p, walk, [&](int n, int rank, int part) { jobs[n] = 8 * rank + (part < 0 ? 0 : part); });
 }
+extern "C" void share(int part, int parts, int* begin, int* end) { aat::part_range(aat::PartId{0, 0, part, parts, 0}, *begin, *end); }
 extern "C" void walks(int rows, int T, int Br, int Bc, int Seq_q, int Seq_k, int* out) {
   for (int t = 0; t < T; ++t) out[t] = rows ? aat::row_walk(t, Br, Bc, Seq_q, Seq_k) : aat::col_walk(t, Br, Bc, Seq_q, Seq_k);
 }
@@ -143,11 +144,20 @@ def test_a_library_without_the_question_is_asked_for_its_workspace_size():
     assert runtime._provided(New(), cfg, 4096, 1, 8, 512, 512, False) == 4096
 
 
-def test_shares_cover_the_walk():
-    for n in range(0, 40):
-        for parts in (2, 3, 4):
-            cuts = [n * p // parts for p in range(parts + 1)]           # part_range
-            assert cuts[0] == 0 and cuts[-1] == n and all(b - a in (n // parts, n // parts + 1) for a, b in zip(cuts, cuts[1:]))
+def test_shares_cover_the_walk(lib):
+    for first in (0, 3, 17):
+        for n in range(0, 70):
+            for parts in (1, 2, 3, 4):
+                begin, end, at = ctypes.c_int(), ctypes.c_int(), first
+                for part in range(parts):
+                    begin.value, end.value = first, first + n
+                    lib.share(part, parts, ctypes.byref(begin), ctypes.byref(end))
+                    assert begin.value == at and end.value - begin.value in (n // parts, n // parts + 1), (first, n, parts, part)
+                    at = end.value
+                assert at == first + n
+    begin, end = ctypes.c_int(5), ctypes.c_int(3)                       # an empty walk
+    lib.share(1, 2, ctypes.byref(begin), ctypes.byref(end))
+    assert begin.value == end.value == 5
 
 
 def test_lengths_in_turn_are_searched_for_once(lib):

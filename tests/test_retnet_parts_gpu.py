@@ -1,11 +1,11 @@
-"""RetNet with decay rates where the longest blocks are walked by several workgroups: lengths at which the library cuts, ragged and
-with either side the longer one, against the oracle's exact form under the rounded-operand rule of oracle/tolerance.py; the order in
-which the parts arrive must not show."""
+"""RetNet with decay rates where the longest blocks are walked by several workgroups: lengths at which the library cuts, whole and
+with a part of a last block, either side the longer one, against the oracle's exact form under the rounded-operand rule of
+oracle/tolerance.py; the order in which the parts arrive must not show."""
 import pytest
 import torch
 
 import attention_autotuner_amd as aat
-from attention_autotuner_amd.autotuner import Runtime, gfx950_space, library, runtime
+from attention_autotuner_amd.autotuner import Runtime, gfx950_space, library, prebuilt, prebuilt_extra, runtime
 from oracle import ref_op, tolerance
 from test_retnet_ragged_gpu import _check, _problem
 
@@ -34,6 +34,52 @@ def test_blocks_in_parts_against_the_oracle(dqk, dv):
     assert cut >= 2 or dqk == 64, "nothing was cut"          # a walk of 17 tiles of 64 columns is not worth an exchange
 
 
+# every RetNet shape that is built, the tuned ones among them: 2112 and 1984 rows leave half a block of 128, 2112 a quarter of one of 256
+BUILT = [c for c in prebuilt.shipping_set(ARCH, prebuilt_extra.parity_configs()) if c.operation in ("ret", "ret_bwd")]
+
+
+@pytest.mark.parametrize("problem", [(1, 2, 2112, 1984), (2, 1, 1984, 2112), (1, 1, 4096, 4096)])
+@pytest.mark.parametrize("dqk,dv", sorted({(c.Kd, c.D) for c in BUILT}))
+def test_every_shape_that_is_cut_against_the_oracle(dqk, dv, problem):
+    cut = [c for c in BUILT if (c.Kd, c.D) == (dqk, dv) and not (problem[2] % c.Bc or problem[3] % c.Bc) and _cuts(Runtime(ARCH, c), problem)]
+    if not cut:
+        pytest.skip("no shape of these head sizes is cut at these lengths")
+    _check(problem, dqk, dv, "decay", 950 + problem[2] % 7, [c for c in cut if c.operation == "ret"], [c for c in cut if c.operation == "ret_bwd"])
+
+
+@pytest.mark.parametrize("op,dqk,dv,br", [("ret", 256, 512, 128), ("ret", 256, 512, 64), ("ret_bwd", 256, 512, 128), ("ret_bwd", 256, 256, 128),
+                                          ("ret_bwd", 64, 64, 64)])
+@pytest.mark.parametrize("sq,sk", [(2112, 2112), (2112, 1984)])
+def test_the_library_cuts_with_the_room_it_asks_for_and_with_no_byte_less(op, dqk, dv, br, sq, sk):
+    """The arrival counts in the workspace say which launches were cut: all of them, blocks that are partial among them."""
+    problem = b, h, _, _ = 1, 2, sq, sk
+    cfg = next(c for c in gfx950_space.rule_ret_configs(op, dqk, dv) if c.Br == br)
+    rt = Runtime(ARCH, cfg)
+    lib = library.load(rt._path(), op)
+    q, k, v, do, _, lg = (t.cuda() for t in _problem(b, h, sq, sk, dqk, dv, "decay", 43))
+    r = torch.full((b, h, sq), 3.0, device="cuda")
+    out = [torch.empty_like(do)] if op == "ret" else [torch.empty_like(t) for t in (q, k, v)]
+    arrays = [q, k, v, lg, out[0], r] if op == "ret" else [q, k, v, lg, do, r, *out]
+    base, size = lib.workspace_size(*problem), lib.decay_workspace_size(*problem, 1 << 40)
+    buf = torch.full((size + 4096,), 0x5a, dtype=torch.uint8, device="cuda")
+    rt.apply(arrays, decay=True, workspace=buf[:size - 1])
+    assert bool((buf[base:] == 0x5a).all())
+    whole = [t.clone() for t in out]
+    rt.apply(arrays, decay=True, workspace=buf[:size])
+    torch.cuda.synchronize()
+    assert bool((buf[size:] == 0x5a).all())
+    launches = 1 if op == "ret" else 3
+    counts = buf[base:base + 256 * (launches + 1)].view(torch.int32).cpu().view(launches + 1, 64)
+    for launch in range(launches):
+        words = counts[launch].tolist()
+        arrived = words.count(words[0])
+        assert 2 <= words[0] <= 4 and arrived % h == 0 and words[:arrived] == [words[0]] * arrived, launch
+        assert set(words[arrived:]) <= {0, 0x5a5a5a5a}, launch
+    for cut, one in zip(out, whole):
+        assert not torch.equal(cut, one) or dqk == 64                     # other sums of fp32 values
+        assert ((cut.float() - one.float()).norm() / one.float().norm()).item() < 1e-3
+
+
 @pytest.mark.parametrize("dqk,dv", [(64, 64), (128, 128), (256, 512)])
 def test_parts_give_the_same_bits_every_time(dqk, dv):
     problem = b, h, sq, sk = 1, 4, 2112, 2112
@@ -50,6 +96,39 @@ def test_parts_give_the_same_bits_every_time(dqk, dv):
         outs = [o, r, *grads]
         first = first or outs
         assert all(torch.equal(a, x) for a, x in zip(first, outs))
+
+
+def test_a_captured_call_replays_its_parts():
+    """The counts are cleared and the orders handed out by the call itself: replays between eager work give the same bits."""
+    problem = b, h, sq, sk = 1, 2, 2112, 2112
+    q, k, v, do, _, lg = (t.cuda() for t in _problem(b, h, sq, sk, 256, 512, "decay", 47))
+    fwd, bwd = (Runtime(ARCH, c) for c in _configs(256, 512, problem))
+    assert _cuts(fwd, problem) and _cuts(bwd, problem)
+    o, r = torch.empty_like(do), torch.empty(b, h, sq, device="cuda")
+    grads = [torch.empty_like(t) for t in (q, k, v)]
+
+    def call():
+        fwd.apply([q, k, v, lg, o, r], decay=True)
+        bwd.apply([q, k, v, lg, do, r, *grads], decay=True)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for seed in range(4):
+        q.copy_(torch.randn(q.shape, generator=torch.Generator().manual_seed(seed)).half())
+        call()
+        torch.cuda.synchronize()
+        want = [t.clone() for t in (o, r, *grads)]
+        for t in (o, r, *grads):
+            t.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, x) for a, x in zip(want, (o, r, *grads))), seed
 
 
 @pytest.mark.parametrize("op", ["ret", "ret_bwd"])
