@@ -709,7 +709,7 @@ def rule_attn_backward_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
 # a pair is 1 to 4 % slower on the mean than the best of five to seven shapes, the shape that used to stand in at lengths
 # like 1344 (64 x 32 tiles, single buffers) 10 % at best and up to a half at d_v 512.  Where the line lies: two blocks of 64
 # rows share a CU as one block of 128 does, so up to 512 of them the dense walk keeps more CUs busy with the smaller ones
-# (B3 H8 S1344 256/256, 504 blocks: 43 us against 67 for 264 blocks of 128 rows); the blocks of a skipping walk differ in length
+# (B3 H8 S1344 256/256, 504 blocks: 66 us against 86 for 264 blocks of 128 rows on 32-row tiles, 102 on 64-row ones); the blocks of a skipping walk differ in length
 # and balance at half as many.  Backward: blocks of 64 kv rows lead everywhere up to d 192 for the same reason, with dS stored.
 #   forward  (Br, Bc, K buffers, V buffers, threads, waves per SIMD)
 #   backward (Br, Bc, threads, buffers of the dV pass' two streams, of the others', waves per SIMD, ds_rows)

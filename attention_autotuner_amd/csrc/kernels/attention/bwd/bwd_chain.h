@@ -74,9 +74,10 @@ struct AttnBwdChain {
 // x1, x2: resident-side matrices (COL: k, v; ROW: q, dO); y1, y2: streamed-side matrices (COL: q, dO;
 // ROW: k, v); all [B*H, S, width] fp16.  COL writes out1 = dV and out2 = dK; ROW writes out2 = dQ.
 // Row statistics [B*H, seq_q] fp32: the row kernel runs first.  It holds dO in registers anyway, so it reads O once on top, makes
-// delta = rowsum(dO * O) and lse2 = lse * log2(e) of its rows and leaves both for the column kernel (a kernel of their own read dO
-// once more, 22 us of 767 for forward and backward at B4 H32 S2048 d 128 causal, 752 without it).  ROW takes o and lse, COL neither.
-//  c2 = softmax_scale * log2(e); out_scale = softmax_scale.
+// delta = rowsum(dO * O) and lse2 = lse * log2(e) of its rows and leaves both for the column kernel.  A kernel of their own read dO
+// once more, 22 us; forward and backward at B4 H32 S2048 d 128 causal with and without it, both in turn on three cards: 767 and 752,
+// 753 and 738, 798 and 793 us.  ROW takes o and lse, COL neither.
+// c2 = softmax_scale * log2(e); out_scale = softmax_scale.
 // OUTS (COL only): 3 = both outputs, 1 = dV only (x2, delta and out2 are not touched), 2 = dK only.
 // GEN: lengths that are multiples of 32 and not of the tiles.  Missing 32-row groups of the last resident block load rows
 // that exist, and are not stored; a wave that owns none that exist keeps the block's copies and barriers going and computes

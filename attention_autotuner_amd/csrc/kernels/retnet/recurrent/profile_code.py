@@ -102,8 +102,8 @@ bool split_pays(long bh, int vdim, int block_kdim, bool wide) {{
   return split < passes + add;
 }}
 
-// Two launches: the decay factors of every (head, chunk), beyond 128 key dims in the launch that makes P, then the scan.  A value slice of 128 dims per
-// block halves the traffic of q and k; where it would leave most of the compute units without a block or vdim does not
+// Two launches: the decay factors of every (head, chunk), beyond 128 key dims in the launch that makes P, then the scan.  A value
+// slice of 128 dims per block halves the traffic of q and k; where it would leave most of the compute units without a block or vdim does not
 // allow it, 64 key dims take slices of 64 and more of them the split kernel, which split_pays() may choose elsewhere too.
 hipError_t launch(const float* q, const float* k, const float* v, const float* decay, float* out, int batch, int heads,
                   int kdim, int vdim, int l, int block_kdim, char* workspace, hipStream_t stream) {{

@@ -73,8 +73,8 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
               "both access patterns of the fp32 chunk tiles are free of LDS bank conflicts");
 
 // ---------------------------------------------------------------------------------------------------
-// Decay factors of one (head, chunk), computed once by retnet_recurrent_factors and shared by every
-// batch entry and value slice.  Vector-ALU instructions do not overlap fp32 MFMAs on this hardware, so
+// Decay factors of one (head, chunk), computed once, by retnet_recurrent_factors or, beyond 128 key dims, by the first blocks of
+// retnet_recurrent_pmat, and shared by every batch entry and value slice.  Vector-ALU instructions do not overlap fp32 MFMAs on this hardware, so
 // everything that depends on the decay alone is taken out of the main kernel.
 //
 // State is kept as T = State / lambda with a per-head scalar lambda (the product of the decays since
@@ -82,7 +82,8 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
 //   O^T = (p_n lambda) (T^T Q) + V P,      T += K diag(w / lambda') V^T,   lambda' = A lambda.
 // When |lambda'| leaves [2^-40, 2^40] (or is zero) the record says so: the kernel then multiplies T by
 // `scale` = A lambda once and lambda restarts at 1.
-//   [0, 4096)     D[g][lane][e]   = prod_{m<j<=n} a_j for m = 8g+4h+e, n = lane%32, h = lane/32 (0 for m > n)
+//   [0, 4096)     D[g][lane][e]   = prod_{m<j<=n} a_j for m = 8g+4h+e, n = lane%32, h = lane/32 (0 for m > n); not written
+//                                   by retnet_recurrent_pmat, which multiplies P by it, and not read after it
 //   [4096, 4224)  W[h][g][e]      = w_m / lambda'      (w_m alone on a rescale)
 //   [4224, 4352)  PNL[n]          = p_n lambda
 //   [4352, 4360)  rescale flag (uint32), scale (float)
@@ -90,8 +91,8 @@ constexpr int kRecFactorBytes = 5120;
 constexpr int kRecFactorW = 4096, kRecFactorPnl = 4224, kRecFactorFlag = 4352;
 
 // decay [H][L] -> factors [H][L/32][kRecFactorBytes], for part `part` of `parts` of head `head`'s sequence, by a block of
-// WAVES waves with 8 bytes of dynamic LDS per chunk.  WITH_D: the D of the records too.  A head's chunks are shared out over the blocks of its row and the waves of a block.  Each block
-// walks lambda from the first chunk to its own last one by itself (a product per thread and chunk, then one wave chains
+// WAVES waves with 8 bytes of dynamic LDS per chunk.  WITH_D: the D of the records too.  A head's chunks are shared out over the
+// blocks of its row and the waves of a block.  Each block walks lambda from the first chunk to its own last one by itself (a product per thread and chunk, then one wave chains
 // them); lambda is known before a record is written, so a record is written once.
 //
 // Bound by latency: a load, the walk (one dependent multiplication and comparison per chunk), a load and 32 products, a store.
@@ -520,8 +521,10 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
 //
 // The first heads * parts blocks of the launch make the records of the decay factors instead, 8 bytes of dynamic LDS per chunk
 // (the kernel below waits for both anyway): D, which P needs, depends on its own chunk only, and every wave forms its 8 rows
-// while its loads are under way, in the order of the records.  B2 H8 L1056 256/512: 94.4 us a call with a
-// launch of its own for the records (5.6 us and the gap behind it), 88.6 like this.
+// while its loads are under way, in the order of the records.  B2 H8 L1056 256/512: 94.4 us a call with a launch of its own for the
+// records (5.6 us and the gap behind it), 88.6 like this.  So also in long sequences, where the room of the records' walk in every
+// block's LDS (48 KB with the static part at 131072 positions) takes places from the P blocks: B1 H8 L65536 256/128 5110 and 4988,
+// B1 H8 L131072 256/64 10210 and 9948, B1 H2 L131072 192/64 9938 and 9871.
 template <int KD>
 __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __restrict__ q, const float* __restrict__ k,
                                                              const float* __restrict__ decay, char* __restrict__ factors,

@@ -348,9 +348,9 @@ template <class Length> inline float parts_estimate_us(long heads, int T, const 
   return 6.4f + us;
 }
 
-// The plan with the smallest estimate; cutting has to gain a twentieth, and a fifth where the pieces of several heads share an XCD and
-// the estimate is least sure (with a twentieth six of 280 such calls lost 3 % and more, up to 17, with a fifth one).  No plan: beyond two rounds of blocks, which even out by
-// themselves; where a part saves less of its block's walk than its exchange takes; where the jobs could not be dealt out to the
+// The plan with the smallest estimate; cutting has to gain a twentieth, and a fifth where the pieces of several heads share an XCD
+// and the estimate is least sure (with a twentieth six of 280 such calls lost more than 3 %, up to 17, with a fifth two, up to 7).
+// No plan: beyond two rounds of blocks, which even out by themselves; where a part saves less of its block's walk than its exchange takes; where the jobs could not be dealt out to the
 // XCDs by heads any more (all of K and V in every L2: B1 H10 S3008 192/192 forward 74 us whole, 96 in such a plan).
 template <class Length> inline PartsPlan plan_parts(long heads, int T, Length&& length, const PartsCost& c) {
   PartsPlan best;

@@ -17,7 +17,10 @@ since; 18 us per forward at H 8, S 2048).
 ``mask[h, i, j] = gamma_h^(i + S_kv - S_q - j)`` on and below that diagonal and 0 above it: the mask is
 built in registers from ``gamma`` ([H], 0.5 <= gamma_h <= 1) instead of being streamed from a
 [H, S_q, S_kv] tensor, and tiles above the diagonal are skipped.  The reference has no such entry (it
-always streams the tensor, python/ops/retnet_interface.py:26-31).
+always streams the tensor, python/ops/retnet_interface.py:26-31).  Where a problem would leave the chip partly idle, the longest
+blocks of rows are walked in parts whose fp32 sums are added up at the end: the same call gives the same bits every time, but
+how the blocks are cut depends on batch size, heads and lengths, and a (batch, head) of another call may differ by the order of
+those additions.
 """
 import torch
 

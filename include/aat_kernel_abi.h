@@ -146,8 +146,8 @@ int kernel_entry_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_
 /* Flash-attention backward: dq, dk, dv from q, k, v, o, dO and the forward's lse (see kernel_entry_lse).
  * No counterpart in the reference, whose MultiHeadAttnFunc.backward is an empty stub
  * (python/ops/attention_interface.py:37-58, README.md:107); this is the entry point that stub would bind.
- * Seq_q and Seq_k must both be multiples of the library's Br and Bc.  workspace_size() bytes of
- * workspace are required (two fp32 values per query row); dq, dk, dv are fully overwritten. */
+ * Seq_q and Seq_k are any multiples of 32.  workspace_size() bytes of workspace are required (two fp32 values per query
+ * row); dq, dk, dv are fully overwritten. */
 float profile_ex(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* dO, float* lse,
                  aat_half* dq, aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k,
                  float softmax_scale, int causal, void* workspace, size_t workspace_bytes, void* stream);
