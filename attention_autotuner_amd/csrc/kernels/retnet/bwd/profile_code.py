@@ -187,6 +187,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_hal
 hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* dO, float* r,
                         aat_half* dq, aat_half* dk, aat_half* dv, int B, int H, int Seq_q, int Seq_k, void* workspace,
                         size_t workspace_bytes, hipStream_t stream) {{
+  aat::touch_thread_storage();
   return launch_passes<true>(q, k, v, nullptr, log2_gamma, dO, r, dq, dk, dv, B, H, Seq_q, Seq_k, aat::MaskWalk(), workspace, workspace_bytes, stream);
 }}
 }}  // namespace

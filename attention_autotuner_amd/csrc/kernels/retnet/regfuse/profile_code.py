@@ -62,6 +62,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* mask, aat_hal
 // Decay-mask variant: the mask is gamma_h^(q + Seq_k - Seq_q - kv) below the diagonal, zero above it.
 hipError_t launch_decay(aat_half* q, aat_half* k, aat_half* v, const float* log2_gamma, aat_half* o, float* r, int B,
                         int H, int Seq_q, int Seq_k, void* workspace, size_t workspace_bytes, hipStream_t stream) {{
+  aat::touch_thread_storage();
   static const hipError_t lds_ok = allow_kernels<true>();
   if (lds_ok != hipSuccess) return lds_ok;
   const size_t at = workspace_size(B, H, Seq_q, Seq_k);

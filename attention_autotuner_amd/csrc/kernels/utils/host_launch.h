@@ -22,6 +22,15 @@ template <class K> inline hipError_t allow_lds(K kernel, int bytes) {
                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
+// Touches thread-local storage of this library, at the start of a call.  After a library with such storage has been loaded (the HIP
+// runtime loads some late), glibc 2.35 sends every access of the thread to the storage of older ones through its slow path until
+// the thread touches a newer one's, and torch looks its allocator, device and stream up there: torch.empty 1.09 us after a call
+// with this, 1.35 without, a whole decay call of 24 blocks (host-bound) 13.3 and 15.5.
+inline void touch_thread_storage() {
+  static thread_local volatile unsigned calls = 0;
+  calls = calls + 1;
+}
+
 // `launch()` enqueues one complete invocation on `stream` and returns a hipError_t.
 template <class F> inline float timed_mean_ms(hipStream_t stream, F launch) {
   hipEvent_t start, stop;

@@ -165,3 +165,13 @@ def test_lengths_in_turn_are_searched_for_once(lib):
     problems = [(h, s, s, 1) for _ in range(3) for s in lengths for h in (8, 32)] + [(8, 64, 128, 1), (8, 64, 128, 2), (8, 64, 128, 1)] * 5
     flat = (ctypes.c_int * (4 * len(problems)))(*[x for p in problems for x in p])
     assert 128 + 2 <= lib.searches(flat, len(problems)) <= 128 + 2 + 16          # sets of four: a few problems push each other out
+
+
+@pytest.mark.parametrize("op", ["ret", "ret_bwd"])
+def test_decay_calls_touch_thread_storage_of_their_library(op):
+    """... which is what keeps torch's own accesses off glibc's slow path on the host (utils/host_launch.h)."""
+    cfg = next(c for o, d, c in RULE if o == op and d == (64, 64))
+    segments = subprocess.run(["readelf", "-lW", codegen.compile_config(cfg, MI355X(), timeout=600)], check=True, capture_output=True, text=True).stdout
+    assert " TLS " in segments
+    entry = codegen.render(cfg).split("hipError_t launch_decay(")[1].split("\n}")[0]
+    assert "aat::touch_thread_storage();" in entry
