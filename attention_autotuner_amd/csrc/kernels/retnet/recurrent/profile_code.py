@@ -96,8 +96,8 @@ bool split_pays(long bh, int vdim, int block_kdim, bool wide) {{
   if (!wide && block_kdim > 64) return true;
   const double pmat = block_kdim > 128 ? 2.0 * bh * block_kdim * 32 * 4 / 5e6 : 0.0;   // P: q and k once more at 5 TB/s
   const double split = pmat + (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : block_kdim == 192 ? 2.45 : 2.6) * rounds(bh * (vdim / 32), kUnits);
-  if (!wide) return split < 3.05 * rounds(bh * (vdim / 64), 2 * kUnits);
-  const double passes = (block_kdim / 128 * 5.8 + block_kdim / 64 % 2 * 4.1) * rounds(bh * (vdim / 128), kUnits);
+  if (!wide) return split < 2.5 * rounds(bh * (vdim / 64), 2 * kUnits);
+  const double passes = (block_kdim / 128 * 4.8 + block_kdim / 64 % 2 * 3.25) * rounds(bh * (vdim / 128), kUnits);
   const double add = block_kdim > 128 ? 3.0 * bh * vdim * 32 * 4 / 8e6 : 0.0;      // two reads and a write, partly from the cache
   return split < passes + add;
 }}

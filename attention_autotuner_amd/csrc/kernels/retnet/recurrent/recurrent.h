@@ -4,14 +4,14 @@
 // (decay, k*v) pairs, one scan per (key dim, value dim) pair, launched by retnet_recurrent_fwd :427-463),
 // same tensors: q, k [B, H, kdim, L], v, out [B, H, vdim, L] (sequence contiguous), decay [H, L].
 //
-// The scan is evaluated chunk by chunk on the fp32 matrix cores instead of element by element on the
+// The scan is evaluated chunk by chunk on the matrix cores instead of element by element on the
 // vector ALU.  For a chunk of 32 positions, with State = S at the end of the previous chunk:
 //   S^T[m][n]  = sum_kd K[kd][m] Q[kd][n]                          (keys m x queries n)
 //   P[m][n]    = S^T[m][n] * prod_{m<j<=n} a_j  (0 for m > n)      exact running products, no logarithms
 //   O^T[vd][n] = p_n * sum_kd State[kd][vd] Q[kd][n] + sum_m V[vd][m] P[m][n],   p_n = prod_{j<=n} a_j
 //   State[kd][vd] = A * State[kd][vd] + sum_m K[kd][m] w_m V[vd][m],   w_m = prod_{j>m} a_j, A = prod_j a_j
 // which is 5 flops per (position, kd, vd) -- what the element-wise recurrence itself costs -- but at the
-// MFMA rate.  No logarithms or divisions: zero and negative decays behave as in the recurrence.
+// matrix cores' rate.  No logarithms or divisions: zero and negative decays behave as in the recurrence.
 //
 // One block owns one (batch, head) and a slice of DVS value dims; wave w owns value dims [32w, 32w+32) of
 // the slice: its State tiles (KD x 32, fp32, in registers for the whole sequence) and its rows of O^T.
@@ -74,8 +74,7 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
 
 // ---------------------------------------------------------------------------------------------------
 // Decay factors of one (head, chunk), computed once, by retnet_recurrent_factors or, beyond 128 key dims, by the first blocks of
-// retnet_recurrent_pmat, and shared by every batch entry and value slice.  Vector-ALU instructions do not overlap fp32 MFMAs on this hardware, so
-// everything that depends on the decay alone is taken out of the main kernel.
+// retnet_recurrent_pmat, and shared by every batch entry and value slice.
 //
 // State is kept as T = State / lambda with a per-head scalar lambda (the product of the decays since
 // the last rescale), so that a chunk's decay does not have to be multiplied into the KD x DVS state:
@@ -178,64 +177,179 @@ __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(co
   rec_factor_records<kRecFactorWaves, true>(decay, factors, L, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
+// ---------------------------------------------------------------------------------------------------
+// Operands of a contraction over 16 key dims or positions (one k-step): element j of half h stands for index 8(j/4)+4h+j%4
+// of the step, the rows that registers 8s .. 8s+7 of a C tile hold, so the registers of one product are an operand of the next.
+//
+// FP32 = false, taken first: an fp32 value is the sum of three bf16 ones (hi, mid, lo: 8 significant bits each, rounded to
+// nearest), and a product the sum of the six largest of their nine, on v_mfma_f32_32x32x16_bf16: 6 x 32 cycles for 16 indices
+// where v_mfma_f32_32x32x2_f32 takes 8 x 64.  What is left out is below 2^-23 of a product and 2^-26 of it on average, less than
+// the rounding of one fp32 addition; bf16 has the range of fp32, so nothing is scaled.  A sum is rounded six times per k-step
+// instead of eight, and results are no further from 64 bits than with fp32 products: relative 2-norm at B8 H32 L512 128/128
+// 7.58e-7 -> 7.26e-7, most of it from the products of decays both have in common; with decays in [0.5, 1] 1.28e-7 -> 9.5e-8; the
+// same with normal or positive values, magnitudes spread over 12 decades along the key dims, or products around 1e-24.
+// An infinity (or a value that rounds to one in bf16) becomes a NaN in its parts: a block that finds a value in its output that
+// is not finite runs once more from the start with FP32 = true.
+// FP32 = true: eight fp32 values and eight v_mfma_f32_32x32x2_f32.
+template <bool FP32> struct RecOp {
+  static constexpr int kParts = FP32 ? 2 : 3;
+  u4v p[kParts];
+};
+typedef __bf16 rec_bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 rec_bf2 __attribute__((ext_vector_type(2)));
+
+// ALONE: where no matrix instruction is under way the remainder x - hi is one v_dot2_f32_bf16 (times -1 and 0, exact) instead of a
+// shift or mask and a subtraction; it shares the matrix core's issue path and waits there for a matrix instruction to end.
+template <bool FP32, bool ALONE = false> AAT_DEV RecOp<FP32> rec_op(f4v a, f4v b) {
+  RecOp<FP32> o;
+  if constexpr (FP32) {
+    __builtin_memcpy(&o.p[0], &a, 16);
+    __builtin_memcpy(&o.p[1], &b, 16);
+  } else {
+    // -1 in one half and 0 in the other; in scalar registers, for as constants the compiler writes both as the inline -1.0
+    uint32_t minus1_lo = 0x0000bf80u, minus1_hi = 0xbf800000u;
+    if constexpr (ALONE) asm("" : "+s"(minus1_lo), "+s"(minus1_hi));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float x0 = i < 2 ? a[2 * i] : b[2 * i - 4], x1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const f2v x = {x0, x1};
+        const rec_bf2 r = __builtin_convertvector(x, rec_bf2);
+        uint32_t bits;
+        __builtin_memcpy(&bits, &r, 4);
+        o.p[t][i] = bits;
+        if constexpr (ALONE) {
+          if (t < 2) {
+            x0 = __builtin_amdgcn_fdot2_f32_bf16(r, __builtin_bit_cast(rec_bf2, minus1_lo), x0, false);
+            x1 = __builtin_amdgcn_fdot2_f32_bf16(r, __builtin_bit_cast(rec_bf2, minus1_hi), x1, false);
+          }
+        } else if (t < 2) {
+          x0 -= __uint_as_float(bits << 16);
+          x1 -= __uint_as_float(bits & 0xffff0000u);
+        }
+      }
+    }
+  }
+  return o;
+}
+AAT_DEV f4v rec_quarter(const f16v& c, int v0) { return f4v{c[v0], c[v0 + 1], c[v0 + 2], c[v0 + 3]}; }
+template <bool FP32> AAT_DEV RecOp<FP32> rec_op_of_c(const f16v& c, int s) {      // registers 8s .. 8s+7
+  return rec_op<FP32>(rec_quarter(c, 8 * s), rec_quarter(c, 8 * s + 4));
+}
+// c += a b over the 16 indices of the step, the small partial products first.
+template <bool FP32> AAT_DEV f16v rec_mma(const RecOp<FP32>& a, const RecOp<FP32>& b, f16v c) {
+  if constexpr (FP32) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c = mfma_32x32x2_f32(__uint_as_float(a.p[j >> 2][j & 3]), __uint_as_float(b.p[j >> 2][j & 3]), c);
+  } else {
+    constexpr int ai[6] = {2, 0, 1, 1, 0, 0}, bi[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+      rec_bf8 x, y;
+      __builtin_memcpy(&x, &a.p[ai[t]], 16);
+      __builtin_memcpy(&y, &b.p[bi[t]], 16);
+      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+    }
+  }
+  return c;
+}
+// Keeps an operand's making where it is written: the compiler moves it to its use otherwise, past a branch in between.
+template <bool FP32> AAT_DEV void rec_pin(RecOp<FP32>& o) {
+#pragma unroll
+  for (int p = 0; p < RecOp<FP32>::kParts; ++p) asm volatile("" : "+v"(o.p[p]));
+}
+// Order of a region of the program: READS LDS reads, then each of a k-step's six matrix instructions with VALU vector instructions behind
+// it, which issue while it runs.  Ends the region.
+template <bool FP32, int READS, int VALU> AAT_DEV void rec_interleave() {
+  if constexpr (!FP32) {
+    if constexpr (READS > 0) __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, VALU, 0);
+    }
+  }
+  sched_fence();
+}
+// The largest bit patterns seen, as signed and as unsigned numbers: beyond the infinities' once a value was not finite.
+struct RecFinite {
+  int32_t pos = 0;
+  uint32_t neg = 0;
+  AAT_DEV void see(const f16v& x) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t b = __float_as_uint(x[i]);
+      pos = max(pos, (int32_t)b);
+      neg = max(neg, b);
+    }
+  }
+  AAT_DEV bool broken() const { return pos >= 0x7f800000 || neg >= 0xff800000u; }
+};
+// Whether any lane of the block says so; also a barrier in front of what the caller does with LDS next.
+AAT_DEV bool rec_any_wave(char* smem, bool x) {
+  const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  int* const flags = reinterpret_cast<int*>(smem);
+  block_sync();
+  flags[wave] = __ballot(x) != 0ull;
+  block_sync();
+  int any = 0;
+  for (int i = 0; i < waves; ++i) any |= flags[i];
+  block_sync();
+  return __builtin_amdgcn_readfirstlane(any) != 0;
+}
+
 template <int KD, int DVS>
 struct RetRecurrent {
   static constexpr int kChunk = 32;                       // positions per step
   static constexpr int kWaves = DVS / 32;
-  static constexpr int kThreads = kWaves * 64 + 64;        // the matrix waves plus one wave that moves the data
+  static constexpr int kThreads = kWaves * 64 + 128;       // the matrix waves plus two that move the data
   static constexpr int kKB = KD / 32;                     // State tiles per wave
-  static constexpr int kGroups = KD / 8;                  // groups of 8 key dims (one (h, e) sweep of a step)
-  static constexpr int kGroupsPerWave = kGroups / kWaves; // share of one wave in the S^T contraction
+  static constexpr int kSteps = KD / 16;                  // k-steps over the key dims
+  static constexpr int kUnits = kSteps / kWaves;          // of them, a wave's share of S^T and of the operands made for all waves
   static constexpr int kKTile = KD * 128, kVTile = DVS * 128;
   static constexpr int kQOff = kKTile, kVOff = 2 * kKTile, kFOff = 2 * kKTile + kVTile;
-  static constexpr int kStage = kFOff + kRecFactorBytes;  // K, Q, V tiles and the decay factors of one chunk
-  static constexpr int kRed = kWaves * 4096;              // one partial S^T tile per wave
-  static constexpr int kOutOff = 2 * kStage + kRed;       // per wave: its 32 x 32 output tile, staged for 16-byte stores
-  static constexpr int kSmemBytes = kOutOff + kWaves * 4096;
+  static constexpr int kStage = kFOff + kRecFactorBytes;  // K, Q, V tiles and decay factors of one chunk
+  static constexpr int kOpOff = 2 * kStage;               // operands of Q, then of K, made for all waves: 3 parts of 1 KB per unit
+  static constexpr int kSmemBytes = kOpOff + 2 * kSteps * 3072;
+  // Once the waves have taken a chunk over, their partial S^T tiles lie where K was (and Q: 64 key dims, four waves), and each wave's
+  // output tile where its rows of V were.
+  static_assert(kWaves * 4096 <= (KD == 64 && DVS == 128 ? 2 : 1) * kKTile, "partial tiles");
   static_assert(KD % 32 == 0 && DVS % 64 == 0 && DVS <= 256, "tile shape");
-  static_assert(kGroups % kWaves == 0, "the S^T contraction must split evenly over the waves");
-  static_assert(kFOff + kRecFactorBytes <= 65536, "tile offsets go into the 16-bit offset field of the LDS reads");
+  static_assert(kSteps % kWaves == 0, "the waves share the k-steps evenly");
   static_assert(kSmemBytes <= 160 * 1024, "LDS");
+  // Byte offset, from kOpOff, of part p of the operand of unit u (Q: k-step u over the key dims; K: k-step u%2 over the positions of State tile u/2).
+  AAT_DEV static constexpr int op_at(bool of_q, int u, int p) { return ((of_q ? 0 : kSteps) + u) * 3072 + p * 1024; }
 };
-
-// LDS reads and stores issued by hand so that their waits can be counted: the compiler answers every
-// dependency on an LDS load with lgkmcnt(0) while an LDS-DMA copy is in flight, and here one is in
-// flight all the time.  LDS operations retire in order, so "at most N younger ones outstanding" is enough.
-AAT_DEV float lds_read_f1_async(uint32_t base, int imm) {
-  float v;
-  asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(base), "i"(imm));
-  return v;
-}
-template <int N, class V> AAT_DEV void lds_wait_younger_f(V& v) {
-  static_assert(N >= 0 && N < 16, "lgkmcnt is a 4-bit counter");
-  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N));
-}
 
 // q, k: [B*H][kdim][L]; v, out: [B*H][vdim][L]; factors: output of retnet_recurrent_factors.  Contracts
 // the first KD key dims (the reference's block_kdim, reference recurrent.h:290,427).  Grid (vdim / DVS, B*H).
-// Compiled for two waves per SIMD's worth of registers (256): then every MFMA takes and leaves its
-// operands in vector registers and nothing has to be moved between register classes.
 //
-// Waves 0 .. DVS/32-1 do the arithmetic; the last wave of the block only moves data: it issues every
-// LDS-DMA copy of the next chunk and stores the previous chunk's output tiles from their LDS staging
-// area.  An LDS-DMA or store instruction holds its wave for 16 to 50 cycles (thousands for a burst), and a
-// matrix wave is the only one on its SIMD: whatever it spends issuing memory instructions the matrix core
-// idles.  The data wave has nothing else to do.
-template <int KD, int DVS>
-__global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void retnet_recurrent_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const char* __restrict__ factors, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
+// Waves 0 .. DVS/32-1 do the arithmetic; the last two waves of the block only move data: they issue every LDS-DMA copy and store
+// the previous chunk's output tiles from their LDS staging area.  An LDS-DMA or store instruction holds its wave for 16 to 50
+// cycles, which a matrix wave would spend with the matrix core idle.
+//
+// A chunk has two phases.  In the first a wave reads its share of K and Q, makes their operands (44 vector instructions for eight
+// values, so once per block and not once per wave) and leaves them in LDS; behind a barrier every wave reads all of them.  The
+// second is a sequence of k-steps: six matrix instructions, with the vector instructions that make a later k-step's operand of
+// T, V or P between them (7 fit behind one) and the LDS reads of the next k-step.
+//
+// Bound by the board's power: 8000 cycles a chunk (120 matrix instructions = 3840, some 950 vector instructions and 450 KB through LDS)
+// run at 2.35 GHz without the memory stream and at 1.8 GHz with it; the stream by itself takes 270 us of the 310 at B8 H32 L2048
+// 128/128.  Whole calls, fp32 products and one data wave before, this kernel now: B8 H32 L2048 128/128 369 -> 310 us (L512 100 -> 77),
+// 64/128 235 -> 213, 64/64 206 -> 164.  Tried and not kept: two
+// chunks' copies under way at all times, at the price of factors read from memory and a fourth barrier, 331 us; non-temporal copies or
+// stores +-3 %.
+template <bool FP32, int KD, int DVS>
+AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                      const char* __restrict__ factors, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
   using T = RetRecurrent<KD, DVS>;
-
-  extern __shared__ __align__(16) char smem[];
+  using Op = RecOp<FP32>;
 
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.y, h = bh % heads;
   const int nchunk = L / T::kChunk;
-  const char* qg = reinterpret_cast<const char*>(q + (size_t)bh * kdim * L);
-  const char* kg = reinterpret_cast<const char*>(k + (size_t)bh * kdim * L);
-  const char* vg = reinterpret_cast<const char*>(v + ((size_t)bh * vdim + (size_t)blockIdx.x * DVS) * L);
   const char* fg = factors + (size_t)h * nchunk * kRecFactorBytes;
   const int pitch = L * 4;
   // Output: a wave's O^T tile goes through LDS so that it leaves as four 16-byte-per-lane stores (8 rows
@@ -244,42 +358,41 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
   // fall on different halves of the banks.
   const int orl = lane >> 3, occ = lane & 7;
 
-  if (wave == T::kWaves) {
-    // ================================ data wave =================================================
+  if (wave >= T::kWaves) {
+    // ================================ data waves ================================================
     // LDS-DMA of a tile of 128-byte rows: instruction i covers positions 8i .. 8i+7, lane l position
     // 8i + l/8, chunk slot l%8.  The source row is rec_pos(position), the source chunk the slot XOR the
     // position's slot term (whose high bit is the parity of i).  Every address below is a scalar base that
-    // moves with the chunk plus a per-lane 32-bit offset computed here once: the loop of this wave must not
-    // contain a single vector instruction -- a vector instruction has to find a gap between the fp32 MFMAs
-    // of the matrix wave that shares the SIMD, and a copy that waits for one took 175 cycles to issue.
+    // moves with the chunk plus a per-lane 32-bit offset computed here once.
+    const char* qg = reinterpret_cast<const char*>(q + (size_t)bh * kdim * L);
+    const char* kg = reinterpret_cast<const char*>(k + (size_t)bh * kdim * L);
+    const char* vg = reinterpret_cast<const char*>(v + ((size_t)bh * vdim + (size_t)blockIdx.x * DVS) * L);
     constexpr int kTileOps = (KD > DVS ? KD : DVS) / 8;
     uint32_t toff[kTileOps];
 #pragma unroll
     for (int i = 0; i < kTileOps; ++i)
       toff[i] = (uint32_t)((8 * i + rec_pos(orl)) * pitch + (occ ^ (((i & 1) << 2) | (orl >> 1))) * 16);
-    const uint32_t lane16off = lane * 16;
     auto dma_one = [&](const char* g_uniform, uint32_t lane_off, char* lds) {   // written out: scalar base + lane offset form
       const uint64_t base = (uint64_t)(uintptr_t)g_uniform;
       const uint32_t dst = (uint32_t)(uintptr_t)(AAT_AS3 char*)lds;
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                    :: "v"(lane_off), "s"(base), "s"(dst) : "memory", "m0");
     };
-    // K and Q are needed first (the partial S^T opens a chunk); V and the decay factors follow.
-    auto dma_kq = [&](int c, int stage) {
-      char* s = smem + stage * T::kStage;
-      const size_t col = (size_t)c * T::kChunk * 4;
+    auto dma_k = [&](int c, int stage) {
 #pragma unroll
-      for (int i = 0; i < KD / 8; ++i) dma_one(kg + col, toff[i], s + i * 1024);
+      for (int i = 0; i < KD / 8; ++i) dma_one(kg + (size_t)c * T::kChunk * 4, toff[i], smem + stage * T::kStage + i * 1024);
+    };
+    auto dma_q = [&](int c, int stage) {
 #pragma unroll
-      for (int i = 0; i < KD / 8; ++i) dma_one(qg + col, toff[i], s + T::kQOff + i * 1024);
+      for (int i = 0; i < KD / 8; ++i) dma_one(qg + (size_t)c * T::kChunk * 4, toff[i], smem + stage * T::kStage + T::kQOff + i * 1024);
     };
     auto dma_vf = [&](int c, int stage) {
-      char* s = smem + stage * T::kStage;
+      char* const s = smem + stage * T::kStage;
 #pragma unroll
       for (int i = 0; i < DVS / 8; ++i) dma_one(vg + (size_t)c * T::kChunk * 4, toff[i], s + T::kVOff + i * 1024);
-      const char* f = fg + (size_t)c * kRecFactorBytes;
 #pragma unroll
-      for (int i = 0; i < kRecFactorBytes / 1024; ++i) dma_one(f + i * 1024, lane16off, s + T::kFOff + i * 1024);
+      for (int i = 0; i < kRecFactorBytes / 1024; ++i)
+        dma_one(fg + (size_t)c * kRecFactorBytes + i * 1024, lane * 16, s + T::kFOff + i * 1024);
     };
     // output tiles of chunk c: one per matrix wave, four 8-row groups each; all reads first, one wait, then
     // the stores back to back, each a scalar base plus one of 16 precomputed lane offsets
@@ -288,14 +401,9 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
     for (int w = 0; w < T::kWaves; ++w)
 #pragma unroll
       for (int i = 0; i < 4; ++i) ooff[w][i] = (uint32_t)(((32 * w + 8 * i + orl) * L + occ * 4) * 4);
-    const char* const oread = smem + T::kOutOff + (orl ^ ((orl >> 2) & 1)) * 128 + occ * 16;
+    const char* const oread = smem + T::kVOff + (orl ^ ((orl >> 2) & 1)) * 128 + occ * 16;
     float* const og = out + ((size_t)bh * vdim + (size_t)blockIdx.x * DVS) * L;
-    auto store_chunk = [&](int c) {
-      f4v x[T::kWaves][4];
-#pragma unroll
-      for (int w = 0; w < T::kWaves; ++w)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[w][i] = *reinterpret_cast<const f4v*>(oread + w * 4096 + i * 1024);
+    const auto store_tiles = [&](const f4v (&x)[T::kWaves][4], int c) {
       wait_lgkm0();
       const uint64_t base = (uint64_t)(uintptr_t)(og + (size_t)c * T::kChunk);
 #pragma unroll
@@ -303,215 +411,264 @@ __global__ __launch_bounds__(DVS * 2 + 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int i = 0; i < 4; ++i) asm volatile("global_store_dwordx4 %0, %1, %2" :: "v"(ooff[w][i]), "v"(x[w][i]), "s"(base) : "memory");
     };
-    dma_kq(0, 0);
-    dma_vf(0, 0);
-    wait_vmcnt<0>();
-    for (int c = 0; c < nchunk; ++c) {
-      const bool more = c + 1 < nchunk;
-      asm volatile("s_barrier" ::: "memory");          // chunk c is in LDS; the matrix waves are done with chunk c-1
-      if (more) dma_kq(c + 1, (c + 1) & 1);
-      if (c > 0) store_chunk(c - 1);                     // staged before this barrier, overwritten after the next one
-      if (more) dma_vf(c + 1, (c + 1) & 1);
-      asm volatile("s_barrier" ::: "memory");          // (the matrix waves' barrier in front of the S^T sum, late in the chunk)
-      wait_vmcnt<0>();                                   // the next chunk has landed, the stores are out
+    // The first requests K and Q, the second V and the factors and stores the output.  Q's place is free from a chunk's second
+    // barrier on, the others' when the chunk is done.  Memory operations of a wave complete in order.
+    constexpr bool kQEarly = T::kWaves * 4096 <= T::kKTile;
+    constexpr int kKOps = KD / 8, kVfOps = DVS / 8 + kRecFactorBytes / 1024;
+    if (wave == T::kWaves) {
+      dma_k(0, 0);
+      dma_q(0, 0);
+      if (kQEarly && nchunk > 1) {
+        dma_q(1, 1);
+        wait_vmcnt<kKOps>();
+      } else {
+        wait_vmcnt<0>();
+      }
+      for (int c = 0; c < nchunk; ++c) {
+        block_sync();                                      // chunk c is in LDS; the matrix waves are done with chunk c-1
+        if (c + 1 < nchunk) {
+          dma_k(c + 1, (c + 1) & 1);
+          if (!kQEarly) dma_q(c + 1, (c + 1) & 1);
+        }
+        block_sync();                                      // they have taken chunk c over
+        if (kQEarly && c + 2 < nchunk) dma_q(c + 2, c & 1);
+        block_sync();                                      // (their partial S^T are in LDS)
+        if (kQEarly && c + 2 < nchunk) wait_vmcnt<kKOps>();
+        else wait_vmcnt<0>();                              // the next chunk has landed
+      }
+      block_sync();
+    } else {
+      f4v x[T::kWaves][4];
+      const auto read_tiles = [&](int c) {
+#pragma unroll
+        for (int w = 0; w < T::kWaves; ++w)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[w][i] = *reinterpret_cast<const f4v*>(oread + (c & 1) * T::kStage + w * 4096 + i * 1024);
+        wait_lgkm0();
+      };
+      dma_vf(0, 0);
+      wait_vmcnt<0>();
+      for (int c = 0; c < nchunk; ++c) {
+        block_sync();
+        if (c > 0) read_tiles(c - 1);
+        if (c + 1 < nchunk) dma_vf(c + 1, (c + 1) & 1);
+        block_sync();
+        if (c > 0) store_tiles(x, c - 1);
+        block_sync();
+        if (c > 0) wait_vmcnt<4 * T::kWaves>();            // the next chunk has landed; the stores may still be under way
+        else wait_vmcnt<0>();
+      }
+      block_sync();                                        // the last chunk's tiles are staged
+      read_tiles(nchunk - 1);
+      store_tiles(x, nchunk - 1);
+      wait_vmcnt<0>();
     }
-    asm volatile("s_barrier" ::: "memory");              // the last chunk's tiles are staged
-    store_chunk(nchunk - 1);
-    return;
+    return false;
   }
 
   // ================================ matrix waves ================================================
-  char* const ost = smem + T::kOutOff + wave * 4096;
-  char* const ow_even = ost + n * 4 + 5 * hi * 128;                         // write base for e even: position 4h + h
-  char* const ow_odd = ost + n * 4 + (3 * hi + 1) * 128;                    // e odd: position 4h + (1 - h)
+  const int ow_even = T::kVOff + wave * 4096 + n * 4 + 5 * hi * 128;        // write offset for e even: position 4h + h
+  const int ow_odd = T::kVOff + wave * 4096 + n * 4 + (3 * hi + 1) * 128;   // e odd: position 4h + (1 - h)
 
-  // Per-lane LDS read addresses of the current stage (moved to the other stage at the end of a chunk).
+  // Per-lane LDS offsets inside a stage.
   //  row read (row 8G+4h+e, column n): the slot term of the row is the compile-time constant
   //  sw(G, e) = 4(G&1) + 2(e&1) + (e>>1), folded into the lane part by XOR; the row goes into the offset.
   //  column read (16-byte chunk 2g+h of row n of a 32-row block): position and slot term are per lane.
-  const uint32_t lds0 = lds_addr(smem);
   const uint32_t row_lane = hi * 128 + (n >> 2) * 16 + (n & 3) * 4;
-  const int wave_rows = wave * T::kGroupsPerWave * 8;                 // first key dim of this wave's share of S^T
-  const int wave_sw = 4 * ((wave * T::kGroupsPerWave) & 1);
   const int cp = rec_pos(n);
-  constexpr int kNumBases = 8 + 8 + 4 + 4 + 4;
-  uint32_t bases[kNumBases];
-  uint32_t* const row4 = bases;            // [8]  State^T Q operand rows
-  uint32_t* const row1 = bases + 8;        // [8]  this wave's rows of the S^T contraction
-  uint32_t* const colb = bases + 16;       // [4]  K columns
-  uint32_t* const colv = bases + 20;       // [4]  V columns of this wave's 32 value dims
-  uint32_t& lane16 = bases[24];
-  uint32_t& wbase = bases[25];
-  uint32_t& pbase = bases[26];
-  uint32_t& sbase = bases[27];
+  uint32_t colb[4];
 #pragma unroll
-  for (int sw = 0; sw < 8; ++sw) {
-    row4[sw] = lds0 + (row_lane ^ (sw << 4));
-    row1[sw] = lds0 + wave_rows * 128 + (row_lane ^ ((sw ^ wave_sw) << 4));
-  }
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    colb[g] = lds0 + cp * 128 + rec_slot(cp, 2 * g + hi) * 16;
-    colv[g] = colb[g] + T::kVOff + wave * 4096;
-  }
-  lane16 = lds0 + lane * 16;
-  wbase = lds0 + hi * 64;
-  pbase = lds0 + n * 4;
-  sbase = lds0;
-  uint32_t redo[T::kWaves - 1];                                       // the other waves' partial tiles
-#pragma unroll
-  for (int t = 0; t < T::kWaves - 1; ++t) redo[t] = lds0 + 2 * T::kStage + ((wave + 1 + t) % T::kWaves) * 4096 + lane * 16;
-  char* const red_mine = smem + 2 * T::kStage + wave * 4096 + lane * 16;
+  for (int g = 0; g < 4; ++g) colb[g] = cp * 128 + rec_slot(cp, 2 * g + hi) * 16;
+  const uint32_t lane16 = lane * 16;
+  // LDS offsets beyond 64 KB do not fit the instructions' offset field: one register for all the operands and partial tiles
+  uint32_t op0 = T::kOpOff + lane16;
+  asm volatile("" : "+v"(op0));
+  char* const ops = smem + op0;
+  char* const ops_own = ops + wave * T::kUnits * 3072;
 
   f16v st[T::kKB];
 #pragma unroll
   for (int i = 0; i < T::kKB; ++i) st[i] = zero16();
+  RecFinite finite;
 
-  // The LDS reads of a chunk form one stream, consumed in order, each issued kPF elements ahead.
-  constexpr int kPF = 6, kRing = kPF + 1;
-  constexpr int nS1 = 8 * T::kGroupsPerWave;              // K and Q row reads of the partial S^T
-  constexpr int nS4 = 16 * T::kKB;                        // Q row reads of State^T Q
-  constexpr int nRedG = T::kWaves;                        // per g: the other waves' partials, then D
-  // Order after State^T Q: the State update comes first (it needs V, w and K only), the sum of the partial
-  // S^T tiles, P and V P sit inside it, before its last 16 matrix instructions.  Whatever a vector phase
-  // needs from the matrix pipe (O^T for its scaling, V P for the staging of the output tile) then left it a
-  // thousand cycles earlier, and the barrier in front of the partial tiles comes late in the chunk.
-  constexpr int jS4 = nS1, jFlag = jS4 + nS4, jV = jFlag + 1, jW = jV + 4, jK1 = jW + 4;
-  constexpr int jRed = jK1 + 4 * (T::kKB - 1), jPnl = jRed + 4 * nRedG, jK2 = jPnl + 1;
-  constexpr int nElem = jK2 + 4;
+  for (int c = 0; c < nchunk; ++c) {
+    char* const sm = smem + (c & 1) * T::kStage;
+    block_sync();      // chunk c is in LDS (the data waves waited for it); every wave is done with chunk c-1
 
-  auto chunk = [&](auto stage_tag, int c) {
-    constexpr int S = decltype(stage_tag)::value;
-    float fr[kRing];
-    f4v vr[kRing];
-    f16v sp = zero16(), oacc = zero16(), pm;
-    f4v vt[4], wv[4];
-    float ka = 0.f;
-
-    auto issue = [&](auto jt) {
-      constexpr int j = decltype(jt)::value, slot = j % kRing;
-      if constexpr (j < nS1) {
-        constexpr int i = j / 2, gg = i / 4, e = i % 4, p0 = 8 * gg + 4 * (e & 1) + (e & 2), sw = (p0 >> 1) & 7;
-        fr[slot] = lds_read_f1_async(row1[sw], (j % 2 ? T::kQOff : 0) + p0 * 128);
-      } else if constexpr (j < jFlag) {
-        constexpr int jj = j - jS4, G = jj / 4, e = jj % 4, p0 = 8 * G + 4 * (e & 1) + (e & 2), sw = (p0 >> 1) & 7;
-        fr[slot] = lds_read_f1_async(row4[sw], T::kQOff + p0 * 128);
-      } else if constexpr (j == jFlag) {
-        vr[slot] = lds_read_f4_async(sbase, T::kFOff + kRecFactorFlag);
-      } else if constexpr (j < jW) {
-        vr[slot] = lds_read_f4_async(colv[j - jV], 0);
-      } else if constexpr (j < jK1) {
-        vr[slot] = lds_read_f4_async(wbase, T::kFOff + kRecFactorW + (j - jW) * 16);
-      } else if constexpr (j < jRed) {
-        constexpr int kb = (j - jK1) / 4, g = (j - jK1) % 4;
-        vr[slot] = lds_read_f4_async(colb[g], kb * 4096);
-      } else if constexpr (j < jPnl) {
-        constexpr int g = (j - jRed) / nRedG, t = (j - jRed) % nRedG;
-        if constexpr (t < T::kWaves - 1) vr[slot] = lds_read_f4_async(redo[t], g * 1024);
-        else vr[slot] = lds_read_f4_async(lane16, T::kFOff + g * 1024);
-      } else if constexpr (j == jPnl) {
-        fr[slot] = lds_read_f1_async(pbase, T::kFOff + kRecFactorPnl);
-      } else {
-        vr[slot] = lds_read_f4_async(colb[j - jK2], (T::kKB - 1) * 4096);
+    // ---- this wave's share of the operands of Q and of K diag(w / lambda')
+    Op qown[T::kUnits], kop[T::kUnits];
+    f4v kx[T::kUnits][2], vx[4];
+    {
+      f4v qx[T::kUnits][2], kc[T::kUnits][2];
+#pragma unroll
+      for (int s = 0; s < T::kUnits; ++s) {
+        const int u = wave * T::kUnits + s;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          // row 16u + 8(j/4) + 4h + j%4
+          const int p0 = 8 * (j >> 2) + 4 * (j & 1) + (j & 2), sw = (p0 >> 1) & 7;
+          const uint32_t at = u * 2048 + p0 * 128 + (row_lane ^ (sw << 4));
+          qx[s][j >> 2][j & 3] = *reinterpret_cast<const float*>(sm + T::kQOff + at);
+          kx[s][j >> 2][j & 3] = *reinterpret_cast<const float*>(sm + at);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          kc[s][i] = *reinterpret_cast<const f4v*>(sm + (u >> 1) * 4096 + cp * 128 + (rec_slot(cp, hi) ^ (4 * (u & 1) + 2 * i)) * 16);
+          if constexpr (!FP32) kc[s][i] *= *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorW + hi * 64 + (2 * (u & 1) + i) * 16);
+        }
       }
+      Op kown[T::kUnits];
+#pragma unroll
+      for (int s = 0; s < T::kUnits; ++s) {
+        qown[s] = rec_op<FP32, true>(qx[s][0], qx[s][1]);
+        kown[s] = rec_op<FP32, true>(kc[s][0], kc[s][1]);
+      }
+#pragma unroll
+      for (int s = 0; s < T::kUnits; ++s)
+#pragma unroll
+        for (int p = 0; p < Op::kParts; ++p) {
+          *reinterpret_cast<u4v*>(ops_own + T::op_at(true, s, p)) = qown[s].p[p];
+          *reinterpret_cast<u4v*>(ops_own + T::op_at(false, s, p)) = kown[s].p[p];
+        }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) vx[g] = *reinterpret_cast<const f4v*>(sm + T::kVOff + wave * 4096 + colb[g]);
+      kop[0] = rec_op<FP32, true>(kx[0][0], kx[0][1]);
+    }
+    block_sync();
+    const auto read_op = [&](bool of_q, int u) {
+      Op o;
+#pragma unroll
+      for (int p = 0; p < Op::kParts; ++p) o.p[p] = *reinterpret_cast<const u4v*>(ops + T::op_at(of_q, u, p));
+      return o;
     };
 
-    auto consume = [&](auto jt) {
-      constexpr int j = decltype(jt)::value, slot = j % kRing, younger = (nElem - 1 - j < kPF) ? nElem - 1 - j : kPF;
-      if constexpr (j < nS1) {
-        lds_wait_younger_f<younger>(fr[slot]);
-        if constexpr (j % 2 == 0) ka = fr[slot];
-        else sp = mfma_32x32x2_f32(ka, fr[slot], sp);
-        if constexpr (j == nS1 - 1) {
+    // From here to the end of the chunk: a region per k-step, its six matrix instructions with the vector instructions that make a
+    // later region's operand between them, and the LDS reads of the next region.
+    // ---- the wave's partial S^T
+    f16v sp = zero16(), oacc = zero16();
+    Op top, qop = read_op(true, 0);
+    sched_fence();
+    static_for<T::kUnits>([&](auto it) {
+      constexpr int s = decltype(it)::value;
+      if constexpr (s + 1 < T::kUnits) kop[s + 1] = rec_op<FP32>(kx[s + 1][0], kx[s + 1][1]);
+      else top = rec_op_of_c<FP32>(st[0], 0);
+      sp = rec_mma<FP32>(kop[s], qown[s], sp);
+      rec_interleave<FP32, 0, 8>();
+    });
+
+    // ---- T^T Q
+    // w / lambda' goes with K, whose operands are made once; FP32: with V as in the kernel below, so that no range is lost to the scale of K
+    const auto update_op = [&](const Op (&vop)[2], int s) {
+      if constexpr (!FP32) return vop[s];
+      const auto w = [&](int g) { return *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorW + hi * 64 + g * 16); };
+      return rec_op<FP32>(vx[2 * s] * w(2 * s), vx[2 * s + 1] * w(2 * s + 1));
+    };
+    Op vop[2], pop[2];
+    static_for<T::kSteps>([&](auto it) {
+      constexpr int ks = decltype(it)::value;
+      Op tnext, qnext;
+      if constexpr (ks + 1 < T::kSteps) {
+        qnext = read_op(true, ks + 1);
+        tnext = rec_op_of_c<FP32>(st[(ks + 1) >> 1], (ks + 1) & 1);
+        rec_pin(tnext);
+      } else {
+        vop[0] = rec_op<FP32>(vx[0], vx[1]);
+        rec_pin(vop[0]);
+      }
+      oacc = rec_mma<FP32>(top, qop, oacc);
+      rec_interleave<FP32, ks + 1 < T::kSteps ? 3 : 0, 8>();
+      if constexpr (ks == 1) {
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            f4v x = {sp[4 * g], sp[4 * g + 1], sp[4 * g + 2], sp[4 * g + 3]};
-            *reinterpret_cast<f4v*>(red_mine + g * 1024) = x;
-          }
-          asm volatile("" ::: "memory");     // the stores stay here, far ahead of the barrier that publishes them
+        for (int g = 0; g < 4; ++g) *reinterpret_cast<f4v*>(sm + wave * 4096 + g * 1024 + lane16) = rec_quarter(sp, 4 * g);
+        sched_fence();
+      }
+      top = tnext;
+      qop = qnext;
+    });
+    f4v dd[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) dd[g] = *reinterpret_cast<const f4v*>(sm + T::kFOff + g * 1024 + lane16);
+    const float pnl = *reinterpret_cast<const float*>(sm + T::kFOff + kRecFactorPnl + n * 4);
+    Op wop = read_op(false, 0);
+    const f4v flag = *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorFlag);
+    if (__builtin_amdgcn_readfirstlane(__float_as_uint(flag[0])) != 0u) {   // lambda left its range: fold it into T
+#pragma unroll
+      for (int kb = 0; kb < T::kKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[kb][i] *= flag[1];
+    }
+
+    // ---- T += K diag(w / lambda') V^T, the positions 0-15 of every State tile first; meanwhile P, and
+    // O^T = (p_n lambda) T^T Q + V P ahead of the last k-step, so that it has left the matrix core when it is stored
+    f4v part[2][T::kWaves - 1];
+    const auto read_partials = [&](int g0) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < T::kWaves - 1; ++t) {
+          const int w = wave + 1 + t < T::kWaves ? wave + 1 + t : wave + 1 + t - T::kWaves;
+          part[g][t] = *reinterpret_cast<const f4v*>(sm + w * 4096 + (g0 + g) * 1024 + lane16);
         }
-      } else if constexpr (j < jFlag) {
-        constexpr int jj = j - jS4;
-        lds_wait_younger_f<younger>(fr[slot]);
-        oacc = mfma_32x32x2_f32(st[jj / 16][jj % 16], fr[slot], oacc);
-      } else if constexpr (j == jFlag) {
-        lds_wait_younger_f<younger>(vr[slot]);
-        if (__builtin_amdgcn_readfirstlane(__float_as_uint(vr[slot][0])) != 0u) {   // lambda left its range: fold it into T
-          const float sc = vr[slot][1];
+    };
+    const auto add_partials = [&](int g0) {                // P of two row groups: the waves' partial sums times D
 #pragma unroll
-          for (int kb = 0; kb < T::kKB; ++kb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) st[kb][i] *= sc;
-        }
-      } else if constexpr (j < jW) {
-        lds_wait_younger_f<younger>(vr[slot]);
-        vt[j - jV] = vr[slot];
-      } else if constexpr (j < jK1) {
-        lds_wait_younger_f<younger>(vr[slot]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) wv[j - jW][e] = vt[j - jW][e] * vr[slot][e];
-      } else if constexpr (j < jRed) {
-        constexpr int kb = (j - jK1) / 4, g = (j - jK1) % 4;
-        lds_wait_younger_f<younger>(vr[slot]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st[kb] = mfma_32x32x2_f32(vr[slot][e], wv[g][e], st[kb]);
-      } else if constexpr (j < jPnl) {
-        constexpr int g = (j - jRed) / nRedG, t = (j - jRed) % nRedG;
-        lds_wait_younger_f<younger>(vr[slot]);
+      for (int g = g0; g < g0 + 2; ++g)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if constexpr (t < T::kWaves - 1) sp[4 * g + e] += vr[slot][e];
-          else pm[4 * g + e] = sp[4 * g + e] * vr[slot][e];
+#pragma unroll
+          for (int t = 0; t < T::kWaves - 1; ++t) sp[4 * g + e] += part[g - g0][t][e];
+          sp[4 * g + e] *= dd[g][e];
         }
-      } else if constexpr (j == jPnl) {
-        lds_wait_younger_f<younger>(fr[slot]);
-        // O^T = (p_n lambda) T^T Q + V P
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[i] *= fr[slot];
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) oacc = mfma_32x32x2_f32(vt[g][e], pm[4 * g + e], oacc);
-      } else {
-        constexpr int kb = T::kKB - 1, g = j - jK2;
-        lds_wait_younger_f<younger>(vr[slot]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st[kb] = mfma_32x32x2_f32(vr[slot][e], wv[g][e], st[kb]);
-        if constexpr (j == nElem - 1) {
-#pragma unroll
-          for (int gg = 0; gg < 4; ++gg)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              *reinterpret_cast<float*>((e & 1 ? ow_odd : ow_even) + (8 * gg + (e & 2)) * 128) = oacc[4 * gg + e];
-          asm volatile("" ::: "memory");     // staged before the barrier that hands it to the data wave
-        }
-      }
     };
-
-    asm volatile("s_barrier" ::: "memory");   // chunk c is in LDS (the data wave waited for it); every wave is done with chunk c-1
-    static_for<kPF>([&](auto jt) { issue(jt); });
     sched_fence();
-    static_for<nElem>([&](auto jt) {
-      constexpr int j = decltype(jt)::value;
-      if constexpr (j + kPF < nElem) {
-        // the partial tiles were stored long before (LDS operations retire in order and younger reads
-        // have been waited for), so a bare barrier is enough before the first read of another wave's tile
-        if constexpr (j + kPF == jRed) asm volatile("s_barrier" ::: "memory");
-        issue(std::integral_constant<int, j + kPF>{});
+    static_for<T::kSteps>([&](auto it) {
+      constexpr int i = decltype(it)::value, kb = i % T::kKB, s = i / T::kKB;
+      Op wnext;
+      if constexpr (i + 1 < T::kSteps) wnext = read_op(false, 2 * ((i + 1) % T::kKB) + (i + 1) / T::kKB);
+      constexpr auto at = [](int x) { return x * T::kSteps / 8; };
+      if constexpr (i == at(0)) vop[1] = rec_op<FP32>(vx[2], vx[3]);
+      if constexpr (i == at(2)) {
+        add_partials(0);
+        read_partials(2);
       }
-      consume(jt);
-      sched_fence();
-    });
+      if constexpr (i == at(3)) pop[0] = rec_op_of_c<FP32>(sp, 0);
+      if constexpr (i == at(4)) add_partials(2);
+      if constexpr (i == at(5)) pop[1] = rec_op_of_c<FP32>(sp, 1);
+      if constexpr (i == at(6)) {
 #pragma unroll
-    for (int i = 0; i < kNumBases; ++i) bases[i] += (S == 0) ? T::kStage : -T::kStage;
-  };
-
-  for (int c = 0; c < nchunk; c += 2) {
-    chunk(std::integral_constant<int, 0>{}, c);
-    if (c + 1 < nchunk) chunk(std::integral_constant<int, 1>{}, c + 1);
+        for (int r = 0; r < 16; ++r) oacc[r] *= pnl;
+      }
+      if constexpr (i == T::kSteps - 1) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) oacc = rec_mma<FP32>(vop[r], pop[r], oacc);
+        sched_fence();
+      }
+      st[kb] = rec_mma<FP32>(wop, update_op(vop, s), st[kb]);
+      rec_interleave<FP32, 3, 8>();
+      if constexpr (i == at(0)) {
+        block_sync();                                      // the partial S^T are in LDS
+        read_partials(0);
+      }
+      wop = wnext;
+    });
+    finite.see(oacc);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        *reinterpret_cast<float*>(sm + (e & 1 ? ow_odd : ow_even) + (8 * g + (e & 2)) * 128) = oacc[4 * g + e];
   }
-  wait_lgkm0();
-  asm volatile("s_barrier" ::: "memory");     // the last chunk's output tiles are staged: the data wave stores them
+  block_sync();               // the last chunk's output tiles are staged: the data wave stores them
+  return finite.broken();
+}
+
+template <int KD, int DVS>
+__global__ __launch_bounds__(DVS * 2 + 128) __attribute__((amdgpu_waves_per_eu(2, 2))) void retnet_recurrent_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    const char* __restrict__ factors, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
+  extern __shared__ __align__(16) char smem[];
+  const bool broken = rec_scan<false, KD, DVS>(smem, q, k, v, factors, out, heads, kdim, vdim, L);
+  if (rec_any_wave(smem, broken)) rec_scan<true, KD, DVS>(smem, q, k, v, factors, out, heads, kdim, vdim, L);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -613,6 +770,19 @@ struct RetRecurrentSplit {
   static_assert(kSmemBytes <= 160 * 1024, "LDS");
 };
 
+// LDS reads and stores issued by hand so that their waits can be counted: the compiler answers every
+// dependency on an LDS load with lgkmcnt(0) while an LDS-DMA copy is in flight, and here one is in
+// flight all the time.  LDS operations retire in order, so "at most N younger ones outstanding" is enough.
+AAT_DEV float lds_read_f1_async(uint32_t base, int imm) {
+  float v;
+  asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(base), "i"(imm));
+  return v;
+}
+template <int N, class V> AAT_DEV void lds_wait_younger_f(V& v) {
+  static_assert(N >= 0 && N < 16, "lgkmcnt is a 4-bit counter");
+  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N));
+}
+
 // Grid: B * H * vdim / 32 blocks, the slices of one (batch, head) on one XCD (they read the same q and k).
 template <int KD, int WK, bool PRE>
 __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void retnet_recurrent_split_kernel(
@@ -630,7 +800,9 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
   const char* fg = factors + (size_t)h * nchunk * kRecFactorBytes;
 
   if (wave == WK) {
-    // data wave: see the kernel above
+    // Every address is a scalar base that moves with the chunk plus a per-lane 32-bit offset computed here once: the loop of this wave
+    // must not contain a single vector instruction -- one has to find a gap between the fp32 MFMAs of the matrix wave that shares
+    // the SIMD, and a copy that waits for one took 175 cycles to issue.
     const char* qg = reinterpret_cast<const char*>(q + (size_t)bh * kdim * L);
     const char* kg = reinterpret_cast<const char*>(k + (size_t)bh * kdim * L);
     const char* vg = reinterpret_cast<const char*>(v + ((size_t)bh * vdim + vd0) * L);

@@ -262,3 +262,66 @@ def test_graph_capture_replays():
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(out, aat.retnet_recurrent_fwd(q2, k2, v2, decay2))
+
+
+# blocks of 128 and of 64 value dims (192 of them, so the split kernel stays away): one chunk, two, an odd number; every head
+@pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(8, 24, 128, 128, 32), (8, 24, 64, 128, 64), (8, 24, 64, 64, 96),
+                                                   (4, 24, 128, 256, 160), (8, 24, 64, 64, 32), (8, 24, 64, 128, 96)])
+def test_blocks_that_split_the_value_dims(b, h, kdim, vdim, seqlen):
+    q, k, v, decay = _inputs(21, b, h, kdim, vdim, seqlen, -0.3, 1.2)
+    decay[0, seqlen // 2] = 0.0
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(h):
+        _close(out[:, head], ref[:, head])
+
+
+# fp32 products in three bf16 parts: values down to where the smallest part of one is a bf16 subnormal, and magnitudes that differ from key dim to
+# key dim; a part lost to a flush or a common scale would show as 2^-8 or 2^-16 of a value
+@pytest.mark.parametrize("k_scale,q_scale,spread", [(1e-30, 1e20, 0.0), (1e30, 1e-20, 0.0), (1.0, 1.0, 12.0)])
+def test_products_in_parts_keep_the_range_of_fp32(k_scale, q_scale, spread):
+    q, k, v, decay = _inputs(22, 8, 24, 128, 128, 64, 0.9, 1.0)
+    per_dim = 10.0 ** ((torch.arange(128) * 37 % 128 / 127.0 - 0.5) * spread).view(1, 1, 128, 1)
+    q, k = (q * q_scale * per_dim).float(), (k * k_scale / per_dim).float()
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(24):
+        _close(out[:, head], ref[:, head])
+
+
+# An infinity or a NaN takes its (batch, head, value slice) from the chunk it lies in on, and nothing else: the rest is as without it,
+# bit for bit in other blocks, within the bound in the chunks before
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+@pytest.mark.parametrize("kdim,vdim", [(128, 128), (64, 128), (64, 64)])
+def test_values_that_are_not_finite(value, which, kdim, vdim):
+    b, h, seqlen, pos = 8, 24, 128, 70
+    q, k, v, decay = _inputs(23, b, h, kdim, vdim, seqlen, 0.9, 1.0)
+    clean = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    bad = dict(q=q, k=k, v=v)
+    bad[which] = bad[which].clone()
+    bad[which][3, 5, 7, pos] = value
+    out = aat.retnet_recurrent_fwd(bad["q"].cuda(), bad["k"].cuda(), bad["v"].cuda(), decay.cuda())
+    rows = slice(7, 8) if which == "v" else slice(None)
+    last = pos + 1 if which == "q" else seqlen
+    assert not torch.isfinite(out[3, 5, rows, pos:last]).any()
+    _close(out[3, 5, :, :64], clean[3, 5, :, :64].cpu())
+    if which == "q":
+        _close(out[3, 5, :, 96:], clean[3, 5, :, 96:].cpu())
+    out[3, 5], clean[3, 5] = 0.0, 0.0
+    assert torch.equal(out, clean)
+
+
+# 3.4e38 rounds to an infinity in bf16, but is none: with small partners every product and sum stays finite
+@pytest.mark.parametrize("which", ["q", "k"])
+@pytest.mark.parametrize("kdim,vdim", [(128, 128), (64, 128), (64, 64)])
+def test_values_beyond_the_largest_of_bf16(which, kdim, vdim):
+    b, h, seqlen, pos = 8, 24, 128, 70
+    q, k, v, decay = _inputs(24, b, h, kdim, vdim, seqlen, 0.9, 1.0)
+    x = {n: t if n == which else t * 1e-6 for n, t in (("q", q), ("k", k), ("v", v))}
+    x[which][3, 5, 7, pos] = 3.4e38
+    out = aat.retnet_recurrent_fwd(x["q"].cuda(), x["k"].cuda(), x["v"].cuda(), decay.cuda())
+    ref = torch.from_numpy(brute.retnet_recurrent(x["q"].numpy(), x["k"].numpy(), x["v"].numpy(), decay.numpy()))
+    assert torch.isfinite(out).all()
+    _close(out[3, 5], ref[3, 5])
+    _close(out[3, 4], ref[3, 4])
