@@ -67,6 +67,8 @@ def _bind_recurrent(lib):
     dims = [_I] * 6                                   # batch, heads, kdim, vdim, l, block_kdim
     lib.retnet_recurrent_workspace_size.restype = _SZ
     lib.retnet_recurrent_workspace_size.argtypes = dims
+    lib.retnet_recurrent_room.restype = _SZ
+    lib.retnet_recurrent_room.argtypes = dims + [_SZ]
     lib.retnet_recurrent_fwd.restype = None
     lib.retnet_recurrent_fwd.argtypes = [_VP] * 5 + dims
     lib.retnet_recurrent_fwd_ex.restype = _I

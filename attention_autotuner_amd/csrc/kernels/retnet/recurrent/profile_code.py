@@ -28,6 +28,12 @@ size_t total_workspace_bytes(int batch, int heads, int vdim, int l, int block_kd
   return block_kdim > 128 ? f + (size_t)batch * heads * vdim * l * sizeof(float) : f;
 }}
 
+// Operands of K and Q and the products P for the kernel that takes them from memory, behind the factors.
+size_t stream_bytes(int batch, int heads, int l, int block_kdim) {{
+  const size_t f = (factor_bytes(heads, l) + 255) / 256 * 256;
+  return f + (size_t)batch * heads * (l / 32) * (4096 + (size_t)(block_kdim / 16) * 6144);
+}}
+
 bool rec_shape_ok(int batch, int heads, int kdim, int vdim, int l, int block_kdim) {{
   return batch > 0 && heads > 0 && l > 0 && l % 32 == 0 && l / 32 <= 4096 && block_kdim >= 64 && block_kdim % 64 == 0 &&
          block_kdim <= kMaxKdim && block_kdim <= kdim && vdim > 0 && vdim % 64 == 0;
@@ -72,8 +78,8 @@ hipError_t launch_split(const float* q, const float* k, const float* v, const fl
   if (ok != hipSuccess) return ok;
   if constexpr (kPre) {{
     const int parts = std::min(32, (l / 32 + 3) / 4);                  // a chunk per wave up to 128 chunks
-    aat::retnet_recurrent_pmat<KD><<<dim3((unsigned)heads * parts + (unsigned)batch * heads * (l / 32)), dim3(256),
-                                     (size_t)(l / 32) * 8, stream>>>(q, k, decay, factors, room, heads, parts, kdim, l);
+    aat::retnet_recurrent_pmat<KD, false><<<dim3((unsigned)heads * parts + (unsigned)batch * heads * (l / 32)), dim3(256),
+                                     (size_t)(l / 32) * 8, stream>>>(q, k, decay, factors, room, nullptr, heads, parts, kdim, l);
   }} else {{
     launch_factors(decay, factors, heads, l, stream);
   }}
@@ -84,34 +90,74 @@ hipError_t launch_split(const float* q, const float* k, const float* v, const fl
   return hipGetLastError();
 }}
 
-// Whether blocks of 32 value dims that split the key dims between their waves take less time than passes over 128 and
-// 64 key dims with 128 (wide) or 64 value dims per block: microseconds per chunk of a round of blocks, times the rounds on 256
-// compute units (a block fills one; two of the 64 x 64 ones share one), and the addition of the passes' outputs.  Blocks of 64
-// value dims and 128 key dims never came out ahead and are not built.  Measured at 2048 positions, whole calls, passes against
-// split: B4 H8 128/256 344 -> 147 us, B4 H12 128/256 347 -> 268, B8 H16 128/256 363 -> 552; B4 H16 64/128 207 -> 142,
-// B8 H32 64/128 262 -> 482; B4 H16 192/256 609 -> 371; B4 H16 256/256 748 -> 391.
-bool split_pays(long bh, int vdim, int block_kdim, bool wide) {{
-  constexpr long kUnits = 256;
-  const auto rounds = [](long blocks, long at_once) {{ return (double)((blocks + at_once - 1) / at_once); }};
-  if (!wide && block_kdim > 64) return true;
-  const double pmat = block_kdim > 128 ? 2.0 * bh * block_kdim * 32 * 4 / 5e6 : 0.0;   // P: q and k once more at 5 TB/s
-  const double split = pmat + (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : block_kdim == 192 ? 2.45 : 2.6) * rounds(bh * (vdim / 32), kUnits);
-  if (!wide) return split < 2.5 * rounds(bh * (vdim / 64), 2 * kUnits);
-  const double passes = (block_kdim / 128 * 4.8 + block_kdim / 64 % 2 * 3.25) * rounds(bh * (vdim / 128), kUnits);
-  const double add = block_kdim > 128 ? 3.0 * bh * vdim * 32 * 4 / 8e6 : 0.0;      // two reads and a write, partly from the cache
-  return split < passes + add;
+template <int KD, int WK>
+hipError_t launch_stream(const float* q, const float* k, const float* v, const float* decay, char* factors, char* room, float* out,
+                         int batch, int heads, int kdim, int vdim, int l, hipStream_t stream) {{
+  using T = aat::RetRecurrentStream<KD, WK>;
+  const auto kernel = &aat::retnet_recurrent_stream_kernel<KD, WK>;
+  static const hipError_t ok = aat::allow_lds(kernel, T::kSmemBytes);
+  if (ok != hipSuccess) return ok;
+  char* const ops = room + (size_t)batch * heads * (l / 32) * 4096;
+  const int parts = std::min(32, (l / 32 + 3) / 4);                    // a chunk per wave up to 128 chunks
+  aat::retnet_recurrent_pmat<KD, true><<<dim3((unsigned)heads * parts + (unsigned)batch * heads * (l / 32)), dim3(256),
+                                         (size_t)(l / 32) * 8, stream>>>(q, k, decay, factors, room, ops, heads, parts, kdim, l);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  kernel<<<dim3((unsigned)batch * heads * (vdim / 32)), dim3(T::kThreads), T::kSmemBytes, stream>>>(q, k, v, factors, room, ops, out,
+                                                                                             heads, kdim, vdim, l);
+  return hipGetLastError();
 }}
 
-// Two launches: the decay factors of every (head, chunk), beyond 128 key dims in the launch that makes P, then the scan.  A value
-// slice of 128 dims per block halves the traffic of q and k; where it would leave most of the compute units without a block or vdim does not
-// allow it, 64 key dims take slices of 64 and more of them the split kernel, which split_pays() may choose elsewhere too.
+// How a problem is scanned, by estimates of each way in microseconds per chunk of 32 positions: time per chunk of a round of blocks, times
+// the rounds on 256 compute units (a block fills one; two of the 64 x 64 ones share one).
+//  passes  over 128 and 64 key dims with 128 (wide) or 64 value dims per block, and the addition of their outputs.  Blocks of 64 value
+//          dims and 128 key dims never came out ahead and are not built.
+//  split   blocks of 32 value dims that split the key dims between their waves.  Measured at 2048 positions, whole calls, passes
+//          against split: B4 H8 128/256 344 -> 147 us, B4 H12 128/256 347 -> 268, B4 H16 64/128 207 -> 142, B4 H16 192/256 609 -> 371.
+//  stream  the same with the operands of K and Q made ahead, where the caller has the room: 20 bytes of traffic per key dim and
+//          position, which go at 7 TB/s while what is made stays in the memory-side cache (12 of them: 256 MB, of which some 110 do it)
+//          and at 3 beyond.  Measured at 1024 positions against the better of the others: 16 (batch, head) pairs and 256 value
+//          dims, 64 / 128 / 192 / 256 key dims 73 -> 46, 72 -> 46, 84 -> 64, 82 -> 64 us; 32 pairs 73 -> 49, 72 -> 62, 89 -> 82, 89 -> 94; 64 pairs and
+//          256 key dims (200 MB) 175 -> 222.
+struct Estimate {{ double passes, split, stream; bool wide; }};
+Estimate estimate(long bh, int vdim, int l, int block_kdim) {{
+  constexpr long kUnits = 256;
+  const auto rounds = [](long blocks, long at_once) {{ return (double)((blocks + at_once - 1) / at_once); }};
+  Estimate e;
+  e.wide = vdim % 128 == 0 && bh * (vdim / 128) >= 192;
+  const double narrow = rounds(bh * (vdim / 32), kUnits);
+  const double pmat = block_kdim > 128 ? 2.0 * bh * block_kdim * 32 * 4 / 5e6 : 0.0;   // P: q and k once more at 5 TB/s
+  e.split = pmat + (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : block_kdim == 192 ? 2.45 : 2.4) * narrow;
+  const double add = block_kdim > 128 ? 3.0 * bh * vdim * 32 * 4 / 8e6 : 0.0;      // two reads and a write, partly from the cache
+  e.passes = e.wide ? (block_kdim / 128 * 4.8 + block_kdim / 64 % 2 * 3.25) * rounds(bh * (vdim / 128), kUnits) + add
+             : block_kdim == 64 ? 2.5 * rounds(bh * (vdim / 64), 2 * kUnits) : 2 * e.split;
+  const double ahead = (double)bh * 32 * (20.0 * block_kdim + 256) / ((double)bh * l * (12.0 * block_kdim + 128) <= 1.1e8 ? 7e6 : 3e6);
+  e.stream = ahead + (block_kdim == 64 ? 1.1 : block_kdim == 128 ? 1.35 : block_kdim == 192 ? 1.75 : narrow > 1 ? 2.1 : 1.8) * narrow;
+  return e;
+}}
+// From 16 chunks on: below that the calls of both ways differ by less than 15 us (4 pairs 64/64 at 512 positions 39 -> 25), and a short
+// call gives the same bits with and without the room.
+bool stream_pays(const Estimate& e, int l) {{ return l >= 512 && e.stream < 0.95 * std::min(e.split, e.passes); }}
+
+// Two launches: the decay factors of every (head, chunk), beyond 128 key dims and with operands made ahead in the launch that makes P, then the scan.
+// A value slice of 128 dims per block halves the traffic of q and k; where it would leave most of the compute units without a block
+// or vdim does not allow it, 64 key dims take slices of 64 and more of them the split kernel, which may be chosen elsewhere too.
 hipError_t launch(const float* q, const float* k, const float* v, const float* decay, float* out, int batch, int heads,
-                  int kdim, int vdim, int l, int block_kdim, char* workspace, hipStream_t stream) {{
+                  int kdim, int vdim, int l, int block_kdim, char* workspace, size_t workspace_bytes, hipStream_t stream) {{
   char* factors = workspace;
   float* part = reinterpret_cast<float*>(workspace + (factor_bytes(heads, l) + 255) / 256 * 256);
   char* const room = reinterpret_cast<char*>(part);
-  const bool wide = vdim % 128 == 0 && (long)batch * heads * (vdim / 128) >= 192;
-  if (split_pays((long)batch * heads, vdim, block_kdim, wide)) {{
+  const Estimate e0 = estimate((long)batch * heads, vdim, l, block_kdim);
+  const bool wide = e0.wide;
+  if (stream_pays(e0, l) && workspace_bytes >= stream_bytes(batch, heads, l, block_kdim)) {{
+    switch (block_kdim) {{
+      case 64: return launch_stream<64, 2>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 128: return launch_stream<128, 4>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      case 192: return launch_stream<192, 3>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+      default: return launch_stream<256, 4>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
+    }}
+  }}
+  if (e0.split < e0.passes) {{
     switch (block_kdim) {{
       case 64: return launch_split<64, 2>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
       case 128: return launch_split<128, 4>(q, k, v, decay, factors, room, out, batch, heads, kdim, vdim, l, stream);
@@ -211,13 +257,19 @@ extern "C" size_t retnet_recurrent_workspace_size(int batch, int heads, int kdim
   return rec_shape_ok(batch, heads, kdim, vdim, l, block_kdim) ? total_workspace_bytes(batch, heads, vdim, l, block_kdim) : 0;
 }}
 
+extern "C" size_t retnet_recurrent_room(int batch, int heads, int kdim, int vdim, int l, int block_kdim, size_t most) {{
+  if (!rec_shape_ok(batch, heads, kdim, vdim, l, block_kdim)) return 0;
+  const size_t need = total_workspace_bytes(batch, heads, vdim, l, block_kdim), more = stream_bytes(batch, heads, l, block_kdim);
+  return stream_pays(estimate((long)batch * heads, vdim, l, block_kdim), l) && more <= most ? std::max(need, more) : need;
+}}
+
 extern "C" int retnet_recurrent_fwd_ex(const float* q, const float* k, const float* v, const float* decay, float* out,
                                        int batch, int heads, int kdim, int vdim, int l, int block_kdim,
                                        void* workspace, size_t workspace_bytes, void* stream) {{
   if (!rec_shape_ok(batch, heads, kdim, vdim, l, block_kdim)) return AAT_ERR_SHAPE;
   if (workspace == nullptr || workspace_bytes < total_workspace_bytes(batch, heads, vdim, l, block_kdim)) return AAT_ERR_WORKSPACE;
   return (int)launch(q, k, v, decay, out, batch, heads, kdim, vdim, l, block_kdim, static_cast<char*>(workspace),
-                     static_cast<hipStream_t>(stream));
+                     workspace_bytes, static_cast<hipStream_t>(stream));
 }}
 
 extern "C" float retnet_recurrent_profile(const float* q, const float* k, const float* v, const float* decay, float* out,
@@ -227,7 +279,7 @@ extern "C" float retnet_recurrent_profile(const float* q, const float* k, const 
   if (workspace == nullptr || workspace_bytes < total_workspace_bytes(batch, heads, vdim, l, block_kdim)) return -1.f;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return aat::timed_mean_ms(s, [&]() {{
-    return launch(q, k, v, decay, out, batch, heads, kdim, vdim, l, block_kdim, static_cast<char*>(workspace), s);
+    return launch(q, k, v, decay, out, batch, heads, kdim, vdim, l, block_kdim, static_cast<char*>(workspace), workspace_bytes, s);
   }});
 }}
 
@@ -241,7 +293,7 @@ extern "C" int retnet_recurrent_fwd_noalloc(const float* q, const float* k, cons
   char* ws = nullptr;
   const hipError_t e = scratch_of_current_device(&ws);
   if (e != hipSuccess) return (int)e;
-  return (int)launch(q, k, v, decay, out, batch, heads, kdim, vdim, l, block_kdim, ws, static_cast<hipStream_t>(stream));
+  return (int)launch(q, k, v, decay, out, batch, heads, kdim, vdim, l, block_kdim, ws, 0, static_cast<hipStream_t>(stream));
 }}
 
 // The reference's own entry point: same name, same arguments, no status, null stream.  An unsupported
@@ -272,7 +324,7 @@ extern "C" void retnet_recurrent_fwd(void* d_q, void* d_k, void* d_v, void* d_de
   }}
   const hipError_t e = launch(static_cast<const float*>(d_q), static_cast<const float*>(d_k), static_cast<const float*>(d_v),
                               static_cast<const float*>(d_decay), static_cast<float*>(d_out), batch, heads, kdim, vdim, l,
-                              block_kdim, ws, nullptr);
+                              block_kdim, ws, 0, nullptr);
   if (e != hipSuccess) std::fprintf(stderr, "retnet_recurrent_fwd: %s\n", hipGetErrorString(e));
 }}
 """

@@ -85,7 +85,7 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
 //                                   by retnet_recurrent_pmat, which multiplies P by it, and not read after it
 //   [4096, 4224)  W[h][g][e]      = w_m / lambda'      (w_m alone on a rescale)
 //   [4224, 4352)  PNL[n]          = p_n lambda
-//   [4352, 4360)  rescale flag (uint32), scale (float)
+//   [4352, 4368)  rescale flag (uint32), scale, lambda, 1 / lambda' (1 on a rescale)
 constexpr int kRecFactorBytes = 5120;
 constexpr int kRecFactorW = 4096, kRecFactorPnl = 4224, kRecFactorFlag = 4352;
 
@@ -165,6 +165,8 @@ AAT_DEV void rec_factor_records(const float* __restrict__ decay, char* __restric
     if (lane == 0) {
       *reinterpret_cast<uint32_t*>(rec + kRecFactorFlag) = rescale ? 1u : 0u;
       *reinterpret_cast<float*>(rec + kRecFactorFlag + 4) = lam_new;
+      *reinterpret_cast<float*>(rec + kRecFactorFlag + 8) = lam;
+      *reinterpret_cast<float*>(rec + kRecFactorFlag + 12) = inv;
     }
   }
 }
@@ -672,9 +674,11 @@ __global__ __launch_bounds__(DVS * 2 + 128) __attribute__((amdgpu_waves_per_eu(2
 }
 
 // ---------------------------------------------------------------------------------------------------
-// P of every (batch, head, chunk) for the kernel below, as C registers: [B*H][L/32][g][lane][e], 4 KB per chunk.  One block
+// P of every (batch, head, chunk) for the kernels below, as C registers: [B*H][L/32][g][lane][e], 4 KB per chunk.  One block
 // per chunk; its waves split the key dims, read q and k straight from memory (rows of 128 bytes, each used once) and wave w adds
 // up row group w and multiplies it by D.  Bound by the read of q and k.
+// OPS: also the operands of Q p_n and K w_m for retnet_recurrent_stream_kernel, [B*H][L/32][KD/16 of Q, KD/16 of K][part][lane][16 B];
+// bound by their 12 bytes per key dim and position (B2 H8 L1056, 256 key dims: 8.8 us without them, 17 with).
 //
 // The first heads * parts blocks of the launch make the records of the decay factors instead, 8 bytes of dynamic LDS per chunk
 // (the kernel below waits for both anyway): D, which P needs, depends on its own chunk only, and every wave forms its 8 rows
@@ -682,10 +686,10 @@ __global__ __launch_bounds__(DVS * 2 + 128) __attribute__((amdgpu_waves_per_eu(2
 // records (5.6 us and the gap behind it), 88.6 like this.  So also in long sequences, where the room of the records' walk in every
 // block's LDS (48 KB with the static part at 131072 positions) takes places from the P blocks: B1 H8 L65536 256/128 5110 and 4988,
 // B1 H8 L131072 256/64 10210 and 9948, B1 H2 L131072 192/64 9938 and 9871.
-template <int KD>
+template <int KD, bool OPS>
 __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __restrict__ q, const float* __restrict__ k,
                                                              const float* __restrict__ decay, char* __restrict__ factors,
-                                                             char* __restrict__ pmat, int heads, int parts, int kdim, int L) {
+                                                             char* __restrict__ pmat, char* __restrict__ ops, int heads, int parts, int kdim, int L) {
   __shared__ __align__(16) f4v part[4][4][64];
   const int records = heads * parts;
   if ((int)blockIdx.x < records) {
@@ -695,37 +699,73 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
   const int lane = threadIdx.x & 63, n = lane & 31, hi = lane >> 5, nchunk = L / 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = xcd_remap(blockIdx.x - records, gridDim.x - records), bh = tile / nchunk, c = tile % nchunk;
-  constexpr int kRows = KD / 4;                       // key dims of one wave
-  const size_t at = ((size_t)bh * kdim + wave * kRows + hi) * L + (size_t)c * 32 + n;
-  const float *qp = q + at, *kp = k + at;
-  float kx[kRows / 2], qx[kRows / 2];
+  constexpr int kUnits = KD / 64;                     // k-steps of 16 key dims of one wave
+  const size_t at = ((size_t)bh * kdim + 16 * kUnits * wave + 4 * hi) * L + (size_t)c * 32 + n;
+  f4v kx[kUnits][2], qx[kUnits][2];                   // rows 16u + 8(j/4) + 4h + j%4 of column n
 #pragma unroll
-  for (int i = 0; i < kRows / 2; ++i) {
-    kx[i] = kp[(size_t)2 * i * L];
-    qx[i] = qp[(size_t)2 * i * L];
+  for (int s = 0; s < kUnits; ++s)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const size_t row = at + (size_t)(16 * s + 8 * (j >> 2) + (j & 3)) * L;
+      kx[s][j >> 2][j & 3] = k[row];
+      qx[s][j >> 2][j & 3] = q[row];
+    }
+  // OPS: K once more, row n of State tiles wave and wave + 4: positions 8g + 4h .. + 3
+  typedef f4v f4v_dword __attribute__((aligned(4)));  // q, k, v may start at any float
+  constexpr int kTiles = KD / 32, kMine = (kTiles + 3) / 4;
+  f4v kr[kMine][4];
+  if constexpr (OPS) {
+#pragma unroll
+    for (int t = 0; t < kMine; ++t) {
+      const int kb = wave + 4 * t < kTiles ? wave + 4 * t : wave % kTiles;
+      const float* const row = k + ((size_t)bh * kdim + 32 * kb + n) * L + (size_t)c * 32 + 4 * hi;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) kr[t][g] = *reinterpret_cast<const f4v_dword*>(row + 8 * g);
+    }
   }
   sched_fence();                                      // all loads in flight before the first product
   const float* const dg = decay + (size_t)(bh % heads) * L + (size_t)c * 32;
-  f4v dsel = {0.f, 0.f, 0.f, 0.f};                    // D of rows 8 wave + 4 hi + e
-  float d = 0.f;
+  f4v dsel = {0.f, 0.f, 0.f, 0.f}, wsel[4];           // D of rows 8 wave + 4 hi + e; w of positions 8g + 4 hi + e
+  float d = 0.f, w = 1.f;
 #pragma unroll
   for (int g = 3; g >= 0; --g) {
     f4v rows[2];
 #pragma unroll
     for (int i = 7; i >= 0; --i) {
       const int m = 8 * g + i;
-      if (m < 31) d *= dg[m + 1];
+      if (m < 31) { d *= dg[m + 1]; w *= dg[m + 1]; }
       d = (m == n) ? 1.f : d;
       rows[i >> 2][i & 3] = d;
+      if constexpr (OPS) wsel[g][i & 3] = i >= 4 ? w : hi ? wsel[g][i & 3] : w;
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) dsel[e] = g == wave ? (hi ? rows[1][e] : rows[0][e]) : dsel[e];
   }
   f16v sp = zero16();
 #pragma unroll
-  for (int i = 0; i < kRows / 2; ++i) sp = mfma_32x32x2_f32(kx[i], qx[i], sp);
+  for (int s = 0; s < kUnits; ++s) sp = rec_mma<true>(rec_op<true>(kx[s][0], kx[s][1]), rec_op<true>(qx[s][0], qx[s][1]), sp);
 #pragma unroll
-  for (int g = 0; g < 4; ++g) part[wave][g][lane] = f4v{sp[4 * g], sp[4 * g + 1], sp[4 * g + 2], sp[4 * g + 3]};
+  for (int g = 0; g < 4; ++g) part[wave][g][lane] = rec_quarter(sp, 4 * g);
+  if constexpr (OPS) {
+    char* const mine = ops + ((size_t)bh * nchunk + c) * (2 * KD / 16) * 3072 + lane * 16;
+    const float pn = d * dg[0];
+#pragma unroll
+    for (int s = 0; s < kUnits; ++s) {
+      const RecOp<false> o = rec_op<false>(qx[s][0] * pn, qx[s][1] * pn);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<u4v*>(mine + (wave * kUnits + s) * 3072 + p * 1024) = o.p[p];
+    }
+#pragma unroll
+    for (int t = 0; t < kMine; ++t)
+      if (wave + 4 * t < kTiles) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const RecOp<false> o = rec_op<false>(kr[t][2 * s] * wsel[2 * s], kr[t][2 * s + 1] * wsel[2 * s + 1]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) *reinterpret_cast<u4v*>(mine + (KD / 16 + 2 * (wave + 4 * t) + s) * 3072 + p * 1024) = o.p[p];
+        }
+      }
+  }
   __syncthreads();
   f4v x = part[0][wave][lane];
 #pragma unroll
@@ -1049,6 +1089,284 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
       for (int e = 0; e < 4; ++e) orow[s][(size_t)e * L + (size_t)(nchunk - 1) * T::kChunk] = x[e];
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------------
+// The split scan with the operands of Q and K made once per (batch, head) ahead of it: retnet_recurrent_pmat leaves them in memory
+// in the order the matrix instructions take them (Q times p_n, K times w_m, three bf16 parts each), and every wave reads those of
+// its own key dims straight into registers, a chunk ahead.  V, P and the factors come through LDS, requested three chunks ahead by
+// a wave of their own, which also adds up and stores the waves' partial sums of O^T: a wave's loads return in order, and one that
+// comes from memory holds up every one behind it.
+//
+// Bound by the chain of a chunk in one wave per SIMD: 52 matrix instructions (24 below 192 key dims) = 1800 (1024) of some 3000 (2600)
+// cycles, the rest the barrier, LDS latency and vector work that a result of the chunk has to wait for; with 256 blocks of 256 key dims the
+// operands, 96 KB per block and chunk from L2, add 15 us of 80.  Whole calls, the split kernel above and this one with its launch ahead:
+// B2 H8 L2048 128/128 135 -> 84 us, B1 H8 L2048 256/128 152 -> 106, B4 H16 L2048 64/128 139 -> 112, B2 H8 L1056 256/512 87.2 -> 79.7.
+// Tried and not kept: 32 key dims per wave, eight waves (B2 H8 L1056 256/512 94); the operands brought into L2 by the data wave's touches
+// (91 against 79 without); partial sums added and stored by the matrix waves (+8); V read straight into registers (+6).
+template <int KD, int WK>
+struct RetRecurrentStream {
+  static constexpr int kChunk = 32;
+  static constexpr int kThreads = WK * 64 + 64;
+  static constexpr int kRows = KD / WK;                    // key dims of one wave
+  static constexpr int kKB = kRows / 32;                   // its State tiles
+  static constexpr int kSteps = 2 * kKB;                   // its k-steps over the key dims; as many (State tile, k-step over the positions)
+  static constexpr int kOwn = (4 + WK - 1) / WK;           // row groups of a C tile it adds up (the last may not exist)
+  static constexpr int kOpBytes = 2 * (KD / 16) * 3072;    // per (batch, head, chunk)
+  static constexpr int kPOff = 4096, kFOff = 8192;
+  static constexpr int kStage = kFOff + kRecFactorBytes - kRecFactorW;      // V, P and the factors (all but D) of one chunk
+  static constexpr int kStages = 4;
+  static constexpr int kSumOff = kStages * kStage;         // two buffers of a partial O^T tile per wave
+  static constexpr int kSmemBytes = kSumOff + 2 * WK * 4096;
+  static_assert(KD % (32 * WK) == 0 && WK >= 2 && WK <= 4 && kKB <= 2, "one or two State tiles per wave");
+};
+
+template <bool FP32, int KD, int WK>
+AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                             const char* __restrict__ factors, const char* __restrict__ pmat, const char* __restrict__ ops,
+                             float* __restrict__ out, int heads, int kdim, int vdim, int L) {
+  using T = RetRecurrentStream<KD, WK>;
+  using Op = RecOp<FP32>;
+  typedef f4v f4v_dword __attribute__((aligned(4)));       // k may start at any float
+
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = xcd_remap(blockIdx.x, gridDim.x), slices = vdim / 32;
+  const int bh = tile / slices, vd0 = tile % slices * 32, h = bh % heads;
+  const int nchunk = L / T::kChunk;
+  const uint32_t lane16 = lane * 16;
+  const char* const og = ops + (size_t)bh * nchunk * T::kOpBytes;
+
+  if (wave == WK) {
+    const char* const vg = reinterpret_cast<const char*>(v + ((size_t)bh * vdim + vd0) * L);
+    const char* const pg = pmat + (size_t)bh * nchunk * 4096;
+    const char* const fg = factors + (size_t)h * nchunk * kRecFactorBytes + kRecFactorW;
+    const int orl = lane >> 3, occ = lane & 7;
+    uint32_t voff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) voff[i] = (uint32_t)((8 * i + rec_pos(orl)) * L * 4 + (occ ^ (((i & 1) << 2) | (orl >> 1))) * 16);
+    const auto copy = [&](const char* g_uniform, uint32_t lane_off, char* lds) {
+      const uint64_t base = (uint64_t)(uintptr_t)g_uniform;
+      const uint32_t dst = (uint32_t)(uintptr_t)(AAT_AS3 char*)lds;
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :: "v"(lane_off), "s"(base), "s"(dst) : "memory", "m0");
+    };
+    const auto request = [&](int c) {
+      char* const s = smem + c % T::kStages * T::kStage;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) copy(vg + (size_t)c * T::kChunk * 4, voff[i], s + i * 1024);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) copy(pg + (size_t)c * 4096 + i * 1024, lane16, s + T::kPOff + i * 1024);
+      copy(fg + (size_t)c * kRecFactorBytes, lane16, s + T::kFOff);
+    };
+    // Output tile of chunk c: the waves' partial sums, registers of a C tile.
+    f4v x[4];
+    const auto add_sums = [&](int c) {
+      const char* const part = smem + T::kSumOff + (c & 1) * WK * 4096 + lane16;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) x[g] = *reinterpret_cast<const f4v*>(part + g * 1024);
+#pragma unroll
+      for (int t = 1; t < WK; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) x[g] += *reinterpret_cast<const f4v*>(part + t * 4096 + g * 1024);
+    };
+    uint32_t ooff[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) ooff[r] = (uint32_t)((8 * (r >> 2) + 4 * hi + (r & 3)) * L + n) * 4;
+    const auto store = [&](int c) {
+      const uint64_t base = (uint64_t)(uintptr_t)(out + ((size_t)bh * vdim + vd0) * L + (size_t)c * T::kChunk);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) asm volatile("global_store_dword %0, %1, %2" :: "v"(ooff[r]), "v"(x[r >> 2][r & 3]), "s"(base) : "memory");
+    };
+    for (int c = 0; c < 3 && c < nchunk; ++c) request(c);
+    if (nchunk > 2) wait_vmcnt<9>();
+    else wait_vmcnt<0>();
+    block_sync();                                          // chunks 0 and 1 have landed
+    for (int c = 0; c < nchunk; ++c) {
+      if (c + 3 < nchunk) request(c + 3);
+      if (c > 0) {
+        add_sums(c - 1);
+        store(c - 1);
+      }
+      // chunk c + 2 has landed: younger than its copies are the stores of two chunks and the copies of chunk c + 3
+      if (c > 1 && c + 3 < nchunk) wait_vmcnt<16 + 9 + 16>();
+      else wait_vmcnt<0>();
+      block_sync();
+    }
+    add_sums(nchunk - 1);
+    store(nchunk - 1);
+    wait_vmcnt<0>();
+    return false;
+  }
+
+  int own[T::kOwn];                                        // this wave's row groups; a missing one repeats its first, with P = V = 0
+#pragma unroll
+  for (int s = 0; s < T::kOwn; ++s) own[s] = wave + s * WK < 4 ? wave + s * WK : wave;
+  const float last = WK != 3 || wave + (T::kOwn - 1) * WK < 4 ? 1.f : 0.f;
+  const char* const og_mine = og + wave * T::kSteps * 3072 + lane16;
+  const int cp = rec_pos(n);
+
+  const auto read_q = [&](int ks, int c) {
+    Op o;
+    if constexpr (FP32) {
+      const float* const row = q + ((size_t)bh * kdim + wave * T::kRows + 16 * ks + 4 * hi) * L + (size_t)c * 32 + n;
+      f4v x[2];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j >> 2][j & 3] = row[(size_t)(8 * (j >> 2) + (j & 3)) * L];
+      o = rec_op<FP32>(x[0], x[1]);
+    } else {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) o.p[p] = *reinterpret_cast<const u4v*>(og_mine + (size_t)c * T::kOpBytes + ks * 3072 + p * 1024);
+    }
+    return o;
+  };
+  const auto read_k = [&](int u, int c) {                  // k-step u%2 over the positions of State tile u/2
+    Op o;
+    if constexpr (FP32) {
+      const float* const row = k + ((size_t)bh * kdim + wave * T::kRows + 32 * (u >> 1) + n) * L + (size_t)c * 32 + 16 * (u & 1) + 4 * hi;
+      o = rec_op<FP32>(*reinterpret_cast<const f4v_dword*>(row), *reinterpret_cast<const f4v_dword*>(row + 8));
+    } else {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) o.p[p] = *reinterpret_cast<const u4v*>(og_mine + (size_t)c * T::kOpBytes + (KD / 16 + u) * 3072 + p * 1024);
+    }
+    return o;
+  };
+  const auto stage_of = [&](int c) { return smem + c % T::kStages * T::kStage; };
+  const auto v_at = [&](const char* sm, int g) { return *reinterpret_cast<const f4v*>(sm + cp * 128 + rec_slot(cp, 2 * g + hi) * 16); };
+  f16v st[T::kKB], oacc = zero16();                        // State / lambda; T^T Q of the chunk that comes next, 0 for the first
+#pragma unroll
+  for (int i = 0; i < T::kKB; ++i) st[i] = zero16();
+  RecFinite finite;
+  Op qop[T::kSteps], kop[T::kSteps], vop[2];               // of the next chunk and of this one
+  // in the order of their first uses: what the compiler waits for at the top of the loop is the worse of this order and the loop's
+#pragma unroll
+  for (int i = 0; i < T::kSteps; ++i) {
+    kop[i] = read_k(i, 0);
+    sched_fence();
+  }
+#pragma unroll
+  for (int i = 0; i < T::kSteps; ++i) {
+    qop[i] = read_q(i, nchunk > 1 ? 1 : 0);
+    sched_fence();
+  }
+  block_sync();                                            // chunks 0 and 1 have landed
+  f4v vx[4], fx;                                           // V, and rescale flag, scale, lambda, 1 / lambda'
+  const auto read_v = [&](const char* sm) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) vx[g] = v_at(sm, g);
+    fx = *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorFlag - kRecFactorW);
+  };
+  const auto make_v = [&](const char* sm, int s) {         // of V w / lambda'; K has the w already, FP32: it has not
+    const auto x = [&](int g) {
+      if constexpr (FP32) return vx[g] * *reinterpret_cast<const f4v*>(sm + T::kFOff + hi * 64 + g * 16);
+      else return vx[g] * fx[3];
+    };
+    return rec_op<FP32>(x(2 * s), x(2 * s + 1));
+  };
+  read_v(stage_of(0));
+  vop[0] = make_v(stage_of(0), 0);
+  vop[1] = make_v(stage_of(0), 1);
+
+  // A step of the loop updates the State with chunk c, finishes chunk c's output and contracts the new State with chunk c+1's Q.
+  // Every operand read ahead is used once and then read again for a chunk later in its place; behind the first branch the
+  // step is one basic block, or the compiler moves those reads to its end.  Vector work goes between matrix instructions that do
+  // not wait for it: the parts of a State tile that is done between those of the next one's update, those of the next chunk's V between the last
+  // of T^T Q.
+  for (int c = 0; c < nchunk; ++c) {
+    const int next = c + 1 < nchunk ? c + 1 : nchunk - 1, next2 = c + 2 < nchunk ? c + 2 : nchunk - 1;
+    const char* const sm = stage_of(c);
+    const float lam = fx[2];
+    if (__builtin_amdgcn_readfirstlane(__float_as_uint(fx[0])) != 0u) {     // lambda left its range: fold it into T
+#pragma unroll
+      for (int kb = 0; kb < T::kKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[kb][i] *= fx[1];
+    }
+
+    // ---- T += K diag(w / lambda') V^T
+    f4v vo[T::kOwn], pm[T::kOwn];
+#pragma unroll
+    for (int t = 0; t < T::kOwn; ++t) {
+      vo[t] = v_at(sm, own[t]);
+      pm[t] = *reinterpret_cast<const f4v*>(sm + T::kPOff + own[t] * 1024 + lane16);
+    }
+    Op top[T::kSteps];
+    static_for<T::kSteps>([&](auto it) {
+      constexpr int u = decltype(it)::value, kb = u >> 1, s = u & 1;
+      if constexpr (u == 0) {
+        if constexpr (FP32) {
+          const float pnl = *reinterpret_cast<const float*>(sm + T::kFOff + kRecFactorPnl - kRecFactorW + n * 4);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[r] *= pnl;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[r] *= lam;
+        }
+      }
+      if constexpr (u >= 2) {
+        top[u - 2] = rec_op_of_c<FP32>(st[0], u - 2);
+        rec_pin(top[u - 2]);
+      }
+      st[kb] = rec_mma<FP32>(kop[u], vop[s], st[kb]);
+      rec_interleave<FP32, 0, u == 0 ? 3 : 8>();
+      kop[u] = read_k(u, next);
+    });
+
+    // ---- O^T = (p_n lambda) T^T Q + V P, over this wave's key dims and positions, and T^T Q of the next chunk
+#pragma unroll
+    for (int t = 0; t < T::kOwn; ++t) {
+      const f4v a = t + 1 < T::kOwn ? vo[t] : vo[t] * last, b = t + 1 < T::kOwn ? pm[t] : pm[t] * last;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) oacc = mfma_32x32x2_f32(a[e], b[e], oacc);
+    }
+    read_v(stage_of(next));
+    constexpr int kMade = T::kSteps - 2;                   // operands of T made so far
+    top[kMade] = rec_op_of_c<FP32>(st[T::kKB - 1], 0);
+    rec_pin(top[kMade]);
+    sched_fence();
+    f16v tq = zero16();
+    static_for<T::kSteps>([&](auto it) {
+      constexpr int ks = decltype(it)::value;
+      if constexpr (ks == 0) {
+        top[kMade + 1] = rec_op_of_c<FP32>(st[T::kKB - 1], 1);
+        rec_pin(top[kMade + 1]);
+      }
+      if constexpr (ks == T::kSteps - 2 && ks > 0) {
+        vop[0] = make_v(stage_of(next), 0);
+        rec_pin(vop[0]);
+      }
+      if constexpr (ks == T::kSteps - 1) {
+        if constexpr (T::kSteps == 2) {
+          vop[0] = make_v(stage_of(next), 0);
+          rec_pin(vop[0]);
+        }
+        vop[1] = make_v(stage_of(next), 1);
+        rec_pin(vop[1]);
+      }
+      tq = rec_mma<FP32>(top[ks], qop[ks], tq);
+      rec_interleave<FP32, 0, T::kSteps == 2 && ks == 1 ? 16 : 8>();
+      qop[ks] = read_q(ks, next2);
+      if constexpr (ks == 0) {
+        finite.see(oacc);
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f4v*>(smem + T::kSumOff + (c & 1) * WK * 4096 + wave * 4096 + g * 1024 + lane16) = rec_quarter(oacc, 4 * g);
+      }
+    });
+    oacc = tq;
+    block_sync();              // chunk c's partial sums are there; chunk c-1's, which the next step overwrites, have been read
+  }
+  return finite.broken();
+}
+
+// Grid: B * H * vdim / 32 blocks, the slices of one (batch, head) on one XCD (they read the same operands).
+template <int KD, int WK>
+__global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void retnet_recurrent_stream_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const char* __restrict__ factors,
+    const char* __restrict__ pmat, const char* __restrict__ ops, float* __restrict__ out, int heads, int kdim, int vdim, int L) {
+  extern __shared__ __align__(16) char smem[];
+  const bool broken = rec_stream_scan<false, KD, WK>(smem, q, k, v, factors, pmat, ops, out, heads, kdim, vdim, L);
+  if (rec_any_wave(smem, broken)) rec_stream_scan<true, KD, WK>(smem, q, k, v, factors, pmat, ops, out, heads, kdim, vdim, L);
 }
 
 }  // namespace aat

@@ -21,6 +21,8 @@ from ..autotuner.runtime import KernelLaunchError
 _ERRORS = {-2: "unsupported shape: L must be a multiple of 32 (at most 131072), block_kdim a multiple of 64 up to 256 "
                "and <= kdim, vdim a multiple of 64",
            -3: "workspace missing or too small"}
+# What a call allocates for itself at most to have K and Q laid out ahead of the scan; a workspace handed in is used as it is.
+_MOST_WORKSPACE = 1 << 30
 
 
 def _library(device_type):
@@ -55,7 +57,8 @@ def retnet_recurrent_fwd(q, k, v, decay, device_type=None, block_kdim=None, out=
     assert out.shape == v.shape and out.dtype == torch.float32 and out.is_contiguous() and out.device == v.device
     need = int(lib.retnet_recurrent_workspace_size(batch, nheads, kdim, vdim, seqlen, block_kdim))
     if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
+        room = int(lib.retnet_recurrent_room(batch, nheads, kdim, vdim, seqlen, block_kdim, _MOST_WORKSPACE))
+        workspace = torch.empty(max(need, room, 1), dtype=torch.uint8, device=q.device)
     with torch.cuda.device(q.device):
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         rc = lib.retnet_recurrent_fwd_ex(*[ctypes.c_void_p(t.data_ptr()) for t in (q, k, v, decay, out)], batch, nheads, kdim,

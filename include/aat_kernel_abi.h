@@ -205,6 +205,13 @@ int retnet_recurrent_fwd_noalloc(const float* q, const float* k, const float* v,
 size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most);
 #endif
 
+#if defined(AAT_OP_RET_RECURRENT)
+/* Bytes of workspace that retnet_recurrent_fwd_ex makes use of for this problem: retnet_recurrent_workspace_size() and, from 512
+ * positions on where it pays, the operands of K and Q made once per (batch, head) (12 bytes per key dim and position), unless they
+ * take more than `most` bytes.  They are optional; results with and without them differ by the order of fp32 additions. */
+size_t retnet_recurrent_room(int batch, int heads, int kdim, int vdim, int l, int block_kdim, size_t most);
+#endif
+
 #ifdef __cplusplus
 }
 #endif

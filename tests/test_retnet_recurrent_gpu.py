@@ -325,3 +325,94 @@ def test_values_beyond_the_largest_of_bf16(which, kdim, vdim):
     assert torch.isfinite(out).all()
     _close(out[3, 5], ref[3, 5])
     _close(out[3, 4], ref[3, 4])
+
+
+def _room(b, h, kdim, vdim, seqlen, most=1 << 40):
+    lib = library.load_recurrent(codegen.compile_config(RetRecurrentConfig(), ARCH))
+    need = lib.retnet_recurrent_workspace_size(b, h, kdim, vdim, seqlen, kdim)
+    return need, lib.retnet_recurrent_room(b, h, kdim, vdim, seqlen, kdim, ctypes.c_size_t(most))
+
+
+# operands of K and Q made ahead of the scan: every number of key dims (192: three waves, the first with two row groups), the fewest chunks that
+# take it, odd and even counts, decays that are 0, negative and that drive the carried product out of its range, against the recurrence
+@pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(1, 2, 64, 64, 512), (1, 3, 64, 192, 544), (2, 2, 128, 64, 576), (1, 2, 128, 320, 544),
+                                                   (1, 2, 192, 64, 544), (2, 1, 192, 128, 512), (1, 2, 256, 64, 512), (1, 3, 256, 128, 544)])
+def test_operands_made_ahead(b, h, kdim, vdim, seqlen):
+    need, room = _room(b, h, kdim, vdim, seqlen)
+    assert room > need                                    # the call has the room and takes it
+    q, k, v, decay = _inputs(25, b, h, kdim, vdim, seqlen, 0.6, 1.05)
+    decay[0, seqlen // 2] = 0.0
+    decay[0, 1::97] = -0.9
+    decay[-1, 64:128] = 0.05                              # leaves the range at once
+    shifted = torch.zeros(h * seqlen + 1, device="cuda")[1:].view(h, seqlen).copy_(decay)
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), shifted)
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(h):
+        _close(out[:, head], ref[:, head])
+    # without the room, and one byte short of it, the split kernel runs; the results differ by the order of additions
+    for nbytes in (need, room - 1):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        held = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda(), workspace=ws)
+        for head in range(h):
+            _close(held[:, head], ref[:, head])
+
+
+def test_the_room_is_offered_where_it_pays_and_not_beyond_what_is_asked_for():
+    for dims in [(2, 8, 256, 512, 1056), (1, 4, 64, 64, 512)]:
+        need, room = _room(*dims)
+        assert room > need and _room(*dims, most=room) == (need, room) and _room(*dims, most=room - 1) == (need, need)
+    for dims in [(8, 32, 128, 128, 2048), (1, 4, 64, 64, 480), (8, 16, 256, 64, 1024)]:
+        need, room = _room(*dims)
+        assert room == need
+    assert _room(1, 4, 64, 64, 500) == (0, 0)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+@pytest.mark.parametrize("kdim", [64, 128, 192, 256])
+def test_values_that_are_not_finite_with_operands_made_ahead(value, which, kdim):
+    b, h, vdim, seqlen, pos = 2, 2, 64, 544, 262
+    assert _room(b, h, kdim, vdim, seqlen)[1] > _room(b, h, kdim, vdim, seqlen)[0]
+    q, k, v, decay = _inputs(26, b, h, kdim, vdim, seqlen, 0.9, 1.0)
+    clean = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    bad = dict(q=q, k=k, v=v)
+    bad[which] = bad[which].clone()
+    bad[which][1, 1, 7, pos] = value
+    out = aat.retnet_recurrent_fwd(bad["q"].cuda(), bad["k"].cuda(), bad["v"].cuda(), decay.cuda())
+    rows = slice(7, 8) if which == "v" else slice(None)
+    last = pos + 1 if which == "q" else seqlen
+    assert not torch.isfinite(out[1, 1, rows, pos:last]).any()
+    _close(out[1, 1, :, :256], clean[1, 1, :, :256].cpu())
+    if which == "q":
+        _close(out[1, 1, :, 288:], clean[1, 1, :, 288:].cpu())
+    out[1, 1], clean[1, 1] = 0.0, 0.0
+    assert torch.equal(out, clean)
+
+
+def test_operands_made_ahead_keep_the_range_of_fp32_and_replay():
+    """Magnitudes over 12 decades along the key dims; then the call in a graph, replayed with eager work in between."""
+    b, h, kdim, vdim, seqlen = 1, 2, 128, 64, 512
+    q, k, v, decay = _inputs(27, b, h, kdim, vdim, seqlen, 0.9, 1.0)
+    per_dim = 10.0 ** ((torch.arange(kdim) * 37 % kdim / (kdim - 1.0) - 0.5) * 12).view(1, 1, kdim, 1)
+    q, k, v, decay = (q * per_dim).float().cuda(), (k / per_dim).float().cuda(), v.cuda(), decay.cuda()
+    out = aat.retnet_recurrent_fwd(q, k, v, decay)
+    ref = torch.from_numpy(brute.retnet_recurrent(*(t.cpu().numpy() for t in (q, k, v, decay))))
+    for head in range(h):
+        _close(out[:, head], ref[:, head])
+    ws = torch.empty(_room(b, h, kdim, vdim, seqlen)[1], dtype=torch.uint8, device="cuda")
+    got = torch.empty_like(v)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        aat.retnet_recurrent_fwd(q, k, v, decay, out=got, workspace=ws)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        aat.retnet_recurrent_fwd(q, k, v, decay, out=got, workspace=ws)
+    for _ in range(3):
+        got.zero_(), ws.fill_(255)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, out)
+        _ = (q * 2).sum().item()
