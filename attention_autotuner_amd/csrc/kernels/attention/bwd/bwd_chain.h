@@ -314,7 +314,38 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
     constexpr bool kVacc = WPE == 1 && (kFitsVec || RT * ((kOut1 ? DT : 0) + (kOut2 ? KT + NT : 0) + NT) * 16 > 256);
     f16v s[RT][NT], dp[RT][kOut2 ? NT : 1];
     qk_gemm_steps<RT, NT, KS, NCK, PF, kVacc>(s, x1f, y1addr, off, [](int) {});
-    if constexpr (kOut2) qk_gemm_steps<RT, NT, DS, NCD, PF, kVacc>(dp, x2f, y2addr, off, [](int) {});
+    // FUSE: the element-wise work rides in the shadow of matrix instructions -- P = exp2(S c2 - lse2) behind those of dP,
+    // dS = P (dP - delta) behind those of dV -- where a phase of its own left the matrix cores idle: of 4800 clocks per
+    // 64-row tile at d 128 that phase was 1093, the matrix instructions need 2048.  Now dP 985, dV 904 (747 and 720 alone: an
+    // LDS read and a vector instruction of one wave do not overlap), the rest of the phase 235 on the tiles of a causal walk,
+    // 4219 in all with one settle per contraction.  B4 H32 S2048 causal 582 -> 559 us (573 of the settle alone), not causal
+    // 987 -> 945, B16 S512 263 -> 254, B2 H16 S1024 68 -> 63.  Not with 192 or more output accumulators: it spills there.
+    constexpr bool FUSE = kVacc && RT == 1 && kOut1 && kOut2 && DT + KT < 12 && 16 % DS == 0 && 16 % (2 * DT) == 0;
+    f4v rows[FUSE ? NT * 4 : 1];                    // lse2, then delta, of the tile's rows: group i is rows 32 (i/4) + 8 (i%4) + 4h ..
+    const auto read_rows = [&](int first) {
+      static_for<FUSE ? NT * 4 : 0>([&](auto it) {
+        constexpr int i = decltype(it)::value;
+        rows[i] = lds_read_f4_async(stat_addr, off + (first + 32 * (i / 4) + 8 * (i % 4)) * 4);
+      });
+    };
+    const auto rows_landed = [&]() {                // older than the reads of the contraction, whose first step has waited for its own
+#pragma unroll
+      for (int i = 0; i < NT * 4; ++i) asm volatile("" : "+v"(rows[i]));
+    };
+    if constexpr (FUSE) {
+      read_rows(0);
+      qk_gemm_steps<RT, NT, DS, NCD, PF, kVacc>(dp, x2f, y2addr, off, [&](int step) {
+        constexpr int kPer = 16 / DS;
+        if (step == 0) rows_landed();
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+          const int v = step * kPer + i;
+          s[0][v / 16][v % 16] = fast_exp2(s[0][v / 16][v % 16] * c2 - rows[v / 4][v % 4]);
+        }
+      });
+    } else if constexpr (kOut2) {
+      qk_gemm_steps<RT, NT, DS, NCD, PF, kVacc>(dp, x2f, y2addr, off, [](int) {});
+    }
 
     // P = exp2(s*c2 - lse2[q]),  dS = P * (dP - delta[q]);  register v of tile t is streamed row 32t + 8(v/4) + 4h + v%4.
     // Only a tile the diagonal crosses runs the masking code.  COL: the statistics of the streamed rows come
@@ -371,21 +402,44 @@ attn_bwd_chain(const half_t* __restrict__ x1, const half_t* __restrict__ x2, con
         }
       });
     };
-    if (diag_tile) softmax_part(std::true_type{});
-    else softmax_part(std::false_type{});
+    if constexpr (FUSE) {
+      if (diag_tile) {                              // the mask of softmax_part on the finished P
+        const int lim = GEN && !causal ? -BY : x0 + wave * WM + n - diag - jt * BY - 4 * h, have = seq_y - jt * BY - 4 * h;
+#pragma unroll
+        for (int v = 0; v < NT * 16; ++v) {
+          const int c = 32 * (v / 16) + 8 * (v % 16 / 4) + v % 4;
+          if (lim > c || (GEN && c >= have)) s[0][v / 16][v % 16] = 0.f;
+        }
+      }
+      read_rows(BY);
+    } else {
+      if (diag_tile) softmax_part(std::true_type{});
+      else softmax_part(std::false_type{});
+    }
 
     // second contractions: COL  dV^T += dO^T P  and  dK^T += Q^T dS;   ROW  dQ^T += K^T dS
     h8 ef[RT][NT][2];
     constexpr bool TAIL = GEN && NT > 1;
     const int live = (seq_y - jt * BY) / 16;        // GEN: groups of 16 streamed rows that exist
     if constexpr (kOut1) {
-      pv_gemm_steps_hl<RT, NT, DT, NCD, PF, false, TAIL>(acc1, ef, z2lo, z2hi, off, [&](int g) {
+      pv_gemm_steps_hl<RT, NT, DT, NCD, PF, FUSE, TAIL>(acc1, ef, z2lo, z2hi, off, [&](int g) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) ef[rt][g >> 1][g & 1] = pack8_rne(s[rt][g >> 1], 8 * (g & 1));
-      }, live);
+      }, live, [&](auto step_tag) {
+        if constexpr (FUSE) {
+          constexpr int step = decltype(step_tag)::value, kPer = 16 / (2 * DT);
+          if constexpr (step == 0) rows_landed();
+#pragma unroll
+          for (int i = 0; i < kPer; ++i) {
+            constexpr int v0 = step * kPer;
+            const int v = v0 + i;
+            dp[0][v / 16][v % 16] = s[0][v / 16][v % 16] * (dp[0][v / 16][v % 16] - rows[v / 4][v % 4]);
+          }
+        }
+      });
     }
     if constexpr (kOut2) {
-      pv_gemm_steps_hl<RT, NT, KT, NCK, PF, false, TAIL>(acc2, ef, z1lo, z1hi, off, [&](int g) {
+      pv_gemm_steps_hl<RT, NT, KT, NCK, PF, FUSE, TAIL>(acc2, ef, z1lo, z1hi, off, [&](int g) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) ef[rt][g >> 1][g & 1] = pack8_rne(dp[rt][g >> 1], 8 * (g & 1));
       }, live);

@@ -160,9 +160,16 @@ AAT_DEV void mfma_32x32x16_vacc_first(f16v& c, h8 a, h8 b) {
 AAT_DEV void mfma_32x32x16_vacc(f16v& c, h8 a, h8 b) {
   asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }
-// 24 wait states: more than the 16 passes + 3 the longest matrix instruction needs before another unit
-// may read its result.
-AAT_DEV void mfma_settle(f16v& c) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(c)); }
+// 12 wait states: what another unit has to leave between this matrix instruction (8 passes) and a read of its result, and
+// what the compiler leaves behind its own.  The tiles of a contraction are settled together, by one wait behind the last
+// instruction: 24 states for each of two tiles were 192 of the 746 clocks of a 64 x 32 x 128 contraction.
+template <int RT, int NT> AAT_DEV void mfma_settle(f16v (&c)[RT][NT]) {
+  asm volatile("s_nop 11" : "+v"(c[RT - 1][NT - 1]));
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(c[rt][nt]));
+}
 
 // S^T = K Q^T over one kv tile.  kaddr[ks] = LDS address of this lane's chunk for k-step ks in score
 // tile 0 of the K buffer (tile nt adds nt*32 rows).  side(step) runs after the MFMA group of each step.
@@ -232,12 +239,7 @@ AAT_DEV void qk_gemm_steps(f16v (&sacc)[RT][NT], const h8 (&qf)[RT][KS], const u
     side(step);
     sched_fence();
   });
-  if constexpr (VACC) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) mfma_settle(sacc[rt][nt]);
-  }
+  if constexpr (VACC) mfma_settle(sacc);
 }
 
 // O^T += V^T P^T over one kv tile.  vlo[dt] / vhi[dt] = LDS addresses this lane presents to the two
@@ -252,9 +254,13 @@ AAT_DEV void qk_gemm_steps(f16v (&sacc)[RT][NT], const h8 (&qf)[RT][KS], const u
 // buf_off must fold to a constant.
 // TAIL: only the first `live` groups of 16 rows exist (wave-uniform, 2 or more).  The others hold copies of rows that do, and
 // a zero P would keep them out of the sums only while they are finite: 0 * inf is NaN.  Their MFMAs are branched around.
-template <int RT, int NT, int DT, int NCV, int PF, bool BLIND = false, bool TAIL = false, class Pack>
+// side(step), step as a constant, runs behind the MFMAs of each step (the caller's element-wise work in their shadow).
+struct NoSide {
+  template <class I> AAT_DEV void operator()(I) const {}
+};
+template <int RT, int NT, int DT, int NCV, int PF, bool BLIND = false, bool TAIL = false, class Pack, class Side = NoSide>
 AAT_DEV void pv_gemm_steps_hl(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const uint32_t (&vlo)[DT],
-                              const uint32_t (&vhi)[DT], int buf_off, Pack&& pack, int live = 2 * NT) {
+                              const uint32_t (&vhi)[DT], int buf_off, Pack&& pack, int live = 2 * NT, Side&& side = Side{}) {
   constexpr int G = NT * 2;              // groups of 16 kv rows
   constexpr int S = G * DT;
   constexpr int kRow16 = 16 * NCV * 16;
@@ -283,6 +289,7 @@ AAT_DEV void pv_gemm_steps_hl(f16v (&oacc)[RT][DT], h8 (&pf)[RT][NT][2], const u
       if (!TAIL || g < 2 || g < live) oacc[rt][dt] = mfma_32x32x16(vf, pf[rt][g / 2][g % 2], oacc[rt][dt]);
     }
     if constexpr (dt == 0 && g + 1 < G) pack(g + 1);
+    side(step_tag);
     sched_fence();
   });
 }
