@@ -4,13 +4,18 @@ The reference has no such wrapper (its attention operator's ``backward`` is empt
 python/ops/attention_interface.py:37-58); the layout follows its RetNet backward wrapper
 (csrc/kernels/retnet/bwd/profile_code.py:1-119).  One library launches two kernels: the row kernel (dQ), which also
 leaves delta = rowsum(dO * O) and lse in base-2 units in the workspace, and the column kernel (dV, dK), which reads them;
-with ``col_split`` the column kernel runs twice, once per output.
+with ``col_split`` the column kernel runs twice, once per output.  At 128 wide heads a column kernel with 256-row blocks
+(bwd_col.h) takes the grids that fill the chip.
 """
 
 global_vars = r"""
 #define AAT_OP_ATTN_BWD 1
 #include "aat_kernel_abi.h"
 #include "kernels/attention/bwd/bwd_chain.h"
+#define AAT_COL_WIDE ({Kd} == 128 && {D} == 128 && {Br} == 128 && {col_split} == 0)   // has the column kernel of 256-row blocks
+#if AAT_COL_WIDE
+#include "kernels/attention/bwd/bwd_col.h"
+#endif
 #include "kernels/utils/host_launch.h"
 
 namespace {{
@@ -45,6 +50,18 @@ bool whole_tiles(int Seq_q, int Seq_k) {{
   return Seq_q % Br == 0 && Seq_k % Br == 0 && Seq_q % Bc == 0 && Seq_k % BcRow == 0;
 }}
 int blocks_of(int rows) {{ return (rows + Br - 1) / Br; }}
+#if AAT_COL_WIDE
+// Whether 256-row column blocks are the faster ones: one takes 1.6 times as long as one of 128 rows and either fills a compute
+// unit, so it is the rounds of blocks over the 256 units that decide.  Measured at 6 lengths from 256 to 8192 and 8 to 512 heads, whole
+// backward, 256-row / 128-row blocks: 2 rounds for 4, 3 for 6, 4 for 8 take 0.93 to 0.95 of the time, one for two 0.92 to 0.94, 3
+// for 5 1.01, 2 for 3 1.03 to 1.05, one for one 1.21 to 1.33.  The blocks of a causal walk differ in length and the longest ones
+// decide as long as there are few: 256 blocks 1.03 to 1.2 (0.93 only at length 256), 384 0.97 to 1.06, 512 and more 0.94 to 0.97.
+bool wide_columns(int BH, int Seq_k, int causal) {{
+  constexpr long kUnits = 256;
+  const long wide = (long)BH * ((Seq_k + aat::AttnBwdCol::BX - 1) / aat::AttnBwdCol::BX), narrow = (long)BH * blocks_of(Seq_k);
+  return 5 * ((wide + kUnits - 1) / kUnits) < 3 * ((narrow + kUnits - 1) / kUnits) && (!causal || wide >= 2 * kUnits);
+}}
+#endif
 size_t stats_bytes(int B, int H, int Seq_q) {{ return (size_t)2 * B * H * Seq_q * sizeof(float); }}
 
 template <int GEN> hipError_t launch_kernels(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* dO, float* lse, aat_half* dq,
@@ -75,6 +92,16 @@ template <int GEN> hipError_t launch_kernels(aat_half* q, aat_half* k, aat_half*
   kernel_dk<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
       K, V, Q, G, nullptr, nullptr, lse2, delta, nullptr, reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #else
+#if AAT_COL_WIDE
+  if (wide_columns(B * H, Seq_k, causal)) {{
+    using W = aat::AttnBwdCol;
+    static const hipError_t ok3 = aat::allow_lds(aat::attn_bwd_col, W::kSmemBytes);
+    if (ok3 != hipSuccess) return ok3;
+    aat::attn_bwd_col<<<dim3(B * H * ((Seq_k + W::BX - 1) / W::BX)), dim3(W::Nthreads), W::kSmemBytes, stream>>>(
+        K, V, Q, G, lse2, delta, reinterpret_cast<H16*>(dv), reinterpret_cast<H16*>(dk), Seq_k, Seq_q, c2, softmax_scale, causal);
+    return hipGetLastError();
+  }}
+#endif
   kernel_col<GEN><<<dim3(B * H * blocks_of(Seq_k)), dim3(Nthreads), TC::kSmemBytes, stream>>>(
       K, V, Q, G, nullptr, nullptr, lse2, delta, reinterpret_cast<H16*>(dv), reinterpret_cast<H16*>(dk), H, Seq_k, Seq_q, c2, softmax_scale, causal);
 #endif

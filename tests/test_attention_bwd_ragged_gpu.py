@@ -54,6 +54,17 @@ def test_two_row_groups_per_wave_and_one_column_kernel_per_output(causal):
         _check(problem, 256, 512, causal, 350 + i, wide)
 
 
+# Heads enough for column blocks of 256 rows (130 or more blocks, 512 when causal): a last block with five 32-row groups, with six, whole
+# blocks, two blocks per head; one query tile, several; either side the longer one
+@pytest.mark.parametrize("problem,causal", [((10, 13, 96, 160), False), ((10, 13, 32, 256), False), ((5, 13, 64, 416), False),
+                                            ((16, 32, 160, 160), True), ((16, 32, 288, 192), True), ((16, 32, 96, 256), True),
+                                            ((8, 32, 352, 416), True)])
+def test_column_blocks_of_256_rows(problem, causal):
+    cfgs = [c for c in gfx950_space.rule_attn_backward_configs(128, 128) if c.Br == 128 and not c.col_split]
+    assert cfgs
+    _check(problem, 128, 128, causal, 370, cfgs[:1])
+
+
 @pytest.mark.parametrize("d", sorted(p[0] for p in gfx950_space.ATTN_BWD_RULE))
 def test_an_infinite_gradient_in_the_last_partial_tile_stays_an_infinity(d):
     """dV = P^T dO; the query rows a tile does not have are copies of its first 32 with P = 0, and 0 * inf must not reach dV."""
