@@ -408,7 +408,7 @@ def backward_reg_estimate(cfg):
     return vec, acc
 
 
-DS_ROWS = (128, 256)          # kv rows per block of the dK kernel that reads a stored dS (64-row query tiles, two stages)
+DS_ROWS = (128, 256)          # kv rows per block of the dK kernel that reads a stored dS (64-row query tiles, two stages or more)
 DS_TILE = 64
 
 

@@ -264,7 +264,7 @@ int main(int argc, char** argv) {
   HIP_OK(hipMalloc(&t.scan, aat::mask_extent_bytes(ps.H, ps.Sq, ps.Sk)));
   HIP_OK(hipMalloc(&t.ds, (size_t)ps.B * ps.H * ps.Sq * ps.Sk * sizeof(half_t)));
 
-  test_retnet_bwd_stored_ds<128, 64, 256, 1, 1, 128, 64, 256, 2, 2>(ps, t);
+  test_retnet_bwd_stored_ds<128, 64, 256, 1, 1, 128, 64, 512, 3, 2>(ps, t);
   test_retnet_bwd_stored_ds<128, 32, 256, 1, 1, 256, 64, 512, 2, 2>(ps, t);
   test_retnet_bwd_stored_ds<128, 64, 256, 1, 1, 256, 64, 512, 2, 2>(ps, t);
   test_retnet_bwd<128, 32, 256, 3, 2, 1>(ps, t);

@@ -28,20 +28,29 @@
 
 namespace aat {
 
-// Kd: width of q/k rows; BX: kv rows per block (32 per wave); BY: query rows per streamed tile; NS: LDS stages.
+// What bounds it is the stream of dS: at B4 H8 S2048 d_qk 256 the causal walk takes 52 us for 142 MB of it, the dense one 90 for 268.
+// Measured without effect on that: two to five tiles in flight (48 to 120 KB), tiles of 32 rows, half the LDS reads (64 kv rows per wave).
+// Where LDS has no room for a second block beside one of four waves with two stages (d_qk 256, 96 KB), a block has eight waves and three
+// stages: 56 -> 52 us causal, 98 -> 91 dense.
+// Looking the writer's ranges up per tile, through loads that drained all copies in flight, cost the walks with ranges more: 86 -> 54.
+//
+// NWD waves share 32 kv rows, Kd / NWD columns of dK each.
+// Kd: width of q/k rows; BX: kv rows per block; BY: query rows per streamed tile; NS: LDS stages, all but one of them on their way.
 template <int Kd, int BX, int BY, int Nthreads, int NS>
 struct RetBwdDk {
-  static constexpr int NW = Nthreads / kWave;
-  static constexpr int DT = Kd / 32, KSTEPS = BY / 16;
+  static constexpr int NW = Nthreads / kWave, NWK = BX / 32, NWD = NW / NWK;
+  static constexpr int DTW = Kd / 32 / NWD, KSTEPS = BY / 16;
   static constexpr int NCZ = Kd / 8, NCS = 8, NSUB = BX / 64;
-  static_assert(Nthreads % kWave == 0 && BX == 32 * NW, "one 32-row group of kv per wave");
-  static_assert(BY == 64 && Kd % 64 == 0 && BX % 64 == 0, "a query tile is one row of dS blocks");
-  static_assert(NS == 2 || NS == 3, "buffers");
+  static_assert(NWD * NWK * kWave == Nthreads && DTW * NWD * 32 == Kd, "32 kv rows by whole 32-column tiles per wave");
+  static_assert((BY == 64 || BY == 32) && Kd % 64 == 0 && BX % 64 == 0, "a query tile is a row of dS blocks or half of one");
+  static_assert(NS >= 2, "buffers");
   using ZDma = TileDma<BY, NCZ, Nthreads, Swz::Rows4>;   // Q tile
-  using SDma = TileDma<BY * NSUB, NCS, Nthreads, Swz::Rows4, 2>;   // dS tile: NSUB consecutive blocks of BY query rows x 64 kv columns
+  static constexpr int kSIters = BY * NSUB * NCS / Nthreads, kSRows = Nthreads / NCS;   // dS tile: LDS-DMA instructions per thread, rows per instruction
+  static_assert(kSIters * Nthreads == BY * NSUB * NCS, "whole 32-row pieces of dS blocks per instruction");
   static constexpr int kZBytes = BY * Kd * 2, kSBytes = BY * BX * 2;
   static constexpr int kStageBytes = kZBytes + kSBytes;
-  static constexpr int kTileInstr = ZDma::kIters + SDma::kIters;
+  static constexpr int kTileInstr = ZDma::kIters + kSIters;
+  static_assert((NS - 2) * kTileInstr < 64, "copies in flight are counted by a 6-bit counter");
   static constexpr int kOStride = Kd * 2 + 16;
   static constexpr int kMainBytes = NS * kStageBytes;
   static constexpr int kEpiBytes = BX * kOStride;
@@ -58,12 +67,13 @@ __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(W
 ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, half_t* __restrict__ dk, int H,
                    int seq_k, int seq_q, int causal, const int* __restrict__ extents, int wr_rows, int wr_cols, BlockParts in_parts = {}) {
   using T = RetBwdDk<Kd, BX, BY, Nthreads, NS>;
-  constexpr int DT = T::DT, KSTEPS = T::KSTEPS, NCZ = T::NCZ, NCS = T::NCS;
+  constexpr int DTW = T::DTW, KSTEPS = T::KSTEPS, NCZ = T::NCZ, NCS = T::NCS;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave % T::NWK, wd = wave / T::NWK;      // the wave's 32 kv rows and its share of the columns
   const int n = lane & 31, h = lane >> 5;
 
   const int Tx = GEN ? (seq_k + BX - 1) / BX : seq_k / BX;
@@ -91,139 +101,148 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
     j_begin = first <= 0 ? 0 : first / BY;
     part_range(id, j_begin, j_end);
   }
-  // walked downwards from the end of the sequence, like the column passes of the chained kernel
-  const auto tile_of = [&](int j) { return j_begin + j_end - 1 - j; };
 
   const char* zg = reinterpret_cast<const char*>(q + (size_t)bh * seq_q * Kd);
   const char* sg = reinterpret_cast<const char*>(ds + ds_block_offset(bh, 0, x0, seq_q, seq_k));
   const size_t s_pitch = (size_t)(seq_k >> 6) * 8192;    // from one row of blocks to the next
   typename T::ZDma zdma;
-  typename T::SDma sdma;
   zdma.init(tid);
-  sdma.init(tid);
   const int wave_base = wave * 64;
-  auto issue = [&](int j, int st) {
-    const int jt = tile_of(j);
+  // dS: LDS row r of the tile is row r % BY of block r / BY; a wave copies eight rows at a time
+  const uint32_t s_lane = (uint32_t)(lane / NCS * 128 + swz<NCS, Swz::Rows4>(lane / NCS, lane % NCS) * 16);
+  auto issue = [&](int jt, int st) {              // walked downwards from the end of the sequence, like the column passes of the chained kernel
     char* base = smem + st * T::kStageBytes;
     zdma.issue(zg + (size_t)jt * T::kZBytes, base, wave_base);
-    if constexpr (GEN) sdma.issue_rows(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base, cols / 64 * BY);   // the dS blocks that exist
-    else sdma.issue(sg + (size_t)jt * s_pitch, base + T::kZBytes, wave_base);
+    const char* const rows = sg + (size_t)(jt * BY / 64) * s_pitch + jt * BY % 64 * 128;
+#pragma unroll
+    for (int i = 0; i < T::kSIters; ++i) {
+      const int r = i * T::kSRows + wave * (kWave / NCS), sub = r / BY;
+      uint64_t src = (uint64_t)(uintptr_t)(rows + r % BY * 128 + (!GEN || sub * 64 < cols ? sub * 8192 : 0));   // a block that does not exist: copies of the first
+      asm volatile("" : "+s"(src));
+      __builtin_amdgcn_global_load_lds((const AAT_AS1 void*)(uintptr_t)(src + s_lane),
+                                       (AAT_AS3 void*)(base + T::kZBytes + (i * Nthreads + wave_base) * 16), 16, 0, 2);
+    }
   };
 
   // LDS addresses inside stage 0: Q^T fragments (A operand, d-tile dt) and this wave's dS columns (B operand);
   // both are transposing reads of rows 4h + (lane%16)/4 of a 16-row step, + 8 rows for the second half
-  uint32_t zaddr[DT], saddr;
+  uint32_t zaddr[DTW], saddr;
   {
-    int zoff[DT];
-    v_frag_offsets<DT, NCZ>(zoff, lane);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) zaddr[dt] = lds_addr(smem + zoff[dt]);
     const int s16 = lane & 15;
-    const int row = (wave >> 1) * 64 + 4 * h + (s16 >> 2);         // block wave/2 of the tile, 64 rows each
-    const int col = (wave & 1) * 32 + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
-    saddr = lds_addr(smem + T::kZBytes + lds_chunk_off<NCS, Swz::Rows4>(row, col >> 3) + (col & 7) * 2);
+    const int row = 4 * h + (s16 >> 2), col = 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
+#pragma unroll
+    for (int dt = 0; dt < DTW; ++dt)
+      zaddr[dt] = lds_addr(smem + lds_chunk_off<NCZ, Swz::Rows4>(row, 4 * (wd * DTW + dt) + (col >> 3)) + (col & 7) * 2);
+    saddr = lds_addr(smem + T::kZBytes + lds_chunk_off<NCS, Swz::Rows4>((wk >> 1) * BY + row, 4 * (wk & 1) + (col >> 3)) + (col & 7) * 2);
   }
   constexpr int kZRow16 = 16 * NCZ * 16, kZRow8 = 8 * NCZ * 16, kSRow16 = 16 * NCS * 16, kSRow8 = 8 * NCS * 16;
 
-  f16v acc[1][DT];
+  f16v acc[1][DTW];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) acc[0][dt] = zero16();
+  for (int dt = 0; dt < DTW; ++dt) acc[0][dt] = zero16();
 
-  if (j_begin < j_end) {
-    issue(j_begin, 0);
-    if constexpr (NS == 3) {
-      if (j_begin + 1 < j_end) issue(j_begin + 1, 1);
-    }
-  }
-  const int my_kv = x0 + wave * 32 + n;           // the kv position this lane owns
-
-  auto q_tile = [&](const int j, auto st_tag) {
-    constexpr int st = decltype(st_tag)::value;
-    constexpr int off = st * T::kStageBytes;
-    const bool more = (j + 1 < j_end);
-    if constexpr (NS == 3) {
-      if (more) wait_vmcnt<T::kTileInstr>();
-      else wait_vmcnt<0>();
-    } else {
-      wait_vmcnt<0>();
-    }
-    block_sync();
-    if constexpr (NS == 3) {
-      if (j + 2 < j_end) issue(j + 2, (st + 2) % 3);
-    } else {
-      if (more) issue(j + 1, st ^ 1);
-    }
-
-    // the kv range the writer covered for the row block this query tile lies in
-    const int jt = tile_of(j);
-    const int wx0 = (jt * BY) / wr_rows * wr_rows;
+  const int my_kv = x0 + wk * 32 + n;             // the kv position this lane owns
+  // The kv range that the writer covered for the row block a query tile lies in.  Lane i holds that of row block 64 w + i, for the 64
+  // the walk is in: looked up per tile, the ranges' loads drained every copy in flight.
+  int window = -1, lane_lo = 0, lane_hi = seq_k;
+  int wr = (j_end * BY - 1) / wr_rows;            // row block of the current tile
+  const auto load_ranges = [&]() {
+    window = wr >> 6;
+    const int wx0 = (window * 64 + lane) * wr_rows;
     const int wrows = GEN && seq_q - wx0 < wr_rows ? seq_q - wx0 : wr_rows;
-    int wlo = 0, whi = seq_k;
-    if (extents != nullptr) {
-      int lo, hi, jb, je;
-      mask_row_range(ext, head, seq_q, wx0, wrows, lo, hi);
-      mask_tile_range(lo, hi, wr_cols, seq_k / wr_cols, jb, je);
-      wlo = jb * wr_cols;
-      whi = je * wr_cols;
-    } else if (causal) {
-      const int last = wx0 + wrows - 1 + diag;
-      const int lim = last < 0 ? 0 : last / wr_cols + 1;
-      whi = lim * wr_cols < seq_k ? lim * wr_cols : seq_k;
+    lane_lo = 0;
+    lane_hi = seq_k;
+    if (wx0 < seq_q) {
+      if (extents != nullptr) {
+        int lo, hi, jb, je;
+        mask_row_range(ext, head, seq_q, wx0, wrows, lo, hi);
+        mask_tile_range(lo, hi, wr_cols, seq_k / wr_cols, jb, je);
+        lane_lo = jb * wr_cols;
+        lane_hi = je * wr_cols;
+      } else if (causal) {
+        const int last = wx0 + wrows - 1 + diag;
+        const int lim = last < 0 ? 0 : last / wr_cols + 1;
+        lane_hi = lim * wr_cols < seq_k ? lim * wr_cols : seq_k;
+      }
     }
-    const bool all_written = wlo <= x0 && x0 + cols <= whi;        // block-uniform (rows that do not exist are not stored)
+    asm volatile("" : "+v"(lane_lo), "+v"(lane_hi));      // waited for here
+  };
+  if (j_begin < j_end) load_ranges();
+
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (j_end - 1 - i >= j_begin) issue(j_end - 1 - i, i);
+
+  int st = 0;
+  for (int jt = j_end - 1; jt >= j_begin; --jt) {
+    if (jt - j_begin >= NS - 2) wait_vmcnt<(NS - 2) * T::kTileInstr>();
+    else wait_vmcnt<0>();
+    block_sync();
+    if (jt - (NS - 1) >= j_begin) issue(jt - (NS - 1), st == 0 ? NS - 1 : st - 1);
+
+    if (jt * BY < wr * wr_rows) --wr;
+    if (wr >> 6 != window) load_ranges();
+    const int wlo = __builtin_amdgcn_readlane(lane_lo, wr & 63), whi = __builtin_amdgcn_readlane(lane_hi, wr & 63);
     const bool mine_written = my_kv >= wlo && my_kv < whi;
 
     // The operand reads are issued as instructions with counted waits (tile_ops.h): in front of an LDS read it can see
-    // the compiler waits for every LDS-DMA copy in flight, i.e. for the next tile this one has just requested.
-    constexpr int PF = 2;
-    static_for<KSTEPS>([&](auto s_tag) {
-      constexpr int s = decltype(s_tag)::value;
-      h4 blo = lds_read_tr_h4_async(saddr, off + s * kSRow16);
-      h4 bhi = lds_read_tr_h4_async(saddr, off + s * kSRow16 + kSRow8);
-      h4 lo[PF], hi[PF];
+    // the compiler waits for every LDS-DMA copy in flight.  All of the tile's B operands are read ahead of its A operands.
+    const uint32_t off = st * T::kStageBytes, sa = saddr + off;
+    uint32_t za[DTW];
 #pragma unroll
-      for (int i = 0; i < PF && i < DT; ++i) {
-        lo[i] = lds_read_tr_h4_async(zaddr[i], off + s * kZRow16);
-        hi[i] = lds_read_tr_h4_async(zaddr[i], off + s * kZRow16 + kZRow8);
+    for (int dt = 0; dt < DTW; ++dt) za[dt] = zaddr[dt] + off;
+    constexpr int S = KSTEPS * DTW, PF = S < 4 ? S : 4;
+    h4 blo[KSTEPS], bhi[KSTEPS], lo[PF], hi[PF];
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) {
+      blo[s] = lds_read_tr_h4_async(sa, s * kSRow16);
+      bhi[s] = lds_read_tr_h4_async(sa, s * kSRow16 + kSRow8);
+    }
+#pragma unroll
+    for (int i = 0; i < PF; ++i) {
+      lo[i] = lds_read_tr_h4_async(za[i % DTW], i / DTW * kZRow16);
+      hi[i] = lds_read_tr_h4_async(za[i % DTW], i / DTW * kZRow16 + kZRow8);
+    }
+    h8 bf;
+    static_for<S>([&](auto i_tag) {
+      constexpr int i = decltype(i_tag)::value, dt = i % DTW;
+      // wait on the slot, take its value, refill it (a copy made before the wait could read a register whose load
+      // has not landed); the B pairs are older: they have landed too
+      lds_wait_younger<2 * ((i + PF - 1 < S) ? PF - 1 : S - 1 - i)>(lo[i % PF], hi[i % PF]);
+      const h4 clo = lo[i % PF], chi = hi[i % PF];
+      if constexpr (i + PF < S) {
+        lo[i % PF] = lds_read_tr_h4_async(za[(i + PF) % DTW], (i + PF) / DTW * kZRow16);
+        hi[i % PF] = lds_read_tr_h4_async(za[(i + PF) % DTW], (i + PF) / DTW * kZRow16 + kZRow8);
       }
-      h8 bf;
-      static_for<DT>([&](auto dt_tag) {
-        constexpr int dt = decltype(dt_tag)::value;
-        // wait on the slot, take its value, refill it (a copy made before the wait could read a register whose load
-        // has not landed); the B pair is older: it has landed too
-        lds_wait_younger<2 * ((dt + PF - 1 < DT) ? PF - 1 : DT - 1 - dt)>(lo[dt % PF], hi[dt % PF]);
-        h4 clo = lo[dt % PF], chi = hi[dt % PF];
-        if constexpr (dt + PF < DT) {
-          lo[dt % PF] = lds_read_tr_h4_async(zaddr[dt + PF], off + s * kZRow16);
-          hi[dt % PF] = lds_read_tr_h4_async(zaddr[dt + PF], off + s * kZRow16 + kZRow8);
-        }
-        if constexpr (dt == 0) {
-          asm volatile("" : "+v"(blo), "+v"(bhi));
-          bf = cat_h4(blo, bhi);
-          if (!all_written) {
-            if (!mine_written) {
+      if constexpr (dt == 0) {
+        constexpr int s = i / DTW;
+        asm volatile("" : "+v"(blo[s]), "+v"(bhi[s]));
+        bf = cat_h4(blo[s], bhi[s]);
 #pragma unroll
-              for (int e = 0; e < 8; ++e) bf[e] = (half_t)0.f;
-            }
-          }
-        }
-        acc[0][dt] = mfma_32x32x16(cat_h4(clo, chi), bf, acc[0][dt]);
-      });
+        for (int e = 0; e < 8; ++e) bf[e] = mine_written ? bf[e] : (half_t)0.f;
+      }
+      acc[0][dt] = mfma_32x32x16(cat_h4(clo, chi), bf, acc[0][dt]);
     });
-  };
-  for (int j = j_begin; j < j_end; j += NS) {
-    static_for<NS>([&](auto k_tag) {
-      constexpr int k = decltype(k_tag)::value;
-      if (k == 0 || j + k < j_end) q_tile(j + k, std::integral_constant<int, k>{});
-    });
+    st = st == NS - 1 ? 0 : st + 1;
   }
 
   wait_vmcnt<0>();
   block_sync();
-  const auto finish = [&]() {
-    const float one[1] = {1.f};
-    store_o_tile<1, DT, Kd, T::kOStride>(acc, one, smem + wave * 32 * T::kOStride,
-                                         dk + ((size_t)bh * seq_k + x0 + wave * 32) * Kd, lane, 32, !GEN || wave * 32 < cols ? 1 : 0);
+  const auto finish = [&]() {                     // the waves' columns meet in LDS, rows leave whole
+#pragma unroll
+    for (int dt = 0; dt < DTW; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const h2 a = pack_rne(acc[0][dt][4 * g], acc[0][dt][4 * g + 1]), b = pack_rne(acc[0][dt][4 * g + 2], acc[0][dt][4 * g + 3]);
+        h4 w;
+        w[0] = a[0]; w[1] = a[1]; w[2] = b[0]; w[3] = b[1];
+        *reinterpret_cast<h4*>(smem + (wk * 32 + n) * T::kOStride + (32 * (wd * DTW + dt) + 8 * g + 4 * h) * 2) = w;
+      }
+    __syncthreads();
+    char* const out = reinterpret_cast<char*>(dk + ((size_t)bh * seq_k + x0) * Kd);
+#pragma unroll 4
+    for (int c = tid; c < (GEN ? cols : BX) * NCZ; c += Nthreads)
+      *reinterpret_cast<u4v*>(out + (size_t)c * 16) = *reinterpret_cast<const u4v*>(smem + c / NCZ * T::kOStride + c % NCZ * 16);
   };
   if (id.parts > 1) {                             // to the end in here: joined again, the two paths' accumulators cost 68 bytes of scratch
     float none[1];

@@ -32,7 +32,10 @@ constexpr int num_stages_dq = {num_stages_dq};
 constexpr int waves_per_eu = {waves_per_eu};
 constexpr int ds_rows = {ds_rows};               // 0, or kv rows per block of the dK kernel that reads a stored dS
 constexpr bool kStoredDs = ds_rows != 0;
-constexpr int kDkRows = kStoredDs ? ds_rows : 128, kDkTile = 64, kDkStages = 2, kDkWaves = 2;
+// The dK kernel has four waves for 128 kv rows and two stages, eight and three where a second such block would not fit into LDS.
+constexpr int kDkRows = kStoredDs ? ds_rows : 128, kDkTile = 64, kDkWaves = 2;
+constexpr bool kDkAlone = kDkRows == 128 && 4 * kDkTile * (Kd + kDkRows) * 2 > 160 * 1024;
+constexpr int kDkThreads = kDkAlone ? 512 : kDkRows * 2, kDkStages = kDkAlone ? 3 : 2;
 // dV columns per block: the whole row when the accumulators fit the 256 accumulation registers that one
 // wave per SIMD has to itself, else 256-column slices over grid.y (each repeats the first contraction).
 constexpr int RTv = Br / (Nthreads / 64) / 32;
@@ -48,9 +51,9 @@ template <bool DECAY, int GEN> constexpr auto kernel_dv = &aat::ret_bwd_chain<Kd
 template <bool DECAY, int GEN> constexpr auto kernel_dk = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Col, waves_per_eu, GEN, DECAY, false>;
 template <bool DECAY, int GEN> constexpr auto kernel_dq = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, GEN, DECAY, false>;
 // stored dS: the row pass that writes it (the plain one again in a library without it), the dK kernel that reads it
-using TKD = aat::RetBwdDk<Kd, kDkRows, kDkTile, kDkRows * 2, kDkStages>;
+using TKD = aat::RetBwdDk<Kd, kDkRows, kDkTile, kDkThreads, kDkStages>;
 template <bool DECAY, int GEN> constexpr auto kernel_dq_ds = &aat::ret_bwd_chain<D, Kd, DKB, Br, Bc, Nthreads, num_stages_ds, num_stages_dq, BwdPass::Row, waves_per_eu, GEN, DECAY, kStoredDs>;
-template <int GEN> constexpr auto kernel_dk_ds = &aat::ret_bwd_dk_from_ds<Kd, kDkRows, kDkTile, kDkRows * 2, kDkStages, kDkWaves, GEN>;
+template <int GEN> constexpr auto kernel_dk_ds = &aat::ret_bwd_dk_from_ds<Kd, kDkRows, kDkTile, kDkThreads, kDkStages, kDkWaves, GEN>;
 static_assert(!kStoredDs || Br % kDkTile == 0, "a query tile of the dK kernel lies inside one block of the row pass");
 
 // The longest blocks of a decay walk in parts (utils/block_parts.h), where the call has room for their slots behind its other
@@ -59,7 +62,7 @@ constexpr bool kPartsFit = aat::parts_fit(RTv, Bc, waves_per_eu, 0);
 using PV = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DVB, Nthreads, 0, false, DVB == 512>;
 using PQ = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, true, DKB == 512>;
 using PK = aat::PartsLaunch<kPartsFit, Br, Bc, Kd + D, DKB, Nthreads, 0, false, DKB == 512>;
-using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkRows * 2, 0, false, false, 109>;    // it streams dS as well
+using PKD = aat::PartsLaunch<true, kDkRows, kDkTile, Kd, Kd, kDkThreads, 0, false, false, 109, kDkRows / 32>;    // it streams dS as well
 struct BwdPlan {{
   aat::PartsPlan dv, dq, dk;
   size_t counts, slots;
@@ -72,7 +75,7 @@ BwdPlan plan_of(int B, int H, int Seq_q, int Seq_k, bool stored) {{
   BwdPlan p{{}};
   if (D == DVB) p.dv = PV::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TV::kSmemBytes));
   p.dq = PQ::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, row_lds));
-  p.dk = stored ? PKD::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(kDkRows / 32, kDkWaves, TKD::kSmemBytes))
+  p.dk = stored ? PKD::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(kDkThreads / 64, kDkWaves, TKD::kSmemBytes))
                 : PK::find(heads, Seq_q, Seq_k, aat::blocks_per_cu(waves, waves_per_eu, TK::kSmemBytes));
   if (p.dv.gain_us + p.dq.gain_us + p.dk.gain_us < aat::kPrepareUs) return BwdPlan{{}};
   const size_t dk = stored ? PKD::slot_bytes(heads, p.dk) : PK::slot_bytes(heads, p.dk);
@@ -165,7 +168,7 @@ template <bool DECAY> hipError_t launch_passes(aat_half* q, aat_half* k, aat_hal
     H16* ds = reinterpret_cast<H16*>(static_cast<char*>(workspace) + ds_offset(H, Seq_q, Seq_k));
     (whole_q ? kernel_dq_ds<DECAY, 0> : kernel_dq_ds<DECAY, 1>)<<<dim3(grid(blocks_of(Seq_q), dq_parts), Kd / DKB), dim3(Nthreads), TQ::kSmemBytesDsOut, stream>>>(
         G, V, K, M, r, DQ, H, Seq_k, Seq_q, causal, log2_gamma, extents, ds, dq_parts);
-    (whole_q && Seq_k % kDkRows == 0 ? kernel_dk_ds<0> : kernel_dk_ds<1>)<<<dim3(grid((Seq_k + kDkRows - 1) / kDkRows, dk_parts)), dim3(kDkRows * 2), TKD::kSmemBytes, stream>>>(
+    (whole_q && Seq_k % kDkRows == 0 ? kernel_dk_ds<0> : kernel_dk_ds<1>)<<<dim3(grid((Seq_k + kDkRows - 1) / kDkRows, dk_parts)), dim3(kDkThreads), TKD::kSmemBytes, stream>>>(
         Q, ds, DK, H, Seq_k, Seq_q, causal, extents, Br, Bc, dk_parts);
   }} else {{
     (whole_k ? kernel_dk<DECAY, 0> : kernel_dk<DECAY, 1>)<<<dim3(grid(blocks_of(Seq_k), dk_parts), Kd / DKB), dim3(Nthreads), TK::kSmemBytes, stream>>>(

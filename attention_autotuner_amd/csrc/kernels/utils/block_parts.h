@@ -411,7 +411,8 @@ class PlanMemory {
 
 // One kind of launch of a library (FIT: its kernel can): its plan, found once per problem, and the order of the plan's jobs.  MEMORY:
 // by how much the launch's tiles are slower than their matrix work (percent).  NUMBERED: the kernel's output tile is in numbered registers.
-template <bool FIT, int Br, int Bc, int Width, int Cols, int Nthreads, int Extra, bool ROWS, bool NUMBERED, int MEMORY = 100>
+// WAVES: for the cost, where a block's waves do not set the rate of its tiles.
+template <bool FIT, int Br, int Bc, int Width, int Cols, int Nthreads, int Extra, bool ROWS, bool NUMBERED, int MEMORY = 100, int WAVES = Nthreads / 64>
 struct PartsLaunch {
   static constexpr int kQuads = Br * Cols / (4 * Nthreads);
   static constexpr size_t kSlotBytes = part_floats<kQuads, Extra, Nthreads>() * sizeof(float);
@@ -423,7 +424,7 @@ struct PartsLaunch {
     if (!FIT) return {};
     static PlanMemory known;
     return known.get(heads, Seq_q, Seq_k, blocks_per_cu, [=] {
-      const PartsCost cost{MEMORY / 100.0 * 2.0 * Br * Bc * Width / 4.5e6, Nthreads / 64, blocks_per_cu, kQuads / parts_at_once(kQuads, NUMBERED), kSlotBytes};
+      const PartsCost cost{MEMORY / 100.0 * 2.0 * Br * Bc * Width / 4.5e6, WAVES, blocks_per_cu, kQuads / parts_at_once(kQuads, NUMBERED), kSlotBytes};
       return plan_parts(heads, blocks(Seq_q, Seq_k), walk(Seq_q, Seq_k), cost);
     });
   }

@@ -472,6 +472,24 @@ def test_backward_with_a_stored_ds_agrees_with_the_one_that_evaluates_it_twice(d
     _grads_close("stored dS decay rates", got, q, k, v, exact, do, r_ref)
 
 
+@pytest.mark.parametrize("sq", [4096, 4288])
+def test_stored_ds_of_64_row_blocks_and_more(sq):
+    """The dK kernel keeps the ranges of 64 row blocks of the dQ pass at a time: exactly 64, and three more; every row block's range differs from
+    its neighbours'."""
+    with_ds, plain = (parity_matrix.ret_bwd_stored_ds_config(64, 128, 64, 32, 128, rows) for rows in (128, 0))
+    b, h, sk = 1, 2, 256
+    q, k, v, do, _, _ = _decay_problem(b, h, sq, sk, 64, 128, seed=sq)
+    row, col = torch.arange(sq).view(1, sq, 1) // 64, torch.arange(sk).view(1, 1, sk) // 64
+    mask = (((row + row // 64) % 4 != col) * torch.tensor([0.125, 0.25]).view(h, 1, 1)).half()
+    fwd = Runtime(ARCH, gfx950_space.default_forward_config("ret", 64, 128, ARCH, sq, sk))
+    _, r_ref = ref_op.retnet_ref(q, k, v, mask, return_r=True)
+    dev = [t.cuda() for t in (q, k, v, mask, do)] + [r_ref.cuda().contiguous()]
+    for mode in (False, "scanned"):
+        got, want = (_bwd_through(cfg, dev, mode, scan_of=fwd) for cfg in (with_ds, plain))
+        assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2]), mode
+        _grads_close(f"stored dS, {sq} rows, walk={mode}", got, q, k, v, mask, do, r_ref)
+
+
 def test_without_room_for_ds_the_library_evaluates_it_twice():
     """The reference-signature entry points have no workspace to give, and a caller of the others may give a small one or
     none: dK then comes from the chained pass, and the results are those of the library built without the stored dS."""
