@@ -676,10 +676,12 @@ def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, pr
 # (few blocks, many blocks) per pair of head sizes, as arguments of AttnBwdConfig behind the head sizes.  Blocks of 64 resident
 # rows are two waves, two of them to a CU; blocks of 128 are four waves that share one stream.  Up to 512 blocks of 64 rows the
 # smaller ones spread over more CUs (B3 H8 S1344 d 128: 112 us against 114 with two more blocks of 128 rows than there are CUs,
-# d 192 156 against 235), beyond that the larger ones stream less (B4 H32 S1984 d 128 non-causal: 1026 against 1027 ... 1148).
-# A causal walk's blocks are of all lengths, and finer ones end together: the line lies at 1600 there (B6 H20 S832 d 128 123
-# against 131 us).  At d 64 the smaller tile leaves room for four blocks to a CU, which lead beyond the line.  On 34 problems
-# the rule is 1 to 2 % slower on the mean than the best of five to eight shapes.
+# d 192 156 against 235), beyond that the larger ones stream less (B4 H32 S1984 d 128 non-causal: 1026 against 1027 ... 1148), and at
+# d 128 from 256 on where they all fit side by side (0.86 ... 0.91 of the time at 360 to 476 blocks of 64 rows; 1.17 and 1.22 where
+# 260 blocks of 128 rows make a second round).  A causal walk's blocks are of all lengths, and finer ones end together: the line lies
+# at 1600 there (from 600 to 1600 blocks the larger ones take 0.99 ... 1.10 of the time at 352 to 2112 rows).  At d 64 the smaller tile
+# leaves room for four blocks to a CU, which lead beyond the line; a causal walk of 800 rows and more keeps the larger tile up to 640 blocks
+# (500 to 624: 1.06 ... 1.13 with the smaller one, 0.86 and 0.92 at 352 and 544 rows).
 ATTN_BWD_RULE = {
     (64, 64): (dict(Br=64, Bc=64, Nthreads=128, num_stages_qk=2, row_waves_per_eu=2, row_Bc=64),
                dict(Br=64, Bc=32, Nthreads=128, num_stages_qk=2, waves_per_eu=2, row_waves_per_eu=2)),
@@ -700,7 +702,10 @@ def rule_attn_backward_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
     if not pair or seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
         return None
     blocks = b * h * -(-seq_k // 64)
-    return pair[blocks > (1600 if causal and dim_qk > 64 else 512)]
+    if causal:
+        return pair[blocks > (1600 if dim_qk > 64 else 640 if seq_k >= 800 else 512)]
+    side_by_side = dim_qk == 128 and blocks > 256 and b * h * -(-seq_k // 128) <= 256
+    return pair[blocks > 512 or side_by_side]
 
 
 # ---- RetNet without a tuned entry ------------------------------------------------------------------------
