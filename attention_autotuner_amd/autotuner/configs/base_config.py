@@ -9,7 +9,8 @@ subclasses, so logs and cache files written by the reference remain readable.
 New on MI355X: ``waves_per_eu`` (resident waves per SIMD the kernel is compiled for),
 ``sw_pipeline`` (software-pipelined schedule: the next tile's first contraction is issued between the
 current tile's exponentials; needs two K and two V buffers) and ``kv_splits`` (number of kv-range
-partitions for long-kv / few-row problems).
+partitions for long-kv / few-row problems) and ``kv_groups`` (waves of a block that share their query rows and take the kv
+units in turn, for launches of few row blocks).
 """
 import os
 
@@ -57,6 +58,7 @@ class BaseConfig:
         self.waves_per_eu = 1
         self.sw_pipeline = 0
         self.kv_splits = 1
+        self.kv_groups = 1
         self.operation = type(self).operation
         self.template_dir = os.path.join(_KERNEL_ROOT, type(self).kernel_subdir) if type(self).kernel_subdir else None
 
@@ -78,6 +80,8 @@ class BaseConfig:
             out.append("p1")
         if getattr(self, "kv_splits", 1) != 1:
             out.append(f"s{self.kv_splits}")
+        if getattr(self, "kv_groups", 1) != 1:
+            out.append(f"g{self.kv_groups}")
         return out
 
     def __repr__(self):
@@ -86,7 +90,7 @@ class BaseConfig:
             body += f",warps_mma1_n={self.warps_mma1_n},warp_mma_n={self.warps_mma_n}"
         extras = self._extras()
         if extras:
-            body += ", " + ", ".join(f"{k}={getattr(self, k)}" for k, d in (("waves_per_eu", 1), ("sw_pipeline", 0), ("kv_splits", 1))
+            body += ", " + ", ".join(f"{k}={getattr(self, k)}" for k, d in (("waves_per_eu", 1), ("sw_pipeline", 0), ("kv_splits", 1), ("kv_groups", 1))
                                      if getattr(self, k, d) != d)
         return f"Config({body})"
 
@@ -112,6 +116,7 @@ class BaseConfig:
         cfg.waves_per_eu = 1
         cfg.sw_pipeline = 0
         cfg.kv_splits = 1
+        cfg.kv_groups = 1
         vars(cfg).update({k: v for k, v in dd.items() if k != "template_dir"})
         cfg.operation = cls.operation
         cfg.template_dir = os.path.join(_KERNEL_ROOT, cls.kernel_subdir)

@@ -29,7 +29,7 @@ def _waves(cfg):
 
 
 def rows_per_wave(cfg):
-    return cfg.Br // _waves(cfg)
+    return cfg.Br * getattr(cfg, "kv_groups", 1) // _waves(cfg)
 
 
 def blocks_per_cu(cfg):
@@ -60,7 +60,8 @@ def forward_lds_bytes(cfg):
         main += (cfg.warps_mma1_n * cfg.Br + cfg.Br) * 4 + 64
         return max(main, cfg.Br * (cfg.D * 2 + 16 * cfg.warps_mma_n))
     epilogue = cfg.Br * (cfg.D * 2 + 16)
-    return max(main, epilogue)
+    handed = (getattr(cfg, "kv_groups", 1) - 1) * cfg.Br * (cfg.D * 4 + 16)      # what waves that share rows hand over
+    return max(main, epilogue, handed)
 
 
 def forward_reg_estimate(cfg):
@@ -116,7 +117,11 @@ def forward_valid(cfg, arch):
     if cfg.fuse_type == "shared":
         if cfg.Nthreads % WAVE or not shared_grid_ok(cfg):
             return False
-    elif cfg.Nthreads % WAVE or cfg.Br % (MFMA_M * _waves(cfg)):
+    elif cfg.Nthreads % WAVE or _waves(cfg) % getattr(cfg, "kv_groups", 1) or cfg.Br % (MFMA_M * (_waves(cfg) // getattr(cfg, "kv_groups", 1))):
+        return False
+    if getattr(cfg, "kv_groups", 1) > 1 and not (cfg.operation == "attn" and cfg.fuse_type == "register" and not cfg.sw_pipeline and cfg.kv_splits == 1 and
+                                                 rows_per_wave(cfg) == MFMA_M and cfg.num_stages_qk == cfg.num_stages_v == 2 and
+                                                 cfg.Bc // unit_rows(cfg) % cfg.kv_groups == 0):
         return False
     if cfg.Bc % 32 or cfg.Kd % 64 or cfg.D % 64:
         return False
@@ -330,6 +335,8 @@ def kv_parts(cfg, arch, b, h, seq_q, seq_k, causal):
     """Into how many parts the library of ``cfg`` cuts the kv range of a problem."""
     if cfg.kv_splits > 1:
         return 1 if causal else cfg.kv_splits
+    if cfg.kv_groups > 1:
+        return 1
     if seq_k < 1024 or b * h * -(-seq_q // cfg.Br) >= 2 * arch.compute_max_core:
         return 1
     return min(range(1, min(64, seq_k // 256) + 1), key=lambda p: forward_estimate_us(cfg, arch, b, h, seq_q, seq_k, causal, p))
@@ -359,11 +366,44 @@ def rule_forward_config(dim_qk, dim_v, arch, b, h, seq_q, seq_k, causal):
     eight waves where K and V stream through once (_streams_once)."""
     if seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
         return None
+    few = few_blocks_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal)
+    if few is not None:
+        return few
     shapes = rule_configs(dim_qk, dim_v)
     if dim_qk + dim_v >= STREAM_WIDTH and _streams_once(b, h, seq_q, seq_k):
         shapes = [c for c in shapes if c.Br == 256 and c.Nthreads == 512] or shapes
     return min(shapes, default=None,
                key=lambda c: forward_estimate_us(c, arch, b, h, seq_q, seq_k, causal, kv_parts(c, arch, b, h, seq_q, seq_k, causal)))
+
+
+# Launches of so few row blocks that one block's walk is their time: 32 rows a block, its waves share them and take the kv units in
+# turn (``kv_groups``).  Per pair of head sizes: (fewest and most kv rows, Bc, threads, waves per SIMD).  Kernel time against the shape
+# taken without them, 165 problems of 2 to 32 heads, 32 to 1536 rows: d 64 0.67 ... 0.98 up to 256 blocks of 32 rows and 0.70 ... 0.82 for the
+# causal walks of 384 and 512 (dense ones 0.9 ... 1.13), d 128 0.62 ... 0.92 up to 256 and 0.8 ... 1.5 beyond.  Short ranges are one tile
+# for every shape: 1.03 ... 1.20 on 128 keys, d 128 0.94 ... 1.08 on 256.  At d 128 a few dozen blocks on 2080 keys lose to kv parts (1.05 ... 1.23),
+# at d 64 they do not (0.82 ... 0.91).  45 problems drawn from these ranges: 0.89 on the mean, 1.02 at most from the shortest range on.
+FEW_BLOCKS = {
+    (64, 64): (160, 2112, 128, 256, 2),
+    (128, 128): (288, 1536, 128, 256, 1),
+}
+
+
+def few_blocks_configs(dim_qk, dim_v):
+    if (dim_qk, dim_v) not in FEW_BLOCKS:
+        return []
+    _, _, bc, nt, wpe = FEW_BLOCKS[dim_qk, dim_v]
+    return [AttnConfig(32, bc, dim_qk, dim_v, dim_qk, 32, 2, 2, nt, True, waves_per_eu=wpe, kv_groups=nt // 64).set_fuse_type("register")]
+
+
+def few_blocks_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
+    """The configuration for an attention forward of few row blocks, or None: a problem with more of them, or of other sizes.  It
+    goes ahead of the entries tuned for other problems, none of which has such a kernel."""
+    cfgs = few_blocks_configs(dim_qk, dim_v)
+    if not cfgs or seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
+        return None
+    least, most = FEW_BLOCKS[dim_qk, dim_v][:2]
+    few = b * h * -(-seq_q // 32) <= (512 if causal and dim_qk == 64 else 256)
+    return cfgs[0] if few and least <= seq_k <= most else None
 
 
 # ---- backward (RetNet) ---------------------------------------------------------------------------------

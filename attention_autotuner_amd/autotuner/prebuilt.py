@@ -37,7 +37,7 @@ def default_configs(arch=None):
             elif op == "attn_bwd":
                 cfgs.append(gfx950_space.default_attn_backward_config(dqk, dv, arch, seq, seq))
         if op == "attn":
-            cfgs += gfx950_space.rule_configs(dqk, dv)
+            cfgs += gfx950_space.rule_configs(dqk, dv) + gfx950_space.few_blocks_configs(dqk, dv)
         if op == "attn_bwd":
             cfgs += gfx950_space.rule_attn_backward_configs(dqk, dv)
         if op == "ret":

@@ -27,14 +27,18 @@ constexpr bool sw_pipeline = {sw_pipeline};      // next tile's QK^T MFMAs inter
 constexpr int unit_rows = sw_pipeline ? Bc : {BlockKSmem2};   // plain schedule: kv rows per scores -> softmax -> PV unit inside a tile of Bc rows
 constexpr float kReferenceScale = 0.125f;        // what the reference kernels hard-code
 
-using Traits = aat::AttnFwdRegfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v>;
+#define AAT_KV_GROUPS {kv_groups}                // > 1: that many waves share their query rows; such a library has one kernel, for any lengths
+using Traits = aat::AttnFwdRegfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, AAT_KV_GROUPS>;
 constexpr int shared_mem = Traits::kSmemBytes;
-const auto kernel = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, sw_pipeline, false>;
-const auto kernel_causal = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, sw_pipeline, true>;
-const auto kernel_causal_paired = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, sw_pipeline, true, false, false, true>;
+#if AAT_KV_GROUPS > 1
+const auto kernel_gen = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, AAT_KV_GROUPS, false, true>;
+#else
+const auto kernel = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, 1, sw_pipeline, false>;
+const auto kernel_causal = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, 1, sw_pipeline, true>;
+const auto kernel_causal_paired = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, 1, sw_pipeline, true, false, false, true>;
 // any lengths that are multiples of 32, causal or not; and the same with the kv range cut into parts
-const auto kernel_gen = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, false, true>;
-const auto kernel_split = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, false, true, true>;
+const auto kernel_gen = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, 1, false, true>;
+const auto kernel_split = &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 1, 1, false, true, true>;
 constexpr int shared_mem_split = Traits::kSmemBytesSplit;
 
 // Persistent variant (a block walks several row blocks, prefetching across them): exists for two K and two V
@@ -49,7 +53,7 @@ using PersistTraits = Traits::Persist<waves_per_eu>;
 constexpr int shared_mem_persist = PersistTraits::kSmemBytes;
 template <bool OK> auto persistent_kernel() {{
   if constexpr (OK)
-    return &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, false, false, false, true>;
+    return &aat::flashattn_fwd_regfuse<Kd, D, Br, Bc, Nthreads, num_stages_qk, num_stages_v, waves_per_eu, unit_rows, 0, 1, false, false, false, true>;
   else
     return static_cast<decltype(kernel)>(nullptr);
 }}
@@ -102,17 +106,22 @@ bool pairs_fill_the_chip(int n) {{
   const int resident = cus * per_cu;
   return n % resident == 0 || n >= 8 * resident;
 }}
+#endif
 
 bool lengths_ok(int B, int H, int Seq_q, int Seq_k) {{ return aat::shape_ok(B, H, Seq_q, Seq_k, 32, 32); }}
-bool whole_tiles(int Seq_q, int Seq_k) {{ return Seq_q % Br == 0 && Seq_k % Bc == 0; }}
+bool whole_tiles(int Seq_q, int Seq_k) {{ return AAT_KV_GROUPS == 1 && Seq_q % Br == 0 && Seq_k % Bc == 0; }}
 int row_blocks(int Seq_q) {{ return (Seq_q + Br - 1) / Br; }}
 
+#if AAT_KV_GROUPS > 1
+int kv_parts(int, int, int, int, int) {{ return 1; }}
+#else
 constexpr aat::ForwardShape kShape = {{Br, Bc, Kd, D, Nthreads / 64, aat::forward_blocks_per_cu(Nthreads / 64, waves_per_eu, shared_mem_split),
                                       (num_stages_qk == 1) + (num_stages_v == 1)}};
 int kv_parts(int B, int H, int Seq_q, int Seq_k, int causal) {{
   if (kv_splits > 1) return causal ? 1 : kv_splits;
   return aat::choose_kv_parts(kShape, B, H, Seq_q, Seq_k, causal);
 }}
+#endif
 size_t split_workspace_bytes(int parts, int B, int H, int Seq_q) {{
   return parts > 1 ? (size_t)parts * B * H * Seq_q * (D + 1) * sizeof(float) : 0;
 }}
@@ -129,6 +138,7 @@ size_t needed_workspace(int B, int H, int Seq_q, int Seq_k, int causal) {{
 hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int H, int Seq_q, int Seq_k,
                   float softmax_scale, int causal, void* workspace, size_t workspace_bytes, hipStream_t stream, float* lse = nullptr) {{
   causal = causal != 0;                          // any value but 0 asks for the causal walk; the general kernel multiplies by it
+#if AAT_KV_GROUPS == 1
   const int parts = kv_parts(B, H, Seq_q, Seq_k, causal);
   if (parts > 1 && workspace != nullptr && workspace_bytes >= split_workspace_bytes(parts, B, H, Seq_q)) {{
     static const hipError_t lds_ok_split = aat::allow_lds(kernel_split, shared_mem_split);
@@ -144,6 +154,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int
         part_o, part_lse, reinterpret_cast<aat::half_t*>(o), lse, (int)rows, parts);
     return hipGetLastError();
   }}
+#endif
   if (!whole_tiles(Seq_q, Seq_k)) {{
     static const hipError_t lds_ok_gen = aat::allow_lds(kernel_gen, shared_mem);
     if (lds_ok_gen != hipSuccess) return lds_ok_gen;
@@ -153,6 +164,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int
         nullptr, 0, causal);
     return hipGetLastError();
   }}
+#if AAT_KV_GROUPS == 1
   const int items = B * H * (Seq_q / Br);
   if (kernel_persist != nullptr && !causal && (Seq_k / Bc) % 2 == 0 && Seq_k <= kPersistMaxKv) {{
     const int resident = resident_blocks();
@@ -178,6 +190,7 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, int B, int
       reinterpret_cast<const aat::half_t*>(q), reinterpret_cast<const aat::half_t*>(k),
       reinterpret_cast<const aat::half_t*>(v), reinterpret_cast<aat::half_t*>(o), lse, H, Seq_k, Seq_q,
       softmax_scale, nullptr, nullptr, 0, causal);
+#endif
   return hipGetLastError();
 }}
 }}  // namespace

@@ -35,16 +35,17 @@
 
 namespace aat {
 
-template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV>
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int KVG = 1>
 struct AttnFwdRegfuse {
   static constexpr int NW = Nthreads / kWave;   // waves per block
-  static constexpr int WM = Br / NW;            // query rows per wave
+  static constexpr int NWR = NW / KVG;          // waves side by side along the rows; KVG waves share theirs
+  static constexpr int WM = Br / NWR;           // query rows per wave
   static constexpr int RT = WM / 32;            // 32-row groups per wave
   static constexpr int NT = Bc / 32;            // score tiles (units) along kv
   static constexpr int KS = Kd / 16;            // MFMA k-steps of S^T = K Q^T
   static constexpr int DT = D / 32;             // output tiles along d
   static constexpr int NCK = Kd / 8, NCV = D / 8;
-  static_assert(Nthreads % kWave == 0 && Br % NW == 0 && WM % 32 == 0, "each wave owns whole 32-row tiles");
+  static_assert(Nthreads % kWave == 0 && NW % KVG == 0 && Br % NWR == 0 && WM % 32 == 0, "each wave owns whole 32-row tiles");
   static_assert(Bc % 32 == 0 && Kd % 64 == 0 && D % 64 == 0, "tile shape");
   static_assert(NSK == 1 || NSK == 2, "K buffers");
   static_assert(NSV == 1 || NSV == 2, "V buffers");
@@ -55,7 +56,10 @@ struct AttnFwdRegfuse {
   static constexpr int kOStride = D * 2 + 16;   // epilogue staging row stride (bytes)
   static constexpr int kMainBytes = NSK * kKBytes + NSV * kVBytes;
   static constexpr int kEpiBytes = Br * kOStride;
-  static constexpr int kSmemBytes = kMainBytes > kEpiBytes ? kMainBytes : kEpiBytes;
+  static constexpr int kHandBytes = WM * (D * 4 + 16);     // what a wave that shares its rows hands over: accumulators, maxima, sums
+  static constexpr int kHandedBytes = (KVG - 1) * NWR * kHandBytes;
+  static constexpr int kMostBytes = kMainBytes > kEpiBytes ? kMainBytes : kEpiBytes;
+  static constexpr int kSmemBytes = kMostBytes > kHandedBytes ? kMostBytes : kHandedBytes;
   static constexpr int kSmemBytesSplit = kMainBytes;   // the partial outputs of a kv split are stored without staging
   // Persistent blocks (PERSIST) stage their output tiles where the copies of the next row block's first kv
   // tile do not land: behind the K/V buffers as far as the LDS budget of a block goes, then in the second K
@@ -140,15 +144,21 @@ template <bool CAUSAL, class F> AAT_DEV void run_tiles(F& tile, int n_full, int 
 // the copies only: memory operations complete in order, so "at most as many outstanding as stores were issued
 // after them" leaves the stores in flight.  Needs two K and two V buffers and an even number of kv tiles (the
 // buffer parity must wrap); plain schedule, non-causal, unsplit.
-template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int WPE = 1, int BU = Bc, int GEN = 0,
+//
+// KVG: that many waves share their rows and take the units of a kv tile in turn; at the end they hand accumulators, maxima and
+// sums to the first of them through LDS.  For launches of so few row blocks that the time is one block's walk: blocks of 32 rows put
+// twice to four times as many CUs to work, and a wave's chain of units is a quarter as long.  Kernel time of 32 rows by four waves
+// against the shape chosen without them: 16 heads, 512 rows, d 64 7.5 -> 6.7 us, causal 9.0 -> 6.8, on 1024 keys 15.4 -> 9.2; d 128
+// 11.6 -> 10.3, 8 heads of 1024 rows causal 21.9 -> 14.3, 24 heads of 32 on 512 11.9 -> 9.9.
+template <int Kd, int D, int Br, int Bc, int Nthreads, int NSK, int NSV, int WPE = 1, int BU = Bc, int GEN = 0, int KVG = 1,
           bool PIPE = false, bool CAUSAL = false, bool SPLIT = false, bool PERSIST = false, bool PAIR = false>
 __global__ void __launch_bounds__(Nthreads) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k,
                       const half_t* __restrict__ v, half_t* __restrict__ o, float* __restrict__ lse,
                       int H, int seq_k, int seq_q, float softmax_scale, float* __restrict__ part_o = nullptr,
                       float* __restrict__ part_lse = nullptr, int n_items = 0, int causal = 1) {
-  using T = AttnFwdRegfuse<Kd, D, Br, Bc, Nthreads, NSK, NSV>;
-  constexpr int RT = T::RT, NT = T::NT, KS = T::KS, DT = T::DT, NCK = T::NCK, NCV = T::NCV, WM = T::WM, NW = T::NW;
+  using T = AttnFwdRegfuse<Kd, D, Br, Bc, Nthreads, NSK, NSV, KVG>;
+  constexpr int RT = T::RT, NT = T::NT, KS = T::KS, DT = T::DT, NCK = T::NCK, NCV = T::NCV, WM = T::WM, NWR = T::NWR;
   constexpr int PF = AAT_PF;                     // operand prefetch distance, in MFMA steps
   // Plain schedule: a kv tile of Bc rows (one copy, one barrier) is worked through in NU units of BU rows, each
   // scores -> softmax -> PV, so the live score tile is RT * BU / 32 accumulator blocks whatever Bc is.
@@ -167,6 +177,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
   constexpr bool ILV = CAUSAL && RT == 2 && !PIPE && NSK == 2 && NSV == 2;
   static_assert(!PIPE || T::kPipeOk, "the pipelined schedule needs 2+2 buffers and unit-aligned K copies");
   static_assert(!GEN || (CAUSAL && !PIPE && !PERSIST && !PAIR), "the general kernel is a form of the causal plain schedule");
+  static_assert(KVG == 1 || (GEN && !SPLIT && !ILV && NSK == 2 && NSV == 2 && NU % KVG == 0), "waves that share rows: the general kernel, one row group a wave");
   static_assert(!SPLIT || GEN, "kv splitting is part of the general kernel");
   using TP = typename T::template Persist<WPE>;
   static_assert(!PERSIST || (!PIPE && !CAUSAL && !SPLIT && TP::kOk), "persistent blocks: plain schedule, 2+2 buffers, room to stage the output");
@@ -178,6 +189,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
+  const int rwave = KVG == 1 ? wave : wave % NWR, kvg = KVG == 1 ? 0 : wave / NWR;   // the wave's place along the rows; the first of its units in a kv tile
 
   const int Tr = GEN ? (seq_q + Br - 1) / Br : seq_q / Br;
   TileDma<Bc, NCK, Nthreads, Swz::Rows16, 0, XA> kdma;
@@ -193,9 +205,9 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
     k_frag_offsets<KS, NCK>(koff, n, h);
     v_frag_offsets<DT, NCV>(voff, lane);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kaddr[ks] = lds_addr(kbuf + koff[ks]);
+    for (int ks = 0; ks < KS; ++ks) kaddr[ks] = lds_addr(kbuf + kvg * NTU * T::kUnitK + koff[ks]);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) vaddr[dt] = lds_addr(vbuf + voff[dt]);
+    for (int dt = 0; dt < DT; ++dt) vaddr[dt] = lds_addr(vbuf + kvg * NTU * T::kUnitV + voff[dt]);
   }
 
   const float c2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, softmax_scale * kLog2e)));   // wave-uniform: a scalar register
@@ -248,8 +260,8 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
     const char* vg = reinterpret_cast<const char*>(v + ((size_t)bh * seq_k + (size_t)tile0 * Bc) * D);
 
     // first row of the wave's first 32-row group inside the block, and the distance to its second group
-    const int wrow0 = ILV ? 32 * wave : wave * WM;
-    const int group_rows = ILV ? 32 * (2 * NW - 1 - 2 * wave) : 32;
+    const int wrow0 = ILV ? 32 * rwave : rwave * WM;
+    const int group_rows = ILV ? 32 * (2 * NWR - 1 - 2 * rwave) : 32;
     int groups = RT;                              // 32-row groups of this wave that exist (its first ones)
     if constexpr (GEN) {
       groups = 0;
@@ -343,9 +355,9 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
         // The matrix phases run at a raised wave priority: with two or three waves on the SIMD the one that has
         // MFMAs to issue goes first and the others' softmax arithmetic fills the gaps, not the other way round
         // (causal forward at three waves per SIMD: -1.4 %; nothing at two).
-        static_for<NU>([&](auto unit_tag) {
-          constexpr int U = decltype(unit_tag)::value;
-          const int kv0 = kv_first + j * Bc + U * BU;   // first kv row of the unit
+        static_for<NU / KVG>([&](auto unit_tag) {
+          constexpr int U = decltype(unit_tag)::value * KVG;   // of the block; the wave's own is kvg further
+          const int kv0 = kv_first + j * Bc + (U + kvg) * BU;  // first kv row of the unit
           constexpr bool TAIL = GEN && MASKED && NTU > 1;   // kv rows of the unit may be missing: they stay out of the second contraction
           if constexpr (ILV) {
             // One body for both row groups; in a unit the early group no longer sees (and the late one does) its
@@ -387,7 +399,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
             return;
           }
           bool wave_sees = true;
-          if constexpr (MASKED) wave_sees = kv0 <= (q0 + wave * WM + WM - 1) * slope + diag;
+          if constexpr (MASKED) wave_sees = kv0 <= (q0 + rwave * WM + WM - 1) * slope + diag;
           if constexpr (GEN) wave_sees = wave_sees && groups > 0 && (!MASKED || kv0 < seq_k);
 
           f16v sacc[RT][NTU];
@@ -522,6 +534,42 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
     } else if constexpr (TP::kSharesBuffers) {
       block_sync();                                // every wave is done with the parity-1 buffers
     }
+    char* const hand = smem + rwave * (KVG - 1) * T::kHandBytes;   // KVG > 1: where the waves of these rows meet
+    if constexpr (KVG > 1) {
+      const auto accumulators = [&](int g) { return reinterpret_cast<f4v*>(hand + g * T::kHandBytes) + lane; };
+      const auto max_and_sum = [&](int g) { return reinterpret_cast<f2v*>(hand + g * T::kHandBytes + RT * DT * 4096) + lane; };
+      if (kvg > 0) {
+        static_for<RT * DT * 4>([&](auto i_tag) {
+          constexpr int i = decltype(i_tag)::value, e = 4 * (i % 4);
+          const f16v& a = oacc[i / 4 / DT][i / 4 % DT];
+          accumulators(kvg - 1)[i * 64] = f4v{a[e], a[e + 1], a[e + 2], a[e + 3]};
+        });
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) max_and_sum(kvg - 1)[rt * 64] = f2v{m_run[rt], l_run[rt]};
+      }
+      block_sync();
+      if (kvg > 0) return;
+#pragma unroll 1
+      for (int g = 0; g < KVG - 1; ++g) {
+        float own[RT], other[RT];                 // weights of what the two have seen; of nothing: 0
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const f2v ml = max_and_sum(g)[rt * 64];
+          const float m = fmaxf(m_run[rt], ml[0]);
+          own[rt] = m_run[rt] == -INFINITY ? 0.f : fast_exp2((m_run[rt] - m) * c2);
+          other[rt] = ml[0] == -INFINITY ? 0.f : fast_exp2((ml[0] - m) * c2);
+          m_run[rt] = m;
+          l_run[rt] = l_run[rt] * own[rt] + ml[1] * other[rt];
+        }
+        static_for<RT * DT * 4>([&](auto i_tag) {
+          constexpr int i = decltype(i_tag)::value, rt = i / 4 / DT, dt = i / 4 % DT;
+          const f4v b = accumulators(g)[i * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[rt][dt][4 * (i % 4) + e] = oacc[rt][dt][4 * (i % 4) + e] * own[rt] + b[e] * other[rt];
+        });
+      }
+      wait_lgkm0();                               // the place is the output's staging area next
+    }
     float inv[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -543,7 +591,7 @@ flashattn_fwd_regfuse(const half_t* __restrict__ q, const half_t* __restrict__ k
                                            o + ((size_t)bh * seq_q + q0 + wave * WM) * D, lane);
     } else {
       // transposed through LDS for 16-byte coalesced stores
-      store_o_tile<RT, DT, D, T::kOStride>(oacc, inv, smem + wave * WM * T::kOStride,
+      store_o_tile<RT, DT, D, T::kOStride>(oacc, inv, KVG > 1 ? hand : smem + wave * WM * T::kOStride,
                                            o + ((size_t)bh * seq_q + q0 + wrow0) * D, lane, group_rows, groups);
     }
     if constexpr (PAIR) {

@@ -50,6 +50,8 @@ def planned(key, make_tuner, default_factory):
         tuner = make_tuner()
         op, key_dim, head_dim = key[0].replace("_decay", ""), key[6], key[7]
         near = NEAR_ENOUGH if gfx950_space.covered_by_rule(op, key_dim, head_dim) else None
+        if op == "attn" and gfx950_space.few_blocks_config(key_dim, head_dim, *key[2:6], key[8]) is not None:
+            near = -1                                      # no other problem's entry
         cc = resolve(tuner, default_factory, near)
         plan = base_tunner._memo[k] = (cc, Runtime(tuner.arch, cc))
     return plan

@@ -44,6 +44,31 @@ def test_every_rule_shape_at_the_edges_of_its_tiles(d, causal):
             assert (lse.cpu() - want_lse)[seen].abs().max().item() <= 1e-3
 
 
+@pytest.mark.parametrize("d", sorted(p[0] for p in gfx950_space.FEW_BLOCKS))
+@pytest.mark.parametrize("causal", [False, True])
+def test_waves_that_share_their_rows(d, causal):
+    """Units of a kv tile that a wave of the group does not have, see or is alone with; rows that see no key; an infinite value."""
+    for i, (b, h, sq, sk) in enumerate(SHAPES):
+        q, k, v = _inputs(b, h, sq, sk, d, 130 + i)
+        want, want_lse = ref_op.attention_ref(q, k, v, None, causal, return_lse=True)
+        if not causal:
+            v[0, 0, sk - 1, 5] = float("inf")
+        qc, kc, vc = (t.cuda() for t in (q, k, v))
+        for cfg in gfx950_space.few_blocks_configs(d, d):
+            print(d, causal, (b, h, sq, sk), cfg, flush=True)
+            o = torch.full((b, h, sq, d), 7.0, dtype=torch.float16, device="cuda")
+            lse = torch.full((b, h, sq), 7.0, device="cuda")
+            Runtime(ARCH, cfg).apply([qc, kc, vc, o], softmax_scale=1 / math.sqrt(d), causal=causal, lse=lse)
+            torch.cuda.synchronize()
+            got, seen = o.float().cpu(), torch.isfinite(want_lse)
+            if not causal:
+                assert (got[0, 0, :, 5] == float("inf")).all()
+                got[0, 0, :, 5] = want[0, 0, :, 5]
+            assert (got - want).abs().max().item() <= 2e-3
+            assert torch.equal(torch.isfinite(lse.cpu()), seen)
+            assert (lse.cpu() - want_lse)[seen].abs().max().item() <= 1e-3
+
+
 @pytest.mark.parametrize("b,h,sq,sk,causal", [(3, 5, 1088, 1088, True), (2, 3, 192, 4160, True), (1, 4, 64, 8192, False), (2, 3, 96, 96, False)])
 def test_the_operator_takes_them_and_its_calls_agree(b, h, sq, sk, causal):
     q, k, v = (t.cuda() for t in _inputs(b, h, sq, sk, 128, 7))
