@@ -95,7 +95,8 @@ class Runtime:
         q, k = torch_array[0], torch_array[1]
         if not q.is_cuda:
             raise KernelLaunchError("kernel libraries run on the GPU only; got CPU tensors")
-        B, H, Sq, Sk = q.shape[0], q.shape[1], q.shape[2], k.shape[2]
+        B, H, Sq = q.shape[:3]
+        Sk = k.shape[2]
         op = self.config.operation
         lib = self._lib
         if lib is None:
@@ -123,9 +124,9 @@ class Runtime:
         # the prototypes are set (library.py), so plain integers convert; the launch goes to the stream that is current
         # on the tensors' device, with that device current
         index = q.device.index
-        other = index != torch.cuda.current_device()
+        previous = torch._C._cuda_getDevice()
+        other = index != previous
         if other:
-            previous = torch.cuda.current_device()
             torch.cuda.set_device(index)
         try:
             stream = torch._C._cuda_getCurrentRawStream(index)
