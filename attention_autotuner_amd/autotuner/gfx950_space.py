@@ -377,33 +377,32 @@ def rule_forward_config(dim_qk, dim_v, arch, b, h, seq_q, seq_k, causal):
 
 
 # Launches of so few row blocks that one block's walk is their time: 32 rows a block, its waves share them and take the kv units in
-# turn (``kv_groups``).  Per pair of head sizes: (fewest and most kv rows, Bc, threads, waves per SIMD).  Kernel time against the shape
-# taken without them, 165 problems of 2 to 32 heads, 32 to 1536 rows: d 64 0.67 ... 0.98 up to 256 blocks of 32 rows and 0.70 ... 0.82 for the
-# causal walks of 384 and 512 (dense ones 0.9 ... 1.13), d 128 0.62 ... 0.92 up to 256 and 0.8 ... 1.5 beyond.  Short ranges are one tile
+# turn (``kv_groups``), or 64 rows by twice as many waves.  Per pair of head sizes, in order of preference: (rows of a block, its waves, waves per SIMD, fewest and most
+# kv rows, most blocks when dense and when causal).  Kernel time against the shape taken without them, 165 problems of 2 to 32 heads, 32 to 1536
+# rows: d 64 0.67 ... 0.98 up to 256 blocks of 32 rows and 0.70 ... 0.82 for the causal walks of 384 and 512, d 128 0.62 ... 0.92 up to 256;
+# blocks of 64 rows up to 256 0.70 ... 0.93 (1.02 ... 1.16 on 512 keys).  Short ranges are one tile
 # for every shape: 1.03 ... 1.20 on 128 keys, d 128 0.94 ... 1.08 on 256.  At d 128 a few dozen blocks on 2080 keys lose to kv parts (1.05 ... 1.23),
-# at d 64 they do not (0.82 ... 0.91).  45 problems drawn from these ranges: 0.89 on the mean, 1.02 at most from the shortest range on.
+# at d 64 they do not (0.82 ... 0.91).
 FEW_BLOCKS = {
-    (64, 64): (160, 2112, 128, 256, 2),
-    (128, 128): (288, 1536, 128, 256, 1),
+    (64, 64): ((32, 4, 2, 160, 2112, 256, 512), (64, 8, 2, 640, 2112, 256, 256)),
+    (128, 128): ((32, 4, 1, 288, 1536, 256, 256), (64, 8, 2, 640, 1536, 256, 256)),
 }
 
 
 def few_blocks_configs(dim_qk, dim_v):
-    if (dim_qk, dim_v) not in FEW_BLOCKS:
-        return []
-    _, _, bc, nt, wpe = FEW_BLOCKS[dim_qk, dim_v]
-    return [AttnConfig(32, bc, dim_qk, dim_v, dim_qk, 32, 2, 2, nt, True, waves_per_eu=wpe, kv_groups=nt // 64).set_fuse_type("register")]
+    return [AttnConfig(br, 128, dim_qk, dim_v, dim_qk, 32, 2, 2, 64 * waves, True, waves_per_eu=wpe, kv_groups=4).set_fuse_type("register")
+            for br, waves, wpe, *_ in FEW_BLOCKS.get((dim_qk, dim_v), ())]
 
 
 def few_blocks_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
     """The configuration for an attention forward of few row blocks, or None: a problem with more of them, or of other sizes.  It
     goes ahead of the entries tuned for other problems, none of which has such a kernel."""
-    cfgs = few_blocks_configs(dim_qk, dim_v)
-    if not cfgs or seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
+    if seq_q % MIN_LENGTH or seq_k % MIN_LENGTH:
         return None
-    least, most = FEW_BLOCKS[dim_qk, dim_v][:2]
-    few = b * h * -(-seq_q // 32) <= (512 if causal and dim_qk == 64 else 256)
-    return cfgs[0] if few and least <= seq_k <= most else None
+    for cfg, (br, _, _, least, most, dense, walked) in zip(few_blocks_configs(dim_qk, dim_v), FEW_BLOCKS.get((dim_qk, dim_v), ())):
+        if least <= seq_k <= most and b * h * -(-seq_q // br) <= (walked if causal else dense):
+            return cfg
+    return None
 
 
 # ---- backward (RetNet) ---------------------------------------------------------------------------------
