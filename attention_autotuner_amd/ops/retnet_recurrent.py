@@ -55,10 +55,9 @@ def retnet_recurrent_fwd(q, k, v, decay, device_type=None, block_kdim=None, out=
     if out is None:
         out = torch.empty_like(v)
     assert out.shape == v.shape and out.dtype == torch.float32 and out.is_contiguous() and out.device == v.device
-    need = int(lib.retnet_recurrent_workspace_size(batch, nheads, kdim, vdim, seqlen, block_kdim))
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        room = int(lib.retnet_recurrent_room(batch, nheads, kdim, vdim, seqlen, block_kdim, _MOST_WORKSPACE))
-        workspace = torch.empty(max(need, room, 1), dtype=torch.uint8, device=q.device)
+    if workspace is None or workspace.numel() * workspace.element_size() < lib.retnet_recurrent_workspace_size(batch, nheads, kdim, vdim, seqlen, block_kdim):
+        room = int(lib.retnet_recurrent_room(batch, nheads, kdim, vdim, seqlen, block_kdim, _MOST_WORKSPACE))      # workspace_size() or more
+        workspace = torch.empty(max(room, 1), dtype=torch.uint8, device=q.device)
     with torch.cuda.device(q.device):
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         rc = lib.retnet_recurrent_fwd_ex(*[ctypes.c_void_p(t.data_ptr()) for t in (q, k, v, decay, out)], batch, nheads, kdim,
