@@ -278,7 +278,8 @@ def side_measurements(aat, arch, Runtime, mk, steps, warmup):
 def retnet_recurrent_measurement(aat, steps, warmup):
     """RetNet recurrent form at the shape of the reference's own bench (benchmarks/retnet/retnet.cu:236:
     B 8, H 32, L 2048, 128 key and value dims, fp32).  5 flops per (position, key dim, value dim): the
-    recurrence's two multiply-adds and one multiply; fp32 MFMA peak 157.3 TFLOP/s."""
+    recurrence's two multiply-adds and one multiply.  The products run as bf16 ones of the operands' parts, so what bounds it
+    is memory; the fraction of the fp32 MFMA peak, 157.3 TFLOP/s, is kept for comparison."""
     import torch
     if not hasattr(aat, "retnet_recurrent_fwd"):
         return {}
@@ -294,6 +295,8 @@ def retnet_recurrent_measurement(aat, steps, warmup):
     nbytes = 4.0 * (q.numel() + k.numel() + v.numel() + out.numel())
     res = extra(t, flops, peak=157.3, gbps=round(nbytes / t.median / 1e6, 1))
     res["frac_of_fp32_mfma_peak"] = res["roofline"]["frac"]
+    res["roofline"] = {"bound": "hbm", "achieved": res["gbps"], "peak": 8000.0, "unit": "GB/s", "frac": round(res["gbps"] / 8000.0, 4),
+                       "algorithmic_bytes": nbytes}
     log(f"retnet recurrent fwd: {t.median:.4f} ms -> {res['tflops']} TFLOP/s ({res['gbps']} GB/s)")
     return {"retnet_recurrent_b8h32s2048_dqk128_dv128_f32": res}
 
