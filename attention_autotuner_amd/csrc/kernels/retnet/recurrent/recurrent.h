@@ -85,7 +85,7 @@ static_assert(rec_row_reads_conflict_free() && rec_column_reads_conflict_free(),
 //                                   by retnet_recurrent_pmat, which multiplies P by it, and not read after it
 //   [4096, 4224)  W[h][g][e]      = w_m / lambda'      (w_m alone on a rescale)
 //   [4224, 4352)  PNL[n]          = p_n lambda
-//   [4352, 4368)  rescale flag (uint32), scale, lambda, 1 / lambda' (1 on a rescale)
+//   [4352, 4360)  rescale flag (uint32), scale
 constexpr int kRecFactorBytes = 5120;
 constexpr int kRecFactorW = 4096, kRecFactorPnl = 4224, kRecFactorFlag = 4352;
 
@@ -165,8 +165,6 @@ AAT_DEV void rec_factor_records(const float* __restrict__ decay, char* __restric
     if (lane == 0) {
       *reinterpret_cast<uint32_t*>(rec + kRecFactorFlag) = rescale ? 1u : 0u;
       *reinterpret_cast<float*>(rec + kRecFactorFlag + 4) = lam_new;
-      *reinterpret_cast<float*>(rec + kRecFactorFlag + 8) = lam;
-      *reinterpret_cast<float*>(rec + kRecFactorFlag + 12) = inv;
     }
   }
 }
@@ -497,7 +495,7 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
     char* const sm = smem + (c & 1) * T::kStage;
     block_sync();      // chunk c is in LDS (the data waves waited for it); every wave is done with chunk c-1
 
-    // ---- this wave's share of the operands of Q and of K diag(w / lambda')
+    // ---- this wave's share of the operands of Q and of K
     Op qown[T::kUnits], kop[T::kUnits];
     f4v kx[T::kUnits][2], vx[4];
     {
@@ -514,10 +512,8 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
           kx[s][j >> 2][j & 3] = *reinterpret_cast<const float*>(sm + at);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < 2; ++i)
           kc[s][i] = *reinterpret_cast<const f4v*>(sm + (u >> 1) * 4096 + cp * 128 + (rec_slot(cp, hi) ^ (4 * (u & 1) + 2 * i)) * 16);
-          if constexpr (!FP32) kc[s][i] *= *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorW + hi * 64 + (2 * (u & 1) + i) * 16);
-        }
       }
       Op kown[T::kUnits];
 #pragma unroll
@@ -559,26 +555,29 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
     });
 
     // ---- T^T Q
-    // w / lambda' goes with K, whose operands are made once; FP32: with V as in the kernel below, so that no range is lost to the scale of K
-    const auto update_op = [&](const Op (&vop)[2], int s) {
-      if constexpr (!FP32) return vop[s];
-      const auto w = [&](int g) { return *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorW + hi * 64 + g * 16); };
-      return rec_op<FP32>(vx[2 * s] * w(2 * s), vx[2 * s + 1] * w(2 * s + 1));
+    // w / lambda' goes with V as in the kernels below, before V is taken apart, at the price of two more operands a chunk: with K, whose
+    // operands are made once, a factor of 2^-36 takes a K of 1e-28 out of fp32 where V has the room for it (B8 H32 L2048 128/128 315 -> 321 us).
+    f4v wx[2];
+    const auto read_w = [&](int s) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) wx[i] = *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorW + hi * 64 + (2 * s + i) * 16);
     };
-    Op vop[2], pop[2];
+    Op vop[2], uop[2], pop[2];                             // V for V P, V w / lambda' for the State
     static_for<T::kSteps>([&](auto it) {
       constexpr int ks = decltype(it)::value;
       Op tnext, qnext;
       if constexpr (ks + 1 < T::kSteps) {
         qnext = read_op(true, ks + 1);
+        if constexpr (ks + 2 == T::kSteps) read_w(0);
         tnext = rec_op_of_c<FP32>(st[(ks + 1) >> 1], (ks + 1) & 1);
         rec_pin(tnext);
       } else {
-        vop[0] = rec_op<FP32>(vx[0], vx[1]);
-        rec_pin(vop[0]);
+        uop[0] = rec_op<FP32>(vx[0] * wx[0], vx[1] * wx[1]);
+        rec_pin(uop[0]);
+        read_w(1);
       }
       oacc = rec_mma<FP32>(top, qop, oacc);
-      rec_interleave<FP32, ks + 1 < T::kSteps ? 3 : 0, 8>();
+      rec_interleave<FP32, ks + 2 < T::kSteps ? 3 : ks + 1 < T::kSteps ? 5 : 2, 8>();
       if constexpr (ks == 1) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) *reinterpret_cast<f4v*>(sm + wave * 4096 + g * 1024 + lane16) = rec_quarter(sp, 4 * g);
@@ -628,7 +627,8 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
       Op wnext;
       if constexpr (i + 1 < T::kSteps) wnext = read_op(false, 2 * ((i + 1) % T::kKB) + (i + 1) / T::kKB);
       constexpr auto at = [](int x) { return x * T::kSteps / 8; };
-      if constexpr (i == at(0)) vop[1] = rec_op<FP32>(vx[2], vx[3]);
+      if constexpr (i == at(0)) uop[1] = rec_op<FP32>(vx[2] * wx[0], vx[3] * wx[1]);
+      if constexpr (i == at(1)) vop[0] = rec_op<FP32>(vx[0], vx[1]);
       if constexpr (i == at(2)) {
         add_partials(0);
         read_partials(2);
@@ -639,13 +639,14 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
       if constexpr (i == at(6)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[r] *= pnl;
+        vop[1] = rec_op<FP32>(vx[2], vx[3]);
       }
       if constexpr (i == T::kSteps - 1) {
 #pragma unroll
         for (int r = 0; r < 2; ++r) oacc = rec_mma<FP32>(vop[r], pop[r], oacc);
         sched_fence();
       }
-      st[kb] = rec_mma<FP32>(wop, update_op(vop, s), st[kb]);
+      st[kb] = rec_mma<FP32>(wop, uop[s], st[kb]);
       rec_interleave<FP32, 3, 8>();
       if constexpr (i == at(0)) {
         block_sync();                                      // the partial S^T are in LDS
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(DVS * 2 + 128) __attribute__((amdgpu_waves_per_eu(2
 // P of every (batch, head, chunk) for the kernels below, as C registers: [B*H][L/32][g][lane][e], 4 KB per chunk.  One block
 // per chunk; its waves split the key dims, read q and k straight from memory (rows of 128 bytes, each used once) and wave w adds
 // up row group w and multiplies it by D.  Bound by the read of q and k.
-// OPS: also the operands of Q p_n and K w_m for retnet_recurrent_stream_kernel, [B*H][L/32][KD/16 of Q, KD/16 of K][part][lane][16 B];
+// OPS: also the operands of Q and K for retnet_recurrent_stream_kernel, [B*H][L/32][KD/16 of Q, KD/16 of K][part][lane][16 B];
 // bound by their 12 bytes per key dim and position (B2 H8 L1056, 256 key dims: 8.8 us without them, 17 with).
 //
 // The first heads * parts blocks of the launch make the records of the decay factors instead, 8 bytes of dynamic LDS per chunk
@@ -725,18 +726,17 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
   }
   sched_fence();                                      // all loads in flight before the first product
   const float* const dg = decay + (size_t)(bh % heads) * L + (size_t)c * 32;
-  f4v dsel = {0.f, 0.f, 0.f, 0.f}, wsel[4];           // D of rows 8 wave + 4 hi + e; w of positions 8g + 4 hi + e
-  float d = 0.f, w = 1.f;
+  f4v dsel = {0.f, 0.f, 0.f, 0.f};                    // D of rows 8 wave + 4 hi + e
+  float d = 0.f;
 #pragma unroll
   for (int g = 3; g >= 0; --g) {
     f4v rows[2];
 #pragma unroll
     for (int i = 7; i >= 0; --i) {
       const int m = 8 * g + i;
-      if (m < 31) { d *= dg[m + 1]; w *= dg[m + 1]; }
+      if (m < 31) d *= dg[m + 1];
       d = (m == n) ? 1.f : d;
       rows[i >> 2][i & 3] = d;
-      if constexpr (OPS) wsel[g][i & 3] = i >= 4 ? w : hi ? wsel[g][i & 3] : w;
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) dsel[e] = g == wave ? (hi ? rows[1][e] : rows[0][e]) : dsel[e];
@@ -748,10 +748,9 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
   for (int g = 0; g < 4; ++g) part[wave][g][lane] = rec_quarter(sp, 4 * g);
   if constexpr (OPS) {
     char* const mine = ops + ((size_t)bh * nchunk + c) * (2 * KD / 16) * 3072 + lane * 16;
-    const float pn = d * dg[0];
 #pragma unroll
     for (int s = 0; s < kUnits; ++s) {
-      const RecOp<false> o = rec_op<false>(qx[s][0] * pn, qx[s][1] * pn);
+      const RecOp<false> o = rec_op<false>(qx[s][0], qx[s][1]);
 #pragma unroll
       for (int p = 0; p < 3; ++p) *reinterpret_cast<u4v*>(mine + (wave * kUnits + s) * 3072 + p * 1024) = o.p[p];
     }
@@ -760,7 +759,7 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
       if (wave + 4 * t < kTiles) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-          const RecOp<false> o = rec_op<false>(kr[t][2 * s] * wsel[2 * s], kr[t][2 * s + 1] * wsel[2 * s + 1]);
+          const RecOp<false> o = rec_op<false>(kr[t][2 * s], kr[t][2 * s + 1]);
 #pragma unroll
           for (int p = 0; p < 3; ++p) *reinterpret_cast<u4v*>(mine + (KD / 16 + 2 * (wave + 4 * t) + s) * 3072 + p * 1024) = o.p[p];
         }
@@ -1093,7 +1092,7 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
 
 // ---------------------------------------------------------------------------------------------------
 // The split scan with the operands of Q and K made once per (batch, head) ahead of it: retnet_recurrent_pmat leaves them in memory
-// in the order the matrix instructions take them (Q times p_n, K times w_m, three bf16 parts each), and every wave reads those of
+// in the order the matrix instructions take them (three bf16 parts each), and every wave reads those of
 // its own key dims straight into registers, a chunk ahead.  V, P and the factors come through LDS, requested three chunks ahead by
 // a wave of their own, which also adds up and stores the waves' partial sums of O^T: a wave's loads return in order, and one that
 // comes from memory holds up every one behind it.
@@ -1250,22 +1249,25 @@ AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const floa
     sched_fence();
   }
   block_sync();                                            // chunks 0 and 1 have landed
-  f4v vx[4], fx;                                           // V, and rescale flag, scale, lambda, 1 / lambda'
+  f4v vx[4], wx[4], fx;                                    // V, w / lambda', and rescale flag, scale in the first two
+  float pnx;                                               // p_n lambda
   const auto read_v = [&](const char* sm) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) vx[g] = v_at(sm, g);
     fx = *reinterpret_cast<const f4v*>(sm + T::kFOff + kRecFactorFlag - kRecFactorW);
+    pnx = *reinterpret_cast<const float*>(sm + T::kFOff + kRecFactorPnl - kRecFactorW + n * 4);
   };
-  const auto make_v = [&](const char* sm, int s) {         // of V w / lambda'; K has the w already, FP32: it has not
-    const auto x = [&](int g) {
-      if constexpr (FP32) return vx[g] * *reinterpret_cast<const f4v*>(sm + T::kFOff + hi * 64 + g * 16);
-      else return vx[g] * fx[3];
-    };
-    return rec_op<FP32>(x(2 * s), x(2 * s + 1));
+  const auto read_w = [&](const char* sm, int s) {
+#pragma unroll
+    for (int g = 2 * s; g < 2 * s + 2; ++g) wx[g] = *reinterpret_cast<const f4v*>(sm + T::kFOff + hi * 64 + g * 16);
   };
+  const auto make_v = [&](int s) { return rec_op<FP32>(vx[2 * s] * wx[2 * s], vx[2 * s + 1] * wx[2 * s + 1]); };   // of V w / lambda'
   read_v(stage_of(0));
-  vop[0] = make_v(stage_of(0), 0);
-  vop[1] = make_v(stage_of(0), 1);
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    read_w(stage_of(0), s);
+    vop[s] = make_v(s);
+  }
 
   // A step of the loop updates the State with chunk c, finishes chunk c's output and contracts the new State with chunk c+1's Q.
   // Every operand read ahead is used once and then read again for a chunk later in its place; behind the first branch the
@@ -1275,7 +1277,7 @@ AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const floa
   for (int c = 0; c < nchunk; ++c) {
     const int next = c + 1 < nchunk ? c + 1 : nchunk - 1, next2 = c + 2 < nchunk ? c + 2 : nchunk - 1;
     const char* const sm = stage_of(c);
-    const float lam = fx[2];
+    const float pnl = pnx;
     if (__builtin_amdgcn_readfirstlane(__float_as_uint(fx[0])) != 0u) {     // lambda left its range: fold it into T
 #pragma unroll
       for (int kb = 0; kb < T::kKB; ++kb)
@@ -1294,14 +1296,8 @@ AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const floa
     static_for<T::kSteps>([&](auto it) {
       constexpr int u = decltype(it)::value, kb = u >> 1, s = u & 1;
       if constexpr (u == 0) {
-        if constexpr (FP32) {
-          const float pnl = *reinterpret_cast<const float*>(sm + T::kFOff + kRecFactorPnl - kRecFactorW + n * 4);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[r] *= pnl;
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[r] *= lam;
-        }
+        for (int r = 0; r < 16; ++r) oacc[r] *= pnl;
       }
       if constexpr (u >= 2) {
         top[u - 2] = rec_op_of_c<FP32>(st[0], u - 2);
@@ -1331,16 +1327,18 @@ AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const floa
         top[kMade + 1] = rec_op_of_c<FP32>(st[T::kKB - 1], 1);
         rec_pin(top[kMade + 1]);
       }
+      if constexpr (ks == (T::kSteps > 2 ? T::kSteps - 3 : 0)) read_w(stage_of(next), 0);
+      if constexpr (ks == T::kSteps - 2) read_w(stage_of(next), 1);
       if constexpr (ks == T::kSteps - 2 && ks > 0) {
-        vop[0] = make_v(stage_of(next), 0);
+        vop[0] = make_v(0);
         rec_pin(vop[0]);
       }
       if constexpr (ks == T::kSteps - 1) {
         if constexpr (T::kSteps == 2) {
-          vop[0] = make_v(stage_of(next), 0);
+          vop[0] = make_v(0);
           rec_pin(vop[0]);
         }
-        vop[1] = make_v(stage_of(next), 1);
+        vop[1] = make_v(1);
         rec_pin(vop[1]);
       }
       tq = rec_mma<FP32>(top[ks], qop[ks], tq);

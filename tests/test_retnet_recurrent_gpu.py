@@ -289,6 +289,25 @@ def test_products_in_parts_keep_the_range_of_fp32(k_scale, q_scale, spread):
         _close(out[:, head], ref[:, head])
 
 
+# Decay factors far from one, next to values at the other end: w / lambda' of 2^-36 beside a K of 1e-28, w of 1e-30 beside a K of 1e-12, p_n of
+# 1e-30 beside a Q of 1e-12.  Their products leave fp32 (or three bf16 parts) and what they are for does not: the factors go with V and with the sum.
+# Blocks of 128 and 64 value dims, and those with operands made ahead.
+@pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(8, 24, 128, 128, 64), (8, 24, 64, 128, 64), (8, 24, 64, 64, 64), (1, 2, 64, 64, 512),
+                                                   (1, 2, 128, 64, 512), (1, 2, 192, 64, 512), (1, 2, 256, 64, 512)])
+@pytest.mark.parametrize("where,factor,k_scale,q_scale,v_scale", [(0, 2.0 ** 36, 1e-28, 1e16, 1e12), (16, 1e-30, 1e-12, 1e12, 1e20),
+                                                                  (32, 1e-30, 1e14, 1e-12, 1e12)])
+def test_decay_factors_beside_values_at_the_other_end(b, h, kdim, vdim, seqlen, where, factor, k_scale, q_scale, v_scale):
+    q, k, v, decay = _inputs(28, b, h, kdim, vdim, seqlen, 1.0, 1.0)
+    q, k, v = (q * q_scale).float(), (k * k_scale).float(), (v * v_scale).float()
+    decay[:, where] = factor
+    if factor < 1:
+        v[..., where:] = 0.0                              # what came before is all there is behind the factor
+    out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
+    ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
+    for head in range(h):
+        _close(out[:, head, :, where:], ref[:, head, :, where:])
+
+
 # An infinity or a NaN takes its (batch, head, value slice) from the chunk it lies in on, and nothing else: the rest is as without it,
 # bit for bit in other blocks, within the bound in the chunks before
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
