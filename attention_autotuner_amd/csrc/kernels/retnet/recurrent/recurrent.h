@@ -184,12 +184,17 @@ __global__ __launch_bounds__(kRecFactorThreads) void retnet_recurrent_factors(co
 // FP32 = false, taken first: an fp32 value is the sum of three bf16 ones (hi, mid, lo: 8 significant bits each, rounded to
 // nearest), and a product the sum of the six largest of their nine, on v_mfma_f32_32x32x16_bf16: 6 x 32 cycles for 16 indices
 // where v_mfma_f32_32x32x2_f32 takes 8 x 64.  What is left out is below 2^-23 of a product and 2^-26 of it on average, less than
-// the rounding of one fp32 addition; bf16 has the range of fp32, so nothing is scaled.  A sum is rounded six times per k-step
+// the rounding of one fp32 addition.  A sum is rounded six times per k-step
 // instead of eight, and results are no further from 64 bits than with fp32 products: relative 2-norm at B8 H32 L512 128/128
 // 7.58e-7 -> 7.26e-7, most of it from the products of decays both have in common; with decays in [0.5, 1] 1.28e-7 -> 9.5e-8; the
 // same with normal or positive values, magnitudes spread over 12 decades along the key dims, or products around 1e-24.
-// An infinity (or a value that rounds to one in bf16) becomes a NaN in its parts: a block that finds a value in its output that
-// is not finite runs once more from the start with FP32 = true.
+// bf16 ends where fp32 does upwards, but at 2^-133 downwards (conversion, v_dot2 and matrix instructions keep subnormals), so the parts of a
+// value below 2^-110 would hold fewer than its 24 bits.  Therefore Q, K and V are multiplied by kRecUp = 2^16, with which every fp32 value
+// there is has parts that are exact; sums carry the powers along (S^T, the State and P 2^32, outputs 2^48: the inputs of the products that
+// follow have more room below than they need) and outputs are scaled back at the end.
+// An infinity (or a value, or a sum, that the scale or bf16's rounding takes there: inputs from 2^112 on, outputs from 2^80, from 2^40
+// where lambda is 2^-40) becomes a NaN in its parts: a block that finds a value in its output that
+// is not finite runs once more from the start with FP32 = true, which scales nothing.
 // FP32 = true: eight fp32 values and eight v_mfma_f32_32x32x2_f32.
 template <bool FP32> struct RecOp {
   static constexpr int kParts = FP32 ? 2 : 3;
@@ -197,6 +202,8 @@ template <bool FP32> struct RecOp {
 };
 typedef __bf16 rec_bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 rec_bf2 __attribute__((ext_vector_type(2)));
+constexpr float kRecUp = 0x1p16f, kRecDown = 0x1p-48f;
+template <bool FP32> AAT_DEV f4v rec_up(f4v x) { return FP32 ? x : x * kRecUp; }
 
 // ALONE: where no matrix instruction is under way the remainder x - hi is one v_dot2_f32_bf16 (times -1 and 0, exact) instead of a
 // shift or mask and a subtraction; it shares the matrix core's issue path and waits there for a matrix instruction to end.
@@ -334,10 +341,11 @@ struct RetRecurrent {
 // second is a sequence of k-steps: six matrix instructions, with the vector instructions that make a later k-step's operand of
 // T, V or P between them (7 fit behind one) and the LDS reads of the next k-step.
 //
-// Bound by the board's power: 8000 cycles a chunk (120 matrix instructions = 3840, some 950 vector instructions and 450 KB through LDS)
-// run at 2.35 GHz without the memory stream and at 1.8 GHz with it; the stream by itself takes 270 us of the 310 at B8 H32 L2048
-// 128/128.  Whole calls, fp32 products and one data wave before, this kernel now: B8 H32 L2048 128/128 369 -> 310 us (L512 100 -> 77),
-// 64/128 235 -> 213, 64/64 206 -> 164.  Tried and not kept: two
+// Bound by the board's power: some 8000 cycles a chunk (120 matrix instructions = 3840, 1100 vector instructions and 450 KB through LDS)
+// run at 2.35 GHz without the memory stream and at 1.8 GHz with it; the stream by itself takes 270 us of the 328 at B8 H32 L2048
+// 128/128.  Whole calls on inputs that change, fp32 products and one data wave before, this kernel now: B8 H32 L2048 128/128 368 -> 328 us
+// (L512 96 -> 87), 64/128 234 -> 222, 64/64 209 -> 184; 170 of the vector instructions and 14 of the 328 us go into the scale and into decay
+// factors that stay with V.  Tried and not kept: two
 // chunks' copies under way at all times, at the price of factors read from memory and a fourth barrier, 331 us; non-temporal copies or
 // stores +-3 %.
 template <bool FP32, int KD, int DVS>
@@ -518,8 +526,8 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
       Op kown[T::kUnits];
 #pragma unroll
       for (int s = 0; s < T::kUnits; ++s) {
-        qown[s] = rec_op<FP32, true>(qx[s][0], qx[s][1]);
-        kown[s] = rec_op<FP32, true>(kc[s][0], kc[s][1]);
+        qown[s] = rec_op<FP32, true>(rec_up<FP32>(qx[s][0]), rec_up<FP32>(qx[s][1]));
+        kown[s] = rec_op<FP32, true>(rec_up<FP32>(kc[s][0]), rec_up<FP32>(kc[s][1]));
       }
 #pragma unroll
       for (int s = 0; s < T::kUnits; ++s)
@@ -529,8 +537,8 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
           *reinterpret_cast<u4v*>(ops_own + T::op_at(false, s, p)) = kown[s].p[p];
         }
 #pragma unroll
-      for (int g = 0; g < 4; ++g) vx[g] = *reinterpret_cast<const f4v*>(sm + T::kVOff + wave * 4096 + colb[g]);
-      kop[0] = rec_op<FP32, true>(kx[0][0], kx[0][1]);
+      for (int g = 0; g < 4; ++g) vx[g] = rec_up<FP32>(*reinterpret_cast<const f4v*>(sm + T::kVOff + wave * 4096 + colb[g]));
+      kop[0] = rec_op<FP32, true>(rec_up<FP32>(kx[0][0]), rec_up<FP32>(kx[0][1]));
     }
     block_sync();
     const auto read_op = [&](bool of_q, int u) {
@@ -548,7 +556,7 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
     sched_fence();
     static_for<T::kUnits>([&](auto it) {
       constexpr int s = decltype(it)::value;
-      if constexpr (s + 1 < T::kUnits) kop[s + 1] = rec_op<FP32>(kx[s + 1][0], kx[s + 1][1]);
+      if constexpr (s + 1 < T::kUnits) kop[s + 1] = rec_op<FP32>(rec_up<FP32>(kx[s + 1][0]), rec_up<FP32>(kx[s + 1][1]));
       else top = rec_op_of_c<FP32>(st[0], 0);
       sp = rec_mma<FP32>(kop[s], qown[s], sp);
       rec_interleave<FP32, 0, 8>();
@@ -659,7 +667,7 @@ AAT_DEV bool rec_scan(char* smem, const float* __restrict__ q, const float* __re
     for (int g = 0; g < 4; ++g)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        *reinterpret_cast<float*>(sm + (e & 1 ? ow_odd : ow_even) + (8 * g + (e & 2)) * 128) = oacc[4 * g + e];
+        *reinterpret_cast<float*>(sm + (e & 1 ? ow_odd : ow_even) + (8 * g + (e & 2)) * 128) = FP32 ? oacc[4 * g + e] : oacc[4 * g + e] * kRecDown;
   }
   block_sync();               // the last chunk's output tiles are staged: the data wave stores them
   return finite.broken();
@@ -750,7 +758,7 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
     char* const mine = ops + ((size_t)bh * nchunk + c) * (2 * KD / 16) * 3072 + lane * 16;
 #pragma unroll
     for (int s = 0; s < kUnits; ++s) {
-      const RecOp<false> o = rec_op<false>(qx[s][0], qx[s][1]);
+      const RecOp<false> o = rec_op<false>(rec_up<false>(qx[s][0]), rec_up<false>(qx[s][1]));
 #pragma unroll
       for (int p = 0; p < 3; ++p) *reinterpret_cast<u4v*>(mine + (wave * kUnits + s) * 3072 + p * 1024) = o.p[p];
     }
@@ -759,7 +767,7 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
       if (wave + 4 * t < kTiles) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-          const RecOp<false> o = rec_op<false>(kr[t][2 * s], kr[t][2 * s + 1]);
+          const RecOp<false> o = rec_op<false>(rec_up<false>(kr[t][2 * s]), rec_up<false>(kr[t][2 * s + 1]));
 #pragma unroll
           for (int p = 0; p < 3; ++p) *reinterpret_cast<u4v*>(mine + (KD / 16 + 2 * (wave + 4 * t) + s) * 3072 + p * 1024) = o.p[p];
         }
@@ -1099,9 +1107,9 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
 //
 // Bound by the chain of a chunk in one wave per SIMD: 52 matrix instructions (24 below 192 key dims) = 1800 (1024) of some 3000 (2600)
 // cycles, the rest the barrier, LDS latency and vector work that a result of the chunk has to wait for; with 256 blocks of 256 key dims the
-// operands, 96 KB per block and chunk from L2, add 15 us of 80.  Whole calls, the split kernel above and this one with its launch ahead:
-// B2 H8 L2048 128/128 135 -> 84 us, B1 H8 L2048 256/128 152 -> 106, B4 H16 L2048 64/128 139 -> 112, B2 H8 L1056 256/512 87.2 -> 79.7.
-// Tried and not kept: 32 key dims per wave, eight waves (B2 H8 L1056 256/512 94); the operands brought into L2 by the data wave's touches
+// operands, 96 KB per block and chunk from L2, add 15 us of 80.  Whole calls on inputs that change, the split kernel above and this one with
+// its launch ahead: B2 H8 L2048 128/128 139 -> 96 us, B1 H8 L2048 256/128 157 -> 120, B4 H4 L1024 64/64 73 -> 48, B2 H8 L1056 256/512 92 -> 89
+// (all operands in the caches: 87 -> 83).  Tried and not kept: 32 key dims per wave, eight waves (B2 H8 L1056 256/512 94); the operands brought into L2 by the data wave's touches
 // (91 against 79 without); partial sums added and stored by the matrix waves (+8); V read straight into registers (+6).
 template <int KD, int WK>
 struct RetRecurrentStream {
@@ -1261,7 +1269,9 @@ AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const floa
 #pragma unroll
     for (int g = 2 * s; g < 2 * s + 2; ++g) wx[g] = *reinterpret_cast<const f4v*>(sm + T::kFOff + hi * 64 + g * 16);
   };
-  const auto make_v = [&](int s) { return rec_op<FP32>(vx[2 * s] * wx[2 * s], vx[2 * s + 1] * wx[2 * s + 1]); };   // of V w / lambda'
+  const auto make_v = [&](int s) {                         // of V w / lambda'
+    return rec_op<FP32>(rec_up<FP32>(vx[2 * s]) * wx[2 * s], rec_up<FP32>(vx[2 * s + 1]) * wx[2 * s + 1]);
+  };
   read_v(stage_of(0));
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -1297,14 +1307,14 @@ AAT_DEV bool rec_stream_scan(char* smem, const float* __restrict__ q, const floa
       constexpr int u = decltype(it)::value, kb = u >> 1, s = u & 1;
       if constexpr (u == 0) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[r] *= pnl;
+        for (int r = 0; r < 16; ++r) oacc[r] = FP32 ? oacc[r] * pnl : oacc[r] * pnl * kRecDown;
       }
       if constexpr (u >= 2) {
         top[u - 2] = rec_op_of_c<FP32>(st[0], u - 2);
         rec_pin(top[u - 2]);
       }
       st[kb] = rec_mma<FP32>(kop[u], vop[s], st[kb]);
-      rec_interleave<FP32, 0, u == 0 ? 3 : 8>();
+      rec_interleave<FP32, 0, u == 0 ? 6 : 8>();
       kop[u] = read_k(u, next);
     });
 

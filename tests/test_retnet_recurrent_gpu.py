@@ -276,16 +276,22 @@ def test_blocks_that_split_the_value_dims(b, h, kdim, vdim, seqlen):
         _close(out[:, head], ref[:, head])
 
 
-# fp32 products in three bf16 parts: values down to where the smallest part of one is a bf16 subnormal, and magnitudes that differ from key dim to
-# key dim; a part lost to a flush or a common scale would show as 2^-8 or 2^-16 of a value
-@pytest.mark.parametrize("k_scale,q_scale,spread", [(1e-30, 1e20, 0.0), (1e30, 1e-20, 0.0), (1.0, 1.0, 12.0)])
-def test_products_in_parts_keep_the_range_of_fp32(k_scale, q_scale, spread):
-    q, k, v, decay = _inputs(22, 8, 24, 128, 128, 64, 0.9, 1.0)
-    per_dim = 10.0 ** ((torch.arange(128) * 37 % 128 / 127.0 - 0.5) * spread).view(1, 1, 128, 1)
-    q, k = (q * q_scale * per_dim).float(), (k * k_scale / per_dim).float()
+# fp32 products in three bf16 parts: Q, K, V, S^T, the State or outputs at the low end of fp32 (2e-37 / 2^24 lies below the smallest bf16
+# subnormal, 9e-41: parts of a value that is not scaled are off by 2e-4 of it), at the high end (the State is held divided by lambda, 2^-40 at the
+# least: 3e26 is as far as fp32 goes), and magnitudes that differ from key dim to key dim.
+# Blocks of 128 and 64 value dims, and those with operands made ahead
+@pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(8, 24, 128, 128, 64), (8, 24, 64, 64, 64), (1, 2, 64, 64, 512), (1, 2, 128, 64, 512),
+                                                   (1, 2, 192, 64, 512), (1, 2, 256, 64, 512)])
+@pytest.mark.parametrize("k_scale,q_scale,v_scale,spread", [(1e-30, 1e20, 1.0, 0.0), (2e-37, 1e26, 1.0, 0.0), (1e26, 2e-37, 1.0, 0.0), (1e20, 1.0, 2e-37, 0.0),
+                                                            (1e-19, 2e-18, 1e25, 0.0), (1e-19, 1e26, 2e-18, 0.0), (1e-15, 1e-15, 2e-7, 0.0),
+                                                            (1e24, 1e-20, 1.0, 0.0), (1.0, 1.0, 1.0, 12.0)])
+def test_products_in_parts_keep_the_range_of_fp32(b, h, kdim, vdim, seqlen, k_scale, q_scale, v_scale, spread):
+    q, k, v, decay = _inputs(22, b, h, kdim, vdim, seqlen, 0.9, 1.0)
+    per_dim = 10.0 ** ((torch.arange(kdim) * 37 % kdim / (kdim - 1.0) - 0.5) * spread).view(1, 1, kdim, 1)
+    q, k, v = (q * q_scale * per_dim).float(), (k * k_scale / per_dim).float(), (v * v_scale).float()
     out = aat.retnet_recurrent_fwd(q.cuda(), k.cuda(), v.cuda(), decay.cuda())
     ref = torch.from_numpy(brute.retnet_recurrent(q.numpy(), k.numpy(), v.numpy(), decay.numpy()))
-    for head in range(24):
+    for head in range(h):
         _close(out[:, head], ref[:, head])
 
 
@@ -333,9 +339,10 @@ def test_values_that_are_not_finite(value, which, kdim, vdim):
 
 # 3.4e38 rounds to an infinity in bf16, but is none: with small partners every product and sum stays finite
 @pytest.mark.parametrize("which", ["q", "k"])
-@pytest.mark.parametrize("kdim,vdim", [(128, 128), (64, 128), (64, 64)])
-def test_values_beyond_the_largest_of_bf16(which, kdim, vdim):
-    b, h, seqlen, pos = 8, 24, 128, 70
+@pytest.mark.parametrize("b,h,kdim,vdim,seqlen", [(8, 24, 128, 128, 128), (8, 24, 64, 128, 128), (8, 24, 64, 64, 128), (4, 6, 64, 64, 512),
+                                                   (4, 6, 128, 64, 512), (4, 6, 192, 64, 512), (4, 6, 256, 64, 512)])
+def test_values_beyond_the_largest_of_bf16(which, b, h, kdim, vdim, seqlen):
+    pos = 70
     q, k, v, decay = _inputs(24, b, h, kdim, vdim, seqlen, 0.9, 1.0)
     x = {n: t if n == which else t * 1e-6 for n, t in (("q", q), ("k", k), ("v", v))}
     x[which][3, 5, 7, pos] = 3.4e38
