@@ -109,7 +109,8 @@ attn_bwd_col(const half_t* __restrict__ k, const half_t* __restrict__ v, const h
     dma.issue(dOg + (size_t)j * T::kYBytes, base + T::kYBytes, wave * 64);
     // every wave copies the statistics (same bytes, same place): uniform instruction counts
     const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(AAT_AS3 char*)(base + 2 * T::kYBytes));
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(stat_off), "s"(statg + (size_t)j * BY * 4) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 ::"s"(dst), "v"(stat_off), "s"(statg + (size_t)j * BY * 4) : "memory", "m0");
   };
 
   // resident operands: this lane's two rows of K and of V as MFMA B fragments

@@ -250,7 +250,8 @@ struct TileDma {
       static_assert(AUX == 0 || !SADDR, "the scalar-base form is written without cache-policy bits");
       const uint32_t dst = __builtin_amdgcn_readfirstlane(
           (uint32_t)(uintptr_t)(AAT_AS3 char*)(lds + (i * NT + wave_base) * 16));
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(lane_off), "s"(base) : "memory");
+      // a wait state between the write of M0 and the copy that reads it; the compiler leaves one in front of its own
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(lane_off), "s"(base) : "memory", "m0");
       return;
     }
     __builtin_amdgcn_global_load_lds((const AAT_AS1 void*)(uintptr_t)(base + lane_off),

@@ -538,3 +538,20 @@ def test_the_library_cuts_the_kv_range_as_the_tile_shape_rule_assumes():
                 assert lib.workspace_size(b, h, sq, sk) == want, (cfg, b, h, sq, sk, parts)
     assert gfx950_space.rule_forward_config(128, 128, ARCH, 3, 12, 1088, 1088, True) is not None
     assert gfx950_space.rule_forward_config(128, 128, ARCH, 1, 1, 128, 80, False) is None       # not whole 32-row groups
+
+
+def test_a_write_of_m0_leaves_a_wait_state_before_the_copy_that_reads_it():
+    """Copies to LDS written by hand: one wait state between the scalar write of M0 and the load (the compiler's own have it), and
+    the compiler knows that M0 has changed."""
+    root = os.path.join(os.path.dirname(codegen.__file__), "..", "csrc")
+    found = 0
+    for folder, _, names in os.walk(root):
+        for name in names:
+            if not name.endswith((".h", ".hip", ".py")):
+                continue
+            text = open(os.path.join(folder, name)).read()
+            for m in re.finditer(r"asm(?: volatile)?\(((?:[^;\"]|\"[^\"]*\")*)\);", text):
+                if re.search(r"\bm0, ", m.group(1)):
+                    found += 1
+                    assert re.search(r"s_mov_b32 m0, %\d\\n\\ts_nop \d\\n", m.group(1)) and m.group(1).rstrip().endswith('"m0"'), (name, m.group(1))
+    assert found >= 5
