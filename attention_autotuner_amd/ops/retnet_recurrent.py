@@ -57,7 +57,13 @@ def retnet_recurrent_fwd(q, k, v, decay, device_type=None, block_kdim=None, out=
     assert out.shape == v.shape and out.dtype == torch.float32 and out.is_contiguous() and out.device == v.device
     if workspace is None or workspace.numel() * workspace.element_size() < lib.retnet_recurrent_workspace_size(batch, nheads, kdim, vdim, seqlen, block_kdim):
         room = int(lib.retnet_recurrent_room(batch, nheads, kdim, vdim, seqlen, block_kdim, _MOST_WORKSPACE))      # workspace_size() or more
-        workspace = torch.empty(max(room, 1), dtype=torch.uint8, device=q.device)
+        try:
+            workspace = torch.empty(max(room, 1), dtype=torch.uint8, device=q.device)
+        except torch.cuda.OutOfMemoryError:
+            need = int(lib.retnet_recurrent_workspace_size(batch, nheads, kdim, vdim, seqlen, block_kdim))
+            if room == need:
+                raise
+            workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)      # K and Q are laid out by every block for itself
     with torch.cuda.device(q.device):
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         rc = lib.retnet_recurrent_fwd_ex(*[ctypes.c_void_p(t.data_ptr()) for t in (q, k, v, decay, out)], batch, nheads, kdim,

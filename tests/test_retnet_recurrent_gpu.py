@@ -442,3 +442,21 @@ def test_operands_made_ahead_keep_the_range_of_fp32_and_replay():
         torch.cuda.synchronize()
         assert torch.equal(got, out)
         _ = (q * 2).sum().item()
+
+
+def test_without_memory_for_operands_made_ahead_a_call_takes_the_least_it_needs(monkeypatch):
+    dims = b, h, kdim, vdim, seqlen = 1, 2, 128, 64, 512
+    need, room = _room(*dims)
+    assert room > need
+    q, k, v, decay = (t.cuda() for t in _inputs(29, *dims, 0.9, 1.0))
+    want = aat.retnet_recurrent_fwd(q, k, v, decay, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+    empty, asked = torch.empty, []
+
+    def no_memory(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            asked.append(size[0])
+            if size[0] > need:
+                raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+    monkeypatch.setattr(torch, "empty", no_memory)
+    assert torch.equal(aat.retnet_recurrent_fwd(q, k, v, decay), want) and asked == [room, need]
