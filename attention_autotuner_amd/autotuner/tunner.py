@@ -55,6 +55,8 @@ class _ForwardTunner(BaseTunner):
         whole = config is None or s["Sq"] % config.Br == 0
         if self.operation == "ret":                       # <..., DECAY>
             return (not flags or flags[-1] == bool(self.decay)) and general in (None, not whole)
+        if getattr(config, "kv_groups", 1) > 1:               # a library of one kernel
+            return True
         if "flashattn_fwd_regfuse" in mangled and len(flags) == 5:     # <..., GEN, PIPE, CAUSAL, SPLIT, PERSIST, PAIR>
             # one general kernel, for both walks, in one part or in several; the others at whole tiles in one part
             parts = 1 if config is None else gfx950_space.kv_parts(config, self.arch, s["B"], s["H"], s["Sq"], s["Sk"], self.causal)
@@ -97,6 +99,22 @@ class AttnTunner(_ForwardTunner):
 
     def __init__(self, arch, torch_array, causal=False, softmax_scale=None):
         super().__init__(arch, torch_array, "attention", causal=causal, softmax_scale=softmax_scale)
+
+    def _few_blocks(self):
+        """What a call of few row blocks launches untuned (waves that share their rows), or None."""
+        k, s = self.problem_key, self.problem_shape
+        cfg = gfx950_space.few_blocks_config(k["dim_qk"], k["dim_v"], s["B"], s["H"], s["Sq"], s["Sk"], self.causal) if _is_rocm(self.arch) else None
+        return cfg if cfg is not None and self._is_valid(cfg) else None
+
+    # Such a problem times that configuration too, whatever the cost model says, which was fitted without any: a tuned entry goes
+    # ahead of the rule from then on and would be the slower of the two otherwise.
+    def get_tuned_configs(self):
+        cfg = self._few_blocks()
+        return super().get_tuned_configs() + ([cfg] if cfg is not None else [])
+
+    def prune(self, configs):
+        shared_rows = [c for c in configs if getattr(c, "kv_groups", 1) > 1]
+        return super().prune([c for c in configs if c not in shared_rows]) + shared_rows
 
     def _ex_args(self):
         scale = self.softmax_scale

@@ -555,3 +555,25 @@ def test_a_write_of_m0_leaves_a_wait_state_before_the_copy_that_reads_it():
                     found += 1
                     assert re.search(r"s_mov_b32 m0, %\d\\n\\ts_nop \d\\n", m.group(1)) and m.group(1).rstrip().endswith('"m0"'), (name, m.group(1))
     assert found >= 5
+
+
+FEW = [((2, 8, 512, 512, 64), False), ((1, 8, 1024, 1024, 128), True), ((3, 5, 32, 160, 64), True), ((1, 12, 768, 1024, 128), False)]
+
+
+@pytest.mark.parametrize("problem,causal", FEW)
+def test_tuning_a_problem_of_few_row_blocks_times_what_it_launches_untuned(problem, causal):
+    """A tuned entry goes ahead of the rule for good: the rule's configuration has to be among what is built and timed."""
+    from attention_autotuner_amd.benchmarks.tune import make_tensors
+    b, h, sq, sk, d = problem
+    pick = gfx950_space.few_blocks_config(d, d, b, h, sq, sk, causal)
+    tuner = AttnTunner(ARCH, make_tensors("attn", b, h, sq, sk, d, d, "meta"), causal=causal)
+    assert tuner.cost_model is not None
+    fitting = [c for c in tuner.get_tuned_configs() if tuner._fits_problem(c)]
+    assert [c for c in fitting if c.kv_groups > 1] == [pick]
+    timed = tuner.prune(fitting)
+    assert pick in timed and (len(timed) < len(fitting) or len(fitting) <= tuner.keep_min)
+    kernels = [k["kernel"] for k in codegen.resource_usage(codegen.compile_config(pick, ARCH, timeout=600)) if "flashattn" in k["kernel"]]
+    assert len(kernels) == 1 and tuner._kernel_matters(kernels[0], pick)
+    # other problems are tuned as before
+    many = AttnTunner(ARCH, make_tensors("attn", 4, 32, 2048, 2048, d, d, "meta"), causal=causal)
+    assert all(c.kv_groups == 1 for c in many.get_tuned_configs())
