@@ -40,6 +40,9 @@ def _bind(lib, op):
     if op == "attn":
         lib.kernel_entry_lse.restype = _I
         lib.kernel_entry_lse.argtypes = [_VP] * 5 + [_I] * 4 + tail
+    if op == "attn_bwd":
+        lib.column_rows.restype = _I
+        lib.column_rows.argtypes = [_I] * 5
     if op in DECAY_OPS:                               # mask slot carries log2(gamma) [H]; dqaccum and causal are gone
         nd = n - 1 if op == "ret_bwd" else n
         lib.profile_decay.restype = _F

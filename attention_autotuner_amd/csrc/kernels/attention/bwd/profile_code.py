@@ -118,6 +118,13 @@ hipError_t launch(aat_half* q, aat_half* k, aat_half* v, aat_half* o, aat_half* 
 extern "C" int abi_version(void) {{ return AAT_ABI_VERSION; }}
 extern "C" const char* config_string(void) {{ return "{config_name}"; }}
 extern "C" size_t workspace_size(int B, int H, int Seq_q, int) {{ return stats_bytes(B, H, Seq_q); }}
+extern "C" int column_rows(int B, int H, int Seq_q, int Seq_k, int causal) {{
+  if (!bwd_shape_ok(B, H, Seq_q, Seq_k)) return 0;
+#if AAT_COL_WIDE
+  if (wide_columns(B * H, Seq_k, causal)) return aat::AttnBwdCol::BX;
+#endif
+  return Br;
+}}
 """
 
 profile_func = r"""

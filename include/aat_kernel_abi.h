@@ -212,6 +212,11 @@ size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most);
 size_t retnet_recurrent_room(int batch, int heads, int kdim, int vdim, int l, int block_kdim, size_t most);
 #endif
 
+#if defined(AAT_OP_ATTN_BWD)
+/* kv rows per block of the column kernel (dV, dK) that a call of this problem launches; 0 for lengths the entry points refuse. */
+int column_rows(int B, int H, int Seq_q, int Seq_k, int causal);
+#endif
+
 #ifdef __cplusplus
 }
 #endif

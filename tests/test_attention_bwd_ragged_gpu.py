@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import attention_autotuner_amd as aat
-from attention_autotuner_amd.autotuner import Runtime, gfx950_space, prebuilt_extra
+from attention_autotuner_amd.autotuner import Runtime, codegen, gfx950_space, library, prebuilt_extra
 from oracle import ref_op, tolerance
 
 pytestmark = pytest.mark.gpu
@@ -62,6 +62,7 @@ def test_two_row_groups_per_wave_and_one_column_kernel_per_output(causal):
 def test_column_blocks_of_256_rows(problem, causal):
     cfgs = [c for c in gfx950_space.rule_attn_backward_configs(128, 128) if c.Br == 128 and not c.col_split]
     assert cfgs
+    assert library.load(codegen.compile_config(cfgs[0], ARCH), "attn_bwd").column_rows(*problem, causal) == 256
     _check(problem, 128, 128, causal, 370, cfgs[:1])
 
 

@@ -577,3 +577,56 @@ def test_tuning_a_problem_of_few_row_blocks_times_what_it_launches_untuned(probl
     # other problems are tuned as before
     many = AttnTunner(ARCH, make_tensors("attn", 4, 32, 2048, 2048, d, d, "meta"), causal=causal)
     assert all(c.kv_groups == 1 for c in many.get_tuned_configs())
+
+
+def test_few_row_blocks_take_shared_rows_within_their_lines_and_ahead_of_other_problems_entries(tmp_path, monkeypatch):
+    """gfx950_space.FEW_BLOCKS at its limits: rows of a block of the pick (32 or 64), None beyond them."""
+    def rows(d, b, h, sq, sk, causal):
+        cfg = gfx950_space.few_blocks_config(d, d, b, h, sq, sk, causal)
+        if cfg is not None:
+            assert cfg.kv_groups == 4 and gfx950_space.forward_valid(cfg, ARCH) and cfg == gfx950_space.rule_forward_config(d, d, ARCH, b, h, sq, sk, causal)
+        return cfg and cfg.Br
+    assert [rows(64, 1, 16, 512, sk, False) for sk in (128, 160, 512, 2112, 2144)] == [None, 32, 32, 32, None]       # 256 blocks of 32 rows
+    assert [rows(64, 1, 17, 512, sk, False) for sk in (608, 640, 2112, 2144)] == [None, 64, 64, None]               # 272, 136 of 64
+    assert [rows(64, 1, 32, 512, sk, causal) for sk, causal in ((512, True), (512, False), (1024, False))] == [32, None, 64]
+    assert rows(64, 1, 33, 512, 1024, True) is rows(64, 1, 33, 512, 1024, False) is None                             # 528, 264 of 64
+    assert [rows(128, 1, 8, 1024, sk, True) for sk in (256, 288, 1536, 1568)] == [None, 32, 32, None]
+    assert [rows(128, 1, 12, 768, sk, False) for sk in (608, 640, 1536, 1568)] == [None, 64, 64, None]
+    assert [rows(d, 1, 2, 512, 512, False) for d in (192, 256)] == [None, None]
+    assert gfx950_space.few_blocks_config(64, 64, 1, 2, 500, 512, False) is gfx950_space.few_blocks_config(64, 128, 1, 2, 512, 512, False) is None
+
+    from attention_autotuner_amd.ops import _resolve
+    base_tunner._memo.clear()
+    monkeypatch.setattr(_resolve, "Runtime", lambda arch, cc: cc)
+    monkeypatch.setenv("AAT_TUNE_ON_MISS", "0")
+    near = AttnConfig(Br=128, Bc=64, Kd=128, D=128, Nthreads=256)
+    for name in ("b4h32q512k512", "b4h32q2048k2048"):
+        with open(tmp_path / f"best_config_attention_MI355X_128_128_{name}_c0.json", "w") as f:
+            json.dump(near.to_dict(), f)
+
+    def planned(b, h, s):
+        def make():
+            t = AttnTunner(ARCH, [torch.empty(b, h, s, 128, dtype=torch.float16, device="meta") for _ in range(4)])
+            t.cache_path = str(tmp_path)
+            return t
+        return _resolve.planned(("attn", ARCH.name, b, h, s, s, 128, 128, False), make,
+                                lambda: gfx950_space.default_forward_config("attn", 128, 128, ARCH, s, s, (b, h, False)))[0]
+    assert planned(1, 12, 512).kv_groups == 4 and planned(4, 24, 512) == near
+    base_tunner._memo.clear()
+
+
+def test_the_library_says_which_column_kernel_a_backward_launches():
+    """256-row column blocks at 128 wide heads: by rounds of blocks over 256 units, causal from 512 blocks on, one output kernel only."""
+    cfgs = {c.Br: c for c in gfx950_space.rule_attn_backward_configs(128, 128) if not c.col_split}
+    lib = library.load(codegen.compile_config(cfgs[128], ARCH, timeout=600), "attn_bwd")
+    # (B, H, Sq, Sk), causal: blocks of 256 and of 128 rows
+    for problem, causal, want in (((4, 32, 2048, 2048), 0, 256), ((4, 32, 2048, 2048), 1, 256),      # 1024, 2048: 4 rounds and 8
+                                  ((2, 64, 256, 256), 0, 128), ((2, 65, 256, 256), 0, 256),          # 128, 256: one and one; 130, 260: one and two
+                                  ((2, 128, 256, 256), 0, 256), ((2, 129, 256, 256), 0, 128),        # 256, 512: one and two; 258, 516: two and three
+                                  ((1, 64, 2048, 2048), 1, 256), ((1, 63, 2048, 2048), 1, 128),      # 512; 504
+                                  ((10, 13, 96, 160), 0, 256), ((16, 32, 96, 256), 1, 256), ((1, 2, 96, 80), 0, 0)):
+        assert lib.column_rows(*problem, causal) == want, (problem, causal)
+    others = [gfx950_space.rule_attn_backward_configs(64, 64)[0]] + ([cfgs[64]] if 64 in cfgs else [])
+    for cfg in others:
+        lib = library.load(codegen.compile_config(cfg, ARCH, timeout=600), "attn_bwd")
+        assert lib.column_rows(4, 32, 2048, 2048, 0) == cfg.Br
