@@ -42,8 +42,8 @@ struct RetBwdDk {
   static constexpr int DTW = Kd / 32 / NWD, KSTEPS = BY / 16;
   static constexpr int NCZ = Kd / 8, NCS = 8, NSUB = BX / 64;
   static_assert(NWD * NWK * kWave == Nthreads && DTW * NWD * 32 == Kd, "32 kv rows by whole 32-column tiles per wave");
-  static_assert((BY == 64 || BY == 32) && Kd % 64 == 0 && BX % 64 == 0, "a query tile is a row of dS blocks or half of one");
-  static_assert(NS >= 2, "buffers");
+  static_assert(BY == 64 && Kd % 64 == 0 && BX % 64 == 0, "a query tile is one row of dS blocks");
+  static_assert(NS == 2 || NS == 3, "buffers");
   using ZDma = TileDma<BY, NCZ, Nthreads, Swz::Rows4>;   // Q tile
   static constexpr int kSIters = BY * NSUB * NCS / Nthreads, kSRows = Nthreads / NCS;   // dS tile: LDS-DMA instructions per thread, rows per instruction
   static_assert(kSIters * Nthreads == BY * NSUB * NCS, "whole 32-row pieces of dS blocks per instruction");
@@ -113,7 +113,7 @@ ret_bwd_dk_from_ds(const half_t* __restrict__ q, const half_t* __restrict__ ds, 
   auto issue = [&](int jt, int st) {              // walked downwards from the end of the sequence, like the column passes of the chained kernel
     char* base = smem + st * T::kStageBytes;
     zdma.issue(zg + (size_t)jt * T::kZBytes, base, wave_base);
-    const char* const rows = sg + (size_t)(jt * BY / 64) * s_pitch + jt * BY % 64 * 128;
+    const char* const rows = sg + (size_t)jt * s_pitch;
 #pragma unroll
     for (int i = 0; i < T::kSIters; ++i) {
       const int r = i * T::kSRows + wave * (kWave / NCS), sub = r / BY;
