@@ -719,8 +719,10 @@ def default_attn_backward_config(dim_qk, dim_v, arch, seq_q=None, seq_k=None, pr
 # d 128 from 256 on where they all fit side by side (0.86 ... 0.91 of the time at 360 to 476 blocks of 64 rows; 1.17 and 1.22 where
 # 260 blocks of 128 rows make a second round).  A causal walk's blocks are of all lengths, and finer ones end together: the line lies
 # at 1600 there (from 600 to 1600 blocks the larger ones take 0.99 ... 1.10 of the time at 352 to 2112 rows).  At d 64 the smaller tile
-# leaves room for four blocks to a CU, which lead beyond the line; a causal walk of 800 rows and more keeps the larger tile up to 640 blocks
-# (500 to 624: 1.06 ... 1.13 with the smaller one, 0.86 and 0.92 at 352 and 544 rows).
+# leaves room for four blocks to a CU, which lead beyond the line.  A causal walk at d 64 keeps the larger tile further (time of the smaller one over
+# it, 18 lengths from 704 to 2048 rows): whole blocks of 64 rows, from 960 rows on, 1.00 ... 1.14 at 560 to 640 blocks and 0.98 ... 1.06 at 650 to 700; of
+# 832 and 896 rows 1.01 ... 1.07 up to 611, 0.97 and 1.02 at 630; with half a block at the end, from 800 rows on, 0.99 ... 1.08 up to 576 and 0.92 ... 1.01
+# around 630; shorter ones 1.0 at 550 and 0.94 ... 0.97 from 594 on.
 ATTN_BWD_RULE = {
     (64, 64): (dict(Br=64, Bc=64, Nthreads=128, num_stages_qk=2, row_waves_per_eu=2, row_Bc=64),
                dict(Br=64, Bc=32, Nthreads=128, num_stages_qk=2, waves_per_eu=2, row_waves_per_eu=2)),
@@ -742,7 +744,8 @@ def rule_attn_backward_config(dim_qk, dim_v, b, h, seq_q, seq_k, causal):
         return None
     blocks = b * h * -(-seq_k // 64)
     if causal:
-        return pair[blocks > (1600 if dim_qk > 64 else 640 if seq_k >= 800 else 512)]
+        line = 1600 if dim_qk > 64 else 512 if seq_k < 800 else 576 if seq_k % 64 else 608 if seq_k < 960 else 640
+        return pair[blocks > line]
     side_by_side = dim_qk == 128 and blocks > 256 and b * h * -(-seq_k // 128) <= 256
     return pair[blocks > 512 or side_by_side]
 

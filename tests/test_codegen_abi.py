@@ -643,3 +643,13 @@ def test_the_library_says_which_column_kernel_a_backward_launches():
     for cfg in others:
         lib = library.load(codegen.compile_config(cfg, ARCH, timeout=600), "attn_bwd")
         assert lib.column_rows(4, 32, 2048, 2048, 0) == cfg.Br
+
+
+def test_the_line_between_the_backward_tiles_of_a_causal_walk_depends_on_its_rows():
+    """d 64: the larger tile up to so many blocks of 64 rows, measured either side (gfx950_space.ATTN_BWD_RULE)."""
+    def streamed(s, heads):
+        return gfx950_space.rule_attn_backward_config(64, 64, 1, heads, s, s, True).Bc
+    for s, heads, larger in ((768, 42, True), (768, 43, False), (800, 44, True), (800, 45, False), (864, 41, True), (864, 45, False),
+                             (896, 43, True), (896, 45, False), (1088, 36, True), (1088, 37, True), (1088, 38, False), (1184, 30, True), (1184, 33, False),
+                             (2048, 20, True), (2048, 21, False)):
+        assert (streamed(s, heads) == 64) == larger, (s, heads)
