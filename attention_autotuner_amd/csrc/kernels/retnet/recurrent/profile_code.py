@@ -111,7 +111,10 @@ hipError_t launch_stream(const float* q, const float* k, const float* v, const f
 // How a problem is scanned, by estimates of each way in microseconds per chunk of 32 positions: time per chunk of a round of blocks, times
 // the rounds on 256 compute units (a block fills one; two of the 64 x 64 ones share one).
 //  passes  over 128 and 64 key dims with 128 (wide) or 64 value dims per block, and the addition of their outputs.  Blocks of 64 value
-//          dims and 128 key dims never came out ahead and are not built.
+//          dims and 128 key dims never came out ahead and are not built.  Measured lines: at 2.75 a chunk for 64 x 64 against stream B5 H6 L4064
+//          64/512 349 -> 298 us, B1 H32 L576 64/512 59 -> 51, B7 H20 L512 64/256 98 either way; the others any higher lose (B3 H16 L736 128/512
+//          99 -> 120 with 5.0 for 4.8, B6 H32 L576 192/128 158 -> 175 with 3.4 for 3.25).  The second pass and the addition are launches of their own: B5 H20
+//          256/256 36.4 against 34.3 us split at 64 positions, 62 against 65 at 160, B6 H32 192/128 40.2 and 38.4 at 96.
 //  split   blocks of 32 value dims that split the key dims between their waves.  Measured at 2048 positions, whole calls, passes
 //          against split: B4 H8 128/256 344 -> 147 us, B4 H12 128/256 347 -> 268, B4 H16 64/128 207 -> 142, B4 H16 192/256 609 -> 371.
 //  stream  the same with the operands of K and Q made ahead, where the caller has the room: 20 bytes of traffic per key dim and
@@ -130,7 +133,8 @@ Estimate estimate(long bh, int vdim, int l, int block_kdim) {{
   e.split = pmat + (block_kdim == 64 ? 1.95 : block_kdim == 128 ? 2.05 : block_kdim == 192 ? 2.45 : 2.4) * narrow;
   const double add = block_kdim > 128 ? 3.0 * bh * vdim * 32 * 4 / 8e6 : 0.0;      // two reads and a write, partly from the cache
   e.passes = e.wide ? (block_kdim / 128 * 4.8 + block_kdim / 64 % 2 * 3.25) * rounds(bh * (vdim / 128), kUnits) + add
-             : block_kdim == 64 ? 2.5 * rounds(bh * (vdim / 64), 2 * kUnits) : 2 * e.split;
+             : block_kdim == 64 ? 2.75 * rounds(bh * (vdim / 64), 2 * kUnits) : 2 * e.split;
+  if (block_kdim > 128) e.passes += 0.3 * 32 / l;                                  // two launches more in a call
   const double ahead = (double)bh * 32 * (20.0 * block_kdim + 256) / ((double)bh * l * (12.0 * block_kdim + 128) <= 1.1e8 ? 7e6 : 3e6);
   e.stream = ahead + (block_kdim == 64 ? 1.1 : block_kdim == 128 ? 1.35 : block_kdim == 192 ? 1.75 : narrow > 1 ? 2.1 : 1.8) * narrow;
   return e;

@@ -384,7 +384,7 @@ def test_operands_made_ahead(b, h, kdim, vdim, seqlen):
 
 
 def test_the_room_is_offered_where_it_pays_and_not_beyond_what_is_asked_for():
-    for dims in [(2, 8, 256, 512, 1056), (1, 4, 64, 64, 512)]:
+    for dims in [(2, 8, 256, 512, 1056), (1, 4, 64, 64, 512), (5, 6, 64, 512, 512)]:
         need, room = _room(*dims)
         assert room > need and _room(*dims, most=room) == (need, room) and _room(*dims, most=room - 1) == (need, need)
     for dims in [(8, 32, 128, 128, 2048), (1, 4, 64, 64, 480), (8, 16, 256, 64, 1024)]:
