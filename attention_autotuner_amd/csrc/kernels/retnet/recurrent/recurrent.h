@@ -15,11 +15,12 @@
 //
 // One block owns one (batch, head) and a slice of DVS value dims; wave w owns value dims [32w, 32w+32) of
 // the slice: its State tiles (KD x 32, fp32, in registers for the whole sequence) and its rows of O^T.
-// v_mfma_f32_32x32x2_f32, lane l, half h = l/32, column j = l%32:
+// Products of 32 x 32 tiles are fp32 matrix instructions (v_mfma_f32_32x32x2_f32) or, where that is the faster way, bf16 ones
+// (v_mfma_f32_32x32x16_bf16) of the operands' parts (RecOp).  Lane l, half h = l/32, column j = l%32 of an fp32 one:
 //   A (32 x 2): lane holds A[j][h];  B (2 x 32): lane holds B[h][j];  C (32 x 32): lane holds C[8g+4h+e][j].
 // The contraction index of a step is free as long as A and B agree, so step (g, e) is given the index
 // 8g+4h+e: then the C registers of one product ARE the A or B operand of the next (State feeds
-// State^T*Q, P feeds V*P) and no value ever changes lanes.
+// State^T*Q, P feeds V*P) and no value ever changes lanes.  The bf16 ones take 16 indices at a time in the same order.
 // S^T is split over the waves along kd (each wave contracts KD/waves key dims), the partial tiles are
 // summed through LDS; every other product is private to its wave.
 #pragma once
@@ -789,9 +790,10 @@ __global__ __launch_bounds__(256) void retnet_recurrent_pmat(const float* __rest
 // (row group g of the C layout goes to wave g % WK), contracts its 8 positions of P with V, and stores its 8
 // rows of the output.  Q is read once per wave and feeds both contractions.
 //
-// Bound by fp32 MFMA like the kernel above; a slice of 32 repeats S^T in every block, so a chunk costs
-// (3 KD + 32) / (2 KD + 32 + KD / 4) of the work of a 128-wide slice, 1.27 times (KD 64) and 1.30 (KD 128), against four times the
-// blocks.  B4 H8 L2048 128/256, 256 blocks: 353 -> 145 us a call.
+// Bound by its fp32 matrix instructions, 64 cycles each: parts made by every wave for itself were slower (B2 H8 L1056 256/512 94 us
+// against 87, made ahead see below).  A slice of 32 repeats S^T in every block, so a chunk has
+// (3 KD + 32) / (2 KD + 32 + KD / 4) of the products of a 128-wide slice, 1.27 times (KD 64) and 1.30 (KD 128), against four times the
+// blocks.  B4 H8 L2048 128/256, 256 blocks: 353 -> 145 us a call (the kernel above with fp32 products).
 // All key dims are contracted in one pass, so nothing is written twice and added.  K, Q, V and the factors are
 // double-buffered; S^T partials reuse the wave's own rows of the consumed Q tile.  The products D of the
 // decays, 4 KB per chunk of which a wave needs the rows of its group, skip LDS, which at KD 256 has no room for them.
@@ -942,7 +944,7 @@ __global__ __launch_bounds__(WK * 64 + 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
   for (int i = 0; i < T::kKB; ++i) st[i] = zero16();
 
-  // One stream of LDS reads per chunk as in the kernel above: rows of K and Q, the previous chunk's O^T
+  // One stream of LDS reads per chunk: rows of K and Q, the previous chunk's O^T
   // partials, flag, V, w, the K columns of one half of the State update, the S^T partials, p_n, the other half.
   constexpr int kPF = 6, kRing = kPF + 1, kOwn = T::kOwn;
   constexpr int nS1 = PRE ? T::kRows / 2 : T::kRows, nUpd = 4 * T::kKB, nHalf = nUpd / 2;

@@ -36,12 +36,15 @@ def _library(device_type):
 
 def workspace_size(nheads, seqlen, device_type=None, batch=1, kdim=128, vdim=128, block_kdim=None):
     """Bytes of workspace one call needs: the decay factors of every (head, 32-position chunk) and, beyond 128
-    key dims, a second output-sized buffer (0 for an unsupported shape)."""
+    key dims, a second output-sized buffer (0 for an unsupported shape).  A call that allocates its own takes more where that
+    makes it faster (retnet_recurrent_room of the library), with results that differ by fp32 rounding."""
     return int(_library(device_type or MI355X()).retnet_recurrent_workspace_size(batch, nheads, kdim, vdim, seqlen,
                                                                                   int(block_kdim or kdim)))
 
 
 def retnet_recurrent_fwd(q, k, v, decay, device_type=None, block_kdim=None, out=None, workspace=None):
+    """``workspace``: at least ``workspace_size()`` bytes, used as it is -- its size may decide how the problem is scanned, and with it the
+    last bits of the result; None: the call allocates what it makes use of, or the least it needs where there is no memory for that."""
     if not (q.is_cuda and k.is_cuda and v.is_cuda and decay.is_cuda):
         raise RuntimeError("retnet_recurrent_fwd runs on the GPU only (HIP kernels); move q, k, v, decay to a cuda device")
     for t in (q, k, v, decay):

@@ -208,7 +208,11 @@ size_t decay_workspace_size(int B, int H, int Seq_q, int Seq_k, size_t most);
 #if defined(AAT_OP_RET_RECURRENT)
 /* Bytes of workspace that retnet_recurrent_fwd_ex makes use of for this problem: retnet_recurrent_workspace_size() and, from 512
  * positions on where it pays, the operands of K and Q made once per (batch, head) (12 bytes per key dim and position), unless they
- * take more than `most` bytes.  They are optional; results with and without them differ by the order of fp32 additions. */
+ * take more than `most` bytes.  They are optional.  Without them the products of such a problem are fp32 matrix instructions, with
+ * them the six largest products of the operands' three bf16 parts (what is left out is below 2^-23 of a product), so the two differ
+ * by fp32 rounding.  Blocks that multiply in parts -- these, and those of 64 and 128 value dims -- hold operands times 2^16: a block that
+ * meets an input of 2^112, an output of 2^80 (2^40 where decays have taken the State's scale to 2^-40), an infinity or a NaN runs once more
+ * with fp32 instructions, for about twice the time and more. */
 size_t retnet_recurrent_room(int batch, int heads, int kdim, int vdim, int l, int block_kdim, size_t most);
 #endif
 
